@@ -161,6 +161,7 @@ int alloc_fields(cmcg_ctx *c, DevFields &f, bool full)
         if (int e = dalloc(c, &f.pot_rnew, n)) return e;
         if (int e = dalloc(c, &f.ntry, n)) return e;
         if (int e = dalloc(c, &f.flags, n)) return e;
+        if (int e = dalloc(c, &f.knew, n)) return e;
     }
     return CMCG_OK;
 }
@@ -285,13 +286,11 @@ static void sort_spec(cmcg_ctx *c, bool fused, SortSpec &sp)
         // ComputeIntermediateEnergy's transfer (cmc_utils.c:382-390) fused into the gather:
         // r <- rnew (the key), rOld <- r, vr <- vrnew, vt <- vtnew.
         // The step's own scratch is not carried: set_velocities3 reads rOld through the
-        // permutation and, of vtold, vrold, Uoldrold and Uoldrnew, only their
-        // combination D, which energy_conservation2 formed and the sort moves (8-word
-        // records).
+        // permutation, and with it the combination D of vtold, vrold, Uoldrold and
+        // Uoldrnew that energy_conservation2 formed (8-word records).
         add_field(sp, f.m, a.m, &f.m, &a.m);
         add_field(sp, f.vrnew, a.vr, &f.vr, &a.vr);
         add_field(sp, f.vtnew, a.vt, &f.vt, &a.vt);
-        add_field(sp, c->sc.sv3_dpre, c->sc.sv3_dpost, nullptr, nullptr);
         add_field(sp, f.r_apo, a.r_apo, &f.r_apo, &a.r_apo);
         add_field(sp, f.r_peri, a.r_peri, &f.r_peri, &a.r_peri);
     } else {
@@ -322,7 +321,8 @@ int run_sort(cmcg_ctx *c, bool fused)
     SortSpec sp;
     sort_spec(c, fused, sp);
     const double *key = fused ? c->f.rnew : c->f.r;
-    hipError_t e = launch_sort_fields(key, c->alt.r, c->f.id, sp.nf, sp.src, sp.dst, c->s, c->sc, c->n_ub, c->stream);
+    hipError_t e = launch_sort_fields(key, c->alt.r, sp.nf, sp.src, sp.dst, c->s, c->sc, c->n_ub,
+                                      fused ? (const int32_t *)c->f.knew : nullptr, c->stream);
     if (e != hipSuccess) { cmcg_report_hip(e, "launch_sort_fields", __FILE__, __LINE__); return CMCG_E_HIP; }
     swap_sorted(c, sp);
     // the old vr/vt buffers are now stale copies; vrnew/vtnew keep their values
@@ -430,7 +430,7 @@ int cmcg_create(cmcg_ctx **out, int device, int64_t n_cap, const cmcg_params *pa
     int e;
     if ((e = alloc_fields(c, c->f, true)) || (e = alloc_fields(c, c->alt, false))) { cmcg_destroy(c); return e; }
     c->alt.phi = c->f.phi; c->alt.sigma = c->f.sigma; c->alt.pot_rnew = c->f.pot_rnew;
-    c->alt.ntry = c->f.ntry; c->alt.flags = c->f.flags;
+    c->alt.ntry = c->f.ntry; c->alt.flags = c->f.flags; c->alt.knew = c->f.knew;
     if ((e = dalloc(c, &c->s, 1))) { cmcg_destroy(c); return e; }
     Scratch &sc = c->sc;
     sc.max_tiles = (n_cap + 2047) / 2048 + 1;
@@ -438,7 +438,8 @@ int cmcg_create(cmcg_ctx **out, int device, int64_t n_cap, const cmcg_params *pa
     sc.max_waves = (n_cap + 2) / 64 + 2;
     sc.max_blocks = (n_cap + 127) / 128 + 2;      // the smallest block of any launch shape: 128 threads
     if (sc.max_blocks < 1024) sc.max_blocks = 1024;   // the stripping passes' fixed grid
-    sc.max_sort_tiles = (n_cap + SORT_TILE - 1) / SORT_TILE + 1;
+    const SortShape sort_max = sort_shape(n_cap);
+    sc.sort_mat_cap = (size_t)sort_max.tiles * sort_max.buckets;
     sc.merge_ends_cap = 2 * (n_cap / 256 + 4);       // two per merge block of set_velocities3 (>= 256 stars)
     sc.sort_aos_cap = n_cap + 4;
     // about two radial-index buckets per star: 2^10 .. 2^23 buckets (at N = 4e6 one per
@@ -449,15 +450,17 @@ int cmcg_create(cmcg_ctx **out, int device, int64_t n_cap, const cmcg_params *pa
     if ((e = dalloc(c, &sc.ridx, (size_t)ridx_entries(sc.ridx_bits))) ||
         (e = dalloc(c, &sc.ridx_tb, (size_t)ridx_tiles(sc.ridx_bits) + 1))) { cmcg_destroy(c); return e; }
     if ((e = dalloc(c, &sc.tile_sums, (size_t)sc.max_tiles * 6)) || (e = dalloc(c, &sc.partials, (size_t)sc.max_blocks * 16)) ||
-        (e = dalloc(c, &sc.keys_a, (size_t)n_cap + 4)) || (e = dalloc(c, &sc.sort_aos, (size_t)(n_cap + 4) * SORT_AOS_WORDS)) || (e = dalloc(c, &sc.sort_long, (size_t)(sc.sort_long_cap = n_cap / (SORT_RUN_SHORT + 1) + 2))) ||
-        (e = dalloc(c, &sc.sort_nlong, 1)) ||
-        (e = dalloc(c, &sc.mid, (size_t)(n_cap + 2) / MID_STEP + 4)) || (e = dalloc(c, &sc.nodes, (size_t)n_cap + 8)) || (e = dalloc(c, &sc.u_old, (size_t)n_cap + 8)) ||
-        (e = dalloc(c, &sc.merge_ends, (size_t)sc.merge_ends_cap)) || (e = dalloc(c, &sc.sv3_dpre, (size_t)n_cap + 6)) || (e = dalloc(c, &sc.sv3_dpost, (size_t)n_cap + 6)) || (e = dalloc(c, &sc.dt_part, (size_t)64 * 16)) || (e = dalloc(c, &sc.coarse, (size_t)ORB_MAX_COARSE + 8)) || (e = dalloc(c, &sc.red2, (size_t)RED2_BLOCKS * 16)) ||
+        (e = dalloc(c, &sc.sort_aos, (size_t)(n_cap + 4) * SORT_AOS_WORDS)) || (e = dalloc(c, &sc.sort_split, SB_MAX_BUCKETS)) ||
+        (e = dalloc(c, &sc.sort_bad, 1)) || (e = dalloc(c, &sc.sort_bkt, (size_t)n_cap + 4)) ||
+        (e = dalloc(c, &sc.sort_mat, sc.sort_mat_cap)) || (e = dalloc(c, &sc.sort_tot, SB_MAX_BUCKETS)) ||
+        (e = dalloc(c, &sc.sort_first, SB_MAX_BUCKETS + 1)) ||
+        (e = dalloc(c, &sc.sort_order, 2 * (size_t)sc.sort_aos_cap)) ||
+        (e = dalloc(c, &sc.mid, (size_t)(n_cap + 2) / MID_STEP + 4)) || (e = dalloc(c, &sc.nodes, (size_t)n_cap + 8)) || (e = dalloc(c, &sc.u_old, 2 * ((size_t)n_cap + 8))) ||
+        (e = dalloc(c, &sc.merge_ends, (size_t)sc.merge_ends_cap)) || (e = dalloc(c, &sc.sv3_dpre, (size_t)n_cap + 6)) || (e = dalloc(c, &sc.dt_part, (size_t)64 * 16)) || (e = dalloc(c, &sc.coarse, (size_t)ORB_MAX_COARSE + 8)) || (e = dalloc(c, &sc.red2, (size_t)RED2_BLOCKS * 16)) ||
         (e = dalloc(c, (char **)&sc.orb_nib, sizeof(NibbleTables<ORB_NIB_POWERS>))) ||
         (e = dalloc(c, (char **)&sc.relax_nib, sizeof(NibbleTables<8>))) ||
-        (e = dalloc(c, (char **)&sc.wb_nib, 2 * sizeof(NibbleTables<RNG_WB_POWERS>))) || (e = dalloc(c, &sc.keys_b, (size_t)n_cap + 4)) ||
-        (e = dalloc(c, &sc.vals_a, (size_t)n_cap + 4)) || (e = dalloc(c, &sc.sort_mm, 2 * SORT_MM_PARTS)) ||
-        (e = dalloc(c, &sc.block_hist, (size_t)sc.max_sort_tiles * 256)) || (e = dalloc(c, &sc.digit_totals, 8 * 256)) ||
+        (e = dalloc(c, (char **)&sc.wb_nib, 2 * sizeof(NibbleTables<RNG_WB_POWERS>))) ||
+        (e = dalloc(c, &sc.vals_a, (size_t)n_cap + 4)) ||
         (e = dalloc(c, &sc.excess_c, (size_t)n_cap + 6)) || (e = dalloc(c, &sc.excess_list, (size_t)n_cap + 2)) ||
         (e = dalloc(c, &sc.sv3_wend, (size_t)n_cap + 2)) || (e = dalloc(c, &sc.sv3_merged, (size_t)n_cap + 2)) ||
         (e = dalloc(c, &sc.sv3_blk, (size_t)sc.max_blocks)) || (e = dalloc(c, &sc.sv3_fallback, 1)) ||
@@ -1097,8 +1100,8 @@ static int enqueue_step(cmcg_ctx *c, int64_t nub, bool graph)
         PhaseTimer t(c, "sort");
         SortSpec sp;
         sort_spec(c, true, sp);
-        hipError_t e = launch_sort_fields(c->f.rnew, c->alt.r, c->f.id, sp.nf, sp.src, sp.dst, c->s, c->sc, nub,
-                                          c->stream);
+        hipError_t e = launch_sort_fields(c->f.rnew, c->alt.r, sp.nf, sp.src, sp.dst, c->s, c->sc, nub,
+                                          (const int32_t *)c->f.knew, c->stream);
         if (e != hipSuccess) { cmcg_report_hip(e, "launch_sort_fields", __FILE__, __LINE__); return CMCG_E_HIP; }
         swap_sorted(c, sp);
     }
@@ -1109,7 +1112,7 @@ static int enqueue_step(cmcg_ctx *c, int64_t nub, bool graph)
     {
         PhaseTimer t(c, "glue_post_sort");
         // the sort above read the old sorted radii from what is now the alternate r
-        LAUNCH(launch_set_velocities3(c->f, c->s, c->kp, c->sc, nub, c->stream, c->alt.r, c->sc.sv3_dpost));
+        LAUNCH(launch_set_velocities3(c->f, c->s, c->kp, c->sc, nub, c->stream, c->alt.r, c->sc.sv3_dpre));
         LAUNCH(launch_compute_energy(c->f, c->s, c->kp, c->sc, nub, c->stream));
         kl<step_end_kernel>(dim3(1), dim3(1), 0, c->stream, c->s);
     }

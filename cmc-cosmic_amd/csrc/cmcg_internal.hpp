@@ -60,6 +60,7 @@ struct DevFields {
     double *rOld, *Uoldrold, *Uoldrnew, *vrold, *vtold, *EI;
     double *sigma, *pot_rnew;
     int32_t *ntry, *flags;
+    int32_t *knew;         // orbit phase: largest k with r_k < rnew among the old nodes, -1 for a star that leaves
 };
 
 struct KParams {
@@ -317,8 +318,9 @@ __device__ __forceinline__ int64_t find_zero_r(const double *__restrict__ r, int
 // unique largest k with r[k] < x, identical to the full-range search.
 template <class N>
 __device__ __forceinline__ double potential_at_n(const N &nd, int64_t n_max, double x, int64_t lo, int64_t hi,
-                                                 bool *bad)
+                                                 bool *bad, int32_t *k_out = nullptr)
 {
+    if (k_out) *k_out = 0;
     if (x == 0.0) return nd.P(0);
     double r1 = nd.R(1);
     if (x < r1) {
@@ -329,6 +331,7 @@ __device__ __forceinline__ double potential_at_n(const N &nd, int64_t n_max, dou
     if (lo == hi - 1) i = lo;
     else i = find_zero_r_n(nd, lo, hi, x);
     if (i > n_max) { *bad = true; return 0.0; }   // x beyond the outer sentinel
+    if (k_out) *k_out = (int32_t)i;
     double ri, pi, ri1, pi1;
     nd.RP(i, ri, pi);
     nd.RP(i + 1, ri1, pi1);
@@ -633,9 +636,9 @@ __device__ __forceinline__ int64_t mid_search(const double2 *__restrict__ mid, i
 // gives the same index as the full-range search.
 template <class N>
 __device__ __forceinline__ double potential_at_coarse_n(const N &nd, int64_t n_max, double x, int64_t lo, int64_t hi,
-                                                        const Coarse &c, bool *bad)
+                                                        const Coarse &c, bool *bad, int32_t *k_out = nullptr)
 {
-    if (x == 0.0 || x < nd.R(1)) return potential_at_n(nd, n_max, x, lo, hi, bad);
+    if (x == 0.0 || x < nd.R(1)) return potential_at_n(nd, n_max, x, lo, hi, bad, k_out);
     int a = 0, b = c.cs;                    // largest s with cr[s] < x (cr[0] = r[0] < x)
     while (a < b) {
         int m = (a + b + 1) >> 1;
@@ -667,7 +670,7 @@ __device__ __forceinline__ double potential_at_coarse_n(const N &nd, int64_t n_m
             }
         }
     }
-    return potential_at_n(nd, n_max, x, lo, hi, bad);
+    return potential_at_n(nd, n_max, x, lo, hi, bad, k_out);
 }
 __device__ __forceinline__ double potential_at_coarse(const double *__restrict__ r, const double *__restrict__ phi,
                                                       int64_t n_max, double x, int64_t lo, int64_t hi,
@@ -682,14 +685,14 @@ __device__ __forceinline__ double potential_at_coarse(const double *__restrict__
 // bracket [lo, hi] (valid when r_lo < x <= r_hi) narrows it further.
 template <class N>
 __device__ __forceinline__ double potential_at_ridx_n(const N &nd, int64_t n_max, double x, int64_t lo, int64_t hi,
-                                                      const RIdx &ri, bool *bad)
+                                                      const RIdx &ri, bool *bad, int32_t *k_out = nullptr)
 {
-    if (x == 0.0 || x < nd.R(1)) return potential_at_n(nd, n_max, x, lo, hi, bad);
+    if (x == 0.0 || x < nd.R(1)) return potential_at_n(nd, n_max, x, lo, hi, bad, k_out);
     int32_t a, b;
     ridx_bracket(ri, x, a, b);
     if (a > lo) lo = a;
     if (b < hi) hi = b;
-    return potential_at_n(nd, n_max, x, lo, hi, bad);
+    return potential_at_n(nd, n_max, x, lo, hi, bad, k_out);
 }
 
 // Narrow a find_zero_Q bracket [lo, hi] with pred(Q(lo)) true and pred(Q(hi)) false

@@ -106,8 +106,8 @@ struct ec2_kernel {
 // that EI reads unchanged for the stars it keeps and sets EI = 0 for the stars it
 // strips, so EI can be formed here, before it, with the same result.
 // It also forms D = vold^2 + 2 (1 - q) (Uoldrold - Uoldrnew), the part of
-// set_velocities3's vnew^2 (cmc_utils.c:242-247) that the sort then carries in place of
-// its four inputs: the same operations in the same order, so the same double.
+// set_velocities3's vnew^2 (cmc_utils.c:242-247) that reaches it through the permutation
+// in place of its four inputs: the same operations in the same order, so the same double.
 struct ec2_ie_kernel {
     static constexpr int LB = 1024, MB = 0;
     static __device__ __forceinline__ void run(KGrid kg_, DevFields f, DevScalars *s, KParams P, double *__restrict__ dpre)
@@ -165,6 +165,7 @@ __device__ void strip_block(DevFields &f, const KParams &P, double Rt, int64_t n
         if (f.r_apo[i] > Rt && f.rnew[i] < 1000000) {
             double m = f.m[i], E = f.E[i], J = f.J[i];
             f.rnew[i] = CMCG_SF_INFINITY; f.vrnew[i] = 0.0; f.vtnew[i] = 0.0;
+            f.knew[i] = -1;
             v[0] += E * m / (double)P.n_star;   // Eescaped
             v[1] += J * m / (double)P.n_star;   // Jescaped
             v[2] += m / (double)P.n_star;       // DTidalMassLoss
@@ -329,7 +330,8 @@ struct old_node_potential_kernel {
     static __device__ __forceinline__ void run(KGrid kg_, const double *__restrict__ r_old,
                                                                      const double2 *__restrict__ nodes,
                                                                      DevScalars *s, double2 *__restrict__ u_old,
-                                                                     const int64_t *__restrict__ ends)
+                                                                     const int64_t *__restrict__ ends,
+                                                                     const double *__restrict__ dpre)
 {
     __shared__ double2 L[MERGE_LDS];
     const int64_t n_old = s->sort_in, n = s->n_max;
@@ -376,22 +378,24 @@ struct old_node_potential_kernel {
             if (i > n) { dev_set_error(s, CMCG_E_BRACKET, sl); v = 0.0; }
             else v = pi + (pi1 - pi) * (1.0 / ri - 1.0 / x) / (1.0 / ri - 1.0 / ri1);
         }
-        u_old[sl] = make_double2(v, x);       // with the radius: set_velocities3 reads both at once
+        // with the radius and D in one 32-byte sector: set_velocities3 reads them at once
+        u_old[2 * sl] = make_double2(v, x);
+        u_old[2 * sl + 1] = make_double2(dpre[sl], 0.0);
     }
 }
 };
 
 constexpr int SV3_COARSE = 1024;      // LDS samples of r for potential(rOld)
 
-// With u_old (the step): potential(rOld) and rOld itself through the sort's permutation,
-// and D (dpost) in place of vtold, vrold, Uoldrold and Uoldrnew.  Without: the
+// With u_old (the step): potential(rOld), rOld itself and D (in place of vtold, vrold,
+// Uoldrold and Uoldrnew) through the sort's permutation.  Without: the
 // reference's fields and a search (the entry point of the reference's name).
 struct sv3_kernel {
     static constexpr int LB = GT, MB = 0;
     static __device__ __forceinline__ void run(KGrid kg_, DevFields f, DevScalars *s, KParams P, double *__restrict__ excess_c,
                                                  int64_t *__restrict__ blk_cnt, const double2 *__restrict__ mid,
                                                  const double2 *__restrict__ nodes, const double2 *__restrict__ u_old,
-                                                 const uint32_t *__restrict__ perm, const double *__restrict__ dpost)
+                                                 const uint32_t *__restrict__ perm)
 {
     __shared__ int cnt;
     __shared__ double cr[SV3_COARSE + 1];
@@ -410,9 +414,10 @@ struct sv3_kernel {
         double m = f.m[i], ri = f.r[i];
         double Unewrold, D;
         if (u_old) {
-            const double2 ux = u_old[perm[i - 1]];
+            const int64_t old = 2 * (int64_t)perm[i - 1];
+            const double2 ux = u_old[old];
+            D = u_old[old + 1].x;
             Unewrold = ux.x + phi_s_own(ri, m, P.inv_nstar, ux.y);
-            D = dpost[i];
         } else {
             const double rO = f.rOld[i];
             bool bad = false;
@@ -735,16 +740,16 @@ hipError_t launch_ie_transfer(const DevFields &f, DevScalars *s, int64_t n_ub, h
     return hipGetLastError();
 }
 hipError_t launch_set_velocities3(const DevFields &f, DevScalars *s, const KParams &P, const Scratch &sc,
-                                  int64_t n_ub, hipStream_t st, const double *r_old_sorted, const double *dpost)
+                                  int64_t n_ub, hipStream_t st, const double *r_old_sorted, const double *dpre)
 {
-    if ((r_old_sorted != nullptr) != (dpost != nullptr)) return hipErrorInvalidValue;
+    if ((r_old_sorted != nullptr) != (dpre != nullptr)) return hipErrorInvalidValue;
     int64_t nb = grid_for(n_ub);
     if (nb > sc.max_blocks) return hipErrorInvalidValue;
     unsigned ge = grid_for(n_ub);
     if (ge > 256) ge = 256;            // the excess-list kernels stride over the list
     kl<sv3_begin_kernel>(dim3(1), dim3(1), 0, st, s, sc.sv3_fallback);
     // the step calls this right after the potential, which left the node table current
-    if (!dpost)
+    if (!dpre)
         if (hipError_t e = launch_mid_build(f, s, sc, n_ub, st)) return e;
     if (r_old_sorted) {
         const int64_t mb = (n_ub + MERGE_BLK - 1) / MERGE_BLK;
@@ -752,11 +757,11 @@ hipError_t launch_set_velocities3(const DevFields &f, DevScalars *s, const KPara
         kl<merge_ends_kernel>(dim3((unsigned)((2 * mb + 255) / 256)), dim3(256), 0, st, r_old_sorted,
                               (const double2 *)sc.nodes, (const DevScalars *)s, sc.merge_ends);
         kl<old_node_potential_kernel>(dim3((unsigned)mb), dim3(MERGE_T), 0, st, r_old_sorted,
-                                      (const double2 *)sc.nodes, s, sc.u_old, (const int64_t *)sc.merge_ends);
+                                      (const double2 *)sc.nodes, s, sc.u_old, (const int64_t *)sc.merge_ends, dpre);
     }
     kl<sv3_kernel>(dim3((unsigned)nb), dim3(GT), 0, st, f, s, P, sc.excess_c, sc.sv3_blk,
                        (const double2 *)sc.mid, (const double2 *)sc.nodes,
-                       r_old_sorted ? (const double2 *)sc.u_old : nullptr, (const uint32_t *)sc.vals_a, dpost);
+                       r_old_sorted ? (const double2 *)sc.u_old : nullptr, (const uint32_t *)sc.vals_a);
     kl<sv3_scan_kernel>(dim3(1), dim3(1024), 0, st, s, sc.sv3_blk, nb);
     kl<sv3_compact_kernel>(dim3((unsigned)nb), dim3(GT), 0, st, s, (const double *)sc.excess_c,
                        (const int64_t *)sc.sv3_blk, sc.excess_list);

@@ -77,6 +77,17 @@ __device__ __forceinline__ void removed(double (&red)[NRED], double Ej, double J
     red[4] = Ej * mj / (double)P.n_star;
 }
 
+// DevFields::knew of a star that stays at r_j (a circular orbit): the nodes below it
+template <class N>
+__device__ __forceinline__ int32_t nodes_below(const N &nd, int64_t j, double rj)
+{
+    int64_t k = j - 1;
+    while (k > 0 && !(nd.R(k) < rj)) k--;
+    return (int32_t)k;
+}
+// ... and of one sampled at x between nodes k and k + 1 (the sort drops radii at or beyond SF_INFINITY)
+__device__ __forceinline__ int32_t knew_of(int32_t k, double x) { return x < CMCG_SF_INFINITY ? k : -1; }
+
 // The part of get_positions_loop after the positive-Q index is known
 // (cmc_evolution_thr.c:832-934).
 template <class N>
@@ -94,12 +105,14 @@ __device__ void sample_star(const N &nd, const DevFields &f, DevScalars *s, cons
     if (o.brent) flags |= CMCG_SF_BRENT;
     if (o.circular) {
         f.rnew[j] = rj; f.vrnew[j] = f.vr[j]; f.vtnew[j] = f.vt[j];
+        f.knew[j] = nodes_below(nd, j, rj);
         flags |= CMCG_SF_CIRCULAR;
         return;
     }
     if (o.ra >= s->Rtidal) {
         f.r_apo[j] = o.ra; f.r_peri[j] = o.rp;
         f.rnew[j] = CMCG_SF_INFINITY; f.vrnew[j] = 0.0; f.vtnew[j] = 0.0;
+        f.knew[j] = -1;
         removed(red, Ej, J, mj, P);
         flags |= CMCG_SF_REMOVED_RT;
         return;
@@ -114,6 +127,7 @@ __device__ void sample_star(const N &nd, const DevFields &f, DevScalars *s, cons
     const double r_lo0 = nd.R(lo0), r_hi0 = nd.R(hi0);
     double X = 0.0, rr = 0.0, vr = 0.0, potr = 0.0;
     int k;
+    int32_t kn = 0;
     bool bad = false;
     for (k = 1; k <= CMCG_N_TRY; k++) {
         X = rng_dbl(rng);
@@ -123,7 +137,7 @@ __device__ void sample_star(const N &nd, const DevFields &f, DevScalars *s, cons
         int64_t lo = lo0, hi = hi0;
         if (!(r_lo0 < rr)) lo = 1;
         if (!(rr <= r_hi0)) hi = n + 1;
-        potr = potential_at_n(nd, n, rr, lo, hi, &bad);
+        potr = potential_at_n(nd, n, rr, lo, hi, &bad, &kn);
         double pot = potr + phi_s_own(rj, mj, P.inv_nstar, rr);
         double drds = 0.25 * (rmax - rmin) * (3.0 - 3.0 * s0 * s0);
         double Q = 2.0 * E - 2.0 * pot - J * J / rr / rr;
@@ -143,6 +157,7 @@ __device__ void sample_star(const N &nd, const DevFields &f, DevScalars *s, cons
     f.r_apo[j] = rmax;
     if (rng_dbl(rng) < 0.5) vr = -vr;
     f.rnew[j] = rr;
+    f.knew[j] = knew_of(kn, rr);
     f.vrnew[j] = vr;
     f.vtnew[j] = J / rr;
     f.pot_rnew[j] = potr;
@@ -169,6 +184,7 @@ struct TryCtx {
 // result of a star's tries
 struct TryOut {
     double X, rr, vr, potr;
+    int32_t kn;        // index of rr among the nodes
     int k;             // tries taken; CMCG_N_TRY + 1 when none was accepted
     bool bad, nan;
 };
@@ -203,12 +219,14 @@ __device__ __forceinline__ bool prepare_star(const N &nd, const DevFields &f, De
     if (o.brent) flags |= CMCG_SF_BRENT;
     if (o.circular) {
         f.rnew[j] = rj; f.vrnew[j] = f.vr[j]; f.vtnew[j] = f.vt[j];
+        f.knew[j] = nodes_below(nd, j, rj);
         flags |= CMCG_SF_CIRCULAR;
         return false;
     }
     if (o.ra >= s->Rtidal) {
         f.r_apo[j] = o.ra; f.r_peri[j] = o.rp;
         f.rnew[j] = CMCG_SF_INFINITY; f.vrnew[j] = 0.0; f.vtnew[j] = 0.0;
+        f.knew[j] = -1;
         flags |= CMCG_SF_REMOVED_RT;      // its removal sums are added by the caller
         return false;
     }
@@ -229,8 +247,8 @@ __device__ __forceinline__ bool prepare_star(const N &nd, const DevFields &f, De
 // st is the state after the try's two draws.
 template <class N>
 __device__ __forceinline__ bool one_try(const N &nd, const Coarse &C, const KParams &P, int64_t n, const TryCtx &tc,
-                                        Rng &st, double &X, double &rr, double &vr, double &potr, bool &bad,
-                                        bool &nan)
+                                        Rng &st, double &X, double &rr, double &vr, double &potr, int32_t &kn,
+                                        bool &bad, bool &nan)
 {
     X = rng_dbl(st);
     const double s0 = 2.0 * X - 1.0;
@@ -239,8 +257,8 @@ __device__ __forceinline__ bool one_try(const N &nd, const Coarse &C, const KPar
     int64_t lo = tc.lo0, hi = tc.hi0;
     if (!(tc.r_lo0 < rr)) lo = 1;
     if (!(rr <= tc.r_hi0)) hi = n + 1;
-    potr = C.ri.t ? potential_at_ridx_n(nd, n, rr, lo, hi, C.ri, &bad)
-                  : potential_at_coarse_n(nd, n, rr, lo, hi, C, &bad);
+    potr = C.ri.t ? potential_at_ridx_n(nd, n, rr, lo, hi, C.ri, &bad, &kn)
+                  : potential_at_coarse_n(nd, n, rr, lo, hi, C, &bad, &kn);
     const double pot = potr + phi_s_own(tc.rj, tc.mj, P.inv_nstar, rr);
     const double drds = 0.25 * (tc.rmax - tc.rmin) * (3.0 - 3.0 * s0 * s0);
     const double Q = 2.0 * tc.E - 2.0 * pot - tc.J * tc.J / rr / rr;
@@ -263,7 +281,7 @@ __device__ void wave_tries(const N &nd, const Coarse &C, const KParams &P, int64
     const int lane = threadIdx.x & 63;
     int next = 1;                         // owner: first try not yet evaluated
     bool bad_acc = false;
-    out.k = 0; out.bad = false; out.nan = false;
+    out.k = 0; out.bad = false; out.nan = false; out.kn = 0;
     out.X = out.rr = out.vr = out.potr = 0.0;
     uint64_t pending = __ballot(need);
     while (pending) {
@@ -283,9 +301,10 @@ __device__ void wave_tries(const N &nd, const Coarse &C, const KParams &P, int64
         if (!idle)
             for (int d = 0; d < 2 * o; d++) (void)rng_int(st);
         double X = 0.0, rr = 0.0, vr = 0.0, potr = 0.0;
+        int32_t kn = 0;
         bool bad = false, nan = false, term = false;
         if (eval) {
-            term = one_try(nd, C, P, n, t, st, X, rr, vr, potr, bad, nan);
+            term = one_try(nd, C, P, n, t, st, X, rr, vr, potr, kn, bad, nan);
             Rng sg = st;
             if (term && !nan && rng_dbl(sg) < 0.5) vr = -vr;    // sign draw after the accepted try
         }
@@ -313,7 +332,7 @@ __device__ void wave_tries(const N &nd, const Coarse &C, const KParams &P, int64
         }
         const int srcl = src < 0 ? lane : src;
         const double sX = __shfl(X, srcl), srr = __shfl(rr, srcl), svr = __shfl(vr, srcl), spot = __shfl(potr, srcl);
-        const int snan = __shfl((int)nan, srcl);
+        const int snan = __shfl((int)nan, srcl), skn = __shfl(kn, srcl);
         Rng ns;
         ns.z0 = __shfl(st.z0, srcl); ns.z1 = __shfl(st.z1, srcl); ns.z2 = __shfl(st.z2, srcl); ns.z3 = __shfl(st.z3, srcl);
         if (owner) {
@@ -321,7 +340,7 @@ __device__ void wave_tries(const N &nd, const Coarse &C, const KParams &P, int64
             const uint64_t upto = (src >= 63 ? ~0ull : ((1ull << (src + 1)) - 1ull)) & span;
             bad_acc |= (bmask & upto) != 0ull;
             if (done) {
-                out.X = sX; out.rr = srr; out.vr = svr; out.potr = spot; out.nan = snan != 0;
+                out.X = sX; out.rr = srr; out.vr = svr; out.potr = spot; out.nan = snan != 0; out.kn = skn;
                 out.k = tw ? next + (src - base) : CMCG_N_TRY + 1;
                 out.bad = bad_acc;
             } else {
@@ -395,11 +414,11 @@ struct orbits_kernel {
             // destroy_obj (cmc_dynamics_helper.c:131-153) + remove_star_center
             f.vr[j] = 0.0; f.vt[j] = 0.0; f.E[j] = 0.0; f.J[j] = 0.0; f.id[j] = 0;
             f.X[j] = 0.0; f.Y[j] = 0.0; f.r_peri[j] = 0.0; f.r_apo[j] = 0.0;
-            f.rnew[j] = CMCG_SF_INFINITY; f.m[j] = 2.2250738585072014e-308;
+            f.rnew[j] = CMCG_SF_INFINITY; f.knew[j] = -1; f.m[j] = 2.2250738585072014e-308;
             f.vrnew[j] = 0.0; f.vtnew[j] = 0.0;
             flags = CMCG_SF_DESTROYED;
         } else if (E >= 0.0) {
-            f.rnew[j] = CMCG_SF_INFINITY; f.vrnew[j] = 0.0; f.vtnew[j] = 0.0;
+            f.rnew[j] = CMCG_SF_INFINITY; f.vrnew[j] = 0.0; f.vtnew[j] = 0.0; f.knew[j] = -1;
             flags = CMCG_SF_REMOVED_E;
         } else {
             if (q_le0(q_sign(rj, mj, P.inv_nstar, rj, f.phi[j], E, J))) {
@@ -437,6 +456,7 @@ struct orbits_kernel {
             f.r_peri[j] = tc.rmin;
             f.r_apo[j] = tc.rmax;
             f.rnew[j] = to.rr;
+            f.knew[j] = knew_of(to.kn, to.rr);
             f.vrnew[j] = to.vr;
             f.vtnew[j] = tc.J / to.rr;
             f.pot_rnew[j] = to.potr;
@@ -719,12 +739,13 @@ struct ridx_clear_kernel {
 // the radial index's marks (nodes 0..n), in one pass over r and phi: node k (node 0
 // stands for "below every bucket") writes its index at its bucket when it is the
 // bucket's last node, and k at every multiple of RIDX_TILE in (bucket(r_k),
-// bucket(r_{k+1})] of the tile table.  The index array must be cleared before.
+// bucket(r_{k+1})] of the tile table.  The index array must be cleared before.  *bad is
+// set where the radii do not ascend (the step's sort then does without their order).
 struct node_index_kernel {
     static constexpr int LB = 1024, MB = 0;
     static __device__ __forceinline__ void run(KGrid kg_, const double *__restrict__ r, const double *__restrict__ phi, DevScalars *s,
                                   double2 *__restrict__ nodes, double2 *__restrict__ mid, uint32_t *__restrict__ t,
-                                  uint32_t *__restrict__ tb, int bits)
+                                  uint32_t *__restrict__ tb, int bits, int32_t *bad)
 {
     const int64_t n = s->n_max;
     const int64_t k = (int64_t)kg_.bid * blockDim.x + threadIdx.x;
@@ -743,7 +764,11 @@ struct node_index_kernel {
         x.lo = (uint64_t)__double_as_longlong(r[1]);
         x.shift = ridx_shift(x.lo, (uint64_t)__double_as_longlong(r[n]), bits);
         if (k >= 1) bk = ridx_bucket(x, rk);
-        if (k < n) bn = ridx_bucket(x, r[k + 1]);
+        if (k < n) {
+            const double rk1 = r[k + 1];
+            bn = ridx_bucket(x, rk1);
+            if (k >= 1 && !(rk <= rk1)) *bad = 1;
+        }
         if (k >= 1 && bn != bk) t[bk] = (uint32_t)k;
     }
     for (int64_t m = (bk + RIDX_TILE) / RIDX_TILE; m * RIDX_TILE <= bn; m++) tb[m] = (uint32_t)k;
@@ -918,7 +943,7 @@ hipError_t launch_node_index(const DevFields &f, DevScalars *s, const Scratch &s
     const int64_t entries = ridx_entries(sc.ridx_bits);
     kl<ridx_clear_kernel>(dim3(512), dim3(256), 0, st, sc.ridx, entries);
     kl<node_index_kernel>(dim3((unsigned)((n_ub + 2 + 255) / 256)), dim3(256), 0, st, f.r, f.phi, s,
-                       (double2 *)sc.nodes, (double2 *)sc.mid, sc.ridx, sc.ridx_tb, sc.ridx_bits);
+                       (double2 *)sc.nodes, (double2 *)sc.mid, sc.ridx, sc.ridx_tb, sc.ridx_bits, sc.sort_bad);
     kl<ridx_scan_kernel>(dim3((unsigned)ridx_tiles(sc.ridx_bits)), dim3(256), 0, st, sc.ridx,
                        (const uint32_t *)sc.ridx_tb, sc.ridx_bits);
     return hipGetLastError();

@@ -1,38 +1,38 @@
 // a1: qsorts_new -> sample_sort at one rank (src/cmc/cmc_sort.c:375-629): order the
 // stars by r ascending (compare_type, :245-250), ties by id (the reference's libc
-// qsort leaves them unordered), drop the r == SF_INFINITY tail
+// qsort leaves them unordered), then by slot; drop the r == SF_INFINITY tail
 // (remove_stripped_stars, :343-354), then refresh r and m (post_sort_comm,
 // src/cmc/cmc_utils.c:2259-2288).
 //
-// Device algorithm: LSD radix sort of one 64-bit word per star: a 32-bit key z on
-// top (the order-preserving bits of r, shifted by the live minimum and scaled so the
-// live range fills 31 bits; the SF_INFINITY tail gets z = 2^32 - 1) and the star's
-// slot below.  Four passes of 8-bit digits over z, each three kernels (tile
-// histogram, per-digit tile scan, stable scatter).  The scatter ranks each 4096-word
-// tile with 64-lane ballot multisplit (stable in tile order), stages the sorted tile
-// in LDS and writes it out digit-run by digit-run, so global writes are coalesced.
-// Runs of equal z are then put in (r, id) order (in place up to 64 words, by a bitonic
-// sort in LDS up to 4096, by a merge sort in global memory beyond: any input sorts),
-// and one gather moves the payload.
+// Device algorithm: a distribution sort in two moves of each star's payload.
+//   count    every star's bucket among B buckets of about SB_AVG stars and a bucket
+//            histogram per tile;
+//   scan     the tiles' offsets inside every bucket (only beyond SB_SMALL_N stars; below,
+//            every scatter block sums the few histogram rows itself);
+//   scatter  each star's fields packed into one 64- or 128-byte record at the next free
+//            place of its bucket (order inside a bucket is free: the buckets are put into
+//            the total order (r, id, slot) next, so the result does not depend on it);
+//   sort     one block per bucket orders its records in LDS and writes every field
+//            coalesced.
+// In the step the bucket comes from the index of the new radius among the old ones, which
+// the orbit phase found with the potential there: a step moves stars along their orbits
+// and changes the density little, so equal cuts of the old order keep nearly equal counts.
+// The general entry point orders radii it knows nothing about and bisects boundaries taken
+// from a sorted sample.  Counts decide only the speed: a bucket beyond the LDS capacity is
+// merge-sorted in global memory by its block.
+//
+// Bound: HBM.  The payload (64 B a star) is read and written twice, 256 B a star, plus 4 B
+// of node indices.  It replaced an LSD radix sort of (key, slot) words, which packed the
+// records, moved the words through four histogram-scan-scatter passes and gathered the
+// records at the end (16 launches, now 3 or 4).  The step's sort, before -> now: N = 1e4
+// 0.099 -> 0.028 ms, 1e5 0.106 -> 0.034, 1e6 0.164 -> 0.092, 4e6 0.399 -> 0.277 (the
+// bucket pass 129 us for 528 MB, 4.1 TB/s; the scatter 112 us for 500 MB).
 #include "kernels.hpp"
 
 namespace {
-constexpr int RS_THREADS = 256;
-constexpr int RS_ITEMS = SORT_TILE / RS_THREADS;
-constexpr int RS_TILE = RS_THREADS * RS_ITEMS;
-constexpr int RS_MAX_FIELDS = 24;
-// LSD passes over z, the top 32 bits of each word; words equal in z are then put in
-// (r, id) order by the run pass (one thread per run up to RUN_SHORT words, one block
-// per longer run: sorting in LDS up to RUN_LONG words, a merge sort beyond).
-constexpr int RS_PASSES = 4;
-constexpr int RS_SHIFT0 = 64 - 8 * RS_PASSES;     // z = word >> RS_SHIFT0
-constexpr uint32_t Z_TAIL = 0xffffffffu;          // z of the SF_INFINITY tail; live z < 2^31
-static_assert(RS_PASSES % 2 == 0, "the sorted words must end in keys_a");
-constexpr int RUN_SHORT = SORT_RUN_SHORT;
-constexpr int RUN_LONG = SORT_RUN_LONG;
-// Packed payload records: W = 8 words (64 B) when the fields and r fit, else 16 (one
-// 128-B line); an odd LDS stride per record keeps the packing free of bank conflicts.
-constexpr int AOS_MAX = SORT_AOS_WORDS;
+constexpr int SB_MAX_FIELDS = 20;
+constexpr uint16_t SB_TAIL = 0xffff;               // bucket number of a star of the SF_INFINITY tail
+constexpr uint64_t KEY_INF = 0x8000000000000000ull | 0x4202a05f20000000ull;   // sortable(1.0e10)
 
 __device__ __forceinline__ uint64_t sortable(double x)
 {
@@ -40,674 +40,695 @@ __device__ __forceinline__ uint64_t sortable(double x)
     return (b >> 63) ? ~b : (b | 0x8000000000000000ull);
 }
 
+// The payload without id: field f goes from src[f] to dst[f].
 struct GatherList {
     int nf;
-    const uint64_t *src[RS_MAX_FIELDS];
-    uint64_t *dst[RS_MAX_FIELDS];
+    const uint64_t *src[SB_MAX_FIELDS];
+    uint64_t *dst[SB_MAX_FIELDS];
 };
 
-__device__ __forceinline__ uint32_t word_slot(uint64_t w) { return (uint32_t)w; }
-__device__ __forceinline__ uint32_t word_z(uint64_t w) { return (uint32_t)(w >> RS_SHIFT0); }
-
-// Minimum and maximum order-preserving key of the live stars (r below SF_INFINITY), one
-// pair per block: mm[2b] = min, mm[2b + 1] = max (~0 and 0 for a block that saw none).
-// rs_prep_kernel combines the pairs; partials per block replace thousands of device-scope
-// atomics on one address arriving from every XCD.  The kernel also zeroes the digit
-// totals (zn words at z) and resets the sort's scalars and long-run counters.
-struct rs_minmax_kernel {
-    static constexpr int LB = 256, MB = 0;
-    static __device__ __forceinline__ void run(KGrid kg_, const double *__restrict__ keysrc, DevScalars *s,
-                                                        uint64_t kinf, unsigned long long *__restrict__ mm,
-                                                        uint32_t *__restrict__ z, int64_t zn, int64_t *__restrict__ n_long)
+// Orders LDS traffic of one wave (its DS operations execute in order; this keeps the
+// compiler from moving them).
+__device__ __forceinline__ void wave_sync()
 {
-    __shared__ unsigned long long rmin[4], rmax[4];
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// Block-wide exclusive scan of one count per thread (lds: blockDim / 64 words, free on
+// return); *total receives the sum.
+__device__ __forceinline__ uint32_t block_excl(uint32_t v, uint32_t *lds, uint32_t *total)
+{
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, nw = blockDim.x >> 6;
+    uint32_t x = v;
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) {
+        const uint32_t y = __shfl_up(x, d, 64);
+        if (lane >= d) x += y;
+    }
+    if (lane == 63) lds[w] = x;
+    __syncthreads();
+    uint32_t off = 0, tot = 0;
+    for (int q = 0; q < nw; q++) {
+        const uint32_t c = lds[q];
+        if (q < w) off += c;
+        tot += c;
+    }
+    __syncthreads();
+    *total = tot;
+    return off + x - v;
+}
+
+// Keys lo..hi cut into `bins` equal parts: a monotone map (the factor is rounded down, so
+// every key stays below `bins`).
+struct Binning {
+    uint64_t lo, mult;
+    int shift;
+    __device__ __forceinline__ Binning(uint64_t lo_, uint64_t hi, int bins) : lo(lo_)
+    {
+        const uint64_t range = hi > lo ? hi - lo : 0;
+        shift = range >> 32 ? 32 - __clzll((long long)range) : 0;
+        mult = (uint64_t)((double)bins * 4294967296.0 / ((double)(range >> shift) + 1.0) * (1.0 - 0x1p-40));
+    }
+    __device__ __forceinline__ uint32_t operator()(uint64_t key) const { return (uint32_t)((((key - lo) >> shift) * mult) >> 32); }
+};
+
+// stars per tile when n stars are cut into nt tiles
+__device__ __forceinline__ int64_t tile_chunk(int64_t n, int64_t nt) { return (n + nt - 1) / nt; }
+
+// Bucket boundaries from a sample (the general entry point): S keys at even strides,
+// ordered in LDS by a counting sort over sub-ranges and ranks inside them; boundary b is
+// the sample at rank b S / B.
+constexpr int SMP_T = 1024, SMP_MAX = 8192, SMP_BINS = 4096;
+struct sb_sample_kernel {
+    static constexpr int LB = SMP_T, MB = 0;
+    static __device__ __forceinline__ void run(KGrid kg_, const double *__restrict__ keysrc, const DevScalars *s, int B,
+                                               uint64_t *__restrict__ split)
+{
+    __shared__ uint64_t key[SMP_MAX];
+    __shared__ uint32_t bin[SMP_BINS + 1];
+    __shared__ uint64_t red[2][SMP_T / 64];
+    __shared__ uint32_t scan[SMP_T / 64];
+    const int t = threadIdx.x;
     const int64_t n = s->n_max_new;
-    const int64_t stride = (int64_t)kg_.nb * blockDim.x;
-    for (int64_t q = (int64_t)kg_.bid * blockDim.x + threadIdx.x; q < zn; q += stride) z[q] = 0u;
-    if (kg_.bid == 0 && threadIdx.x == 0) {
-        s->sort_n = 0;
-        s->sort_in = n;
-        n_long[0] = 0;
-    }
-    unsigned long long lo = ~0ull, hi = 0ull;
-    auto take = [&](uint64_t k) {
-        if (k < kinf) {
-            lo = k < lo ? k : lo;
-            hi = k > hi ? k : hi;
+    const int S = n < SMP_MAX ? (int)n : SMP_MAX;
+    for (int q = t; q <= SMP_BINS; q += SMP_T) bin[q] = 0;
+    uint64_t k[SMP_MAX / SMP_T];
+    uint64_t lo = ~0ull, hi = 0ull;
+#pragma unroll
+    for (int u = 0; u < SMP_MAX / SMP_T; u++) {
+        const int q = u * SMP_T + t;
+        k[u] = ~0ull;
+        if (q < S) {
+            k[u] = sortable(keysrc[1 + (int64_t)q * n / S]);
+            if (k[u] > KEY_INF) k[u] = KEY_INF;               // the tail: one value above every live key
+            lo = k[u] < lo ? k[u] : lo;
+            hi = k[u] > hi ? k[u] : hi;
         }
-    };
-    int64_t i = (int64_t)kg_.bid * blockDim.x + threadIdx.x;
-    for (; i + 3 * stride < n; i += 4 * stride) {       // four independent loads in flight
-        const uint64_t k0 = sortable(keysrc[i + 1]), k1 = sortable(keysrc[i + stride + 1]);
-        const uint64_t k2 = sortable(keysrc[i + 2 * stride + 1]), k3 = sortable(keysrc[i + 3 * stride + 1]);
-        take(k0); take(k1); take(k2); take(k3);
     }
-    for (; i < n; i += stride) take(sortable(keysrc[i + 1]));
-    for (int off = 32; off > 0; off >>= 1) {
-        const unsigned long long a = __shfl_down(lo, off, 64), b = __shfl_down(hi, off, 64);
+    for (int o = 32; o > 0; o >>= 1) {
+        const uint64_t a = __shfl_xor(lo, o, 64), b = __shfl_xor(hi, o, 64);
         lo = a < lo ? a : lo;
         hi = b > hi ? b : hi;
     }
-    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-    if (lane == 0) { rmin[w] = lo; rmax[w] = hi; }
+    if ((t & 63) == 0) { red[0][t >> 6] = lo; red[1][t >> 6] = hi; }
     __syncthreads();
-    if (threadIdx.x == 0) {
-        for (int q = 1; q < 4; q++) {
-            lo = rmin[q] < lo ? rmin[q] : lo;
-            hi = rmax[q] > hi ? rmax[q] : hi;
+    for (int q = 0; q < SMP_T / 64; q++) {
+        lo = red[0][q] < lo ? red[0][q] : lo;
+        hi = red[1][q] > hi ? red[1][q] : hi;
+    }
+    const Binning bn_of(lo, hi, SMP_BINS);
+    auto bin_of = [&](uint64_t x) { return bn_of(x); };
+    uint32_t at[SMP_MAX / SMP_T];
+#pragma unroll
+    for (int u = 0; u < SMP_MAX / SMP_T; u++)
+        if (u * SMP_T + t < S) at[u] = atomicAdd(&bin[bin_of(k[u])], 1u);
+    __syncthreads();
+    constexpr int PER = SMP_BINS / SMP_T;
+    uint32_t c[PER], sum = 0, tot;
+#pragma unroll
+    for (int q = 0; q < PER; q++) { c[q] = bin[t * PER + q]; sum += c[q]; }
+    uint32_t run = block_excl(sum, scan, &tot);
+#pragma unroll
+    for (int q = 0; q < PER; q++) { bin[t * PER + q] = run; run += c[q]; }
+    if (t == 0) bin[SMP_BINS] = (uint32_t)S;
+    __syncthreads();
+#pragma unroll
+    for (int u = 0; u < SMP_MAX / SMP_T; u++)
+        if (u * SMP_T + t < S) key[bin[bin_of(k[u])] + at[u]] = k[u];
+    __syncthreads();
+    // boundary b: the sample of rank b S / B, found among its bin's keys
+    for (int b = t; b < B; b += SMP_T) {
+        uint64_t v = 0;
+        if (b > 0 && S > 0) {
+            const uint32_t rank = (uint32_t)((int64_t)b * S / B);
+            const uint32_t bn = bin_of(key[rank]), e0 = bin[bn], e1 = bin[bn + 1];
+            v = key[rank];
+            for (uint32_t p = e0; p < e1; p++) {
+                uint32_t less = 0;
+                for (uint32_t q = e0; q < e1; q++) less += key[q] < key[p] || (key[q] == key[p] && q < p);
+                if (e0 + less == rank) { v = key[p]; break; }
+            }
         }
-        mm[2 * kg_.bid] = lo;
-        mm[2 * kg_.bid + 1] = hi;
+        split[b] = v;
     }
 }
 };
 
-// Blocks of rs_minmax_kernel for a sort over `ntiles` tiles (the same count on both sides).
-__host__ __device__ __forceinline__ int minmax_parts(int64_t ntiles)
-{
-    return ntiles * 4 < SORT_MM_PARTS ? (int)(ntiles * 4) : SORT_MM_PARTS;
-}
-
-// Words from slots 1..n plus the four global digit histograms, and the first pass's
-// per-tile histogram (a block's words are that pass's tile); with `aos` the payload
-// fields of each slot, and r itself after them, are packed into one 128-byte record,
-// so the final gather reads one record per star instead of one cache line per field.
-template <int W>
-struct rs_prep_kernel {
-    static constexpr int LB = RS_THREADS, MB = 0;
-    static __device__ __forceinline__ void run(KGrid kg_, const double *__restrict__ keysrc, DevScalars *s,
-                                                             uint64_t *__restrict__ words,
-                                                             uint32_t *__restrict__ digit_totals,
-                                                             uint64_t *__restrict__ aos, GatherList g, uint64_t kinf,
-                                                             const unsigned long long *__restrict__ mm,
-                                                             uint32_t *__restrict__ block_hist, int64_t ntiles)
-{
-    constexpr int P0 = 8 - RS_PASSES;      // first byte sorted on
-    __shared__ uint32_t h[RS_PASSES][256];
-    constexpr int LD = W + 1;
-    __shared__ uint64_t recs[RS_THREADS * LD];         // one chunk of packed records
-    const int t = threadIdx.x;
-    for (int p = 0; p < RS_PASSES; p++) h[p][t] = 0;
-    // combine the per-block (min, max) pairs of rs_minmax_kernel
-    __shared__ unsigned long long red[2][RS_THREADS / 64];
+// The step's bucket of a star: its index among the old nodes, cut into B equal parts
+// (monotone in the new radius while the old radii ascend; when they do not, every star
+// goes to the last bucket, which the merge sort orders).
+struct StepBucket {
+    double f;
+    int B;
+    bool unordered;
+    __device__ __forceinline__ StepBucket(int64_t n, int B_, bool un) : f((double)B_ / (double)(n + 1)), B(B_), unordered(un) {}
+    __device__ __forceinline__ uint32_t operator()(int32_t knew) const
     {
-        unsigned long long lo = ~0ull, hi = 0ull;
-        for (int q = t; q < minmax_parts(kg_.nb); q += RS_THREADS) {
-            const unsigned long long a = mm[2 * q], b = mm[2 * q + 1];
-            lo = a < lo ? a : lo;
-            hi = b > hi ? b : hi;
-        }
-        for (int off = 32; off > 0; off >>= 1) {
-            const unsigned long long a = __shfl_down(lo, off, 64), b = __shfl_down(hi, off, 64);
-            lo = a < lo ? a : lo;
-            hi = b > hi ? b : hi;
-        }
-        if ((t & 63) == 0) { red[0][t >> 6] = lo; red[1][t >> 6] = hi; }
+        if (knew < 0) return SB_TAIL;
+        const int b = (int)((double)knew * f);
+        return unordered || b >= B ? B - 1 : b;
     }
-    __syncthreads();
-    // z = (key - min) >> S with S chosen so the live range fits 31 bits
-    uint64_t kmin = red[0][0], kmax = red[1][0];
-    for (int q = 1; q < RS_THREADS / 64; q++) {
-        kmin = red[0][q] < kmin ? red[0][q] : kmin;
-        kmax = red[1][q] > kmax ? red[1][q] : kmax;
-    }
-    int S = 0;
-    if (kmax >= kmin) {
-        const uint64_t range = kmax - kmin;
-        const int bits = range ? 64 - __clzll((long long)range) : 0;
-        S = bits > 31 ? bits - 31 : 0;
-    } else {
-        kmin = 0;      // no live star
-    }
-    __syncthreads();
-    const int64_t n = s->n_max_new;
-    const int64_t base = (int64_t)kg_.bid * RS_TILE;
-    auto key_word = [&](double r, int64_t i) {
-        const uint64_t k = sortable(r);
-        const uint32_t z = k >= kinf ? Z_TAIL : (uint32_t)((k - kmin) >> S);
-        const uint64_t w = ((uint64_t)z << RS_SHIFT0) | (uint64_t)(uint32_t)(i + 1);
-        words[i] = w;
-        for (int p = P0; p < 8; p++) atomicAdd(&h[p - P0][(w >> (8 * p)) & 255], 1u);
-    };
-    if (aos && g.nf == W - 1) {
-        // the usual full record, software-pipelined: the next chunk's field loads are in
-        // flight while this chunk goes through LDS
-        uint64_t v[W - 1];
-        double kr = 0.0;
-        auto load = [&](int64_t i) {
-            if (i < n) {
-#pragma unroll
-                for (int f = 0; f < W - 1; f++) v[f] = g.src[f][i + 1];
-                kr = keysrc[i + 1];
-            }
-        };
-        load(base + t);
-        for (int u = 0; u < RS_ITEMS; u++) {
-            const int64_t i0 = base + u * RS_THREADS;
-            if (i0 >= n) break;                          // block-uniform
-            const int64_t i = i0 + t;
-            if (i < n) {
-                key_word(kr, i);
-#pragma unroll
-                for (int f = 0; f < W - 1; f++) recs[LD * t + f] = v[f];
-                recs[LD * t + W - 1] = (uint64_t)__double_as_longlong(kr);
-            }
-            if (u + 1 < RS_ITEMS) load(i + RS_THREADS);
-            __syncthreads();
-            const int64_t cnt = n - i0 < RS_THREADS ? n - i0 : RS_THREADS;
-            uint64_t *dst = aos + (int64_t)W * i0;
-            for (int w = t; w < cnt * W; w += RS_THREADS) dst[w] = recs[LD * (w / W) + w % W];
-            __syncthreads();
-        }
-    } else {
-        for (int u = 0; u < RS_ITEMS; u++) {
-            const int64_t i0 = base + u * RS_THREADS;
-            const int64_t i = i0 + t;
-            if (i < n) key_word(keysrc[i + 1], i);
-            if (aos && i0 < n) {        // block-uniform: pack the chunk through LDS, write it contiguously
-                if (i < n) {
-                    for (int f = 0; f < g.nf; f++) recs[LD * t + f] = g.src[f][i + 1];
-                    recs[LD * t + g.nf] = (uint64_t)__double_as_longlong(keysrc[i + 1]);
-                }
-                __syncthreads();
-                const int64_t cnt = n - i0 < RS_THREADS ? n - i0 : RS_THREADS;
-                uint64_t *dst = aos + (int64_t)W * i0;
-                // whole records (unused words included): partial writes cost more
-                for (int w = t; w < cnt * W; w += RS_THREADS) dst[w] = recs[LD * (w / W) + w % W];
-                __syncthreads();
-            }
-        }
-    }
-    __syncthreads();
-    block_hist[(int64_t)t * ntiles + kg_.bid] = h[0][t];
-    for (int p = P0; p < 8; p++)
-        if (h[p - P0][t]) atomicAdd(&digit_totals[p * 256 + t], h[p - P0][t]);
-}
 };
 
-struct rs_hist_kernel {
-    static constexpr int LB = RS_THREADS, MB = 0;
-    static __device__ __forceinline__ void run(KGrid kg_, const uint64_t *__restrict__ keys, DevScalars *s,
-                                                             int shift, uint32_t *__restrict__ block_hist,
-                                                             int64_t ntiles)
+// Tile histograms over the buckets (row `tile` of mat), the step's form.
+template <int BM>
+struct sb_count_step_kernel {
+    static constexpr int LB = 1024, MB = 0;
+    static __device__ __forceinline__ void run(KGrid kg_, const int32_t *__restrict__ knew, DevScalars *s,
+                                               const int32_t *__restrict__ bad, int B, uint32_t *__restrict__ mat)
 {
-    __shared__ uint32_t h[256];
+    __shared__ uint32_t hist[BM];
     const int t = threadIdx.x;
-    h[t] = 0;
-    __syncthreads();
     const int64_t n = s->n_max_new;
-    const int64_t base = (int64_t)kg_.bid * RS_TILE;
-    uint64_t k[RS_ITEMS];                   // every load of the tile in flight before the counting
-#pragma unroll
-    for (int u = 0; u < RS_ITEMS; u++) {
-        const int64_t i = base + u * RS_THREADS + t;
-        k[u] = i < n ? keys[i] : 0ull;
-    }
-#pragma unroll
-    for (int u = 0; u < RS_ITEMS; u++)
-        if (base + u * RS_THREADS + t < n) atomicAdd(&h[(k[u] >> shift) & 255], 1u);
+    if (kg_.bid == 0 && t == 0) s->sort_in = n;
+    const StepBucket bucket(n, B, *bad != 0);
+    for (int b = t; b < B; b += 1024) hist[b] = 0;
+    const int64_t chunk = tile_chunk(n, kg_.nb);
+    const int64_t i0 = (int64_t)kg_.bid * chunk, i1 = i0 + chunk < n ? i0 + chunk : n;
     __syncthreads();
-    block_hist[(int64_t)t * ntiles + kg_.bid] = h[t];
+    for (int64_t c = i0; c < i1; c += 4 * 1024) {
+        int32_t k[4];
+#pragma unroll
+        for (int u = 0; u < 4; u++) {                     // independent loads in flight
+            const int64_t i = c + u * 1024 + t;
+            k[u] = i < i1 ? knew[i + 1] : -1;
+        }
+#pragma unroll
+        for (int u = 0; u < 4; u++)
+            if (k[u] >= 0) atomicAdd(&hist[bucket(k[u])], 1u);
+    }
+    __syncthreads();
+    for (int b = t; b < B; b += 1024) mat[(int64_t)kg_.bid * B + b] = hist[b];
 }
 };
 
-// One block per digit: exclusive scan of that digit's tile counts, plus the digit's
-// global base (sum of the lower digits' totals for this pass).
-struct rs_scan_kernel {
-    static constexpr int LB = RS_THREADS, MB = 0;
-    static __device__ __forceinline__ void run(KGrid kg_, uint32_t *__restrict__ block_hist, int64_t ntiles,
-                                                             const uint32_t *__restrict__ totals)
+// The same from the radii, and every star's bucket: the number of boundaries
+// split[1..B-1] at or below its key.
+template <int BM>
+struct sb_count_kernel {
+    static constexpr int LB = 1024, MB = 0;
+    static __device__ __forceinline__ void run(KGrid kg_, const double *__restrict__ keysrc, DevScalars *s,
+                                               const uint64_t *__restrict__ split, int B, uint16_t *__restrict__ bkt,
+                                               uint32_t *__restrict__ mat)
 {
-    __shared__ uint32_t red[RS_THREADS];
+    __shared__ uint64_t spl[BM];
+    __shared__ uint32_t hist[BM];
     const int t = threadIdx.x;
-    const int d = kg_.bid;
-    red[t] = t < d ? totals[t] : 0u;
-    __syncthreads();
-    for (int off = RS_THREADS / 2; off > 0; off >>= 1) {
-        if (t < off) red[t] += red[t + off];
-        __syncthreads();
+    const int64_t n = s->n_max_new;
+    if (kg_.bid == 0 && t == 0) s->sort_in = n;
+    for (int b = t; b < B; b += 1024) {
+        spl[b] = split[b];
+        hist[b] = 0;
     }
-    const uint32_t dbase = red[0];
+    int top = 1;
+    while (top < B) top <<= 1;
+    const int64_t chunk = tile_chunk(n, kg_.nb);
+    const int64_t i0 = (int64_t)kg_.bid * chunk, i1 = i0 + chunk < n ? i0 + chunk : n;
     __syncthreads();
-    uint32_t *row = block_hist + (int64_t)d * ntiles;
-    const int64_t chunk = (ntiles + RS_THREADS - 1) / RS_THREADS;
-    const int64_t b0 = (int64_t)t * chunk;
-    uint32_t sum = 0;
-    for (int64_t b = b0; b < b0 + chunk && b < ntiles; b++) sum += row[b];
-    red[t] = sum;
+    for (int64_t c = i0; c < i1; c += 4 * 1024) {
+        uint64_t k[4];
+#pragma unroll
+        for (int u = 0; u < 4; u++) {                     // independent loads in flight
+            const int64_t i = c + u * 1024 + t;
+            k[u] = i < i1 ? sortable(keysrc[i + 1]) : ~0ull;
+        }
+        int at[4] = {0, 0, 0, 0};
+        for (int st = top >> 1; st > 0; st >>= 1) {
+#pragma unroll
+            for (int u = 0; u < 4; u++) {
+                const int m = at[u] + st;
+                if (m < B && spl[m] <= k[u]) at[u] = m;
+            }
+        }
+#pragma unroll
+        for (int u = 0; u < 4; u++) {
+            const int64_t i = c + u * 1024 + t;
+            if (i >= i1) continue;
+            const bool live = k[u] < KEY_INF;
+            bkt[i] = live ? (uint16_t)at[u] : SB_TAIL;
+            if (live) atomicAdd(&hist[at[u]], 1u);
+        }
+    }
     __syncthreads();
-    // inclusive Hillis-Steele scan of the per-thread sums
-    for (int off = 1; off < RS_THREADS; off <<= 1) {
-        uint32_t v = t >= off ? red[t - off] : 0u;
-        __syncthreads();
-        red[t] += v;
-        __syncthreads();
-    }
-    uint32_t run = dbase + red[t] - sum;
-    for (int64_t b = b0; b < b0 + chunk && b < ntiles; b++) {
-        uint32_t c = row[b];
-        row[b] = run;
-        run += c;
-    }
+    for (int b = t; b < B; b += 1024) mat[(int64_t)kg_.bid * B + b] = hist[b];
 }
 };
 
-// Stable scatter of one 4096-word tile.  Wave w ranks the contiguous sub-tile
-// [w*1024, (w+1)*1024) on its own (ballot matching of the 8 digit bits, a per-wave
-// digit counter in LDS updated by the highest lane of each match group), so the
-// item loop needs no block barrier; the (digit, wave) counts then give each wave's
-// offset inside the tile's digit runs.  Index order (wave, item, lane) is the tile's
-// index order, so equal digits keep their order.
-struct rs_scatter_kernel {
-    static constexpr int LB = RS_THREADS, MB = 0;
-    static __device__ __forceinline__ void run(KGrid kg_, const uint64_t *__restrict__ words_in,
-                                                                uint64_t *__restrict__ words_out, DevScalars *s,
-                                                                int shift, const uint32_t *__restrict__ tile_off,
-                                                                int64_t ntiles)
+// The tiles' exclusive offsets inside every bucket, in place, and the bucket totals.  A
+// block takes 64 buckets; its 16 waves take consecutive groups of tiles, lane = bucket.
+struct sb_scan_kernel {
+    static constexpr int LB = 1024, MB = 0;
+    static __device__ __forceinline__ void run(KGrid kg_, uint32_t *__restrict__ mat, uint32_t *__restrict__ totals, int B,
+                                               int nt)
 {
-    constexpr int NW = RS_THREADS / 64;
-    __shared__ uint64_t swords[RS_TILE];
-    __shared__ uint32_t wcnt[NW][256];
-    __shared__ uint32_t dstart[256];       // 38 KB in all: four blocks per CU
+    constexpr int PER = SB_MAX_TILES / 16;
+    __shared__ uint32_t part[16][64];
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    const int b = kg_.bid * 64 + lane;
+    const int per = (nt + 15) / 16, t0 = w * per;
+    uint32_t c[PER], sum = 0;
+#pragma unroll
+    for (int q = 0; q < PER; q++) {
+        c[q] = q < per && t0 + q < nt && b < B ? mat[(int64_t)(t0 + q) * B + b] : 0u;
+        sum += c[q];
+    }
+    part[w][lane] = sum;
+    __syncthreads();
+    uint32_t run = 0, tot = 0;
+    for (int q = 0; q < 16; q++) {
+        if (q < w) run += part[q][lane];
+        tot += part[q][lane];
+    }
+#pragma unroll
+    for (int q = 0; q < PER; q++)
+        if (q < per && t0 + q < nt && b < B) {
+            mat[(int64_t)(t0 + q) * B + b] = run;
+            run += c[q];
+        }
+    if (w == 0 && b < B) totals[b] = tot;
+}
+};
+
+// Records of W words: r, id, slot, then the first W - 3 payload fields.  A wave packs 64
+// stars at a time through its own LDS patch (odd stride: no bank conflicts), so whole
+// records leave in each store instruction; the next 64 stars' loads are in flight
+// meanwhile.  knew: the step's form (bkt is not read).  scanned: mat holds the tiles'
+// offsets and totals the bucket totals (sb_scan_kernel); otherwise both are formed here
+// from the raw histogram rows.  Bound by HBM: 500 MB in 112 us at N = 4e6.
+constexpr int SC_T = 512, SC_W = SC_T / 64;
+template <int W, int BM>
+struct sb_scatter_kernel {
+    static constexpr int LB = SC_T, MB = 0;
+    static __device__ __forceinline__ void run(KGrid kg_, const double *__restrict__ keysrc,
+                                               const uint64_t *__restrict__ id, const DevScalars *s,
+                                               const uint16_t *__restrict__ bkt, const int32_t *__restrict__ knew,
+                                               const int32_t *__restrict__ bad, const uint32_t *__restrict__ mat,
+                                               const uint32_t *__restrict__ totals, uint32_t *__restrict__ first, int B,
+                                               int scanned, uint64_t *__restrict__ aos, GatherList g)
+{
+    constexpr int NF = W - 3, LD = W + 1, PC = W / 2;
+    static_assert(SB_SMALL_BUCKETS <= SC_T, "one bucket per thread without the scan pass");
+    __shared__ uint32_t next[BM];
+    __shared__ uint64_t patch[SC_W][64 * LD];
+    __shared__ uint32_t place[SC_W][64];
+    __shared__ uint32_t lds[SC_W];
     const int t = threadIdx.x, lane = t & 63, w = t >> 6;
     const int64_t n = s->n_max_new;
-    const int64_t base = (int64_t)kg_.bid * RS_TILE;
-    const int64_t wbase = base + (int64_t)w * (64 * RS_ITEMS);
-    for (int d = lane; d < 256; d += 64) wcnt[w][d] = 0;
-    uint64_t k[RS_ITEMS];
-    uint32_t rank[RS_ITEMS];
-    const uint64_t lt_mask = (1ull << lane) - 1ull;
-    // every load of the wave's sub-tile in flight before the ranking
+    const int tile = kg_.bid, nt = kg_.nb;
+    // the tile's first free place in every bucket; tile 0 also writes the buckets' first
+    // places and the number of stars to first[0..B].  Every load is issued before the first
+    // use (a thread's buckets one after another would cost a memory latency each).
+    {
+        constexpr int PER = (BM + SC_T - 1) / SC_T;
+        const int per = (B + SC_T - 1) / SC_T;
+        uint32_t tot[PER], off[PER], sum = 0, all;
 #pragma unroll
-    for (int u = 0; u < RS_ITEMS; u++) {
-        const int64_t i = wbase + u * 64 + lane;
-        k[u] = i < n ? words_in[i] : 0ull;
-    }
-    // this tile's output base of every digit
-    __shared__ uint32_t dout[256];
-    dout[t] = tile_off[(int64_t)t * ntiles + kg_.bid];
-#pragma unroll
-    for (int u = 0; u < RS_ITEMS; u++) {
-        int64_t i = wbase + u * 64 + lane;
-        bool valid = i < n;
-        uint32_t d = (uint32_t)((k[u] >> shift) & 255);
-        uint64_t peers = __ballot(valid);
-#pragma unroll
-        for (int b = 0; b < 8; b++) {
-            bool bit = (d >> b) & 1u;
-            uint64_t bal = __ballot(bit);
-            peers &= bit ? bal : ~bal;
+        for (int q = 0; q < PER; q++) {
+            const int b = t * per + q;
+            const bool in = q < per && b < B;
+            tot[q] = in && scanned ? totals[b] : 0u;
+            off[q] = in && scanned ? mat[(int64_t)tile * B + b] : 0u;
         }
-        uint32_t before = valid ? wcnt[w][d] : 0u;
-        rank[u] = before + (uint32_t)__popcll(peers & lt_mask);
-        if (valid && (peers >> lane) == 1ull) wcnt[w][d] = before + (uint32_t)__popcll(peers);
-    }
-    __syncthreads();
-    // per digit (thread t = digit): the waves' offsets and the tile total
-    uint32_t tot = 0;
-    for (int w2 = 0; w2 < NW; w2++) {
-        uint32_t c = wcnt[w2][t];
-        wcnt[w2][t] = tot;
-        tot += c;
-    }
-    // exclusive scan of the tile's digit counts
-    dstart[t] = tot;
-    __syncthreads();
-    for (int off = 1; off < 256; off <<= 1) {
-        uint32_t x = t >= off ? dstart[t - off] : 0u;
-        __syncthreads();
-        dstart[t] += x;
+        if (!scanned && t < B) {                           // B <= SC_T here: one bucket per thread
+            uint32_t c[SB_SMALL_TILES];
+#pragma unroll
+            for (int r = 0; r < SB_SMALL_TILES; r++) c[r] = r < nt ? mat[(int64_t)r * B + t] : 0u;
+#pragma unroll
+            for (int r = 0; r < SB_SMALL_TILES; r++) {
+                if (r < tile) off[0] += c[r];
+                tot[0] += c[r];
+            }
+        }
+#pragma unroll
+        for (int q = 0; q < PER; q++) sum += tot[q];
+        uint32_t base = block_excl(sum, lds, &all);
+#pragma unroll
+        for (int q = 0; q < PER; q++) {
+            const int b = t * per + q;
+            if (q < per && b < B) {
+                next[b] = base + off[q];
+                if (tile == 0) first[b] = base;
+            }
+            base += tot[q];
+        }
+        if (tile == 0 && t == 0) first[B] = all;
         __syncthreads();
     }
-    uint32_t incl = dstart[t];
-    __syncthreads();
-    dstart[t] = incl - tot;
-    __syncthreads();
-    for (int u = 0; u < RS_ITEMS; u++) {
-        int64_t i = wbase + u * 64 + lane;
-        if (i < n) {
-            uint32_t d = (uint32_t)((k[u] >> shift) & 255);
-            uint32_t p = dstart[d] + wcnt[w][d] + rank[u];
-            swords[p] = k[u];
+    const int64_t chunk = tile_chunk(n, nt);
+    const int64_t i0 = (int64_t)tile * chunk, i1 = i0 + chunk < n ? i0 + chunk : n;
+    const StepBucket bucket(n, B, knew && *bad != 0);
+    uint64_t v[NF], kr = 0, vid = 0;
+    uint32_t bk = SB_TAIL;
+    auto load = [&](int64_t i) {
+        bk = SB_TAIL;
+        if (i < i1) {
+            bk = knew ? bucket(knew[i + 1]) : bkt[i];
+            kr = (uint64_t)__double_as_longlong(keysrc[i + 1]);
+            vid = id[i + 1];
+#pragma unroll
+            for (int f = 0; f < NF; f++) v[f] = f < g.nf ? g.src[f][i + 1] : 0ull;
         }
-    }
-    __syncthreads();
-    const int64_t cnt_tile = n - base < RS_TILE ? n - base : RS_TILE;
-    for (int u = 0; u < RS_ITEMS; u++) {
-        int p = u * RS_THREADS + t;
-        if (p < cnt_tile) {
-            uint64_t word = swords[p];
-            uint32_t d = (uint32_t)((word >> shift) & 255);
-            int64_t g = (int64_t)dout[d] + (p - (int64_t)dstart[d]);
-            words_out[g] = word;
+    };
+    uint64_t *mine = patch[w];
+    load(i0 + w * 64 + lane);
+    for (int64_t c = i0 + w * 64; c < i1; c += SC_T) {             // wave-uniform
+        uint32_t p = ~0u;
+        if (bk != SB_TAIL) {
+            p = atomicAdd(&next[bk], 1u);
+            mine[LD * lane] = kr;
+            mine[LD * lane + 1] = vid;
+            mine[LD * lane + 2] = (uint64_t)(c + lane + 1);
+#pragma unroll
+            for (int f = 0; f < NF; f++) mine[LD * lane + 3 + f] = v[f];
         }
+        place[w][lane] = p;
+        load(c + SC_T + lane);
+        wave_sync();
+#pragma unroll
+        for (int u = 0; u < PC; u++) {
+            const int task = u * 64 + lane, rec = task / PC, pc = task % PC;
+            const uint32_t q = place[w][rec];
+            if (q != ~0u)
+                *(ulonglong2 *)(aos + (int64_t)W * q + 2 * pc) =
+                    ulonglong2{mine[LD * rec + 2 * pc], mine[LD * rec + 2 * pc + 1]};
+        }
+        wave_sync();
     }
 }
 };
 
-// Runs of words equal in z (live stars only: the tail has z = Z_TAIL) are put in
-// (r, id) order, r read back through the slot.  Run starts sort runs of up to
-// RUN_SHORT words themselves (insertion sort) and list longer ones for
-// rs_long_runs_kernel.
-__device__ __forceinline__ bool key_id_less(uint64_t ka, int64_t ia, uint64_t kb, int64_t ib)
+// ---------------------------------------------------------------- one bucket
+// Records a, b of a bucket in the order (r, id, slot).
+template <int W>
+__device__ __forceinline__ bool rec_less(const uint64_t *__restrict__ rec, uint32_t a, uint32_t b)
 {
-    return ka < kb || (ka == kb && ia < ib);
+    const uint64_t *x = rec + (int64_t)W * a, *y = rec + (int64_t)W * b;
+    const uint64_t ka = sortable(__longlong_as_double((long long)x[0])), kb = sortable(__longlong_as_double((long long)y[0]));
+    if (ka != kb) return ka < kb;
+    const int64_t ia = (int64_t)x[1], ib = (int64_t)y[1];
+    return ia < ib || (ia == ib && x[2] < y[2]);
 }
 
-struct rs_runs_kernel {
-    static constexpr int LB = 1024, MB = 0;
-    static __device__ __forceinline__ void run(KGrid kg_, uint64_t *__restrict__ words, const double *__restrict__ keysrc,
-                               const int64_t *__restrict__ id, DevScalars *s, int64_t *__restrict__ long_runs,
-                               int64_t *__restrict__ n_long, int64_t long_cap)
+// the same with the keys known
+template <int W>
+__device__ __forceinline__ bool key_less(const uint64_t *__restrict__ rec, uint64_t ka, uint32_t a, uint64_t kb, uint32_t b)
 {
-    const int64_t i = (int64_t)kg_.bid * blockDim.x + threadIdx.x;
-    const int64_t n = s->n_max_new;
-    if (i > n || n <= 0) return;       // n <= 0: sort_n stays 0
-    // the words at i - 1, i and i + 1, loaded together (indices clamped into [0, n),
-    // the clamped ones are not compared)
-    const uint64_t wp = words[i > 0 ? i - 1 : 0];
-    const uint64_t wi = words[i < n ? i : n - 1];
-    const uint64_t wn = words[i + 1 < n ? i + 1 : n - 1];
-    // the number of live stars: the position where the words reach the tail's z (runs
-    // reorder words of one z only, so the z sequence read here is final)
-    const bool below_prev = i == 0 || word_z(wp) != Z_TAIL;
-    const bool below_here = i < n && word_z(wi) != Z_TAIL;
-    if (below_prev && !below_here) s->sort_n = i;
-    if (i + 1 >= n) return;
-    const uint32_t z = word_z(wi);
-    if (z == Z_TAIL) return;
-    if (word_z(wn) != z) return;
-    if (i > 0 && word_z(wp) == z) return;
-    int64_t e = i + 1;
-    while (e + 1 < n && word_z(words[e + 1]) == z && e - i < RUN_SHORT) e++;
-    if (e + 1 < n && word_z(words[e + 1]) == z) {
-        unsigned long long slot = atomicAdd((unsigned long long *)n_long, 1ull);
-        if ((int64_t)slot < long_cap) long_runs[slot] = i;          // the list holds n / 65 runs
-        else dev_set_error(s, CMCG_E_STATE, i + 1);
-        return;
-    }
-    for (int64_t a = i + 1; a <= e; a++) {
-        const uint64_t wa = words[a];
-        const uint32_t va = word_slot(wa);
-        const uint64_t ka = sortable(keysrc[va]);
-        const int64_t ida = id[va];
-        int64_t b = a - 1;
-        while (b >= i) {
-            const uint64_t wb = words[b];
-            const uint32_t vb = word_slot(wb);
-            if (!key_id_less(ka, ida, sortable(keysrc[vb]), id[vb])) break;
-            words[b + 1] = wb;
-            b--;
-        }
-        words[b + 1] = wa;
-    }
+    return ka < kb || (ka == kb && a != b && rec_less<W>(rec, a, b));
 }
-};
 
-// Long runs: one block per run (grid-stride over the list), bitonic sort by (r, id)
-// in LDS, padded to a power of two with all-ones entries.  Every word of a run has
-// the run's z, so only the slots travel.
-constexpr int LR_T = 256;
-// Bitonic sort by (r, id) of words[i .. i + len) (len <= RUN_LONG, one z) in LDS.
-__device__ void lds_sort_run(uint64_t *__restrict__ words, const double *__restrict__ keysrc,
-                             const int64_t *__restrict__ id, int64_t i, int64_t len, uint32_t z,
-                             uint64_t *sk, int64_t *sid, uint32_t *sv)
+constexpr int BS_T = 512, BS_BINS = 2048, BS_RANK = 48;
+
+// Bitonic sort in LDS of the first cnt entries (cnt <= CAP, a power of two), idx indexing
+// the records; the rest of the next power of two is padded with keys above every live one.
+template <int W, int CAP>
+__device__ void bitonic(const uint64_t *__restrict__ rec, uint64_t *key, uint16_t *idx, int cnt)
 {
-    const int t = threadIdx.x;
     int P = 1;
-    while (P < len) P <<= 1;
-    for (int q = t; q < P; q += LR_T) {
-        if (q < len) {
-            const uint32_t v = word_slot(words[i + q]);
-            sk[q] = sortable(keysrc[v]);
-            sv[q] = v;
-            sid[q] = id[v];
-        } else {
-            sk[q] = ~0ull;
-            sid[q] = INT64_MAX;
-            sv[q] = 0u;
-        }
-    }
+    while (P < cnt) P <<= 1;
+    for (int q = cnt + threadIdx.x; q < P; q += BS_T) { key[q] = ~0ull; idx[q] = 0xffff; }
     __syncthreads();
     for (int kk = 2; kk <= P; kk <<= 1)
         for (int j = kk >> 1; j > 0; j >>= 1) {
-            for (int q = t; q < P; q += LR_T) {
+            for (int q = threadIdx.x; q < P; q += BS_T) {
                 const int x = q ^ j;
                 if (x > q) {
+                    const uint64_t ka = key[q], kb = key[x];
+                    const uint16_t a = idx[q], b = idx[x];
                     const bool up = (q & kk) == 0;
-                    const bool gt = key_id_less(sk[x], sid[x], sk[q], sid[q]);
-                    if (gt == up) {
-                        uint64_t tk = sk[q]; sk[q] = sk[x]; sk[x] = tk;
-                        int64_t ti = sid[q]; sid[q] = sid[x]; sid[x] = ti;
-                        uint32_t tv = sv[q]; sv[q] = sv[x]; sv[x] = tv;
-                    }
+                    const bool gt = ka == ~0ull || kb == ~0ull ? kb < ka : key_less<W>(rec, kb, b, ka, a);
+                    if (gt == up) { key[q] = kb; key[x] = ka; idx[q] = b; idx[x] = a; }
                 }
             }
             __syncthreads();
         }
-    for (int q = t; q < len; q += LR_T) words[i + q] = ((uint64_t)z << RS_SHIFT0) | sv[q];
-    __syncthreads();
 }
 
-// Runs longer than RUN_LONG: chunks of RUN_LONG sorted in LDS, then bottom-up merges
-// between words and tmp (the same positions of the second key buffer), each merge
-// split among the threads along its merge path.
-__device__ __forceinline__ bool word_less(uint64_t wa, uint64_t wb, const double *__restrict__ keysrc,
-                                          const int64_t *__restrict__ id)
-{
-    const uint32_t va = word_slot(wa), vb = word_slot(wb);
-    return key_id_less(sortable(keysrc[va]), id[va], sortable(keysrc[vb]), id[vb]);
-}
-
-__device__ void merge_sort_run(uint64_t *__restrict__ words, uint64_t *__restrict__ tmp,
-                               const double *__restrict__ keysrc, const int64_t *__restrict__ id, int64_t i,
-                               int64_t len, uint32_t z, uint64_t *sk, int64_t *sid, uint32_t *sv)
+// A bucket beyond the LDS capacity: pieces of CAP sorted in LDS, then bottom-up merges of
+// record numbers between two global arrays (ord and tmp), each merge split among the
+// threads along its merge path.  The order ends in the returned array.
+template <int W, int CAP>
+__device__ uint32_t *merge_bucket(const uint64_t *__restrict__ rec, uint64_t *key, uint16_t *idx, int64_t cnt,
+                                  uint32_t *ord, uint32_t *tmp)
 {
     const int t = threadIdx.x;
-    for (int64_t c = 0; c < len; c += RUN_LONG)
-        lds_sort_run(words, keysrc, id, i + c, len - c < RUN_LONG ? len - c : RUN_LONG, z, sk, sid, sv);
-    uint64_t *src = words + i, *dst = tmp + i;
-    for (int64_t w = RUN_LONG; w < len; w <<= 1) {
-        for (int64_t p = 0; p < len; p += 2 * w) {
-            const int64_t la = len - p < w ? len - p : w;
-            const int64_t lb = len - p - la < w ? len - p - la : w;
-            const uint64_t *A = src + p, *B = src + p + la;
+    for (int64_t c = 0; c < cnt; c += CAP) {
+        const int m = (int)(cnt - c < CAP ? cnt - c : CAP);
+        for (int q = t; q < m; q += BS_T) {
+            key[q] = sortable(__longlong_as_double((long long)rec[W * (c + q)]));
+            idx[q] = (uint16_t)q;
+        }
+        __syncthreads();
+        bitonic<W, CAP>(rec + W * c, key, idx, m);
+        for (int q = t; q < m; q += BS_T) ord[c + q] = (uint32_t)(c + idx[q]);
+        __syncthreads();
+    }
+    for (int64_t w = CAP; w < cnt; w <<= 1) {
+        for (int64_t p = 0; p < cnt; p += 2 * w) {
+            const int64_t la = cnt - p < w ? cnt - p : w;
+            const int64_t lb = cnt - p - la < w ? cnt - p - la : w;
+            const uint32_t *A = ord + p, *B = ord + p + la;
             const int64_t L = la + lb;
-            const int64_t d0 = L * t / LR_T, d1 = L * (t + 1) / LR_T;
-            // merge path: the first d0 outputs hold A[0, ia) and B[0, d0 - ia); A
-            // goes first on equal keys.  A[m] is among them iff A[m] <= B[d0 - 1 - m].
+            const int64_t d0 = L * t / BS_T, d1 = L * (t + 1) / BS_T;
+            // the first d0 outputs hold A[0, ia) and B[0, d0 - ia); A[m] is among them
+            // iff it does not follow B[d0 - 1 - m]
             int64_t a_lo = d0 > lb ? d0 - lb : 0, a_hi = d0 < la ? d0 : la;
             while (a_lo < a_hi) {
                 const int64_t m = (a_lo + a_hi) >> 1;
-                if (!word_less(B[d0 - 1 - m], A[m], keysrc, id)) a_lo = m + 1;
+                if (!rec_less<W>(rec, B[d0 - 1 - m], A[m])) a_lo = m + 1;
                 else a_hi = m;
             }
             int64_t ia = a_lo, ib = d0 - a_lo;
             for (int64_t d = d0; d < d1; d++) {
-                const bool takeA = ib >= lb || (ia < la && !word_less(B[ib], A[ia], keysrc, id));
-                dst[p + d] = takeA ? A[ia++] : B[ib++];
+                const bool takeA = ib >= lb || (ia < la && !rec_less<W>(rec, B[ib], A[ia]));
+                tmp[p + d] = takeA ? A[ia++] : B[ib++];
             }
         }
         __syncthreads();
-        uint64_t *x = src; src = dst; dst = x;
+        uint32_t *x = ord; ord = tmp; tmp = x;
     }
-    if (src != words + i)
-        for (int64_t q = t; q < len; q += LR_T) words[i + q] = src[q];
-    __syncthreads();
+    return ord;
 }
 
-// One block per listed run (grid-stride over the list): its length by bisection (words
-// are ordered by z), then the LDS bitonic sort, or the merge sort beyond RUN_LONG words.
-struct rs_long_runs_kernel {
-    static constexpr int LB = LR_T, MB = 0;
-    static __device__ __forceinline__ void run(KGrid kg_, uint64_t *__restrict__ words, uint64_t *__restrict__ tmp,
-                                                            const double *__restrict__ keysrc,
-                                                            const int64_t *__restrict__ id, DevScalars *s,
-                                                            const int64_t *__restrict__ long_runs,
-                                                            const int64_t *__restrict__ n_long, int64_t long_cap)
+// Block b orders bucket b and writes its stars' fields.  In LDS: the keys are counted
+// into BS_BINS equal parts of the bucket's key range, placed part by part, and each takes
+// its rank among the few keys of its part; a part of more than BS_RANK keys (many equal
+// radii, a very uneven bucket) sends the bucket through the bitonic sort instead.  The
+// sorted records are then read back in output order, W/2 lanes per record, and leave
+// through LDS with one coalesced store per field.  Bound by HBM (528 MB in 129 us at
+// N = 4e6); holding the records in registers between the two reads, or 256 threads a
+// block, changed nothing.
+template <int W, int CAP>
+struct sb_sort_kernel {
+    static constexpr int LB = BS_T, MB = 0;
+    static __device__ __forceinline__ void run(KGrid kg_, DevScalars *s, const uint32_t *__restrict__ place, int32_t *bad,
+                                               const uint64_t *__restrict__ aos, uint32_t *__restrict__ order, int64_t n_cap,
+                                               double *__restrict__ r_out, uint64_t *__restrict__ id_out,
+                                               uint32_t *__restrict__ perm, GatherList g)
 {
-    __shared__ uint64_t sk[RUN_LONG];
-    __shared__ int64_t sid[RUN_LONG];
-    __shared__ uint32_t sv[RUN_LONG];
-    __shared__ int64_t len_s;
-    const int64_t nl = n_long[0] < long_cap ? n_long[0] : long_cap;
-    const int64_t n = s->n_max_new;
-    const int t = threadIdx.x;
-    for (int64_t r = kg_.bid; r < nl; r += kg_.nb) {
-        const int64_t i = long_runs[r];
-        const uint32_t z = word_z(words[i]);
-        if (t == 0) {
-            // the last index with the run's z: words[lo] has it, words[hi] not (or lo == hi)
-            int64_t lo = i, hi = i + RUN_LONG < n - 1 ? i + RUN_LONG : n - 1;
-            if (word_z(words[hi]) == z) { lo = hi; hi = n - 1; }     // more than RUN_LONG words
-            if (word_z(words[hi]) == z) lo = hi;
-            while (hi - lo > 1) {
-                const int64_t m = lo + ((hi - lo) >> 1);
-                if (word_z(words[m]) == z) lo = m;
-                else hi = m;
+    constexpr int NF = W - 3, PC = W / 2, ITEMS = CAP / BS_T;
+    constexpr int SN = 256 * 8 / W;                                 // records staged at a time: 16 KB
+    constexpr int STAGE = SN * PC + SN * PC / 32;                   // 16-byte pieces, one pad per 32
+    constexpr int BUF = 2 * STAGE > CAP ? 2 * STAGE : CAP;
+    static_assert(CAP % BS_T == 0 && (CAP & (CAP - 1)) == 0, "LDS capacity");
+    __shared__ __align__(16) uint64_t buf[BUF];                     // keys, later the staged records
+    __shared__ uint16_t idx[CAP], fin[CAP];
+    __shared__ uint32_t bin[BS_BINS + 1];
+    __shared__ uint32_t lds[BS_T / 64];
+    __shared__ uint64_t red[2][BS_T / 64];
+    __shared__ uint32_t worst;
+    const int t = threadIdx.x, nb = kg_.nb, b = kg_.bid;
+    const uint32_t first = place[b], mine = place[b + 1] - first;
+    if (b == 0 && t == 0) {
+        const uint32_t tot = place[nb];
+        if (bad) *bad = 0;
+        s->sort_n = tot;
+        s->n_max = tot;
+        s->n_max_new = tot;                                // no block of this launch reads them
+        r_out[(int64_t)tot + 1] = CMCG_SF_INFINITY;        // the outer sentinel (potential_calculate sets it again)
+    }
+    if (!mine) return;
+    const int64_t cnt = mine;
+    const uint64_t *rec = aos + (int64_t)W * first;
+    const uint32_t *ord = nullptr;                         // global order of a bucket beyond CAP
+    if (cnt > CAP) {
+        ord = merge_bucket<W, CAP>(rec, buf, idx, cnt, order + first, order + n_cap + first);
+    } else {
+        uint64_t k[ITEMS], lo = ~0ull, hi = 0ull;
+        uint32_t at[ITEMS];
+#pragma unroll
+        for (int u = 0; u < ITEMS; u++) {
+            const int e = u * BS_T + t;
+            k[u] = 0;
+            if (e < cnt) {
+                k[u] = sortable(__longlong_as_double((long long)rec[(int64_t)W * e]));
+                lo = k[u] < lo ? k[u] : lo;
+                hi = k[u] > hi ? k[u] : hi;
             }
-            len_s = lo - i + 1;
+        }
+        for (int o = 32; o > 0; o >>= 1) {
+            const uint64_t x = __shfl_xor(lo, o, 64), y = __shfl_xor(hi, o, 64);
+            lo = x < lo ? x : lo;
+            hi = y > hi ? y : hi;
+        }
+        if ((t & 63) == 0) { red[0][t >> 6] = lo; red[1][t >> 6] = hi; }
+        for (int q = t; q <= BS_BINS; q += BS_T) bin[q] = 0;
+        if (t == 0) worst = 0;
+        __syncthreads();
+        for (int q = 0; q < BS_T / 64; q++) {
+            lo = red[0][q] < lo ? red[0][q] : lo;
+            hi = red[1][q] > hi ? red[1][q] : hi;
+        }
+        const Binning bin_of(lo, hi, BS_BINS);
+#pragma unroll
+        for (int u = 0; u < ITEMS; u++)
+            if (u * BS_T + t < cnt) at[u] = atomicAdd(&bin[bin_of(k[u])], 1u);
+        __syncthreads();
+        constexpr int PER = BS_BINS / BS_T;
+        uint32_t c[PER], sum = 0, mx = 0, dummy;
+#pragma unroll
+        for (int q = 0; q < PER; q++) {
+            c[q] = bin[t * PER + q];
+            sum += c[q];
+            mx = c[q] > mx ? c[q] : mx;
+        }
+        if (mx > BS_RANK) worst = mx;                      // any value above BS_RANK will do
+        uint32_t run = block_excl(sum, lds, &dummy);
+#pragma unroll
+        for (int q = 0; q < PER; q++) { bin[t * PER + q] = run; run += c[q]; }
+        if (t == 0) bin[BS_BINS] = (uint32_t)cnt;
+        __syncthreads();
+        const bool uneven = worst > BS_RANK;
+#pragma unroll
+        for (int u = 0; u < ITEMS; u++) {
+            const int e = u * BS_T + t;
+            if (e < cnt) {
+                const uint32_t p = uneven ? (uint32_t)e : bin[bin_of(k[u])] + at[u];
+                buf[p] = k[u];
+                idx[p] = (uint16_t)e;
+                at[u] = p;
+            }
         }
         __syncthreads();
-        const int64_t len = len_s;
-        __syncthreads();
-        if (len <= RUN_LONG) lds_sort_run(words, keysrc, id, i, len, z, sk, sid, sv);
-        else merge_sort_run(words, tmp, keysrc, id, i, len, z, sk, sid, sv);
-    }
-}
-};
-
-// The sorted permutation goes to perm (slot of the star now at position i), r and the
-// payload fields to their destinations.
-struct rs_gather_kernel {
-    static constexpr int LB = 256, MB = 0;
-    static __device__ __forceinline__ void run(KGrid kg_, const uint64_t *__restrict__ words, DevScalars *s,
-                                                        const double *__restrict__ keysrc, double *__restrict__ r_out,
-                                                        uint32_t *__restrict__ perm, GatherList g)
-{
-    int64_t i = (int64_t)kg_.bid * blockDim.x + threadIdx.x;
-    const int64_t n = s->sort_n;
-    if (i == 0) { s->n_max = n; s->n_max_new = n; }     // no block reads them
-    if (i > n) return;
-    if (i == n) {   // the outer sentinel (potential_calculate sets it again)
-        r_out[n + 1] = CMCG_SF_INFINITY;
-        return;
-    }
-    const uint32_t src = word_slot(words[i]);
-    perm[i] = src;
-    r_out[i + 1] = keysrc[src];
-    for (int f = 0; f < g.nf; f++) g.dst[f][i + 1] = g.src[f][src];
-}
-};
-
-template <int W>
-struct rs_gather_aos_kernel {
-    static constexpr int LB = 256, MB = 0;
-    static __device__ __forceinline__ void run(KGrid kg_, const uint64_t *__restrict__ words, DevScalars *s,
-                                               double *__restrict__ r_out, uint32_t *__restrict__ perm,
-                                               const uint64_t *__restrict__ aos, GatherList g)
-{
-    // The block's 256 records are read cooperatively, W/2 lanes per record (one
-    // 16-byte piece each, so each load instruction covers whole records), through LDS;
-    // then each thread writes its star's fields, coalesced across the block.
-    constexpr int PC = W / 2;                          // 16-byte pieces per record
-    __shared__ ulonglong2 recs[256 * PC + 256 * PC / 32];   // one pad slot per 32 pieces
-    __shared__ uint32_t ssrc[256];
-    const int t = threadIdx.x;
-    const int64_t i = (int64_t)kg_.bid * 256 + t;
-    const int64_t n = s->sort_n;
-    if (i == 0) { s->n_max = n; s->n_max_new = n; }     // no block reads them
-    uint32_t src = 0;
-    if (i < n) {
-        src = word_slot(words[i]);
-        perm[i] = src;
-    } else if (i == n) {
-        r_out[n + 1] = CMCG_SF_INFINITY;
-    }
-    ssrc[t] = src;
-    __syncthreads();
-    const int64_t live = n - (int64_t)kg_.bid * 256;   // stars of this block (may be <= 0)
+        if (uneven) {
+            bitonic<W, CAP>(rec, buf, idx, (int)cnt);
+            for (int q = t; q < cnt; q += BS_T) fin[q] = idx[q];
+        } else {
 #pragma unroll
-    for (int u = 0; u < PC; u++) {
-        const int task = u * 256 + t, sl = task / PC, pc = task % PC;
-        if (sl < live) {
-            const ulonglong2 *rec = (const ulonglong2 *)(aos + (int64_t)W * (ssrc[sl] - 1));
-            recs[task + task / 32] = 2 * pc <= g.nf ? rec[pc] : ulonglong2{0ull, 0ull};    // fields, then r in word nf
+            for (int u = 0; u < ITEMS; u++) {
+                const int e = u * BS_T + t;
+                if (e < cnt) {
+                    const uint32_t bn = bin_of(k[u]), e0 = bin[bn], e1 = bin[bn + 1];
+                    uint32_t rank = e0;
+                    for (uint32_t q = e0; q < e1; q++)
+                        if (q != at[u]) rank += key_less<W>(rec, buf[q], idx[q], k[u], (uint32_t)e);
+                    fin[rank] = (uint16_t)e;
+                }
+            }
         }
     }
     __syncthreads();
-    if (i >= n) return;
-    uint64_t w[W];
+    ulonglong2 *stage = (ulonglong2 *)buf;
+    for (int64_t c0 = 0; c0 < cnt; c0 += SN) {
+        const int live = (int)(cnt - c0 < SN ? cnt - c0 : SN);
 #pragma unroll
-    for (int q = 0; q < PC; q++) {
-        const int task = t * PC + q;
-        const ulonglong2 v = recs[task + task / 32];
-        w[2 * q] = v.x;
-        w[2 * q + 1] = v.y;
-    }
+        for (int u = 0; u < SN * PC / BS_T; u++) {
+            const int task = u * BS_T + t, sl = task / PC, pc = task % PC;
+            if (sl < live) {
+                const uint32_t e = ord ? ord[c0 + sl] : fin[c0 + sl];
+                stage[task + task / 32] = *(const ulonglong2 *)(rec + (int64_t)W * e + 2 * pc);
+            }
+        }
+        __syncthreads();
+        if (t < live) {
+            uint64_t w[W];
 #pragma unroll
-    for (int f = 0; f < W; f++) {
-        if (f < g.nf) g.dst[f][i + 1] = w[f];
-        if (f == g.nf) r_out[i + 1] = __longlong_as_double((long long)w[f]);
+            for (int q = 0; q < PC; q++) {
+                const int task = t * PC + q;
+                const ulonglong2 x = stage[task + task / 32];
+                w[2 * q] = x.x;
+                w[2 * q + 1] = x.y;
+            }
+            const int64_t i = (int64_t)first + c0 + t;
+            r_out[i + 1] = __longlong_as_double((long long)w[0]);
+            id_out[i + 1] = w[1];
+            perm[i] = (uint32_t)w[2];
+#pragma unroll
+            for (int f = 0; f < NF; f++)
+                if (f < g.nf) g.dst[f][i + 1] = w[3 + f];
+        }
+        __syncthreads();
     }
 }
 };
 
+// The payload fields beyond a record's, through the permutation.
+struct sb_rest_kernel {
+    static constexpr int LB = 256, MB = 0;
+    static __device__ __forceinline__ void run(KGrid kg_, const DevScalars *s, const uint32_t *__restrict__ perm, int f0,
+                                               GatherList g)
+{
+    const int64_t i = (int64_t)kg_.bid * 256 + threadIdx.x;
+    if (i >= s->sort_n) return;
+    const uint32_t src = perm[i];
+    for (int f = f0; f < g.nf; f++) g.dst[f][i + 1] = g.src[f][src];
+}
+};
+
+template <int W, int BM, int CAP>
+hipError_t sort_launch(const double *key_src, double *r_dst, const uint64_t *id_src, uint64_t *id_dst, const GatherList &g,
+                       DevScalars *s, const Scratch &sc, const SortShape &sh, int64_t n_ub, const int32_t *knew,
+                       hipStream_t st)
+{
+    if (knew) {
+        kl<sb_count_step_kernel<BM>>(dim3((unsigned)sh.tiles), dim3(1024), 0, st, knew, s, (const int32_t *)sc.sort_bad,
+                                     sh.buckets, sc.sort_mat);
+    } else {
+        kl<sb_sample_kernel>(dim3(1), dim3(SMP_T), 0, st, key_src, (const DevScalars *)s, sh.buckets, sc.sort_split);
+        kl<sb_count_kernel<BM>>(dim3((unsigned)sh.tiles), dim3(1024), 0, st, key_src, s, (const uint64_t *)sc.sort_split,
+                                sh.buckets, sc.sort_bkt, sc.sort_mat);
+    }
+    const int scanned = !sh.small;
+    if (scanned)
+        kl<sb_scan_kernel>(dim3((unsigned)((sh.buckets + 63) / 64)), dim3(1024), 0, st, sc.sort_mat, sc.sort_tot,
+                           sh.buckets, sh.tiles);
+    kl<sb_scatter_kernel<W, BM>>(dim3((unsigned)sh.tiles), dim3(SC_T), 0, st, key_src, id_src, (const DevScalars *)s,
+                                 (const uint16_t *)sc.sort_bkt, knew, (const int32_t *)sc.sort_bad,
+                                 (const uint32_t *)sc.sort_mat, (const uint32_t *)sc.sort_tot, sc.sort_first, sh.buckets,
+                                 scanned, sc.sort_aos, g);
+    kl<sb_sort_kernel<W, CAP>>(dim3((unsigned)sh.buckets), dim3(BS_T), 0, st, s, (const uint32_t *)sc.sort_first,
+                               knew ? sc.sort_bad : (int32_t *)nullptr, (const uint64_t *)sc.sort_aos, sc.sort_order,
+                               sc.sort_aos_cap, r_dst, id_dst, sc.vals_a, g);
+    if (g.nf > W - 3)
+        kl<sb_rest_kernel>(dim3((unsigned)((n_ub + 255) / 256)), dim3(256), 0, st, (const DevScalars *)s,
+                           (const uint32_t *)sc.vals_a, W - 3, g);
+    return hipGetLastError();
+}
 } // namespace
 
 // Sort slots 1..n_max_new by (key field, id).  src/dst are parallel lists of payload
-// fields; key_src is the field holding the radii to sort by; r_dst receives them sorted.
-hipError_t launch_sort_fields(const double *key_src, double *r_dst, const int64_t *id_src, int nf,
-                              const uint64_t *const *src, uint64_t *const *dst, DevScalars *s, const Scratch &sc,
-                              int64_t n_ub, hipStream_t st)
+// fields, id the last of them; key_src is the field holding the radii to sort by; r_dst
+// receives them sorted.  knew: the radii's indices among the old nodes that the orbit
+// phase left (the step's sort), or null.
+hipError_t launch_sort_fields(const double *key_src, double *r_dst, int nf, const uint64_t *const *src,
+                              uint64_t *const *dst, DevScalars *s, const Scratch &sc, int64_t n_ub,
+                              const int32_t *knew, hipStream_t st)
 {
-    if (nf > RS_MAX_FIELDS) return hipErrorInvalidValue;
-    GatherList g;
-    g.nf = nf;
-    for (int f = 0; f < nf; f++) { g.src[f] = src[f]; g.dst[f] = dst[f]; }
-    for (int f = nf; f < RS_MAX_FIELDS; f++) { g.src[f] = nullptr; g.dst[f] = nullptr; }
-    // packed records hold the fields and r after them
-    uint64_t *aos = (nf < AOS_MAX && sc.sort_aos && n_ub <= sc.sort_aos_cap) ? sc.sort_aos : nullptr;
-    const bool narrow = nf < 8;          // fields and r in 8 words
-    int64_t ntiles = (n_ub + RS_TILE - 1) / RS_TILE;
-    if (ntiles < 1) ntiles = 1;
-    if (ntiles > sc.max_sort_tiles) return hipErrorInvalidValue;
-    const uint64_t kinf = 0x8000000000000000ull | 0x4202a05f20000000ull;   // sortable(1.0e10)
-    unsigned long long *mm = (unsigned long long *)sc.sort_mm;
-    kl<rs_minmax_kernel>(dim3((unsigned)minmax_parts(ntiles)), dim3(256), 0, st, key_src, s, kinf,
-                       mm, sc.digit_totals, (int64_t)(8 * 256), sc.sort_nlong);
-    // an even number of passes: the sorted words end in keys_a
-    uint64_t *kin = sc.keys_a, *kout = sc.keys_b;
-    if (narrow)
-        kl<rs_prep_kernel<8>>(dim3((unsigned)ntiles), dim3(RS_THREADS), 0, st, key_src, s, kin,
-                           sc.digit_totals, aos, g, kinf, (const unsigned long long *)mm, sc.block_hist, ntiles);
-    else
-        kl<rs_prep_kernel<AOS_MAX>>(dim3((unsigned)ntiles), dim3(RS_THREADS), 0, st, key_src, s, kin,
-                           sc.digit_totals, aos, g, kinf, (const unsigned long long *)mm, sc.block_hist, ntiles);
-    for (int pass = 8 - RS_PASSES; pass < 8; pass++) {
-        int shift = 8 * pass;
-        if (pass > 8 - RS_PASSES)          // the first pass's tile counts come from rs_prep_kernel
-            kl<rs_hist_kernel>(dim3((unsigned)ntiles), dim3(RS_THREADS), 0, st, kin, s, shift,
-                           sc.block_hist, ntiles);
-        kl<rs_scan_kernel>(dim3(256), dim3(RS_THREADS), 0, st, sc.block_hist, ntiles,
-                           (const uint32_t *)(sc.digit_totals + 256 * pass));
-        kl<rs_scatter_kernel>(dim3((unsigned)ntiles), dim3(RS_THREADS), 0, st, kin, kout, s, shift,
-                           (const uint32_t *)sc.block_hist, ntiles);
-        uint64_t *tk = kin; kin = kout; kout = tk;
-    }
-    unsigned g1 = (unsigned)((n_ub + 256) / 256);
-    kl<rs_runs_kernel>(dim3(g1), dim3(256), 0, st, kin, key_src, id_src, s, sc.sort_long,
-                       sc.sort_nlong, sc.sort_long_cap);
-    kl<rs_long_runs_kernel>(dim3(64), dim3(LR_T), 0, st, kin, kout, key_src, id_src, s,
-                       (const int64_t *)sc.sort_long, (const int64_t *)sc.sort_nlong, sc.sort_long_cap);
-    if (aos && narrow)
-        kl<rs_gather_aos_kernel<8>>(dim3(g1), dim3(256), 0, st, (const uint64_t *)kin, s, r_dst,
-                           sc.vals_a, (const uint64_t *)aos, g);
-    else if (aos)
-        kl<rs_gather_aos_kernel<AOS_MAX>>(dim3(g1), dim3(256), 0, st, (const uint64_t *)kin, s, r_dst,
-                           sc.vals_a, (const uint64_t *)aos, g);
-    else
-        kl<rs_gather_kernel>(dim3(g1), dim3(256), 0, st, (const uint64_t *)kin, s, key_src, r_dst,
-                           sc.vals_a, g);
-    return hipGetLastError();
+    if (nf < 1 || nf - 1 > SB_MAX_FIELDS || n_ub > sc.sort_aos_cap) return hipErrorInvalidValue;
+    GatherList g{};
+    g.nf = nf - 1;
+    for (int f = 0; f < g.nf; f++) { g.src[f] = src[f]; g.dst[f] = dst[f]; }
+    const SortShape sh = sort_shape(n_ub);
+    if ((size_t)sh.tiles * sh.buckets > sc.sort_mat_cap) return hipErrorInvalidValue;
+    const uint64_t *id_src = src[nf - 1];
+    uint64_t *id_dst = dst[nf - 1];
+    const bool small = sh.small;
+    // Records: 8 words hold r, id, slot and five fields (the step's sort); a wider payload
+    // takes 16 words, and its buckets, cut from a sample, get twice the LDS capacity.
+    if (g.nf <= 5)
+        return small ? sort_launch<8, SB_SMALL_BUCKETS, 2048>(key_src, r_dst, id_src, id_dst, g, s, sc, sh, n_ub, knew, st)
+                     : sort_launch<8, SB_MAX_BUCKETS, 2048>(key_src, r_dst, id_src, id_dst, g, s, sc, sh, n_ub, knew, st);
+    return small ? sort_launch<16, SB_SMALL_BUCKETS, 4096>(key_src, r_dst, id_src, id_dst, g, s, sc, sh, n_ub, knew, st)
+                 : sort_launch<16, SB_MAX_BUCKETS, 4096>(key_src, r_dst, id_src, id_dst, g, s, sc, sh, n_ub, knew, st);
 }

@@ -10,12 +10,28 @@
 // orbit sampler: most LDS samples of any launch variant; lane jumps l 2^20 by nibble
 // tables of the powers 2^ORB_NIB_B0 .. 2^(ORB_NIB_B0 + ORB_NIB_POWERS - 1)
 constexpr int ORB_MAX_COARSE = 2048;
-// sort payload records: 16 words (128 B, one cache line) per star
+// sort payload records: at most 16 words (128 B, one cache line) per star
 constexpr int SORT_AOS_WORDS = 16;
-constexpr int SORT_RUN_SHORT = 64;   // runs of equal sort keys up to this length are ordered in place
-constexpr int SORT_TILE = 4096;      // words per tile of the radix passes (2048: 4% slower)
-constexpr int SORT_RUN_LONG = 4096;  // ... up to this length in LDS; longer ones by a merge sort
-constexpr int SORT_MM_PARTS = 1024;   // blocks of the sort's min/max pass, one (min, max) pair each
+// The sort's shape: buckets of about SB_AVG stars, at most SB_MAX_BUCKETS (their boundaries
+// and counters fill LDS), and the tiles that its count and scatter passes cut the stars
+// into.  Up to SB_SMALL_N stars the histogram is small enough for every scatter block to
+// sum it, one launch less (at N = 1e5 the whole sort takes 34 us, a launch about 4); there
+// a tile is down to one star per thread, for the shortest chain of loads.
+constexpr int SB_AVG = 1024, SB_MAX_BUCKETS = 8192, SB_MAX_TILES = 512;
+constexpr int64_t SB_SMALL_N = 131072;
+constexpr int SB_SMALL_BUCKETS = (int)(SB_SMALL_N / SB_AVG), SB_SMALL_TILES = 32;
+struct SortShape { int buckets, tiles; bool small; };
+inline SortShape sort_shape(int64_t n_ub)
+{
+    SortShape sh;
+    const int64_t b = (n_ub + SB_AVG - 1) / SB_AVG;
+    sh.buckets = b < 1 ? 1 : b > SB_MAX_BUCKETS ? SB_MAX_BUCKETS : (int)b;
+    sh.small = n_ub <= SB_SMALL_N;
+    const int64_t per = sh.small ? 512 : 2048, most = sh.small ? SB_SMALL_TILES : SB_MAX_TILES;
+    const int64_t t = (n_ub + per - 1) / per;
+    sh.tiles = t < 1 ? 1 : t > most ? (int)most : (int)t;
+    return sh;
+}
 constexpr int RED2_BLOCKS = 64;
 constexpr int ORB_NIB_B0 = 20, ORB_NIB_POWERS = 6;
 
@@ -45,26 +61,26 @@ struct Scratch {
     double *partials;
     int64_t max_blocks;
     // sort
-    uint64_t *keys_a, *keys_b;  // sort words: 32-bit normalised key of r above the 32-bit slot
     uint32_t *vals_a;           // sorted permutation: slot of the star now at each position
-    uint64_t *sort_mm;          // live key (min, max) per block of the min/max pass: 2 * SORT_MM_PARTS
-    uint32_t *block_hist;       // 256 * max_sort_tiles
-    uint32_t *digit_totals;     // 8 * 256
-    int64_t max_sort_tiles;
+    uint64_t *sort_split;       // bucket boundaries (order-preserving keys of r), SB_MAX_BUCKETS
+    int32_t *sort_bad;          // the radii that the orbit phase read do not ascend
+    uint16_t *sort_bkt;         // bucket of every star
+    uint32_t *sort_mat;         // tile histograms over the buckets
+    size_t sort_mat_cap;
+    uint32_t *sort_tot;         // bucket totals
+    uint32_t *sort_first;       // first place of every bucket, and the number of stars kept
+    uint32_t *sort_order;       // record numbers of buckets beyond the LDS capacity: 2 * sort_aos_cap
     uint64_t *sort_aos;         // packed payload records, SORT_AOS_WORDS words per star
-    int64_t *sort_long;         // starts of runs of equal key prefixes longer than SORT_RUN_SHORT
-    int64_t *sort_nlong;        // number of listed runs
-    int64_t sort_long_cap;
     double2 *mid;               // (r, phi) at every 16th node (search middle level)
     double2 *nodes;             // packed (r, phi) of every node, for the searches
     float2 *pred;               // learned apsides proposals (log r_peri, log r_apo) per star
     uint32_t *ridx;             // radial index: nodes below each bucket of r (ridx_nb + 2 entries)
     uint32_t *ridx_tb;          // its value at every RIDX_TILE-th bucket
     int ridx_bits;              // log2 of the bucket count
-    double2 *u_old;             // (new potential, radius) at each old sorted radius (set_velocities3)
+    double2 *u_old;             // (new potential, radius), (D, -) at each old sorted radius (set_velocities3)
     int64_t *merge_ends;        // set_velocities3: node index of both ends of each merge block
     int64_t merge_ends_cap;
-    double *sv3_dpre, *sv3_dpost; // vold^2 + 2(1-q)(Uoldrold - Uoldrnew) per star, before and after the step's sort
+    double *sv3_dpre;           // D = vold^2 + 2(1-q)(Uoldrold - Uoldrnew) per star, in the order before the step's sort
     unsigned long long *dt_part;  // the step's time step: 64 slots, 128 bytes apart, of complemented dt minima
     double2 *coarse;            // orbit sampler's (r, phi) samples, copied into LDS by every block
     void *orb_nib;              // orbit sampler's GF(2) nibble tables (constant per context)
@@ -159,9 +175,9 @@ hipError_t launch_find_zero_Q(const DevFields &f, DevScalars *s, const KParams &
                               const int64_t *j, const int64_t *kmin, const int64_t *kmax,
                               const double *E, const double *J, int64_t *out, hipStream_t st);
 
-hipError_t launch_sort_fields(const double *key_src, double *r_dst, const int64_t *id_src, int nf,
-                              const uint64_t *const *src, uint64_t *const *dst, DevScalars *s, const Scratch &sc,
-                              int64_t n_ub, hipStream_t st);
+hipError_t launch_sort_fields(const double *key_src, double *r_dst, int nf, const uint64_t *const *src,
+                              uint64_t *const *dst, DevScalars *s, const Scratch &sc, int64_t n_ub,
+                              const int32_t *knew, hipStream_t st);
 
 hipError_t launch_step_begin(DevScalars *s, hipStream_t st);
 hipError_t launch_after_dynamics(DevScalars *s, hipStream_t st);
@@ -176,7 +192,7 @@ hipError_t launch_ie_transfer(const DevFields &f, DevScalars *s, int64_t n_ub, h
 // r_old_sorted: the radii the sort of this step read (old sorted order), or nullptr
 hipError_t launch_set_velocities3(const DevFields &f, DevScalars *s, const KParams &P, const Scratch &sc,
                                   int64_t n_ub, hipStream_t st, const double *r_old_sorted = nullptr,
-                                  const double *dpost = nullptr);
+                                  const double *dpre = nullptr);
 hipError_t launch_compute_energy(const DevFields &f, DevScalars *s, const KParams &P, const Scratch &sc,
                                  int64_t n_ub, hipStream_t st);
 
