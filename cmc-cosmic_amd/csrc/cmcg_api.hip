@@ -449,7 +449,7 @@ int cmcg_create(cmcg_ctx **out, int device, int64_t n_cap, const cmcg_params *pa
     while (sc.ridx_bits < 23 && ((int64_t)1 << sc.ridx_bits) < 2 * (n_cap + 2)) sc.ridx_bits++;
     if ((e = dalloc(c, &sc.ridx, (size_t)ridx_entries(sc.ridx_bits))) ||
         (e = dalloc(c, &sc.ridx_tb, (size_t)ridx_tiles(sc.ridx_bits) + 1))) { cmcg_destroy(c); return e; }
-    if ((e = dalloc(c, &sc.tile_sums, (size_t)sc.max_tiles * 6)) || (e = dalloc(c, &sc.partials, (size_t)sc.max_blocks * 16)) ||
+    if ((e = dalloc(c, &sc.tile_sums, (size_t)sc.max_tiles * 12)) || (e = dalloc(c, &sc.partials, (size_t)sc.max_blocks * 16)) ||
         (e = dalloc(c, &sc.sort_aos, (size_t)(n_cap + 4) * SORT_AOS_WORDS)) || (e = dalloc(c, &sc.sort_split, SB_MAX_BUCKETS)) ||
         (e = dalloc(c, &sc.sort_bad, 1)) || (e = dalloc(c, &sc.sort_bkt, (size_t)n_cap + 4)) ||
         (e = dalloc(c, &sc.sort_mat, sc.sort_mat_cap)) || (e = dalloc(c, &sc.sort_tot, SB_MAX_BUCKETS)) ||
@@ -465,11 +465,11 @@ int cmcg_create(cmcg_ctx **out, int device, int64_t n_cap, const cmcg_params *pa
         (e = dalloc(c, &sc.sv3_wend, (size_t)n_cap + 2)) || (e = dalloc(c, &sc.sv3_merged, (size_t)n_cap + 2)) ||
         (e = dalloc(c, &sc.sv3_blk, (size_t)sc.max_blocks)) || (e = dalloc(c, &sc.sv3_fallback, 1)) ||
         (e = dalloc(c, &sc.strip_done, 1)) || (e = dalloc(c, &sc.chain_x, (size_t)n_cap + 8)) ||
-        (e = dalloc(c, &sc.chain_g, (size_t)n_cap + 8)) || (e = dalloc(c, &sc.chain_mk, (size_t)n_cap + 8)) ||
+        (e = dalloc(c, &sc.chain_g, (size_t)n_cap + 8)) ||
         (e = dalloc(c, &sc.defer_list, (size_t)P.defer_cap)) || (e = dalloc(c, &sc.defer_kfirst, (size_t)P.defer_cap)) ||
         (e = dalloc(c, &sc.chain_scal, 4)) || (e = dalloc(c, &sc.chain_len, 4)) || (e = dalloc(c, &sc.chain_fbad, 8)) ||
         (e = dalloc(c, &sc.esa_idx, (size_t)sc.esa_max)) || (e = dalloc(c, &sc.esa_racc, (size_t)sc.esa_max)) ||
-        (e = dalloc(c, &sc.esa_v, (size_t)sc.esa_max)) || (e = dalloc(c, &sc.esa_n, 4)) || (e = dalloc(c, &sc.esa_raw_idx, 2048)) || (e = dalloc(c, &sc.esa_raw_part, 3 * 2048)) || (e = dalloc(c, &sc.rng_base, 2)) || (e = dalloc(c, &sc.rng_wave, (size_t)sc.max_waves)) || (e = dalloc(c, &sc.rng_seeded, 1)) ||
+        (e = dalloc(c, &sc.esa_v, (size_t)sc.esa_max)) || (e = dalloc(c, &sc.esa_n, 8)) || (e = dalloc(c, &sc.esa_raw_idx, 2 * 2048)) || (e = dalloc(c, &sc.esa_raw_part, 2 * 3 * 2048)) || (e = dalloc(c, &sc.rng_base, 2)) || (e = dalloc(c, &sc.rng_wave, (size_t)sc.max_waves)) || (e = dalloc(c, &sc.rng_seeded, 1)) ||
         (e = dalloc(c, &c->T, 1))) {
         cmcg_destroy(c);
         return e;
@@ -1107,7 +1107,7 @@ static int enqueue_step(cmcg_ctx *c, int64_t nub, bool graph)
     }
     {
         PhaseTimer t(c, "potential");
-        LAUNCH(launch_potential(c->f, c->s, c->kp, nub, c->sc, c->stream));
+        LAUNCH(launch_potential(c->f, c->s, c->kp, nub, c->sc, c->stream, false));   // the sort has just set N_MAX
     }
     {
         PhaseTimer t(c, "glue_post_sort");

@@ -54,6 +54,7 @@ struct EsaArgs {
     int64_t *first_bad;         // [1] first element that violates the recurrence (L: none)
     const int64_t *Lp;
     int slack;                  // error bound widened by 2^slack (0; a test hook raises it)
+    int64_t extra;              // the start value is only an estimate, as uncertain as this many more elements
     // per tile
     double *tsumP, *tpreP;      // estimated sums of s*x and their exclusive prefixes
     int64_t *tcnt, *ttail;      // sensitive count; regular sum after the tile's last sensitive element
@@ -112,9 +113,10 @@ __device__ double block_excl_sum(double v, double *lds, double *total)
     return off + ex;
 }
 
+// by a group of CT threads (a block, or half a block that gives each half its own lds)
 __device__ Seg block_excl_seg(Seg v, Seg *lds, Seg *total)
 {
-    const int t = threadIdx.x, lane = t & 63, w = t >> 6, nw = blockDim.x >> 6;
+    const int t = threadIdx.x % CT, lane = t & 63, w = t >> 6, nw = CT >> 6;
     Seg x = v;
 #pragma unroll
     for (int d = 1; d < 64; d <<= 1) {
@@ -164,11 +166,11 @@ __device__ __forceinline__ double err_bound(int64_t j, double vmax, int slack)
 }
 
 // binade of the chain value before element j, or INT32_MIN when its error interval
-// straddles binades; before element 0 the value is v0 exactly
-__device__ __forceinline__ int start_binade(int64_t j, double v0, double P, int slack)
+// straddles binades; before element 0 the value is v0 (exactly, when extra is 0)
+__device__ __forceinline__ int start_binade(int64_t j, double v0, double P, int slack, int64_t extra)
 {
-    if (j == 0) return interval_binade(v0, 0.0);
-    return interval_binade(P, err_bound(j, fmax(fabs(v0), fabs(P)), slack));
+    if (j == 0 && extra == 0) return interval_binade(v0, 0.0);
+    return interval_binade(P, err_bound(j + extra, fmax(fabs(v0), fabs(P)), slack));
 }
 
 // regular increment of an element in units of 2^(bp-52), or sensitive: bp, bq are the
@@ -199,18 +201,24 @@ struct TileItems {
 constexpr int TILE_LDS = CTILE + CTILE / 8;
 __device__ __forceinline__ int tile_slot(int i) { return i + (i >> 3); }
 
-__device__ __forceinline__ void load_tile(const double *__restrict__ x, double sign, int64_t base, int64_t L,
-                                          double *tbuf, double (&sx)[CI])
+// src(j): element j's x.  The loads are issued on their own, as early as the caller can:
+// after a launch each misses L2, and a chain of such misses is what a small cluster's
+// passes wait for.
+template <class Src>
+__device__ __forceinline__ void fetch_tile(const Src &src, int64_t base, int64_t L, double (&v)[CI])
 {
-    const int t = threadIdx.x;
-    double v[CI];                           // every load in flight before the LDS writes
 #pragma unroll
     for (int u = 0; u < CI; u++) {
-        const int64_t j = base + u * CT + t;
-        v[u] = j < L ? x[j] : 0.0;
+        const int64_t j = base + u * CT + threadIdx.x;
+        v[u] = j < L ? src(j) : 0.0;
     }
+}
+
+__device__ __forceinline__ void spread_tile(const double (&v)[CI], double sign, double *tbuf, double (&sx)[CI])
+{
+    const int t = threadIdx.x;
 #pragma unroll
-    for (int u = 0; u < CI; u++) tbuf[tile_slot(u * CT + t)] = base + u * CT + t < L ? sign * v[u] : 0.0;
+    for (int u = 0; u < CI; u++) tbuf[tile_slot(u * CT + t)] = sign * v[u];
     __syncthreads();
 #pragma unroll
     for (int u = 0; u < CI; u++) sx[u] = tbuf[tile_slot(t * CI + u)];
@@ -233,17 +241,17 @@ __device__ __forceinline__ void store_tile(double *__restrict__ g, int64_t base,
 }
 
 // Classification of one tile (items past the end are regular with R = 0), from the
-// estimated prefixes before the tile and before the next one.  Every kernel
+// fetched elements (v) and the estimated prefixes before the tile and before the next one.  Every kernel
 // classifies through this function on the same inputs, so they agree element for
 // element; the binade at a tile start is taken from the same expression in both tiles
 // that meet there.  Nearly always a thread's whole range of
 // values lies in one binade, checked once with the bound at its last element: then
 // only the ties remain to be found.
-__device__ void tile_classify(const EsaArgs &a, int64_t tile, int64_t L, double v0, TileItems &it, double *lds,
-                              double *tbuf, double pre_t, double pre_t1)
+__device__ __forceinline__ void tile_classify(const EsaArgs &a, const double (&v)[CI], int64_t tile, int64_t L, double v0,
+                                              TileItems &it, double *lds, double *tbuf, double pre_t, double pre_t1)
 {
     const int64_t j0 = tile * CTILE + (int64_t)threadIdx.x * CI;
-    load_tile(a.x, a.sign, tile * CTILE, L, tbuf, it.sx);
+    spread_tile(v, a.sign, tbuf, it.sx);
     double acc = 0.0;
 #pragma unroll
     for (int u = 0; u < CI; u++) acc += it.sx[u];
@@ -266,14 +274,14 @@ __device__ void tile_classify(const EsaArgs &a, int64_t tile, int64_t L, double 
     int bt = INT32_MIN;
     if (j0 < L) {
         const double vmax = fmax(fabs(v0), fmax(fabs(Pmin), fabs(Pmax)));
-        const double err = err_bound(jl, vmax, a.slack);
+        const double err = err_bound(jl + a.extra, vmax, a.slack);
         const double lo = fmin(Pmin, j0 == 0 ? v0 : Pmin) - err, hi = fmax(Pmax, j0 == 0 ? v0 : Pmax) + err;
         if (lo > 0.0 || hi < 0.0) {
             const int b1 = binade_of(lo), b2 = binade_of(hi);
             if (b1 == b2) bt = b1;
         }
-        if (j0 == 0 && bt != interval_binade(v0, 0.0)) bt = INT32_MIN;
-        if (edge && bt != start_binade(jl, v0, Pn, a.slack)) bt = INT32_MIN;
+        if (j0 == 0 && bt != start_binade(0, v0, v0, a.slack, a.extra)) bt = INT32_MIN;
+        if (edge && bt != start_binade(jl, v0, Pn, a.slack, a.extra)) bt = INT32_MIN;
     }
     if (bt != INT32_MIN) {
 #pragma unroll
@@ -288,7 +296,7 @@ __device__ void tile_classify(const EsaArgs &a, int64_t tile, int64_t L, double 
         return;
     }
     P = P0;
-    int bp = start_binade(j0, v0, P, a.slack);
+    int bp = start_binade(j0, v0, P, a.slack, a.extra);
 #pragma unroll
     for (int u = 0; u < CI; u++) {
         const int64_t j = j0 + u;
@@ -297,7 +305,7 @@ __device__ void tile_classify(const EsaArgs &a, int64_t tile, int64_t L, double 
         it.bp[u] = bp;
         if (j < L) {
             const double Pe = edge && j + 1 == jl ? Pn : Pq;
-            const int bq = start_binade(j + 1, v0, Pe, a.slack);
+            const int bq = start_binade(j + 1, v0, Pe, a.slack, a.extra);
             if (classify(it.sx[u], bp, bq, &it.R[u])) {
                 it.sens |= 1u << u;
                 it.R[u] = 0;
@@ -409,35 +417,38 @@ __device__ void tile_prefixes(const double *__restrict__ tsumP, int64_t t, doubl
     *pre_t1 = tree_sum(p1, lds);
 }
 
-// self_prefix: form the tile prefixes here (and store this tile's in tpreP for the
-// later passes); otherwise read them from tpreP (esa_tile_scan_kernel).
-struct esa_classify_kernel {
-    static constexpr int LB = CT, MB = 0;
-    static __device__ __forceinline__ void run(KGrid kg_, EsaArgs a, int self_prefix)
+// elements as they lie in memory
+struct ArraySrc {
+    const double *__restrict__ x;
+    __device__ __forceinline__ double operator()(int64_t j) const { return x[j]; }
+};
+
+// LDS of the classification and the rebuild
+struct ChainLds {
+    double d[CT / 64];
+    Seg s[CT / 64];
+    double tbuf[TILE_LDS];
+    double lastv[CT];
+};
+
+// One tile classified: its segment aggregate, and its sensitive elements appended to the
+// chain's list.  v0: the start value (or its estimate).  Returns false in a thread that
+// holds an element below zero, infinite or NaN.
+__device__ __forceinline__ bool classify_tile(const EsaArgs &a, const double (&v)[CI], int64_t tile, int64_t L, double v0,
+                                              double pre_t, double pre_t1, ChainLds &sh)
 {
-    __shared__ double ldsd[CT / 64];
-    __shared__ Seg ldss[CT / 64];
-    __shared__ double tbuf[TILE_LDS];
-    const int64_t L = *a.Lp;
-    const int64_t tile = kg_.bid;
-    if (tile * CTILE >= L) return;
-    double pre_t, pre_t1;
-    if (self_prefix) {
-        tile_prefixes(a.tsumP, tile, ldsd, &pre_t, &pre_t1);
-        if (threadIdx.x == 0) a.tpreP[tile] = pre_t;
-    } else {
-        pre_t = a.tpreP[tile];
-        pre_t1 = a.tpreP[tile + 1];
-    }
     TileItems it;
-    tile_classify(a, tile, L, *a.v0p, it, ldsd, tbuf, pre_t, pre_t1);
+    tile_classify(a, v, tile, L, v0, it, sh.d, sh.tbuf, pre_t, pre_t1);
+    bool ok = true;
+#pragma unroll
+    for (int u = 0; u < CI; u++) ok = ok && a.sign * it.sx[u] >= 0.0 && a.sign * it.sx[u] < __builtin_inf();
     Seg tot;
-    const Seg pre = block_excl_seg(items_seg(it), ldss, &tot);
+    const Seg pre = block_excl_seg(items_seg(it), sh.s, &tot);
     if (threadIdx.x == 0) {
         a.tcnt[tile] = tot.cnt;
         a.ttail[tile] = tot.sum;
     }
-    if (!it.sens) return;
+    if (!it.sens) return ok;
     int64_t cur = pre.sum;
     const int64_t j0 = tile * CTILE + (int64_t)threadIdx.x * CI;
     for (int u = 0; u < CI; u++) {
@@ -454,6 +465,35 @@ struct esa_classify_kernel {
             cur += it.R[u];
         }
     }
+    return ok;
+}
+
+// the estimated prefixes of a tile and the next: formed here (and this tile's stored in
+// tpreP for the later passes), or read from tpreP (esa_tile_scan_kernel)
+__device__ __forceinline__ void get_prefixes(const EsaArgs &a, int64_t tile, int self_prefix, double *lds, double *pre_t,
+                                             double *pre_t1)
+{
+    if (self_prefix) {
+        tile_prefixes(a.tsumP, tile, lds, pre_t, pre_t1);
+        if (threadIdx.x == 0) a.tpreP[tile] = *pre_t;
+    } else {
+        *pre_t = a.tpreP[tile];
+        *pre_t1 = a.tpreP[tile + 1];
+    }
+}
+
+struct esa_classify_kernel {
+    static constexpr int LB = CT, MB = 0;
+    static __device__ __forceinline__ void run(KGrid kg_, EsaArgs a, int self_prefix)
+{
+    __shared__ ChainLds sh;
+    const int64_t L = *a.Lp;
+    const int64_t tile = kg_.bid;
+    if (tile * CTILE >= L) return;
+    double v[CI], pre_t, pre_t1;
+    fetch_tile(ArraySrc{a.x}, tile * CTILE, L, v);
+    get_prefixes(a, tile, self_prefix, sh.d, &pre_t, &pre_t1);
+    classify_tile(a, v, tile, L, *a.v0p, pre_t, pre_t1, sh);
 }
 };
 
@@ -509,22 +549,11 @@ __device__ void esa_walk_block(const EsaArgs &a, int64_t ns, const double *lpre,
     }
 }
 
-// One block: the tiles' sensitive offsets and open-segment carries (a segmented scan
-// of the tile aggregates), then the ordered list of the sensitive elements and the
-// walk.  The list is the classification's appended one put in order by index when it
-// holds every sensitive element; otherwise (more than RAW_CAP, never for an ordinary
-// cluster) this block classifies the tiles again one after another and lists them in
-// order, slowly but exactly.
-struct esa_walk_kernel {
-    static constexpr int LB = CT, MB = 0;
-    static __device__ __forceinline__ void run(KGrid kg_, EsaArgs a)
+// The tiles' sensitive offsets and open-segment carries (a segmented scan of the tile
+// aggregates), by a group of CT threads; returns the chain's total.
+__device__ Seg walk_scan(const EsaArgs &a, int64_t nt, Seg *lds)
 {
-    __shared__ Seg lds[CT / 64];
-    __shared__ int64_t ridx[RAW_CAP];
-    __shared__ double lpre[RAW_CAP], lsx[RAW_CAP];
-    const int t = threadIdx.x;
-    const int64_t L = *a.Lp;
-    const int64_t nt = (L + CTILE - 1) / CTILE;
+    const int t = threadIdx.x % CT;
     const int64_t chunk = (nt + CT - 1) / CT;
     const int64_t b0 = (int64_t)t * chunk;
     Seg tot;
@@ -559,17 +588,61 @@ struct esa_walk_kernel {
             run = seg_then(run, Seg{a.ttail[b], a.tcnt[b]});
         }
     }
-    const int64_t ns = tot.cnt;
-    if (t == 0) *a.s_n = ns;
+    if (t == 0) *a.s_n = tot.cnt;
     __syncthreads();                                // (also makes the block's global writes visible to it)
+    return tot;
+}
+
+// LDS of the walk: the appended list put in order
+struct WalkLds {
+    Seg s[CT / 64];
+    int64_t idx[RAW_CAP];
+    double pre[RAW_CAP], sx[RAW_CAP];
+};
+
+// The appended list (ns <= RAW_CAP entries) put in order by index.
+__device__ void walk_list(const EsaArgs &a, int64_t ns, WalkLds &sh)
+{
+    const int t = threadIdx.x % CT;
+    for (int64_t e = t; e < ns; e += CT) sh.idx[e] = a.raw_idx[e];
+    __syncthreads();
+    for (int64_t e = t; e < ns; e += CT) {
+        const int64_t j = sh.idx[e];
+        int64_t rank = 0;
+        for (int64_t q = 0; q < ns; q++) rank += sh.idx[q] < j;      // the indices are distinct
+        const int64_t tile = j / CTILE;
+        const int64_t pre = a.raw_part[e] + (rank == a.toff[tile] ? a.tcarry[tile] : 0);
+        a.s_idx[rank] = j;
+        sh.pre[rank] = seg_value(pre, a.raw_bp[e]);
+        sh.sx[rank] = a.raw_sx[e];
+    }
+    __syncthreads();
+}
+
+// One block: the scan, then the ordered list of the sensitive elements and the walk.  The
+// list is the classification's appended one when it holds every sensitive element;
+// otherwise (more than RAW_CAP, never for an ordinary cluster) this block classifies the
+// tiles again one after another and lists them in order, slowly but exactly.
+struct esa_walk_kernel {
+    static constexpr int LB = CT, MB = 0;
+    static __device__ __forceinline__ void run(KGrid kg_, EsaArgs a)
+{
+    __shared__ WalkLds sh;
+    const int t = threadIdx.x;
+    const int64_t L = *a.Lp;
+    const int64_t nt = (L + CTILE - 1) / CTILE;
+    const Seg tot = walk_scan(a, nt, sh.s);
+    const int64_t ns = tot.cnt;
     if (ns > RAW_CAP) {
         __shared__ double ldsd[CT / 64];
         __shared__ double tbuf[TILE_LDS];
         for (int64_t tile = 0; tile < nt; tile++) {
             TileItems it;
-            tile_classify(a, tile, L, *a.v0p, it, ldsd, tbuf, a.tpreP[tile], a.tpreP[tile + 1]);
+            double v[CI];
+            fetch_tile(ArraySrc{a.x}, tile * CTILE, L, v);
+            tile_classify(a, v, tile, L, *a.v0p, it, ldsd, tbuf, a.tpreP[tile], a.tpreP[tile + 1]);
             Seg ttot;
-            const Seg pre = block_excl_seg(items_seg(it), lds, &ttot);
+            const Seg pre = block_excl_seg(items_seg(it), sh.s, &ttot);
             int64_t k = a.toff[tile] + pre.cnt;
             int64_t cur = pre.sum + (pre.cnt ? 0 : a.tcarry[tile]);
             const int64_t j0 = tile * CTILE + (int64_t)t * CI;
@@ -590,56 +663,34 @@ struct esa_walk_kernel {
         esa_walk_block(a, ns, nullptr, nullptr);
         return;
     }
-    for (int64_t e = t; e < ns; e += CT) ridx[e] = a.raw_idx[e];
-    __syncthreads();
-    for (int64_t e = t; e < ns; e += CT) {
-        const int64_t j = ridx[e];
-        int64_t rank = 0;
-        for (int64_t q = 0; q < ns; q++) rank += ridx[q] < j;      // the indices are distinct
-        const int64_t tile = j / CTILE;
-        const int64_t pre = a.raw_part[e] + (rank == a.toff[tile] ? a.tcarry[tile] : 0);
-        a.s_idx[rank] = j;
-        lpre[rank] = seg_value(pre, a.raw_bp[e]);
-        lsx[rank] = a.raw_sx[e];
-    }
-    __syncthreads();
-    esa_walk_block(a, ns, lpre, lsx);
+    walk_list(a, ns, sh);
+    esa_walk_block(a, ns, sh.pre, sh.sx);
 }
 };
 
-// Parallel rebuild of every element from the last sensitive value before it,
-// verification of the recurrence against the values actually written (the value
-// before a tile is rebuilt exactly as the previous tile wrote it), and the first
-// violation.
-struct esa_rebuild_kernel {
-    static constexpr int LB = CT, MB = 0;
-    static __device__ __forceinline__ void run(KGrid kg_, EsaArgs a)
+// Parallel rebuild of one tile from the last sensitive value before every element, and
+// verification of the recurrence against the values rebuilt (the value before a tile is
+// rebuilt exactly as the previous tile's block rebuilds it).  vc: the start value that
+// the classification used, v0: the exact one.  nv: the thread's values; *before: the
+// value before its first element.  Returns the thread's first violation, or L.
+// s_v: the values of the ns_eff listed sensitive elements.
+__device__ __forceinline__ int64_t rebuild_tile(const EsaArgs &a, const double (&v)[CI], int64_t tile, int64_t L, double vc,
+                                                double v0, const double *s_v, int64_t ns_eff, ChainLds &sh, TileItems &it,
+                                                double (&nv)[CI], double *before)
 {
-    __shared__ double ldsd[CT / 64];
-    __shared__ Seg ldss[CT / 64];
-    __shared__ double lastv[CT];
-    __shared__ double tbuf[TILE_LDS];
-    const int64_t L = *a.Lp;
-    const int64_t tile = kg_.bid;
     const int64_t base = tile * CTILE;
-    if (base >= L) return;
-    const double v0 = *a.v0p;
     const int t = threadIdx.x;
-    int64_t ns_eff = *a.s_n;
-    if (ns_eff > a.smax) ns_eff = a.smax;
-    TileItems it;
-    tile_classify(a, tile, L, v0, it, ldsd, tbuf, a.tpreP[tile], a.tpreP[tile + 1]);
-    Seg tot;
-    const Seg pre = block_excl_seg(items_seg(it), ldss, &tot);
     const int64_t toff = a.toff[tile], tcarry = a.tcarry[tile];
+    tile_classify(a, v, tile, L, vc, it, sh.d, sh.tbuf, a.tpreP[tile], a.tpreP[tile + 1]);
+    Seg tot;
+    const Seg pre = block_excl_seg(items_seg(it), sh.s, &tot);
     int64_t k = toff + pre.cnt;                       // rank of the next sensitive element
     int64_t cur = pre.sum + (pre.cnt ? 0 : tcarry);
     const int64_t j0 = base + (int64_t)t * CI;
-    double nv[CI];
 #pragma unroll
     for (int u = 0; u < CI; u++) {
         if ((it.sens >> u) & 1) {
-            nv[u] = k < ns_eff ? a.s_v[k] : it.pa[u];
+            nv[u] = k < ns_eff ? s_v[k] : it.pa[u];
             k++;
             cur = 0;
         } else {
@@ -648,39 +699,58 @@ struct esa_rebuild_kernel {
             if (kk >= ns_eff) {
                 nv[u] = it.pa[u];
             } else {
-                const double b = kk >= 0 ? a.s_v[kk] : v0;
+                const double b = kk >= 0 ? s_v[kk] : v0;
                 nv[u] = cur == 0 ? b : b + seg_value(cur, it.bp[u]);
             }
         }
     }
-    lastv[t] = nv[CI - 1];
+    sh.lastv[t] = nv[CI - 1];
     __syncthreads();
-    double before;
+    double prev;
     if (t > 0) {
-        before = lastv[t - 1];
+        prev = sh.lastv[t - 1];
     } else if (tile == 0) {
-        before = v0;
+        prev = v0;
     } else {
         const int64_t kk = toff - 1;
-        if (kk >= ns_eff) before = it.pa[0] - it.sx[0];        // past the list: already left to the repair
-        else if (kk >= 0 && a.s_idx[kk] == base - 1) before = a.s_v[kk];
+        if (kk >= ns_eff) prev = it.pa[0] - it.sx[0];        // past the list: already left to the repair
+        else if (kk >= 0 && a.s_idx[kk] == base - 1) prev = s_v[kk];
         else {
-            const double b = kk >= 0 ? a.s_v[kk] : v0;
-            before = tcarry == 0 ? b : b + seg_value(tcarry, it.bp[0]);
+            const double b = kk >= 0 ? s_v[kk] : v0;
+            // (a tile past the chain's end classifies nothing: its run has the binade of b)
+            prev = tcarry == 0 ? b : b + seg_value(tcarry, base < L ? it.bp[0] : binade_of(b));
         }
     }
+    *before = prev;
     int64_t bad = L;
 #pragma unroll
     for (int u = 0; u < CI; u++) {
         const int64_t j = j0 + u;
         if (j < L) {
-            const double want = before + it.sx[u];
+            const double want = prev + it.sx[u];
             if (want != nv[u] && j < bad) bad = j;
         }
-        before = nv[u];
+        prev = nv[u];
     }
+    return bad;
+}
+
+struct esa_rebuild_kernel {
+    static constexpr int LB = CT, MB = 0;
+    static __device__ __forceinline__ void run(KGrid kg_, EsaArgs a)
+{
+    __shared__ ChainLds sh;
+    const int64_t L = *a.Lp;
+    const int64_t tile = kg_.bid;
+    if (tile * CTILE >= L) return;
+    const double v0 = *a.v0p;
+    TileItems it;
+    double v[CI], nv[CI], before;
+    fetch_tile(ArraySrc{a.x}, tile * CTILE, L, v);
+    const int64_t ns = *a.s_n;
+    const int64_t bad = rebuild_tile(a, v, tile, L, v0, v0, a.s_v, ns < a.smax ? ns : a.smax, sh, it, nv, &before);
     if (bad < L) atomicMin((unsigned long long *)&a.first_bad[1], (unsigned long long)bad);
-    store_tile(a.g, base, L, tbuf, nv);
+    store_tile(a.g, tile * CTILE, L, sh.tbuf, nv);
 }
 };
 
@@ -733,140 +803,386 @@ struct pot_count_kernel {
 }
 };
 
-struct PotWork {
-    double *xa, *ga;           // chain buffers (increments, values)
-    double *Mk;                // chain B result: M_{N-1-j}
-    double *scal;              // [0] 0.0  [1] Mtotal
-    int64_t *len;              // [0] L_A  [1] L_B  [2] L_C
-    int64_t *fbad;             // 2 per chain
+// The three chains of the potential.  A and B are classified together: chain B starts
+// from the total mass, whose estimate (the tile sums of A) is good enough to tell the
+// binades (EsaArgs::extra), so B need not wait for A's walk; one block then walks A and B.
+// Chain A needs only its last value, so it is never rebuilt: for masses that are not
+// negative the bound on the estimate is rigorous, and any other mass takes the repair.
+// B's rebuild forms chain C's increments at once (M_k is not stored), and C's rebuild
+// writes the potential and the node tables.  Eight launches; each chain by itself took
+// five, and the counts and copies five more.  The phase: 0.109 -> 0.070 ms at N = 1e4, where
+// a launch costs 4 to 5 us whatever it does, 0.128 -> 0.090 at 1e6, 0.242 -> 0.179 at 4e6
+// (there the passes over memory bound it: 42, 41 and 34 us for the A and B classification
+// and the two rebuilds).
+struct PotArgs {
+    const double *m;
+    double *r, *phi;
+    DevScalars *s;
+    double nstar;
+    double *xc;                 // chain C's increments
+    double *scal;               // [0] 0.0 (C's start), [1] Mtotal (B's start), [2] its estimate
+    // nonzero: the chains go through the repair.  A kernel reads only the words that earlier
+    // kernels set: [0] classification and [1] lists of A and B, [2] rebuild of B, [3] list
+    // and [4] rebuild of C
+    int64_t *flag;
+    double2 *nodes, *mid;       // packed (r, phi) of every node and of every MID_STEP-th
+    int counted;                // N_MAX from the count of radii below SF_INFINITY (pot_count_kernel)
+    EsaArgs a, b, c;
+    __device__ __forceinline__ int64_t lb(int64_t n) const { return n > 1 ? n - 1 : 0; }
+    __device__ __forceinline__ bool flagged(int words) const
+    {
+        int64_t any = 0;
+        for (int q = 0; q < words; q++) any |= flag[q];
+        return any != 0;
+    }
+};
+struct SrcA {
+    const double *__restrict__ m;
+    __device__ __forceinline__ double operator()(int64_t j) const { return m[1 + j]; }
+};
+// star_m[k] / clus.N_STAR, k = N - j
+struct SrcB {
+    const double *__restrict__ m;
+    int64_t n;
+    double nstar;
+    __device__ __forceinline__ double operator()(int64_t j) const { return m[n - j] / nstar; }
 };
 
-// N_MAX from the count, the chain lengths, and the sentinels before the recurrence
-// reads r[N+1] (cmc_utils.c:713-714)
-struct pot_setup_kernel {
-    static constexpr int LB = 1024, MB = 0;
-    static __device__ __forceinline__ void run(KGrid kg_, DevScalars *s, PotWork w, double *__restrict__ r, double *__restrict__ phi)
+// the total mass from chain A's last value (cmc_utils.c:703)
+__device__ __forceinline__ double pot_mass(const KParams &P, double mprev) { return mprev * P.madhoc + P.cenma_m * P.madhoc; }
+
+// The tile sums of A and B, N_MAX and the sentinels (cmc_utils.c:713-714), the chains'
+// flags and lists cleared.
+struct pot_sums_kernel {
+    static constexpr int LB = CT, MB = 0;
+    static __device__ __forceinline__ void run(KGrid kg_, PotArgs p)
 {
-    int64_t n = s->first_inf - 1;
-    s->n_max = n;
-    w.len[0] = n;                       // A: k = 1..N
-    w.len[1] = n > 1 ? n - 1 : 0;       // B: k = N..2 gives M_{N-1}..M_1
-    w.len[2] = n;                       // C: k = N..1
-    w.scal[0] = 0.0;
-    r[n + 1] = CMCG_SF_INFINITY;
-    phi[n + 1] = 0.0;
+    __shared__ double lds[CT / 64];
+    const int64_t n = p.counted ? p.s->first_inf - 1 : p.s->n_max;
+    const int64_t base = (int64_t)kg_.bid * CTILE;
+    if (kg_.bid == 0 && threadIdx.x == 0) {
+        if (p.counted) p.s->n_max = n;               // the other blocks read first_inf
+        p.scal[0] = 0.0;
+        for (int q = 0; q < 5; q++) p.flag[q] = 0;
+        *p.a.raw_n = 0;
+        *p.b.raw_n = 0;
+        *p.c.raw_n = 0;
+        p.r[n + 1] = CMCG_SF_INFINITY;
+        p.phi[n + 1] = 0.0;
+    }
+    const SrcA sa{p.m};
+    const SrcB sb{p.m, n, p.nstar};
+    double va[CI], vb[CI];
+#pragma unroll
+    for (int u = 0; u < CI; u++) {
+        const int64_t j = base + u * CT + threadIdx.x;
+        va[u] = j < n ? sa(j) : 0.0;
+        vb[u] = j < p.lb(n) ? sb(j) : 0.0;
+    }
+    double ta = 0.0, tb = 0.0;
+#pragma unroll
+    for (int u = 0; u < CI; u++) { ta += va[u]; tb -= vb[u]; }
+    ta = tree_sum(ta, lds);
+    tb = tree_sum(tb, lds);
+    if (threadIdx.x == 0) {
+        p.a.tsumP[kg_.bid] = ta;
+        p.b.tsumP[kg_.bid] = tb;
+    }
 }
 };
+
+// Blocks 0 .. tiles - 1 classify chain A's tiles, the rest chain B's.
+struct pot_classify_ab_kernel {
+    static constexpr int LB = CT, MB = 0;
+    static __device__ __forceinline__ void run(KGrid kg_, PotArgs p, KParams P, int self_prefix)
+{
+    __shared__ ChainLds sh;
+    const int64_t n = p.s->n_max, nt = kg_.nb / 2;
+    const bool isb = kg_.bid >= nt;
+    const int64_t tile = isb ? kg_.bid - nt : kg_.bid;
+    if (tile * CTILE >= n) return;
+    double v[CI], pre_t, pre_t1;
+    if (isb) fetch_tile(SrcB{p.m, n, p.nstar}, tile * CTILE, p.lb(n), v);
+    else fetch_tile(SrcA{p.m}, tile * CTILE, n, v);
+    // the total mass as chain A's sums estimate it, by the same sums in every block of B
+    const int64_t live = (n + CTILE - 1) / CTILE;
+    double est = 0.0;
+    if (isb)
+        for (int64_t q = threadIdx.x; q < live; q += CT) est += p.a.tsumP[q];
+    get_prefixes(isb ? p.b : p.a, tile, self_prefix, sh.d, &pre_t, &pre_t1);
+    bool ok;
+    if (isb) {
+        est = pot_mass(P, tree_sum(est, sh.d));
+        if (tile == 0 && threadIdx.x == 0) p.scal[2] = est;
+        EsaArgs b = p.b;
+        b.extra = n;
+        ok = classify_tile(b, v, tile, p.lb(n), est, pre_t, pre_t1, sh);
+    } else {
+        ok = classify_tile(p.a, v, tile, n, 0.0, pre_t, pre_t1, sh);
+    }
+    if (!ok) p.flag[0] = 1;
+}
+};
+
+__device__ __forceinline__ double lane_value(double x, int lane)
+{
+    const long long b = __double_as_longlong(x);
+    const unsigned lo = __builtin_amdgcn_readlane((unsigned)b, lane), hi = __builtin_amdgcn_readlane((unsigned)(b >> 32), lane);
+    return __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
+}
+
+// The walk over ns listed elements from v, by one whole wave: 64 elements at a time in
+// its lanes' registers, so that the chain of additions waits on no memory.  s_v (which may
+// be pre or sx) receives the value after each element; every lane returns the last.
+__device__ __forceinline__ double pot_walk(int64_t ns, double v, const double *pre, const double *sx, double *s_v)
+{
+    const int lane = threadIdx.x & 63;
+    for (int64_t c = 0; c < ns; c += 64) {
+        const int cnt = (int)(ns - c < 64 ? ns - c : 64);
+        const double p = lane < cnt ? pre[c + lane] : 0.0, x = lane < cnt ? sx[c + lane] : 0.0;
+        double mine = 0.0;
+        for (int k = 0; k < cnt; k++) {
+            const double pk = lane_value(p, k), pred = pk == 0.0 ? v : v + pk;
+            v = pred + lane_value(x, k);
+            if (lane == k) mine = v;
+        }
+        if (lane < cnt) s_v[c + lane] = mine;
+    }
+    return v;
+}
 
 // after chain A: Mtotal, Rtidal (cmc_utils.c:703-707), NaN check (:688-691)
-__device__ __forceinline__ void pot_total(DevScalars *s, const KParams &P, const double *__restrict__ ga, PotWork &w)
+__device__ __forceinline__ void pot_total(const PotArgs &p, const KParams &P, double mprev)
 {
-    int64_t n = s->n_max;
-    double mprev = n > 0 ? ga[n - 1] : 0.0;
-    if (isnan(mprev)) dev_set_error(s, CMCG_E_NAN, n);
-    double Mtotal = mprev * P.madhoc + P.cenma_m * P.madhoc;
+    DevScalars *s = p.s;
+    if (isnan(mprev)) dev_set_error(s, CMCG_E_NAN, s->n_max);
+    const double Mtotal = pot_mass(P, mprev);
     s->Mtotal = Mtotal;
     s->Rtidal = P.orbit_r * pow(Mtotal, 1.0 / 3.0);
-    w.scal[1] = Mtotal;
+    p.scal[1] = Mtotal;
 }
 
-// chain B increments (star_m[k] / clus.N_STAR, k = N - j) and their tile sums; the
-// first thread also finishes chain A (Mtotal, the start value of chain B), which the
-// increments do not use
-struct prep_b_kernel {
-    static constexpr int LB = CT, MB = 0;
-    static __device__ __forceinline__ void run(KGrid kg_, const double *__restrict__ m, DevScalars *s, double nstar,
-                                                    double *__restrict__ x, KParams P, const double *__restrict__ ga,
-                                                    PotWork w, EsaArgs e)
+// Chains A and B: half the block puts each list in order, then one wave walks A, finishes
+// the total mass and walks B from it.  (Block by block, B's list after A's walk: 21 us at
+// N = 4e6 instead of 17; B walked again by every block of its rebuild: no faster in all.)
+struct pot_walk_ab_kernel {
+    static constexpr int LB = 2 * CT, MB = 0;
+    static __device__ __forceinline__ void run(KGrid kg_, PotArgs p, KParams P)
 {
-    __shared__ double lds[CT / 64];
-    if (kg_.bid == 0 && threadIdx.x == 0) pot_total(s, P, ga, w);
-    const int64_t n = s->n_max;
-    const int64_t L = n > 1 ? n - 1 : 0;
-    const int64_t base = (int64_t)kg_.bid * CTILE;
-    double mv[CI];
-#pragma unroll
-    for (int u = 0; u < CI; u++) {
-        const int64_t j = base + u * CT + threadIdx.x;
-        mv[u] = j < L ? m[n - j] : 0.0;
+    __shared__ WalkLds sh[2];
+    __shared__ Seg tot[2];
+    const int64_t n = p.s->n_max, nt = (n + CTILE - 1) / CTILE;
+    if (p.flag[0]) return;                            // the repair runs the chains itself
+    const int h = threadIdx.x / CT;
+    const EsaArgs &c = h ? p.b : p.a;
+    const Seg mine = walk_scan(c, nt, sh[h].s);
+    if (threadIdx.x % CT == 0) tot[h] = mine;
+    __syncthreads();
+    if (tot[0].cnt > RAW_CAP || tot[1].cnt > RAW_CAP) {
+        if (threadIdx.x == 0) p.flag[1] = 1;
+        return;
     }
-    double acc = 0.0;
-#pragma unroll
-    for (int u = 0; u < CI; u++) {
-        const int64_t j = base + u * CT + threadIdx.x;
-        if (j < L) {
-            const double v = mv[u] / nstar;
-            x[j] = v;
-            acc += e.sign * v;
-        }
-    }
-    esa_tile_sums(e, L, acc, lds, kg_.bid);
+    walk_list(c, mine.cnt, sh[h]);
+    if (threadIdx.x >= 64) return;
+    double v = pot_walk(tot[0].cnt, 0.0, sh[0].pre, sh[0].sx, sh[0].pre);
+    if (tot[0].sum != 0) v += seg_value(tot[0].sum, binade_of(v));   // the run after the last stays in one binade
+    if (threadIdx.x == 0) pot_total(p, P, v);
+    pot_walk(tot[1].cnt, pot_mass(P, v), sh[1].pre, sh[1].sx, p.b.s_v);
 }
 };
 
-// p_k = M_k * (1/r_k - 1/r_{k+1}) with the reference's roundings, and their tile sums;
-// chain C runs on w = -phi, w_k = fl(w_{k+1} + p_k)
-struct prep_c_kernel {
+// Chain B rebuilt and verified; from the enclosed masses chain C's increments
+// p_k = M_k * (1/r_k - 1/r_{k+1}), k = N - j, with the reference's roundings, and their
+// tile sums; chain C runs on w = -phi, w_k = fl(w_{k+1} + p_k).  M_k is the value before
+// B's element j.
+struct pot_rebuild_b_kernel {
     static constexpr int LB = CT, MB = 0;
-    static __device__ __forceinline__ void run(KGrid kg_, const double *__restrict__ r, DevScalars *s,
-                                                    const double *__restrict__ Mk, double *__restrict__ x, EsaArgs e)
+    static __device__ __forceinline__ void run(KGrid kg_, PotArgs p)
 {
-    __shared__ double lds[CT / 64];
-    const int64_t n = s->n_max;
-    const int64_t base = (int64_t)kg_.bid * CTILE;
-    double Mv[CI], rk[CI], rk1[CI];
-    const double Mtot = s->Mtotal;
+    __shared__ ChainLds sh;
+    const int64_t n = p.s->n_max;
+    const int64_t tile = kg_.bid, base = tile * CTILE;
+    const int t = threadIdx.x;
+    if (base >= n || p.flag[0] || p.flag[1]) return;
+    EsaArgs b = p.b;
+    b.extra = n;
+    const int64_t lb = p.lb(n);
+    double v[CI], rk[CI], rk1[CI];
+    fetch_tile(SrcB{p.m, n, p.nstar}, base, lb, v);
 #pragma unroll
     for (int u = 0; u < CI; u++) {
-        const int64_t j = base + u * CT + threadIdx.x;
-        const int64_t k = n - j;
-        Mv[u] = rk[u] = rk1[u] = 1.0;
-        if (j < n) {
-            Mv[u] = k == n ? Mtot : Mk[n - 1 - k];
-            rk[u] = r[k];
-            rk1[u] = r[k + 1];
-        }
+        const int64_t j = base + u * CT + t;
+        rk[u] = j < n ? p.r[n - j] : 1.0;
+        rk1[u] = j < n ? p.r[n - j + 1] : 1.0;
     }
-    double acc = 0.0;
+    TileItems it;
+    double nv[CI], before;
+    const int64_t bad = rebuild_tile(b, v, tile, lb, p.scal[2], p.scal[1], b.s_v, *b.s_n, sh, it, nv, &before);
+    if (bad < lb) p.flag[2] = 1;
+    // 1/r_k - 1/r_{k+1} of the tile through LDS
+    __syncthreads();                                  // tbuf free
+#pragma unroll
+    for (int u = 0; u < CI; u++) sh.tbuf[tile_slot(u * CT + t)] = 1.0 / rk[u] - 1.0 / rk1[u];
+    __syncthreads();
+    double x[CI], acc = 0.0;
 #pragma unroll
     for (int u = 0; u < CI; u++) {
-        const int64_t j = base + u * CT + threadIdx.x;
-        if (j < n) {
-            const double v = Mv[u] * (1.0 / rk[u] - 1.0 / rk1[u]);
-            x[j] = v;
-            acc += e.sign * v;
-        }
+        x[u] = (u == 0 ? before : nv[u > 0 ? u - 1 : 0]) * sh.tbuf[tile_slot(t * CI + u)];
+        if (base + (int64_t)t * CI + u < n) acc += x[u];
     }
-    esa_tile_sums(e, n, acc, lds, kg_.bid);
+    const double tot = tree_sum(acc, sh.d);           // (a barrier: every thread is past its reads of tbuf)
+    if (t == 0) p.c.tsumP[tile] = tot;
+    store_tile(p.xc, base, n, sh.tbuf, x);
 }
 };
 
-// phi[k] = -g[n-k] (k = 1..n) and phi[0] (cmc_utils.c:729); thread t handles node
-// k = t for k = 0..n+1 and also writes the packed (r, phi) node table and its every
-// MID_STEP-th entry, which the searches of set_velocities3 and the orbit phase read.
-struct phi_out_kernel {
-    static constexpr int LB = 1024, MB = 0;
-    static __device__ __forceinline__ void run(KGrid kg_, const double *__restrict__ r, double *__restrict__ phi, DevScalars *s, KParams P,
-                               const double *__restrict__ g, double2 *__restrict__ nodes, double2 *__restrict__ mid)
+struct pot_classify_c_kernel {
+    static constexpr int LB = CT, MB = 0;
+    static __device__ __forceinline__ void run(KGrid kg_, PotArgs p, int self_prefix)
 {
-    const int64_t k = (int64_t)kg_.bid * blockDim.x + threadIdx.x;
-    const int64_t n = s->n_max;
-    if (k > n + 1) return;
-    double p;
-    if (k == 0) {
-        // no stars: phi[1] is the sentinel 0
-        p = (n == 0 ? 0.0 : -g[n - 1]) + P.cenma_m * P.madhoc / r[1];
-        phi[0] = p;
-    } else if (k <= n) {
-        p = -g[n - k];
-        phi[k] = p;
-        if (isnan(p)) dev_set_error(s, CMCG_E_NAN, k);
-    } else {
-        p = 0.0;                                  // phi[n + 1], set with r[n + 1] by pot_setup
+    __shared__ ChainLds sh;
+    const int64_t n = p.s->n_max, tile = kg_.bid;
+    if (tile * CTILE >= n || p.flagged(3)) return;
+    double v[CI], pre_t, pre_t1;
+    fetch_tile(ArraySrc{p.xc}, tile * CTILE, n, v);
+    get_prefixes(p.c, tile, self_prefix, sh.d, &pre_t, &pre_t1);
+    classify_tile(p.c, v, tile, n, 0.0, pre_t, pre_t1, sh);
+}
+};
+
+struct pot_walk_c_kernel {
+    static constexpr int LB = CT, MB = 0;
+    static __device__ __forceinline__ void run(KGrid kg_, PotArgs p)
+{
+    __shared__ WalkLds sh;
+    if (p.flagged(3)) return;
+    Seg tot;
+    tot = walk_scan(p.c, (p.s->n_max + CTILE - 1) / CTILE, sh.s);
+    if (tot.cnt > RAW_CAP) {
+        if (threadIdx.x == 0) p.flag[3] = 1;
+        return;
     }
-    const double2 v = make_double2(r[k], p);
-    nodes[k] = v;
-    if (k % MID_STEP == 0) mid[k / MID_STEP] = v;
+    walk_list(p.c, tot.cnt, sh);
+    if (threadIdx.x < 64) pot_walk(tot.cnt, 0.0, sh.pre, sh.sx, p.c.s_v);
+}
+};
+
+// phi_k into the potential and the node tables, which the searches of set_velocities3 and
+// the orbit phase read
+__device__ __forceinline__ void put_node(const PotArgs &p, int64_t k, double r, double phi)
+{
+    const double2 v = make_double2(r, phi);
+    p.nodes[k] = v;
+    if (k % MID_STEP == 0) p.mid[k / MID_STEP] = v;
+}
+// nodes 0 (cmc_utils.c:729; phi1 = phi[1], the sentinel's 0 when there are no stars) and n + 1
+__device__ __forceinline__ void put_ends(const PotArgs &p, const KParams &P, int64_t n, double phi1)
+{
+    const double p0 = phi1 + P.cenma_m * P.madhoc / p.r[1];
+    p.phi[0] = p0;
+    put_node(p, 0, p.r[0], p0);
+    put_node(p, n + 1, CMCG_SF_INFINITY, 0.0);
+}
+
+// Chain C rebuilt and verified, phi_k = -w_k, k = N - j, and the node tables.
+struct pot_rebuild_c_kernel {
+    static constexpr int LB = CT, MB = 0;
+    static __device__ __forceinline__ void run(KGrid kg_, PotArgs p, KParams P)
+{
+    __shared__ ChainLds sh;
+    const int64_t n = p.s->n_max;
+    const int64_t tile = kg_.bid, base = tile * CTILE;
+    const int t = threadIdx.x;
+    if (p.flagged(4)) return;
+    if (n == 0 && kg_.bid == 0 && t == 0) put_ends(p, P, n, 0.0);
+    if (base >= n) return;
+    TileItems it;
+    double v[CI], rk[CI], nv[CI], before;
+    fetch_tile(ArraySrc{p.xc}, base, n, v);
+#pragma unroll
+    for (int u = 0; u < CI; u++) {
+        const int64_t j = base + u * CT + t;
+        rk[u] = j < n ? p.r[n - j] : 1.0;
+    }
+    const int64_t bad = rebuild_tile(p.c, v, tile, n, 0.0, 0.0, p.c.s_v, *p.c.s_n, sh, it, nv, &before);
+    if (bad < n) p.flag[4] = 1;
+    __syncthreads();                                  // tbuf free
+#pragma unroll
+    for (int u = 0; u < CI; u++) sh.tbuf[tile_slot(t * CI + u)] = nv[u];
+    __syncthreads();
+#pragma unroll
+    for (int u = 0; u < CI; u++) {
+        const int i = u * CT + t;
+        const int64_t k = n - (base + i);
+        if (k < 1) break;
+        const double ph = -sh.tbuf[tile_slot(i)];
+        p.phi[k] = ph;
+        if (isnan(ph)) dev_set_error(p.s, CMCG_E_NAN, k);
+        put_node(p, k, rk[u], ph);
+        if (k == 1) put_ends(p, P, n, ph);
+    }
+}
+};
+
+// The repair (a mass below zero, infinite or NaN, a list beyond RAW_CAP, a violated
+// recurrence: never an ordinary cluster; the test hook forces it): the three recurrences
+// themselves, one thread over chunks that the block stages through LDS.
+constexpr int FIX_CHUNK = 2 * WALK_T;
+struct pot_finish_kernel {
+    static constexpr int LB = WALK_T, MB = 0;
+    static __device__ __forceinline__ void run(KGrid kg_, PotArgs p, KParams P)
+{
+    __shared__ double x[FIX_CHUNK], y[FIX_CHUNK];
+    __shared__ double va, vm;
+    if (!p.flagged(5)) return;
+    const int64_t n = p.s->n_max;
+    const int t = threadIdx.x;
+    if (t == 0) va = 0.0;
+    for (int64_t c = 0; c < n; c += FIX_CHUNK) {
+        const int cnt = (int)(n - c < FIX_CHUNK ? n - c : FIX_CHUNK);
+        for (int i = t; i < cnt; i += WALK_T) x[i] = p.m[1 + c + i];
+        __syncthreads();
+        if (t == 0) {
+            double v = va;
+            for (int i = 0; i < cnt; i++) v = v + x[i];
+            va = v;
+        }
+        __syncthreads();
+    }
+    if (t == 0) {
+        pot_total(p, P, va);
+        vm = p.scal[1];
+        va = 0.0;
+    }
+    for (int64_t c = 0; c < n; c += FIX_CHUNK) {
+        const int cnt = (int)(n - c < FIX_CHUNK ? n - c : FIX_CHUNK);
+        for (int i = t; i < cnt; i += WALK_T) {
+            const int64_t k = n - (c + i);
+            x[i] = p.m[k] / p.nstar;
+            y[i] = 1.0 / p.r[k] - 1.0 / p.r[k + 1];
+        }
+        __syncthreads();
+        if (t == 0) {
+            double M = vm, w = va;
+            for (int i = 0; i < cnt; i++) {
+                w = w + M * y[i];
+                M = M - x[i];
+                y[i] = w;
+            }
+            vm = M;
+            va = w;
+        }
+        __syncthreads();
+        for (int i = t; i < cnt; i += WALK_T) {
+            const int64_t k = n - (c + i);
+            const double ph = -y[i];
+            p.phi[k] = ph;
+            if (isnan(ph)) dev_set_error(p.s, CMCG_E_NAN, k);
+            put_node(p, k, p.r[k], ph);
+        }
+        __syncthreads();
+    }
+    if (t == 0) put_ends(p, P, n, n > 0 ? -va : 0.0);
 }
 };
 
@@ -904,10 +1220,11 @@ hipError_t run_chain(const EsaArgs &e, int64_t n_ub, hipStream_t st, bool summed
 
 // The chains' per-tile and list buffers in the context's scratch (tile_sums: six
 // 8-byte words per tile).
-EsaArgs esa_args(const Scratch &sc, int slack)
+// set: 0 or 1, for two chains that are classified together
+EsaArgs esa_args(const Scratch &sc, int slack, int set = 0)
 {
-    double *tb = sc.tile_sums;
     const int64_t T = sc.max_tiles;
+    double *tb = sc.tile_sums + 6 * T * set;
     EsaArgs e{};
     e.slack = slack;
     e.tsumP = tb;
@@ -921,11 +1238,11 @@ EsaArgs esa_args(const Scratch &sc, int slack)
     e.s_v = sc.esa_v;
     e.s_n = sc.esa_n;
     e.smax = sc.esa_max;
-    e.raw_n = sc.esa_n + 1;
-    e.raw_idx = sc.esa_raw_idx;
-    e.raw_part = (int64_t *)sc.esa_raw_part;
-    e.raw_bp = (int32_t *)(sc.esa_raw_part + RAW_CAP);
-    e.raw_sx = sc.esa_raw_part + 2 * RAW_CAP;
+    e.raw_n = sc.esa_n + 1 + set;
+    e.raw_idx = sc.esa_raw_idx + RAW_CAP * set;
+    e.raw_part = (int64_t *)sc.esa_raw_part + 3 * RAW_CAP * set;
+    e.raw_bp = (int32_t *)(e.raw_part + RAW_CAP);
+    e.raw_sx = (double *)(e.raw_part + 2 * RAW_CAP);
     return e;
 }
 } // namespace
@@ -1048,43 +1365,48 @@ struct mpc_take_kernel {
 }
 };
 
+// count: N_MAX is to be counted from the radii (the step's sort has just left it)
 hipError_t launch_potential(const DevFields &f, DevScalars *s, const KParams &P, int64_t n_ub,
-                            const Scratch &sc, hipStream_t st)
+                            const Scratch &sc, hipStream_t st, bool count)
 {
-    int64_t ntiles = (n_ub + CTILE - 1) / CTILE + 1;
-    if (ntiles > sc.max_tiles) return hipErrorInvalidValue;
-    PotWork w;
-    w.xa = sc.chain_x;
-    w.ga = sc.chain_g;
-    w.Mk = sc.chain_mk;
-    w.scal = sc.chain_scal;
-    w.len = sc.chain_len;
-    w.fbad = sc.chain_fbad;
-    // a test hook widens the classification's error bound, which sends most elements
-    // through the fallback paths
-    const EsaArgs e = esa_args(sc, P.chain_k_drop);
-    const unsigned g1 = (unsigned)((n_ub + 256) / 256);
-    const dim3 gt((unsigned)(n_ub > 0 ? (n_ub + CTILE - 1) / CTILE : 1));
-    kl<pot_init_kernel>(dim3(1), dim3(1), 0, st, s);
-    if (n_ub > 0) kl<pot_count_kernel>(dim3(g1), dim3(256), 0, st, f.r, s);
-    kl<pot_setup_kernel>(dim3(1), dim3(1), 0, st, s, w, f.r, f.phi);
-    // chain A: total mass, straight over star_m[1..N]
-    EsaArgs ae = e;
-    ae.x = f.m + 1; ae.g = w.ga; ae.sign = 1.0; ae.v0p = w.scal + 0; ae.first_bad = w.fbad + 0; ae.Lp = w.len + 0;
-    if (hipError_t err = run_chain(ae, n_ub, st)) return err;
-    // chain B: enclosed mass, iterated directly in Mk (chain C's input)
-    EsaArgs be = e;
-    be.x = w.xa; be.g = w.Mk; be.sign = -1.0; be.v0p = w.scal + 1; be.first_bad = w.fbad + 2; be.Lp = w.len + 1;
-    kl<prep_b_kernel>(gt, dim3(CT), 0, st, f.m, s, (double)P.n_star, w.xa, P, (const double *)w.ga, w,
-                       be);
-    if (hipError_t err = run_chain(be, n_ub, st, true)) return err;
-    // chain C: w = -phi
-    EsaArgs ce = e;
-    ce.x = w.xa; ce.g = w.ga; ce.sign = 1.0; ce.v0p = w.scal + 0; ce.first_bad = w.fbad + 4; ce.Lp = w.len + 2;
-    kl<prep_c_kernel>(gt, dim3(CT), 0, st, f.r, s, (const double *)w.Mk, w.xa, ce);
-    if (hipError_t err = run_chain(ce, n_ub, st, true)) return err;
-    kl<phi_out_kernel>(dim3((unsigned)((n_ub + 2 + 255) / 256)), dim3(256), 0, st, f.r, f.phi, s, P,
-                       (const double *)w.ga, (double2 *)sc.nodes, (double2 *)sc.mid);
+    const int64_t ntiles = n_ub > 0 ? (n_ub + CTILE - 1) / CTILE : 1;
+    if (ntiles + 1 > sc.max_tiles) return hipErrorInvalidValue;
+    // a test hook widens the classification's error bound, which sends the chains through
+    // the repair
+    PotArgs p;
+    p.m = f.m; p.r = f.r; p.phi = f.phi; p.s = s;
+    p.nstar = (double)P.n_star;
+    p.xc = sc.chain_x;
+    p.scal = sc.chain_scal;
+    p.flag = sc.chain_fbad;
+    p.nodes = sc.nodes; p.mid = sc.mid;
+    p.counted = count;
+    p.a = esa_args(sc, P.chain_k_drop, 0);
+    p.b = esa_args(sc, P.chain_k_drop, 1);
+    p.a.sign = 1.0;
+    p.b.sign = -1.0;
+    p.c = p.a;                                       // A's tile sums and list are free when C needs its own
+    p.c.raw_n = sc.esa_n + 3;
+    p.a.s_n = sc.esa_n + 4; p.a.s_idx = sc.esa_idx + RAW_CAP;   // walked at the same time as B's
+    const dim3 gt((unsigned)ntiles), bt(CT);
+    const int self_prefix = ntiles <= SELF_PREFIX_MAX;
+    if (count) {
+        kl<pot_init_kernel>(dim3(1), dim3(1), 0, st, s);
+        if (n_ub > 0) kl<pot_count_kernel>(dim3((unsigned)((n_ub + 255) / 256)), dim3(256), 0, st, (const double *)f.r, s);
+    }
+    kl<pot_sums_kernel>(gt, bt, 0, st, p);
+    if (!self_prefix) {
+        kl<esa_tile_scan_kernel>(dim3(1), dim3(WALK_T), 0, st, p.a, ntiles);
+        kl<esa_tile_scan_kernel>(dim3(1), dim3(WALK_T), 0, st, p.b, ntiles);
+    }
+    kl<pot_classify_ab_kernel>(dim3((unsigned)(2 * ntiles)), bt, 0, st, p, P, self_prefix);
+    kl<pot_walk_ab_kernel>(dim3(1), dim3(2 * CT), 0, st, p, P);
+    kl<pot_rebuild_b_kernel>(gt, bt, 0, st, p);
+    if (!self_prefix) kl<esa_tile_scan_kernel>(dim3(1), dim3(WALK_T), 0, st, p.c, ntiles);
+    kl<pot_classify_c_kernel>(gt, bt, 0, st, p, self_prefix);
+    kl<pot_walk_c_kernel>(dim3(1), bt, 0, st, p);
+    kl<pot_rebuild_c_kernel>(gt, bt, 0, st, p, P);
+    kl<pot_finish_kernel>(dim3(1), dim3(WALK_T), 0, st, p, P);
     return hipGetLastError();
 }
 

@@ -43,9 +43,9 @@ __host__ __device__ constexpr int64_t ridx_tiles(int bits) { return (ridx_entrie
 struct Scratch {
     // potential chains: per-tile int128 sums and prefixes plus a boundary value
     // (48 B per tile), chain increments / iterates / enclosed masses per star
-    double *tile_sums;         // 6 words per tile (potential chains)
+    double *tile_sums;         // two sets of 6 words per tile (potential chains)
     int64_t max_tiles;
-    double *chain_x, *chain_g, *chain_mk;
+    double *chain_x, *chain_g;
     double *chain_scal;         // 4 doubles
     int64_t *chain_len;         // 4
     int64_t *chain_fbad;        // 6
@@ -53,8 +53,8 @@ struct Scratch {
     int64_t *esa_idx;
     double *esa_racc;           // regular sum before each listed element
     double *esa_v;
-    int64_t *esa_n;             // [0] sensitive count, [1] appended count, [2] two arrival counters
-    int64_t *esa_raw_idx;       // appended sensitive elements (unordered), 2048
+    int64_t *esa_n;             // [0] sensitive count, [1]..[3] appended counts, [4] the total mass chain's [0]
+    int64_t *esa_raw_idx;       // appended sensitive elements (unordered), 2048 for each set
     double *esa_raw_part;       // their in-tile regular sums (int64), binades (int32) and s x
     int64_t esa_max;
     // deterministic block partials: 8 doubles per block
@@ -108,7 +108,7 @@ struct Scratch {
 };
 
 hipError_t launch_potential(const DevFields &f, DevScalars *s, const KParams &P, int64_t n_ub,
-                            const Scratch &sc, hipStream_t st);
+                            const Scratch &sc, hipStream_t st, bool count = true);
 hipError_t launch_mass_percent(const DevFields &f, DevScalars *s, const KParams &P, int64_t n_ub, const Scratch &sc,
                                const double *pc, int count, int bh_include, double itm, double minimum_r,
                                void *out, hipStream_t st);
