@@ -60,22 +60,6 @@ struct cmcg_ctx {
     void *cen_buf = nullptr;     // cmcg_central_calculate results (allocated on first use)
 };
 
-// t[b][c][q][v] = XOR of the columns of matrix power b0 + b selected by nibble v at
-// bits 4q..4q+3 of state word c (the device's build_nibble_tables, done once here)
-template <int NB>
-static void fill_nibble_tables(const RngTable &ht, int b0, NibbleTables<NB> &nt)
-{
-    for (int b = 0; b < NB; b++)
-        for (int cc = 0; cc < 4; cc++)
-            for (int q = 0; q < 8; q++)
-                for (int v = 0; v < 16; v++) {
-                    uint32_t o = 0;
-                    for (int i = 0; i < 4; i++)
-                        if ((v >> i) & 1) o ^= ht.col[b0 + b][cc][4 * q + i];
-                    nt.t[b][cc][q][v] = o;
-                }
-}
-
 static void invalidate_graphs(cmcg_ctx *c)
 {
     for (auto &g : c->graph)
@@ -402,6 +386,79 @@ void noalloc_setup(int device)
 }
 }  // namespace
 
+// ---- the jump tables (JumpLevel) ----
+// Constants of the generator (2.9 MB): one allocation on each GPU, filled when the first
+// context is created there, read by every context's kernels and freed with the last one.
+
+namespace {
+JumpTables *g_jump_ptr[NOALLOC_MAX_DEVICES];
+int g_jump_users[NOALLOC_MAX_DEVICES];
+
+// t of one level: the unit's matrix `m` (columns), d = 0..63 of it by repeated products
+void fill_jump_level(const uint32_t m[4][32], JumpLevel *levels, int level)
+{
+    JumpLevel &L = levels[level];
+    const bool lanes = jump_over_lanes(level);
+    uint32_t col[4][32];
+    for (int c = 0; c < 4; c++)
+        for (int i = 0; i < 32; i++) col[c][i] = 1u << i;
+    for (int d = 0; d < 64; d++)
+        for (int c = 0; c < 4; c++) {
+            for (int q = 0; q < 8; q++)
+                for (int v = 0; v < 16; v++) {
+                    uint32_t o = 0;
+                    for (int i = 0; i < 4; i++)
+                        if ((v >> i) & 1) o ^= col[c][4 * q + i];
+                    L.t[jump_index(lanes, c, q, v, d)] = o;
+                }
+            for (int i = 0; i < 32; i++) col[c][i] = host_matvec(m[c], col[c][i]);
+        }
+}
+
+// With `device` current: its jump tables, filled for the first user (null: failed).
+const JumpTables *jump_acquire(int device, const RngTable &T)
+{
+    if (device < 0 || device >= NOALLOC_MAX_DEVICES) return nullptr;
+    std::lock_guard<std::mutex> lk(g_scratch_mu);
+    if (g_jump_ptr[device]) {
+        g_jump_users[device]++;
+        return g_jump_ptr[device];
+    }
+    auto h = std::make_unique<JumpTables>();
+    uint32_t m[4][32];
+    for (int k = 0; k < JL_PAIR_N; k++) {       // 3 64^k = 2^(6k) + 2^(6k + 1)
+        for (int c = 0; c < 4; c++)
+            for (int i = 0; i < 32; i++) m[c][i] = host_matvec(T.col[6 * k][c], T.col[6 * k + 1][c][i]);
+        fill_jump_level(m, h->level, JL_PAIR + k);
+    }
+    for (int k = 0; k < JL_SLOT_N; k++) fill_jump_level(T.col[20 + 6 * k], h->level, JL_SLOT + k);
+    fill_jump_level(T.col[66], h->level, JL_PHASE);
+    for (int k = 0; k < JL_STEP_N; k++)
+        if (72 + 6 * k < 128) fill_jump_level(T.col[72 + 6 * k], h->level, JL_STEP + k);
+    for (int b = 0; b < ORB_NIB_POWERS; b++)
+        for (int c = 0; c < 4; c++)
+            for (int q = 0; q < 8; q++)
+                for (int v = 0; v < 16; v++) h->orbit.t[b][c][q][v] = host_matvec(T.col[ORB_NIB_B0 + b][c], (uint32_t)v << (4 * q));
+    void *ptr = nullptr;
+    if (hipMalloc(&ptr, sizeof(JumpTables)) != hipSuccess) return nullptr;
+    if (hipMemcpy(ptr, h.get(), sizeof(JumpTables), hipMemcpyHostToDevice) != hipSuccess) {
+        hipFree(ptr);
+        return nullptr;
+    }
+    g_jump_users[device] = 1;
+    return g_jump_ptr[device] = (JumpTables *)ptr;
+}
+
+// ... and their end of use (the user's work on the device has ended)
+void jump_release(int device)
+{
+    std::lock_guard<std::mutex> lk(g_scratch_mu);
+    if (--g_jump_users[device] > 0) return;
+    hipFree(g_jump_ptr[device]);
+    g_jump_ptr[device] = nullptr;
+}
+}  // namespace
+
 int cmcg_create(cmcg_ctx **out, int device, int64_t n_cap, const cmcg_params *params)
 {
     if (!out || !params || n_cap < 1 || params->n_star < 1 || params->avekernel < 1) return CMCG_E_ARG;
@@ -435,7 +492,6 @@ int cmcg_create(cmcg_ctx **out, int device, int64_t n_cap, const cmcg_params *pa
     Scratch &sc = c->sc;
     sc.max_tiles = (n_cap + 2047) / 2048 + 1;
     sc.esa_max = 1 << 16;
-    sc.max_waves = (n_cap + 2) / 64 + 2;
     sc.max_blocks = (n_cap + 127) / 128 + 2;      // the smallest block of any launch shape: 128 threads
     if (sc.max_blocks < 1024) sc.max_blocks = 1024;   // the stripping passes' fixed grid
     const SortShape sort_max = sort_shape(n_cap);
@@ -457,9 +513,6 @@ int cmcg_create(cmcg_ctx **out, int device, int64_t n_cap, const cmcg_params *pa
         (e = dalloc(c, &sc.sort_order, 2 * (size_t)sc.sort_aos_cap)) ||
         (e = dalloc(c, &sc.mid, (size_t)(n_cap + 2) / MID_STEP + 4)) || (e = dalloc(c, &sc.nodes, (size_t)n_cap + 8)) || (e = dalloc(c, &sc.u_old, 2 * ((size_t)n_cap + 8))) ||
         (e = dalloc(c, &sc.merge_ends, (size_t)sc.merge_ends_cap)) || (e = dalloc(c, &sc.sv3_dpre, (size_t)n_cap + 6)) || (e = dalloc(c, &sc.dt_part, (size_t)64 * 16)) || (e = dalloc(c, &sc.coarse, (size_t)ORB_MAX_COARSE + 8)) || (e = dalloc(c, &sc.red2, (size_t)RED2_BLOCKS * 16)) ||
-        (e = dalloc(c, (char **)&sc.orb_nib, sizeof(NibbleTables<ORB_NIB_POWERS>))) ||
-        (e = dalloc(c, (char **)&sc.relax_nib, sizeof(NibbleTables<8>))) ||
-        (e = dalloc(c, (char **)&sc.wb_nib, 2 * sizeof(NibbleTables<RNG_WB_POWERS>))) ||
         (e = dalloc(c, &sc.vals_a, (size_t)n_cap + 4)) ||
         (e = dalloc(c, &sc.excess_c, (size_t)n_cap + 6)) || (e = dalloc(c, &sc.excess_list, (size_t)n_cap + 2)) ||
         (e = dalloc(c, &sc.sv3_wend, (size_t)n_cap + 2)) || (e = dalloc(c, &sc.sv3_merged, (size_t)n_cap + 2)) ||
@@ -469,7 +522,9 @@ int cmcg_create(cmcg_ctx **out, int device, int64_t n_cap, const cmcg_params *pa
         (e = dalloc(c, &sc.defer_list, (size_t)P.defer_cap)) || (e = dalloc(c, &sc.defer_kfirst, (size_t)P.defer_cap)) ||
         (e = dalloc(c, &sc.chain_scal, 4)) || (e = dalloc(c, &sc.chain_len, 4)) || (e = dalloc(c, &sc.chain_fbad, 8)) ||
         (e = dalloc(c, &sc.esa_idx, (size_t)sc.esa_max)) || (e = dalloc(c, &sc.esa_racc, (size_t)sc.esa_max)) ||
-        (e = dalloc(c, &sc.esa_v, (size_t)sc.esa_max)) || (e = dalloc(c, &sc.esa_n, 8)) || (e = dalloc(c, &sc.esa_raw_idx, 2 * 2048)) || (e = dalloc(c, &sc.esa_raw_part, 2 * 3 * 2048)) || (e = dalloc(c, &sc.rng_base, 2)) || (e = dalloc(c, &sc.rng_wave, (size_t)sc.max_waves)) || (e = dalloc(c, &sc.rng_seeded, 1)) ||
+        (e = dalloc(c, &sc.esa_v, (size_t)sc.esa_max)) || (e = dalloc(c, &sc.esa_n, 8)) ||
+        (e = dalloc(c, &sc.esa_raw_idx, 2 * 2048)) || (e = dalloc(c, &sc.esa_raw_part, 2 * 3 * 2048)) ||
+        (e = dalloc(c, &sc.rng_base, 3)) || (e = dalloc(c, &sc.rng_seeded, 1)) ||
         (e = dalloc(c, &c->T, 1))) {
         cmcg_destroy(c);
         return e;
@@ -477,25 +532,10 @@ int cmcg_create(cmcg_ctx **out, int device, int64_t n_cap, const cmcg_params *pa
     RngTable *ht = new RngTable;
     build_table(*ht);
     c->seeded = host_seed(params->seed);
-    // the orbit sampler's per-lane jumps by l 2^20 (l < 64): nibble tables of the
-    // matrix powers 2^20 .. 2^25, t[b][c][q][v] = column XOR for nibble v at bits 4q..
-    auto *nib = new NibbleTables<ORB_NIB_POWERS>;
-    fill_nibble_tables(*ht, ORB_NIB_B0, *nib);
-    // the relaxation's per-lane jumps by 3 l (l < 64): matrix powers 2^0 .. 2^7
-    auto *rnib = new NibbleTables<8>;
-    fill_nibble_tables(*ht, 0, *rnib);
-    // the wave-base jumps (offsets 3 t 2^6 and t 2^26 within a block)
-    auto *wnib = new NibbleTables<RNG_WB_POWERS>[2];
-    fill_nibble_tables(*ht, 6, wnib[0]);
-    fill_nibble_tables(*ht, 26, wnib[1]);
     bool ok = hipMemcpy(c->T, ht, sizeof(RngTable), hipMemcpyHostToDevice) == hipSuccess &&
-              hipMemcpy(sc.rng_seeded, &c->seeded, sizeof(Rng), hipMemcpyHostToDevice) == hipSuccess &&
-              hipMemcpy(sc.orb_nib, nib, sizeof(*nib), hipMemcpyHostToDevice) == hipSuccess &&
-              hipMemcpy(sc.relax_nib, rnib, sizeof(*rnib), hipMemcpyHostToDevice) == hipSuccess &&
-              hipMemcpy(sc.wb_nib, wnib, 2 * sizeof(NibbleTables<RNG_WB_POWERS>), hipMemcpyHostToDevice) == hipSuccess;
-    delete[] wnib;
-    delete rnib;
-    delete nib;
+              hipMemcpy(sc.rng_seeded, &c->seeded, sizeof(Rng), hipMemcpyHostToDevice) == hipSuccess;
+    if (ok) sc.jump = jump_acquire(device, *ht);
+    ok = ok && sc.jump;
     delete ht;
     if (!ok) { cmcg_destroy(c); return CMCG_E_HIP; }
     *out = c;
@@ -517,6 +557,7 @@ int cmcg_destroy(cmcg_ctx *c)
     if (c->flush_buf) hipFree(c->flush_buf);
     if (c->mpc_buf) hipFree(c->mpc_buf);
     if (c->cen_buf) hipFree(c->cen_buf);
+    if (c->sc.jump) jump_release(c->device);
     if (c->stream) hipStreamDestroy(c->stream);
     delete c;
     return CMCG_OK;
@@ -822,9 +863,9 @@ int cmcg_relax(cmcg_ctx *c, double dt, uint64_t step)
     {
         PhaseTimer t(c, "relax");
         kl<set_dt_step_kernel>(dim3(1), dim3(1), 0, c->stream, c->s, dt, (int64_t)step);
-        LAUNCH(launch_rng_bases(c->T, c->s, c->sc, c->stream));
+        LAUNCH(launch_rng_bases(c->s, c->sc, c->stream));
         LAUNCH(launch_sigma(c->f, c->s, c->kp, c->n_ub, c->stream));
-        LAUNCH(launch_relax(c->f, c->s, c->kp, c->T, c->sc, c->n_ub, c->stream));
+        LAUNCH(launch_relax(c->f, c->s, c->kp, c->sc, c->n_ub, c->stream));
     }
     return cmcg_sync(c);
 }
@@ -846,7 +887,7 @@ int cmcg_orbits(cmcg_ctx *c, uint64_t step, cmcg_orbit_stats *stats)
     {
         PhaseTimer t(c, "orbits");
         kl<set_dt_step_kernel>(dim3(1), dim3(1), 0, c->stream, c->s, __builtin_nan(""), (int64_t)step);
-        LAUNCH(launch_rng_bases(c->T, c->s, c->sc, c->stream));
+        LAUNCH(launch_rng_bases(c->s, c->sc, c->stream));
         hipEvent_t ka = nullptr, kb = nullptr;
         kernel_events(c, "orbits_kernel", ka, kb);
         LAUNCH(launch_orbits(c->f, c->s, c->kp, c->T, c->sc, c->n_ub, c->stream, c->learned ? &c->mlp : nullptr,
@@ -1058,12 +1099,12 @@ static int enqueue_step(cmcg_ctx *c, int64_t nub, bool graph)
         PhaseTimer t(c, "timestep");
         LAUNCH(launch_step_begin(c->s, c->stream));                 // also starts the time step's minimum
         // calc_sigma_r with simul_relax_new, then Dt and the RNG bases
-        LAUNCH(launch_timestep_sigma(c->f, c->s, c->kp, c->T, c->sc, nub, c->stream));
+        LAUNCH(launch_timestep_sigma(c->f, c->s, c->kp, c->sc, nub, c->stream));
     }
     {
         // relaxation with energy_conservation1 fused in
         PhaseTimer t(c, "relax");
-        LAUNCH(launch_relax(c->f, c->s, c->kp, c->T, c->sc, nub, c->stream, true, c->relax_threads));
+        LAUNCH(launch_relax(c->f, c->s, c->kp, c->sc, nub, c->stream, true, c->relax_threads));
         LAUNCH(launch_after_dynamics(c->s, c->stream));
     }
     {
@@ -1565,7 +1606,7 @@ int cmcg_rng_draws(cmcg_ctx *c, int phase, uint64_t step, int64_t first, int64_t
     double *d = nullptr;
     if (hipMalloc(&d, (size_t)count * ndraw * 8) != hipSuccess) return CMCG_E_NOMEM;
     int rc = CMCG_OK;
-    if (launch_rng_bases_step(c->T, c->s, c->sc, (int64_t)step, c->stream) ||
+    if (launch_rng_bases_step(c->s, c->sc, (int64_t)step, c->stream) ||
         launch_rng_draws(c->T, c->sc.rng_base, phase, first, count, ndraw, d, c->stream) ||
         hipMemcpyAsync(out, d, (size_t)count * ndraw * 8, hipMemcpyDeviceToHost, c->stream) || sync(c))
         rc = CMCG_E_HIP;
@@ -1766,7 +1807,7 @@ int cmcg_autotune(cmcg_ctx *c, int reps, int32_t *variant, int32_t *threads, int
         double total = 0.0;
         for (int it = 0; it <= reps; it++) {      // the first run warms up and is not timed
             hipEvent_t ea = it ? a : nullptr, eb = it ? b : nullptr;
-            if (launch_rng_bases(c->T, c->s, c->sc, c->stream) != hipSuccess ||
+            if (launch_rng_bases(c->s, c->sc, c->stream) != hipSuccess ||
                 launch_orbits(c->f, c->s, c->kp, c->T, c->sc, c->n_ub, c->stream, c->learned ? &c->mlp : nullptr,
                               c->margin, ea, eb, v, c->pred_fixed) != hipSuccess ||
                 sync(c) != hipSuccess) { rc = CMCG_E_HIP; break; }
@@ -1932,7 +1973,7 @@ int cmcg_autotune_relax(cmcg_ctx *c, int reps, int32_t *threads, double *ms_best
         double total = 0.0;
         for (int it = 0; it <= reps && !rc; it++) {      // the first run warms up and is not timed
             if (it && hipEventRecord(a, c->stream) != hipSuccess) { rc = CMCG_E_HIP; break; }
-            if (launch_relax(c->f, c->s, c->kp, c->T, c->sc, c->n_ub, c->stream, true, RELAX_SHAPES[v]) != hipSuccess) {
+            if (launch_relax(c->f, c->s, c->kp, c->sc, c->n_ub, c->stream, true, RELAX_SHAPES[v]) != hipSuccess) {
                 rc = CMCG_E_HIP;
                 break;
             }

@@ -119,97 +119,100 @@ __device__ __forceinline__ Rng rng_jump(const RngTable *__restrict__ T, Rng s, u
     return s;
 }
 
-// Block-cooperative jump: s advanced by 2^(row0 + k) steps for every k < nbits (<= 64)
-// with bit k of `bits` set.  Every thread of the block calls it (blockDim.x >= 128).
-// The block first stages the columns of those matrix powers in LDS (cols: 128 * nbits
-// words), then thread (c, i) = (t / 32, t % 32), t < 128, keeps word c of the state
-// and contributes column i of a power when bit i of the word is set: an XOR over the
-// 32 lanes is the product, and the chain of products never waits on memory.  The
-// four words advance independently.  res: an LDS slot for the result.
-__device__ __forceinline__ Rng rng_jump_block(const RngTable *__restrict__ T, Rng s, uint64_t bits, int row0,
-                                              int nbits, uint32_t *cols, Rng *res)
+// Jumps of a wave-uniform state.  Level L of the jump tables holds, for d = 0..63, the
+// GF(2) matrix of d U_L steps (U_L the level's unit), stored as its products with the 16
+// values v of every 4-bit piece q of state word c.  Over the lanes, d = lane, the tables
+// are t[c][q][v][d]: a jump is 32 coalesced loads and XORs, and no lookup waits on another
+// (through per-block LDS tables of single powers a lane's jump took six to eight dependent
+// rounds of 32 lookups: 192 to 256 LDS reads and about 1000 vector instructions a wave).
+// Offsets beyond 63 units take the next levels' digits (units grow by 64), the same for the
+// whole wave; those levels are t[d][c][q][v], 2 KB a digit.
+struct JumpLevel { uint32_t t[4 * 8 * 16 * 64]; };
+constexpr int JL_PAIR = 0, JL_PAIR_N = 6;       // units 3 64^k: relaxation pairs (k = 0 over the lanes)
+constexpr int JL_SLOT = 6, JL_SLOT_N = 6;       // units 2^20 64^k: orbit slots
+constexpr int JL_PHASE = 12;                    // unit 2^66: 16 of them from the pairs to the slots of a step
+constexpr int JL_STEP = 13, JL_STEP_N = 10;     // units 2^72 64^k: steps
+constexpr int JL_COUNT = JL_STEP + JL_STEP_N;
+__host__ __device__ constexpr bool jump_over_lanes(int level) { return level == JL_PAIR; }
+__host__ __device__ constexpr int jump_index(bool lanes, int c, int q, int v, int d)
 {
-    const int t = threadIdx.x;
-    const uint32_t *src = &T->col[row0][0][0];
-    for (int e = t; e < nbits * 128; e += blockDim.x)
-        if ((bits >> (e >> 7)) & 1ull) cols[e] = src[e];
-    __syncthreads();
-    if (t < 128) {
-        const int c = t >> 5, i = t & 31;
-        uint32_t z = c == 0 ? s.z0 : c == 1 ? s.z1 : c == 2 ? s.z2 : s.z3;
-        for (int k = 0; k < nbits; k++) {
-            if (!((bits >> k) & 1ull)) continue;
-            uint32_t v = cols[k * 128 + t] & (0u - ((z >> i) & 1u));
-#pragma unroll
-            for (int d = 16; d > 0; d >>= 1) v ^= __shfl_xor(v, d, 32);
-            z = v;
-        }
-        if (i == 0) {
-            if (c == 0) res->z0 = z;
-            else if (c == 1) res->z1 = z;
-            else if (c == 2) res->z2 = z;
-            else res->z3 = z;
-        }
-    }
-    __syncthreads();
-    const Rng out = *res;
-    __syncthreads();          // cols and res free again
-    return out;
+    return lanes ? ((c * 8 + q) * 16 + v) * 64 + d : ((d * 4 + c) * 8 + q) * 16 + v;
 }
 
-// In-wave jumps through LDS: for the NB matrix powers T^(2^b), b = b0..b0+NB-1, and
-// each state word, tab[b][c][q][v] is the product of the matrix with the nibble v
-// placed at bits 4q..4q+3, so a 32x32 GF(2) product is 8 table lookups.  Lanes of a
-// wave read 16 consecutive words per lookup: no bank conflicts.
-template <int NB>
-struct NibbleTables { uint32_t t[NB][4][8][16]; };
-
-template <int NB>
-__device__ void build_nibble_tables(const RngTable *__restrict__ T, int b0, NibbleTables<NB> &lt)
+// `lane` steps of the unit of a level over the lanes, from z (uniform over the wave)
+__device__ __forceinline__ Rng jump_digit(const JumpLevel &L, const Rng &z, uint32_t lane)
 {
-    for (int idx = threadIdx.x; idx < NB * 4 * 8 * 16; idx += blockDim.x) {
-        const int v = idx & 15, q = (idx >> 4) & 7, c = (idx >> 7) & 3, b = idx >> 9;
-        const uint32_t *col = T->col[b0 + b][c];
+    auto word = [&](int c, uint32_t x) {
         uint32_t o = 0;
-        for (int i = 0; i < 4; i++)
-            if ((v >> i) & 1) o ^= col[4 * q + i];
-        lt.t[b][c][q][v] = o;
-    }
-    __syncthreads();
-}
-
-// copy of tables built once per context (same contents as build_nibble_tables): 16-byte
-// loads, no column XORs per block
-template <int NB>
-__device__ void copy_nibble_tables(const NibbleTables<NB> *__restrict__ src, NibbleTables<NB> &lt)
-{
-    constexpr int NQ = (int)(sizeof(NibbleTables<NB>) / sizeof(uint4));
-    const uint4 *s4 = reinterpret_cast<const uint4 *>(src);
-    uint4 *d4 = reinterpret_cast<uint4 *>(&lt);
-    for (int q = threadIdx.x; q < NQ; q += blockDim.x) d4[q] = s4[q];
-    __syncthreads();
-}
-
-__device__ __forceinline__ uint32_t nib_matvec(const uint32_t (&tab)[8][16], uint32_t v)
-{
-    uint32_t o = 0;
 #pragma unroll
-    for (int q = 0; q < 8; q++) o ^= tab[q][(v >> (4 * q)) & 15u];
-    return o;
+        for (int q = 0; q < 8; q++) o ^= L.t[jump_index(true, c, q, (x >> (4 * q)) & 15u, lane)];
+        return o;
+    };
+    return Rng{word(0, z.z0), word(1, z.z1), word(2, z.z2), word(3, z.z3)};
 }
-
-// advance by off * 2^b0 steps, off < 2^NB
-template <int NB>
-__device__ __forceinline__ Rng rng_jump_lds(const NibbleTables<NB> &lt, Rng s, uint32_t off)
+__device__ __forceinline__ Rng rng_uniform(const Rng &z)
 {
-    for (int b = 0; b < NB; b++) {
+    auto u = [](uint32_t x) { return (uint32_t)__builtin_amdgcn_readfirstlane((int)x); };
+    return Rng{u(z.z0), u(z.z1), u(z.z2), u(z.z3)};
+}
+// A uniform jump by a whole wave (every lane active): lane 8 c + q looks up piece q of
+// word c, so it is one load and a XOR over eight lanes.  (As 32 scalar loads the compiler
+// waits for nearly each: 8 us a jump from cold caches.)
+__device__ __forceinline__ Rng jump_wave(const JumpLevel &L, const Rng &z, uint32_t d)
+{
+    const int i = threadIdx.x & 31, c = i >> 3, q = i & 7;
+    const uint32_t zc = c == 0 ? z.z0 : c == 1 ? z.z1 : c == 2 ? z.z2 : z.z3;
+    uint32_t o = L.t[jump_index(false, c, q, (zc >> (4 * q)) & 15u, d)];
+#pragma unroll
+    for (int m = 1; m < 8; m <<= 1) o ^= (uint32_t)__shfl_xor((int)o, m, 64);
+    auto word = [&](int lane) { return (uint32_t)__builtin_amdgcn_readlane((int)o, lane); };
+    return Rng{word(0), word(8), word(16), word(24)};
+}
+// the same for an offset w (uniform) of any number of digits
+__device__ __forceinline__ Rng jump_uniform(const JumpLevel *__restrict__ L, int levels, Rng z, uint64_t w)
+{
+    for (int k = 0; k < levels && w; k++, w >>= 6) {
+        const uint32_t d = (uint32_t)w & 63u;
+        if (d) z = jump_wave(L[k], z, d);
+    }
+    return z;
+}
+// The orbit sampler's lanes jump through LDS instead: for the matrix powers 2^20 .. 2^25
+// and each state word, t[b][c][q][v] is the product of the matrix with the value v of the
+// word's 4-bit piece q, so a 32x32 GF(2) product is 8 lookups.  The sampler waits on
+// gathers, not on these, while the table loads above evict its nodes from the L1 (1071 ->
+// 1172 us at N = 4e6), and as a pass before it they took 58 us.
+constexpr int ORB_NIB_B0 = 20, ORB_NIB_POWERS = 6;
+struct NibbleTables { uint32_t t[ORB_NIB_POWERS][4][8][16]; };
+__device__ __forceinline__ Rng rng_jump_lds(const NibbleTables &lt, Rng s, uint32_t off)
+{
+    auto matvec = [](const uint32_t (&tab)[8][16], uint32_t v) {
+        uint32_t o = 0;
+#pragma unroll
+        for (int q = 0; q < 8; q++) o ^= tab[q][(v >> (4 * q)) & 15u];
+        return o;
+    };
+    for (int b = 0; b < ORB_NIB_POWERS; b++) {
         if (!((off >> b) & 1u)) continue;
-        s.z0 = nib_matvec(lt.t[b][0], s.z0);
-        s.z1 = nib_matvec(lt.t[b][1], s.z1);
-        s.z2 = nib_matvec(lt.t[b][2], s.z2);
-        s.z3 = nib_matvec(lt.t[b][3], s.z3);
+        s.z0 = matvec(lt.t[b][0], s.z0);
+        s.z1 = matvec(lt.t[b][1], s.z1);
+        s.z2 = matvec(lt.t[b][2], s.z2);
+        s.z3 = matvec(lt.t[b][3], s.z3);
     }
     return s;
+}
+// what a device holds of them
+struct JumpTables {
+    JumpLevel level[JL_COUNT];
+    NibbleTables orbit;
+};
+
+// The state of the lane's pair: the wave's first is number 64 w after base.  Every lane of
+// the wave calls it.
+__device__ __forceinline__ Rng jump_lanes(const JumpLevel *__restrict__ L, int levels, const Rng &base, uint32_t w)
+{
+    const Rng z = jump_uniform(L + 1, levels - 1, rng_uniform(base), (uint32_t)__builtin_amdgcn_readfirstlane((int)w));
+    return jump_digit(L[0], z, threadIdx.x & 63u);
 }
 
 // Workgroups are dispatched round-robin over the 8 XCDs, each with its own L2.  This
@@ -383,7 +386,15 @@ __device__ __forceinline__ int64_t find_zero_Q(const double *__restrict__ r, con
     return find_zero_Q_n(SplitNodes{r, phi}, rj, mj, inv_nstar, kmin, kmax, E, J);
 }
 
-// cmc_orbit.c:722-740 set_a_b
+// cmc_orbit.c:722-740 set_a_b, from the interval's two nodes (k > 0)
+__device__ __forceinline__ void set_a_b_nodes(double rj, double mj, const KParams &P, double rk, double pk, double rk1,
+                                              double pk1, double *a, double *b)
+{
+    double Uk = pk + phi_s_own(rj, mj, P.inv_nstar, rk);
+    double Uk1 = pk1 + phi_s_own(rj, mj, P.inv_nstar, rk1);
+    *a = (Uk1 - Uk) / (1. / rk1 - 1. / rk);
+    *b = (Uk / rk1 - Uk1 / rk) / (1. / rk1 - 1. / rk);
+}
 template <class N>
 __device__ __forceinline__ void set_a_b_n(const N &nd, double rj, double mj, const KParams &P, int64_t k,
                                           double *a, double *b)
@@ -397,10 +408,7 @@ __device__ __forceinline__ void set_a_b_n(const N &nd, double rj, double mj, con
         double rk, pk, rk1, pk1;
         nd.RP(k, rk, pk);
         nd.RP(k + 1, rk1, pk1);
-        double Uk = pk + phi_s_own(rj, mj, P.inv_nstar, rk);
-        double Uk1 = pk1 + phi_s_own(rj, mj, P.inv_nstar, rk1);
-        *a = (Uk1 - Uk) / (1. / rk1 - 1. / rk);
-        *b = (Uk / rk1 - Uk1 / rk) / (1. / rk1 - 1. / rk);
+        set_a_b_nodes(rj, mj, P, rk, pk, rk1, pk1, a, b);
     }
 }
 __device__ __forceinline__ void set_a_b(const double *__restrict__ r, const double *__restrict__ phi,
@@ -566,24 +574,6 @@ __device__ __forceinline__ int64_t coarse_k(const Coarse &c, int s)
     return k < c.n1 ? k : c.n1;
 }
 
-// Index near radius x: the LDS sample interval holding x, then linear interpolation
-// in log r inside it (r is sorted; only an estimate, every use is verified).
-__device__ __forceinline__ int64_t coarse_index_estimate(const Coarse &c, double x)
-{
-    int a = 0, b = c.cs;
-    while (a < b) {
-        int m = (a + b + 1) >> 1;
-        if (c.cr[m] < x) a = m;
-        else b = m - 1;
-    }
-    if (a >= c.cs) return c.n1;
-    int64_t ka = coarse_k(c, a), kb = coarse_k(c, a + 1);
-    float la = __logf((float)c.cr[a]), lb = __logf((float)c.cr[a + 1]), lx = __logf((float)x);
-    float fr = lb > la ? (lx - la) / (lb - la) : 0.f;
-    fr = fr >= 0.f ? (fr > 1.f ? 1.f : fr) : 0.f;      // also maps NaN to 0
-    return ka + (int64_t)(fr * (float)(kb - ka));
-}
-
 // Largest t in [t0, t1] with eval(mid[t]) true, or t0 - 1 if there is none, for a
 // predicate that is true then false over [t0, t1].  eval also returns a key, negative
 // where the predicate holds, that varies smoothly with t; k_lo and k_hi are the keys
@@ -679,44 +669,37 @@ __device__ __forceinline__ double potential_at_coarse(const double *__restrict__
     return potential_at_coarse_n(SplitNodes{r, phi}, n_max, x, lo, hi, c, bad);
 }
 
-// potential(x) with the index search started from the radial index: one bucket read
-// gives a bracket of a few nodes (the answer is the unique largest k with r_k < x,
-// so any valid bracket gives the full-range search's index), then the caller's
-// bracket [lo, hi] (valid when r_lo < x <= r_hi) narrows it further.
-template <class N>
-__device__ __forceinline__ double potential_at_ridx_n(const N &nd, int64_t n_max, double x, int64_t lo, int64_t hi,
-                                                      const RIdx &ri, bool *bad, int32_t *k_out = nullptr)
+// potential(x) through the radial index: the node below x's bucket and the two after it
+// (one index word, then three node loads that do not wait for each other) hold the
+// interval unless the bucket holds more nodes, which a bisection up to the next bucket's
+// first node settles.  The interval is the unique largest i with r_i < x that the
+// full-range search returns.  r1: the innermost radius.
+__device__ __forceinline__ double potential_at_ridx(const double2 *__restrict__ nodes, int64_t n_max, double r1, double x,
+                                                    const RIdx &ri, bool *bad, int32_t *k_out)
 {
-    if (x == 0.0 || x < nd.R(1)) return potential_at_n(nd, n_max, x, lo, hi, bad, k_out);
-    int32_t a, b;
-    ridx_bracket(ri, x, a, b);
-    if (a > lo) lo = a;
-    if (b < hi) hi = b;
-    return potential_at_n(nd, n_max, x, lo, hi, bad, k_out);
-}
-
-// Narrow a find_zero_Q bracket [lo, hi] with pred(Q(lo)) true and pred(Q(hi)) false
-// (pred monotone over the bracket) to the mid-node interval holding the sign change.
-// q_lo, q_hi: Q at the bracket ends when known (they guide the first probes only).
-template <bool POSITIVE>
-__device__ __forceinline__ void mid_narrow_q(const Coarse &c, double rj, double mj, double inv, double E, double J,
-                                             int64_t &lo, int64_t &hi, double q_lo = 0.0, double q_hi = 0.0)
-{
-    if (!c.mid) return;
-    const int64_t t0 = (lo + MID_STEP) / MID_STEP, t1 = (hi - 1) / MID_STEP;
-    if (t0 > t1) return;
-    // key negative where the predicate holds: Q for Q < 0, -Q for Q > 0
-    double k_lo = POSITIVE ? -q_lo : q_lo, k_hi = POSITIVE ? -q_hi : q_hi;
-    if (!(k_lo < 0.0 && k_hi >= 0.0)) { k_lo = -1.0; k_hi = 1.0; }
-    const int64_t t = mid_search(c.mid, t0, t1, k_lo, k_hi, [&](double2 e, double &k) {
-        double q;
-        const int sg = q_sign(rj, mj, inv, e.x, e.y, E, J, &q);
-        k = POSITIVE ? -q : q;
-        return POSITIVE ? q_gt0(sg) : q_lt0(sg);
-    });
-    if (t < t0) { hi = MID_STEP * t0; return; }
-    lo = MID_STEP * t;
-    if (MID_STEP * (t + 1) < hi) hi = MID_STEP * (t + 1);
+    const PackedNodes nd{nodes};
+    if (x == 0.0 || x < r1) return potential_at_n(nd, n_max, x, 1, n_max + 1, bad, k_out);
+    const uint32_t b = ridx_bucket(ri, x);
+    int32_t i = (int32_t)ri.t[b];
+    const double2 *__restrict__ at = nodes + i;              // nodes holds two entries past n_max + 1
+    double2 u = at[0], v = at[1];
+    const double2 w = at[2];
+    if (!(i >= n_max || v.x >= x)) {
+        if (w.x >= x) {
+            i++;
+            u = v;
+            v = w;
+        } else {
+            const int32_t hi = (int32_t)ri.t[b + 1] + 1;
+            i = i + 2 >= hi - 1 ? i + 2 : (int32_t)find_zero_r_n(nd, i + 2, hi, x);
+            u = nodes[i];
+            v = nodes[i + 1];
+        }
+    }
+    *k_out = i;
+    if (u.x > x || v.x < x) { *bad = true; return 0.0; }
+    if (i == 0) return v.y;
+    return u.y + (v.y - u.y) * (1.0 / u.x - 1.0 / x) / (1.0 / u.x - 1.0 / v.x);
 }
 
 // A guess of the radius where Q changes sign between nodes (ra, pa) and (rb, pb),
@@ -750,50 +733,41 @@ __device__ __forceinline__ double interp_root(double ra, double pa, double rb, d
 // find_zero_Q's answer on a bracket [lo, hi] whose ends have the bisection's
 // predicate true and false (POSITIVE: the apocentre, predicate Q > 0; otherwise the
 // pericentre, Q < 0), for a Q with one sign change on the bracket: interpolation
-// steps (interp_root on the current bracket ends, turned into a node bracket by the
-// radial index and probed at its two ends) narrow it, then a bisection in the nodes
-// finishes.  Every index kept is a probed node, so the answer is the unique sign
-// change, the index the full-range bisection returns.  (rl, pl), (rh, ph): nodes lo
-// and hi.
-template <bool POSITIVE, class N>
-__device__ __forceinline__ int64_t ridx_zero_Q(const N &nd, const RIdx &ri, double rj, double mj, double inv,
-                                               double E, double J, int64_t lo, int64_t hi, double rl, double pl,
-                                               double rh, double ph)
+// steps (interp_root on the current bracket ends, turned into a node by the radial index,
+// that node and the two after it loaded together and probed in order) narrow it, then a
+// bisection in the nodes finishes.  Every index kept is a probed node, so the answer is
+// the unique sign change, the index the full-range bisection returns.  (rl, pl), (rh, ph):
+// nodes lo and hi on entry, nodes k and k + 1 of the answer k on return: the caller reads
+// no node again.  (The sampler is bound by the rate of such gathers, 64 lines to a wave's
+// load; probing the two ends of the index's bracket, with its ends and the answer's nodes
+// read for themselves, took about 12 a search, this about 5.)
+template <bool POSITIVE>
+__device__ __forceinline__ int64_t ridx_zero_Q(const double2 *__restrict__ nodes, const RIdx &ri, double rj, double mj,
+                                               double inv, double E, double J, int64_t lo, int64_t hi, double &rl,
+                                               double &pl, double &rh, double &ph)
 {
-    auto pred = [&](double r, double p) {
-        const int sg = q_sign(rj, mj, inv, r, p, E, J);
-        return POSITIVE ? q_gt0(sg) : q_lt0(sg);
-    };
     int32_t l = (int32_t)lo, h = (int32_t)hi;
-    for (int it = 0; it < 3 && h - l > 8; it++) {
+    // node k probed: true when the bracket's lower end moved to it
+    auto probe = [&](int32_t k, const double2 &v) {
+        const int sg = q_sign(rj, mj, inv, v.x, v.y, E, J);
+        const bool in = POSITIVE ? q_gt0(sg) : q_lt0(sg);
+        if (in) { l = k; rl = v.x; pl = v.y; }
+        else { h = k; rh = v.x; ph = v.y; }
+        return in;
+    };
+    for (int it = 0; it < 3 && h - l > 1; it++) {
         const double rg = interp_root(rl, pl, rh, ph, rj, mj, inv, E, J, !POSITIVE);
-        int32_t a, b;
+        int32_t a = l + ((h - l) >> 1);            // no usable guess: a bisection step
         if (rg > rl && rg < rh) {
-            ridx_bracket(ri, rg, a, b);
-            a = a < l ? l : (a > h ? h : a);
-            b = b > h ? h : (b < l ? l : b);
-        } else {
-            a = b = l + ((h - l) >> 1);        // no usable guess: a bisection step
+            const int32_t g = (int32_t)ri.t[ridx_bucket(ri, rg)];
+            a = g < l ? l : (g > h - 1 ? h - 1 : g);
         }
-        if (a > l && a < h) {
-            double r, p;
-            nd.RP(a, r, p);
-            if (pred(r, p)) { l = a; rl = r; pl = p; }
-            else { h = a; rh = r; ph = p; }
-        }
-        if (b > l && b < h) {
-            double r, p;
-            nd.RP(b, r, p);
-            if (pred(r, p)) { l = b; rl = r; pl = p; }
-            else { h = b; rh = r; ph = p; }
-        }
+        const double2 u = nodes[a], v = nodes[a + 1], w = nodes[a + 2];
+        if ((a == l || probe(a, u)) && a + 1 < h && probe(a + 1, v) && a + 2 < h) probe(a + 2, w);
     }
     while (h - l > 1) {
         const int32_t m = l + ((h - l) >> 1);
-        double r, p;
-        nd.RP(m, r, p);
-        if (pred(r, p)) l = m;
-        else h = m;
+        probe(m, nodes[m]);
     }
     return l;
 }
@@ -803,15 +777,15 @@ struct OrbitRS { double rp, ra, dQdrp, dQdra; int64_t kmin, kmax; int circular; 
 
 // cmc_orbit.c:413-540 calc_orbit_new after get_positive_Q_index has produced ktemp
 // (an index with Q > 0; ktemp < 0 means "no positive Q": circular orbit).
-// HAS_C: the LDS samples, radial index and learned proposal of Cr are available.  (A
-// template flag rather than a null test of a pointer: comparing the address of a
-// private object with null is not folded on this target and keeps the object in
+// HAS_C: the LDS samples, radial index and learned proposal of Cr are available, and pj is
+// phi at j.  (A template flag rather than a null test of a pointer: comparing the address
+// of a private object with null is not folded on this target and keeps the object in
 // scratch memory.)
 template <class N, bool HAS_C>
 __device__ __forceinline__ OrbitRS calc_orbit_core(const N &nd, const double *__restrict__ r,
                                                    const double *__restrict__ phi, int64_t n_max, int64_t j,
                                                    double rj, double mj, const KParams &P, double E, double J,
-                                                   int64_t ktemp, const Coarse &Cr)
+                                                   int64_t ktemp, const Coarse &Cr, double pj = 0.0)
 {
     OrbitRS o;
     o.brent = 0; o.linscan = 0; o.err = 0; o.hint_hits = 0; o.hint_misses = 0;
@@ -819,69 +793,71 @@ __device__ __forceinline__ OrbitRS calc_orbit_core(const N &nd, const double *__
         o.rp = o.ra = rj; o.kmin = o.kmax = j; o.dQdrp = o.dQdra = 0.0; o.circular = 1;
         return o;
     }
-    // Q is negative at the centre, positive on one interval around ktemp and negative
-    // far out (r^3 dPhi/dr = r M(r) increases), so the index bisection's result is
-    // the unique sign change of its bracket; the LDS samples narrow both brackets
-    // to one sample interval before the bisection in global memory.
-    int64_t kp_lo = 0, kp_hi = ktemp, ka_lo = ktemp, ka_hi = n_max + 1;
-    bool got_p = false, got_a = false;
-    bool vp = false, va = false;       // bracket ends checked: Q(lo), Q(hi) have the bisection's signs
-    double qp_lo = 0.0, qp_hi = 0.0, qa_lo = 0.0, qa_hi = 0.0;   // Q at sample ends (search guidance only)
-    if (HAS_C && Cr.hint) {
-        // learned proposals: the index range of the predicted apsis +- margin (in
-        // log r), padded by 2, accepted only when Q has the bisection's signs at its ends
+    int64_t kmin, kmax;
+    double rp0, pp0, rp1, pp1;         // nodes kmin, kmin + 1
+    double ra0, pa0, ra1, pa1;         // nodes kmax, kmax + 1
+    if constexpr (HAS_C) {
+        // Q is negative at the centre, positive on one interval around ktemp (= j here) and
+        // negative far out (r^3 dPhi/dr = r M(r) increases), so the index bisection's result
+        // is the unique sign change of its bracket; the LDS samples narrow both brackets
+        // to one sample interval before the interpolation search in global memory.
         const double inv = P.inv_nstar;
-        const float ep = __expf(Cr.margin);
-        // node index just below / at or above radius x: exact bounds from the radial
-        // index, estimates padded by two nodes from the LDS samples otherwise
-        auto below = [&](double x) -> int64_t {
-            if (Cr.ri.t) { int32_t a, b; ridx_bracket(Cr.ri, x, a, b); return a; }
-            return coarse_index_estimate(Cr, x) - 2;
-        };
-        auto above = [&](double x) -> int64_t {
-            if (Cr.ri.t) { int32_t a, b; ridx_bracket(Cr.ri, x, a, b); return b; }
-            return coarse_index_estimate(Cr, x) + 2;
-        };
-        int64_t lo = below((double)(__expf(Cr.lrp) / ep));
-        int64_t hi = above((double)(__expf(Cr.lrp) * ep));
-        lo = lo < 0 ? 0 : lo;
-        hi = hi > ktemp ? ktemp : hi;
-        if (lo < hi && q_lt0(q_sign(rj, mj, inv, nd.R(lo), nd.P(lo), E, J)) &&
-            (hi == ktemp || q_ge0(q_sign(rj, mj, inv, nd.R(hi), nd.P(hi), E, J)))) {
-            kp_lo = lo; kp_hi = hi; got_p = vp = true; o.hint_hits++;
-        } else {
-            o.hint_misses++;
-        }
-        lo = below((double)(__expf(Cr.lra) / ep));
-        hi = above((double)(__expf(Cr.lra) * ep));
-        lo = lo < ktemp ? ktemp : lo;
-        hi = hi > n_max + 1 ? n_max + 1 : hi;
-        if (lo < hi && (lo == ktemp || q_gt0(q_sign(rj, mj, inv, nd.R(lo), nd.P(lo), E, J))) &&
-            !q_gt0(q_sign(rj, mj, inv, nd.R(hi), nd.P(hi), E, J))) {
-            ka_lo = lo; ka_hi = hi; got_a = va = true; o.hint_hits++;
-        } else {
-            o.hint_misses++;
-        }
-    }
-    if (HAS_C) {
-        const double inv = P.inv_nstar;
-        // a verified learned bracket is narrowed by the LDS samples inside it: the
-        // sample bisection runs over those samples only
-        auto narrow = [&](int64_t &lo, int64_t &hi, bool positive) {
-            const int s0 = (int)(lo / Cr.stride) + 1, s1 = (int)((hi - 1) / Cr.stride);
-            if (s0 > s1 || s1 > Cr.cs) return;
-            int a = s0 - 1, b = s1;                    // sample a: predicate true (a = s0 - 1: node lo)
-            while (a < b) {
-                const int m = (a + b + 1) >> 1;
-                const int sg = q_sign(rj, mj, inv, Cr.cr[m], Cr.cphi[m], E, J);
-                if (positive ? q_gt0(sg) : q_lt0(sg)) a = m;
-                else b = m - 1;
+        int64_t kp_lo = 0, kp_hi = ktemp, ka_lo = ktemp, ka_hi = n_max + 1;
+        bool got_p = false, got_a = false;
+        bool vp = false, va = false;   // bracket ends checked: Q(lo), Q(hi) have the bisection's signs
+        rp1 = ra0 = rj;
+        pp1 = pa0 = pj;
+        if (Cr.hint) {
+            // learned proposals: the index range of the predicted apsis +- margin (in
+            // log r), accepted only when Q has the bisection's signs at its ends
+            const float ep = __expf(Cr.margin);
+            int32_t a, b;
+            ridx_bracket(Cr.ri, (double)(__expf(Cr.lrp) / ep), a, b);
+            int64_t lo = a < 0 ? 0 : a;
+            ridx_bracket(Cr.ri, (double)(__expf(Cr.lrp) * ep), a, b);
+            int64_t hi = b > ktemp ? ktemp : b;
+            if (lo < hi && q_lt0(q_sign(rj, mj, inv, nd.R(lo), nd.P(lo), E, J)) &&
+                (hi == ktemp || q_ge0(q_sign(rj, mj, inv, nd.R(hi), nd.P(hi), E, J)))) {
+                kp_lo = lo; kp_hi = hi; got_p = vp = true; o.hint_hits++;
+            } else {
+                o.hint_misses++;
             }
-            if (a >= s0) lo = coarse_k(Cr, a);
-            if (a < s1) hi = coarse_k(Cr, a + 1);
-        };
-        if (got_p) narrow(kp_lo, kp_hi, false);
-        if (got_a) narrow(ka_lo, ka_hi, true);
+            ridx_bracket(Cr.ri, (double)(__expf(Cr.lra) / ep), a, b);
+            lo = a < ktemp ? ktemp : a;
+            ridx_bracket(Cr.ri, (double)(__expf(Cr.lra) * ep), a, b);
+            hi = b > n_max + 1 ? n_max + 1 : b;
+            if (lo < hi && (lo == ktemp || q_gt0(q_sign(rj, mj, inv, nd.R(lo), nd.P(lo), E, J))) &&
+                !q_gt0(q_sign(rj, mj, inv, nd.R(hi), nd.P(hi), E, J))) {
+                ka_lo = lo; ka_hi = hi; got_a = va = true; o.hint_hits++;
+            } else {
+                o.hint_misses++;
+            }
+            // a verified learned bracket is narrowed by the LDS samples inside it: the
+            // sample bisection runs over those samples only
+            auto narrow = [&](int64_t &lo, int64_t &hi, bool positive) {
+                const int s0 = (int)(lo / Cr.stride) + 1, s1 = (int)((hi - 1) / Cr.stride);
+                if (s0 > s1 || s1 > Cr.cs) return;
+                int a = s0 - 1, b = s1;                    // sample a: predicate true (a = s0 - 1: node lo)
+                while (a < b) {
+                    const int m = (a + b + 1) >> 1;
+                    const int sg = q_sign(rj, mj, inv, Cr.cr[m], Cr.cphi[m], E, J);
+                    if (positive ? q_gt0(sg) : q_lt0(sg)) a = m;
+                    else b = m - 1;
+                }
+                if (a >= s0) lo = coarse_k(Cr, a);
+                if (a < s1) hi = coarse_k(Cr, a + 1);
+            };
+            if (got_p) {
+                narrow(kp_lo, kp_hi, false);
+                nd.RP(kp_lo, rp0, pp0);
+                nd.RP(kp_hi, rp1, pp1);
+            }
+            if (got_a) {
+                narrow(ka_lo, ka_hi, true);
+                nd.RP(ka_lo, ra0, pa0);
+                nd.RP(ka_hi, ra1, pa1);
+            }
+        }
         if (!got_p && ktemp >= 1 && q_lt0(q_sign(rj, mj, inv, Cr.cr[0], Cr.cphi[0], E, J))) {
             int a = 0, b = (int)((ktemp - 1) / Cr.stride);
             const int top = b;
@@ -891,51 +867,63 @@ __device__ __forceinline__ OrbitRS calc_orbit_core(const N &nd, const double *__
                 else b = m - 1;
             }
             kp_lo = coarse_k(Cr, a);
-            kp_hi = a < top ? coarse_k(Cr, a + 1) : ktemp;
+            rp0 = Cr.cr[a];
+            pp0 = Cr.cphi[a];
+            if (a < top) {
+                kp_hi = coarse_k(Cr, a + 1);
+                rp1 = Cr.cr[a + 1];
+                pp1 = Cr.cphi[a + 1];
+            }
             vp = true;
-            (void)q_sign(rj, mj, inv, Cr.cr[a], Cr.cphi[a], E, J, &qp_lo);
-            if (a < top) (void)q_sign(rj, mj, inv, Cr.cr[a + 1], Cr.cphi[a + 1], E, J, &qp_hi);
         }
         const int sb = (int)(ktemp / Cr.stride) + 1;
         if (!got_a && sb <= Cr.cs && !q_gt0(q_sign(rj, mj, inv, Cr.cr[Cr.cs], Cr.cphi[Cr.cs], E, J))) {
             va = true;
-            if (!q_gt0(q_sign(rj, mj, inv, Cr.cr[sb], Cr.cphi[sb], E, J))) {
-                ka_hi = coarse_k(Cr, sb);
-            } else {
-                int a = sb, b = Cr.cs - 1;
-                while (a < b) {
-                    int m = (a + b + 1) >> 1;
-                    if (q_gt0(q_sign(rj, mj, inv, Cr.cr[m], Cr.cphi[m], E, J))) a = m;
-                    else b = m - 1;
-                }
+            int a = sb - 1, b = Cr.cs - 1;                 // sample a: Q > 0 (a = sb - 1: node ktemp)
+            while (a < b) {
+                int m = (a + b + 1) >> 1;
+                if (q_gt0(q_sign(rj, mj, inv, Cr.cr[m], Cr.cphi[m], E, J))) a = m;
+                else b = m - 1;
+            }
+            if (a >= sb) {
                 ka_lo = coarse_k(Cr, a);
-                ka_hi = coarse_k(Cr, a + 1);
-                (void)q_sign(rj, mj, inv, Cr.cr[a], Cr.cphi[a], E, J, &qa_lo);
-                (void)q_sign(rj, mj, inv, Cr.cr[a + 1], Cr.cphi[a + 1], E, J, &qa_hi);
+                ra0 = Cr.cr[a];
+                pa0 = Cr.cphi[a];
+            }
+            ka_hi = coarse_k(Cr, a + 1);
+            ra1 = Cr.cr[a + 1];
+            pa1 = Cr.cphi[a + 1];
+        }
+        // verified brackets: interpolation search through the radial index; otherwise the
+        // full-range bisection (which also settles the direction itself)
+        const double2 *nodes = nd.rp;
+        if (vp) {
+            kmin = ridx_zero_Q<false>(nodes, Cr.ri, rj, mj, inv, E, J, kp_lo, kp_hi, rp0, pp0, rp1, pp1);
+        } else {
+            kmin = find_zero_Q_n(nd, rj, mj, inv, kp_lo, kp_hi, E, J);
+            if (kmin >= 0) {
+                nd.RP(kmin, rp0, pp0);
+                nd.RP(kmin + 1, rp1, pp1);
             }
         }
-    }
-    // verified brackets: interpolation search through the radial index; otherwise the
-    // middle table and a bisection (which also settles the direction itself)
-    const bool ri = HAS_C && Cr.ri.t;
-    int64_t kmin, kmax;
-    if (ri && vp) {
-        double rl, pl, rh, ph;
-        nd.RP(kp_lo, rl, pl);
-        nd.RP(kp_hi, rh, ph);
-        kmin = ridx_zero_Q<false>(nd, Cr.ri, rj, mj, P.inv_nstar, E, J, kp_lo, kp_hi, rl, pl, rh, ph);
+        if (va) {
+            kmax = ridx_zero_Q<true>(nodes, Cr.ri, rj, mj, inv, E, J, ka_lo, ka_hi, ra0, pa0, ra1, pa1);
+        } else {
+            kmax = find_zero_Q_n(nd, rj, mj, inv, ka_lo, ka_hi, E, J);
+            if (kmax >= 0) {
+                nd.RP(kmax, ra0, pa0);
+                nd.RP(kmax + 1, ra1, pa1);
+            }
+        }
     } else {
-        if (vp && HAS_C) mid_narrow_q<false>(Cr, rj, mj, P.inv_nstar, E, J, kp_lo, kp_hi, qp_lo, qp_hi);
-        kmin = find_zero_Q_n(nd, rj, mj, P.inv_nstar, kp_lo, kp_hi, E, J);
-    }
-    if (ri && va) {
-        double rl, pl, rh, ph;
-        nd.RP(ka_lo, rl, pl);
-        nd.RP(ka_hi, rh, ph);
-        kmax = ridx_zero_Q<true>(nd, Cr.ri, rj, mj, P.inv_nstar, E, J, ka_lo, ka_hi, rl, pl, rh, ph);
-    } else {
-        if (va && HAS_C) mid_narrow_q<true>(Cr, rj, mj, P.inv_nstar, E, J, ka_lo, ka_hi, qa_lo, qa_hi);
-        kmax = find_zero_Q_n(nd, rj, mj, P.inv_nstar, ka_lo, ka_hi, E, J);
+        kmin = find_zero_Q_n(nd, rj, mj, P.inv_nstar, 0, ktemp, E, J);
+        kmax = find_zero_Q_n(nd, rj, mj, P.inv_nstar, ktemp, n_max + 1, E, J);
+        if (kmin >= 0 && kmax >= 0) {
+            nd.RP(kmin, rp0, pp0);
+            nd.RP(kmin + 1, rp1, pp1);
+            nd.RP(kmax, ra0, pa0);
+            nd.RP(kmax + 1, ra1, pa1);
+        }
     }
     if (kmin < 0 || kmax < 0) {
         o.err = CMCG_E_BRACKET;
@@ -944,11 +932,12 @@ __device__ __forceinline__ OrbitRS calc_orbit_core(const N &nd, const double *__
     }
     double a, b, rmin, rmax, inside_sqrt;
     bool bad = false;
-    set_a_b_n(nd, rj, mj, P, kmin, &a, &b);
+    if (kmin == 0) set_a_b_n(nd, rj, mj, P, 0, &a, &b);
+    else set_a_b_nodes(rj, mj, P, rp0, pp0, rp1, pp1, &a, &b);
     inside_sqrt = a * a - 2.0 * J * J * (b - E);
     if (inside_sqrt < 0.0) {
         rmin = -1.0 * J * J / a;
-        if ((rmin < nd.R(kmin)) || (rmin > nd.R(kmin + 1))) {
+        if ((rmin < rp0) || (rmin > rp1)) {
             const RootVr rv = find_root_vr(r, phi, rj, mj, P.inv_nstar, P.cenma_m * P.madhoc, kmin, E, J);
             rmin = rv.root;
             bad |= rv.bad != 0;
@@ -958,11 +947,12 @@ __device__ __forceinline__ OrbitRS calc_orbit_core(const N &nd, const double *__
         rmin = J * J / (-a + sqrt(inside_sqrt));
     }
     double dQdr_min = 2.0 * J * J / (rmin * rmin * rmin) + 2.0 * a / (rmin * rmin);
-    set_a_b_n(nd, rj, mj, P, kmax, &a, &b);
+    if (kmax == 0) set_a_b_n(nd, rj, mj, P, 0, &a, &b);
+    else set_a_b_nodes(rj, mj, P, ra0, pa0, ra1, pa1, &a, &b);
     inside_sqrt = a * a - 2.0 * J * J * (b - E);
     if (inside_sqrt < 0.0) {
         rmax = -a / (2.0 * (b - E));
-        if ((rmax < nd.R(kmax)) || (rmax > nd.R(kmax + 1))) {
+        if ((rmax < ra0) || (rmax > ra1)) {
             const RootVr rv = find_root_vr(r, phi, rj, mj, P.inv_nstar, P.cenma_m * P.madhoc, kmax, E, J);
             rmax = rv.root;
             bad |= rv.bad != 0;

@@ -12,9 +12,11 @@
 // thread would stall the whole phase, so such stars are deferred: a grid-wide
 // search finds the same first positive index, and a tail kernel finishes them.
 //
-// The phase is bound by dependent gathers into the sorted (r, phi) table (16 B per
-// probe, ~(2 + tries) * log2 N probes per star), which at N = 4e6 is 64 MB and lives
-// in L2/MALL; the compulsory HBM traffic is 96 B/star.
+// The phase is bound by the rate of gathers into the sorted (r, phi) table (16 B a node,
+// a line each: about 5 a search and 4 a try), which at N = 4e6 is 64 MB and lives in
+// L2/MALL, by their latency and by the FP64 work of the exact apsides and tries; the
+// compulsory HBM traffic is 96 B/star.  Sampler at N = 4e6: 1071 us with about 12 gathers
+// a search and 6 a try (71 load instructions a wave), 873 now.
 #include "kernels.hpp"
 
 namespace {
@@ -177,8 +179,7 @@ __device__ void sample_star(const N &nd, const DevFields &f, DevScalars *s, cons
 
 // what a star's tries need (set by prepare_star)
 struct TryCtx {
-    double rmin, rmax, F, E, J, rj, mj, r_lo0, r_hi0;
-    int64_t lo0, hi0;
+    double rmin, rmax, F, E, J, rj, mj;
 };
 
 // result of a star's tries
@@ -209,10 +210,10 @@ __device__ __forceinline__ int nth_set_bit(uint64_t m, int q)
 template <class N>
 __device__ __forceinline__ bool prepare_star(const N &nd, const DevFields &f, DevScalars *s, const KParams &P,
                                              const Coarse &C, int64_t n, int64_t j, double rj, double mj,
-                                             double E, double J, int64_t ktemp, int &flags, int &hits, int &misses,
+                                             double E, double J, double pj, int &flags, int &hits, int &misses,
                                              TryCtx &tc)
 {
-    OrbitRS o = calc_orbit_core<N, true>(nd, f.r, f.phi, n, j, rj, mj, P, E, J, ktemp, C);
+    OrbitRS o = calc_orbit_core<N, true>(nd, f.r, f.phi, n, j, rj, mj, P, E, J, j, C, pj);
     if (o.err) dev_set_error(s, o.err, j);
     hits = o.hint_hits;
     misses = o.hint_misses;
@@ -236,17 +237,13 @@ __device__ __forceinline__ bool prepare_star(const N &nd, const DevFields &f, De
     const double g2 = sqrt(-3.0 * (tc.rmax - tc.rmin) / o.dQdra);
     tc.F = 1.2 * (g1 >= g2 ? g1 : g2);
     tc.E = E; tc.J = J; tc.rj = rj; tc.mj = mj;
-    tc.lo0 = o.kmin < 1 ? 1 : o.kmin;
-    tc.hi0 = o.kmax + 1 > n + 1 ? n + 1 : o.kmax + 1;
-    tc.r_lo0 = nd.R(tc.lo0);
-    tc.r_hi0 = nd.R(tc.hi0);
     return true;
 }
 
 // One try (cmc_evolution_thr.c:862-886) from the state at its first draw; on return
 // st is the state after the try's two draws.
-template <class N>
-__device__ __forceinline__ bool one_try(const N &nd, const Coarse &C, const KParams &P, int64_t n, const TryCtx &tc,
+__device__ __forceinline__ bool one_try(const double2 *__restrict__ nodes, const RIdx &ri, double r1, const KParams &P,
+                                        int64_t n, const TryCtx &tc,
                                         Rng &st, double &X, double &rr, double &vr, double &potr, int32_t &kn,
                                         bool &bad, bool &nan)
 {
@@ -254,11 +251,7 @@ __device__ __forceinline__ bool one_try(const N &nd, const Coarse &C, const KPar
     const double s0 = 2.0 * X - 1.0;
     const double g0 = tc.F * rng_dbl(st);
     rr = 0.5 * (tc.rmin + tc.rmax) + 0.25 * (tc.rmax - tc.rmin) * (3.0 * s0 - s0 * s0 * s0);
-    int64_t lo = tc.lo0, hi = tc.hi0;
-    if (!(tc.r_lo0 < rr)) lo = 1;
-    if (!(rr <= tc.r_hi0)) hi = n + 1;
-    potr = C.ri.t ? potential_at_ridx_n(nd, n, rr, lo, hi, C.ri, &bad, &kn)
-                  : potential_at_coarse_n(nd, n, rr, lo, hi, C, &bad, &kn);
+    potr = potential_at_ridx(nodes, n, r1, rr, ri, &bad, &kn);
     const double pot = potr + phi_s_own(tc.rj, tc.mj, P.inv_nstar, rr);
     const double drds = 0.25 * (tc.rmax - tc.rmin) * (3.0 - 3.0 * s0 * s0);
     const double Q = 2.0 * tc.E - 2.0 * pot - tc.J * tc.J / rr / rr;
@@ -274,8 +267,8 @@ __device__ __forceinline__ bool one_try(const N &nd, const Coarse &C, const KPar
 // All lanes of the wave call this together (convergent).  need: this lane's star
 // samples; wctx: the wave's 64 try constants in LDS (slot = lane, written before a
 // block barrier); rng: this lane's substream state before its star's first try.
-template <int CAP, class N>
-__device__ void wave_tries(const N &nd, const Coarse &C, const KParams &P, int64_t n, bool need,
+template <int CAP>
+__device__ void wave_tries(const double2 *__restrict__ nodes, const RIdx &ri, const KParams &P, int64_t n, bool need,
                            const TryCtx *__restrict__ wctx, Rng rng, TryOut &out)
 {
     const int lane = threadIdx.x & 63;
@@ -283,6 +276,7 @@ __device__ void wave_tries(const N &nd, const Coarse &C, const KParams &P, int64
     bool bad_acc = false;
     out.k = 0; out.bad = false; out.nan = false; out.kn = 0;
     out.X = out.rr = out.vr = out.potr = 0.0;
+    const double r1 = nodes[1].x;
     uint64_t pending = __ballot(need);
     while (pending) {
         const int R = __popcll(pending);
@@ -304,7 +298,7 @@ __device__ void wave_tries(const N &nd, const Coarse &C, const KParams &P, int64
         int32_t kn = 0;
         bool bad = false, nan = false, term = false;
         if (eval) {
-            term = one_try(nd, C, P, n, t, st, X, rr, vr, potr, kn, bad, nan);
+            term = one_try(nodes, ri, r1, P, n, t, st, X, rr, vr, potr, kn, bad, nan);
             Rng sg = st;
             if (term && !nan && rng_dbl(sg) < 0.5) vr = -vr;    // sign draw after the accepted try
         }
@@ -352,32 +346,32 @@ __device__ void wave_tries(const N &nd, const Coarse &C, const KParams &P, int64
     }
 }
 
-// Slot j draws from offset j 2^20; the wave's first slot starts at the per-wave state
-// and lane l jumps l 2^20 (l < 2^6) through the LDS tables.  With learned brackets
-// the network's prediction proposes both find_zero_Q brackets.
-// MINB: blocks per CU the register allocation must allow (1: no constraint; 1024 /
-// THREADS: four waves per SIMD, at the cost of some spilled registers)
+// Slot j draws from offset j 2^20 (base[2]: the state of slot 1): the wave jumps to its
+// first slot, its lanes on through the LDS tables.  With learned brackets the network's
+// prediction proposes both find_zero_Q brackets.
+// MINB: blocks per CU the register allocation must allow (1: no constraint; 5 blocks of 256
+// threads: five waves per SIMD, 96 registers)
 template <int THREADS, int COARSE, int CAP, int MINB>
 struct orbits_kernel {
     static constexpr int LB = THREADS, MB = MINB;
     static __device__ __forceinline__ void run(KGrid kg_, DevFields f, DevScalars *s, KParams P,
-                                                             const RngTable *__restrict__ T,
-                                                             const Rng *__restrict__ wave_base,
+                                                             const JumpTables *__restrict__ jump,
+                                                             const Rng *__restrict__ base,
                                                              double *__restrict__ partials,
                                                              int64_t *__restrict__ defer_list,
                                                              const float2 *__restrict__ pred, float margin,
                                                              const double2 *__restrict__ mid,
                                                              const double2 *__restrict__ nodes,
                                                              const double2 *__restrict__ coarse,
-                                                             const NibbleTables<ORB_NIB_POWERS> *__restrict__ nib,
                                                              const uint32_t *__restrict__ ridx, int ridx_bits)
 {
     // the jump tables are needed only for the lanes' first states, the try constants
     // only after the apsides: one LDS area serves both
     __shared__ union alignas(16) Share {
-        NibbleTables<ORB_NIB_POWERS> lt;
+        NibbleTables lt;
         TryCtx ctx[THREADS];
     } sh;
+    TryCtx *const ctx = sh.ctx;
     __shared__ double cr[COARSE + 1], cphi[COARSE + 1];
     const int64_t n = s->n_max;
     Coarse C;
@@ -386,23 +380,24 @@ struct orbits_kernel {
     C.hint = false; C.lrp = C.lra = 0.f; C.margin = margin;
     C.mid = mid;
     C.ri.t = nullptr;
-    if (ridx && n >= 1) C.ri = ridx_of(ridx, nodes, n, ridx_bits);
-    // both tables are built once per phase: contiguous copies
+    if (n >= 1) C.ri = ridx_of(ridx, nodes, n, ridx_bits);
+    // built once per phase: a contiguous copy
     for (int sI = threadIdx.x; sI <= COARSE; sI += blockDim.x) {
         const double2 v = coarse[sI];
         cr[sI] = v.x;
         cphi[sI] = v.y;
     }
     {
-        constexpr int NQ = (int)(sizeof(NibbleTables<ORB_NIB_POWERS>) / sizeof(uint4));
-        const uint4 *src = reinterpret_cast<const uint4 *>(nib);
+        constexpr int NQ = (int)(sizeof(NibbleTables) / sizeof(uint4));
+        const uint4 *src = reinterpret_cast<const uint4 *>(&jump->orbit);
         uint4 *dst = reinterpret_cast<uint4 *>(&sh.lt);
         for (int q = threadIdx.x; q < NQ; q += blockDim.x) dst[q] = src[q];
     }
-    __syncthreads();
     const int64_t j = 1 + xcd_block(kg_) * blockDim.x + threadIdx.x;
-    Rng rng{};
-    if (j <= n) rng = rng_jump_lds<ORB_NIB_POWERS>(sh.lt, wave_base[(j - 1) >> 6], (uint32_t)((j - 1) & 63));
+    Rng rng = jump_uniform(jump->level + JL_SLOT + 1, JL_SLOT_N - 1, rng_uniform(base[2]),
+                           (uint32_t)__builtin_amdgcn_readfirstlane((int)((j - 1) >> 6)));
+    __syncthreads();
+    rng = rng_jump_lds(sh.lt, rng, (uint32_t)((j - 1) & 63));
     __syncthreads();                           // the tables are dead from here
     bool need = false;
     int flags = 0, ntry = 0, hits = 0, misses = 0;
@@ -421,7 +416,8 @@ struct orbits_kernel {
             f.rnew[j] = CMCG_SF_INFINITY; f.vrnew[j] = 0.0; f.vtnew[j] = 0.0; f.knew[j] = -1;
             flags = CMCG_SF_REMOVED_E;
         } else {
-            if (q_le0(q_sign(rj, mj, P.inv_nstar, rj, f.phi[j], E, J))) {
+            const double pj = f.phi[j];
+            if (q_le0(q_sign(rj, mj, P.inv_nstar, rj, pj, E, J))) {
                 // linear-scan case: finished by the deferred path
                 flags = CMCG_SF_LINSCAN;
                 unsigned long long slot = atomicAdd((unsigned long long *)&s->n_defer, 1ull);
@@ -434,20 +430,20 @@ struct orbits_kernel {
                     C.lrp = y.x;
                     C.lra = y.y;
                 }
-                need = prepare_star(PackedNodes{nodes}, f, s, P, C, n, j, rj, mj, E, J, j, flags, hits, misses,
-                                    sh.ctx[threadIdx.x]);
+                need = prepare_star(PackedNodes{nodes}, f, s, P, C, n, j, rj, mj, E, J, pj, flags, hits, misses,
+                                    ctx[threadIdx.x]);
             }
         }
     }
     __syncthreads();                           // try constants visible to the wave
     // every lane of the wave takes part, stars or not
     TryOut to;
-    wave_tries<CAP>(PackedNodes{nodes}, C, P, n, need, sh.ctx + (threadIdx.x & ~63), rng, to);
+    wave_tries<CAP>(nodes, C.ri, P, n, need, ctx + (threadIdx.x & ~63), rng, to);
     double red[NRED];
     for (int i = 0; i < NRED; i++) red[i] = 0.0;
     if (j <= n) {
         if (need) {
-            const TryCtx &tc = sh.ctx[threadIdx.x];
+            const TryCtx &tc = ctx[threadIdx.x];
             if (to.bad) dev_set_error(s, CMCG_E_BRACKET, j);
             if (to.nan) dev_set_error(s, CMCG_E_NAN, j);
             else if (to.k == CMCG_N_TRY + 1) dev_set_error(s, CMCG_E_NTRY, j);
@@ -858,28 +854,29 @@ struct coarse_build_kernel {
 // Launch shapes of the orbit sampler that the autotuner chooses from: threads per
 // block, LDS samples of the (r, phi) table, and the most lanes one star's tries get
 // in a round (64: all idle lanes; fewer: less speculative work).  Every variant gives
-// the same stars; only the block order of the escape sums differs.  (Asking the
-// compiler for 5 waves per SIMD instead of 4 spills about 100 VGPRs and ran 40%
-// slower.)
-using OrbFn = void (*)(dim3, dim3, hipStream_t, DevFields, DevScalars *, KParams, const RngTable *, const Rng *,
-                       double *, int64_t *, const float2 *, float, const double2 *, const double2 *, const double2 *,
-                       const NibbleTables<ORB_NIB_POWERS> *, const uint32_t *, int);
+// the same stars; only the block order of the escape sums differs.
+using OrbFn = void (*)(dim3, dim3, hipStream_t, DevFields, DevScalars *, KParams, const JumpTables *,
+                       const Rng *, double *, int64_t *, const float2 *, float, const double2 *, const double2 *, const double2 *,
+                       const uint32_t *, int);
 template <int THREADS, int COARSE, int CAP, int MINB>
-void orbits_launch(dim3 g, dim3 b, hipStream_t st, DevFields f, DevScalars *s, KParams P, const RngTable *T,
-                   const Rng *wb, double *partials, int64_t *defer, const float2 *pred, float margin,
+void orbits_launch(dim3 g, dim3 b, hipStream_t st, DevFields f, DevScalars *s, KParams P, const JumpTables *jump,
+                   const Rng *base, double *partials, int64_t *defer, const float2 *pred, float margin,
                    const double2 *mid, const double2 *nodes, const double2 *coarse,
-                   const NibbleTables<ORB_NIB_POWERS> *nib, const uint32_t *ridx, int ridx_bits)
+                   const uint32_t *ridx, int ridx_bits)
 {
-    kl<orbits_kernel<THREADS, COARSE, CAP, MINB>>(g, b, 0, st, f, s, P, T, wb, partials, defer, pred, margin, mid, nodes,
-                                                  coarse, nib, ridx, ridx_bits);
+    kl<orbits_kernel<THREADS, COARSE, CAP, MINB>>(g, b, 0, st, f, s, P, jump, base, partials, defer, pred, margin, mid, nodes,
+                                                  coarse, ridx, ridx_bits);
 }
 struct OrbVariant { OrbFn fn; int threads, coarse, cap, minb; };
 #define ORB_V(T, C, K, M) {orbits_launch<T, C, K, M>, T, C, K, M}
 const OrbVariant kOrbVariants[] = {
-    ORB_V(256, 1024, 64, 1), ORB_V(256, 512, 64, 1), ORB_V(256, 2048, 64, 1), ORB_V(128, 1024, 64, 1),
+    // the first is the default: five waves per SIMD hide the gathers best and at most four
+    // lanes per star waste few tries.  Sampler time, default / the same unconstrained / with
+    // 64 lanes: N = 4e6 873 / 972 / 1020 us, 1e6 225 / 246 / 262, 3e5 75 / 87 / 99, 1e4 40 / 41 / 46.
+    ORB_V(256, 1024, 4, 5),  ORB_V(256, 512, 64, 1), ORB_V(256, 2048, 64, 1), ORB_V(128, 1024, 64, 1),
     ORB_V(512, 1024, 64, 1), ORB_V(128, 512, 64, 1), ORB_V(256, 1024, 2, 1),  ORB_V(256, 1024, 4, 1),
-    ORB_V(256, 1024, 8, 1),  ORB_V(256, 512, 4, 1),  ORB_V(256, 1024, 4, 4),  ORB_V(256, 1024, 8, 4),
-    ORB_V(256, 512, 4, 4)};
+    ORB_V(256, 1024, 8, 1),  ORB_V(256, 512, 4, 1),  ORB_V(256, 1024, 64, 1), ORB_V(256, 512, 4, 5),
+    ORB_V(256, 1024, 8, 5)};
 #undef ORB_V
 constexpr int ORB_NVARIANTS = sizeof(kOrbVariants) / sizeof(kOrbVariants[0]);
 
@@ -900,7 +897,6 @@ hipError_t launch_orbits(const DevFields &f, DevScalars *s, const KParams &P, co
     if (nblocks < 1) nblocks = 1;
     if (nblocks > sc.max_blocks) return hipErrorInvalidValue;
     int jb1 = 20 + bits_needed((uint64_t)n_ub);
-    if (hipError_t e = launch_rng_wave_bases(T, sc, 1, n_ub, st)) return e;
     if (hipError_t e = launch_node_index(f, s, sc, n_ub, st)) return e;
     if (V.coarse > ORB_MAX_COARSE) return hipErrorInvalidValue;
     kl<coarse_build_kernel>(dim3((unsigned)((V.coarse + 256) / 256)), dim3(256), 0, st,
@@ -913,10 +909,10 @@ hipError_t launch_orbits(const DevFields &f, DevScalars *s, const KParams &P, co
         pred = sc.pred;
     }
     if (ev_a) hipEventRecord(ev_a, st);
-    V.fn(dim3((unsigned)nblocks), dim3(V.threads), st, f, s, P, T, (const Rng *)sc.rng_wave,
+    V.fn(dim3((unsigned)nblocks), dim3(V.threads), st, f, s, P, sc.jump, (const Rng *)sc.rng_base,
                        sc.partials, sc.defer_list, pred, margin, (const double2 *)sc.mid,
                        (const double2 *)sc.nodes, (const double2 *)sc.coarse,
-                       (const NibbleTables<ORB_NIB_POWERS> *)sc.orb_nib, (const uint32_t *)sc.ridx, sc.ridx_bits);
+                       (const uint32_t *)sc.ridx, sc.ridx_bits);
     if (ev_b) hipEventRecord(ev_b, st);
     kl<defer_prepare_kernel>(dim3(1), dim3(DEFER_T), 0, st, s, sc.defer_list, sc.defer_kfirst, P.defer_cap);
     kl<defer_search_kernel>(dim3(256, 4), dim3(256), 0, st, f, s, P, (const int64_t *)sc.defer_list,

@@ -29,55 +29,30 @@ __device__ __forceinline__ double calc_n_local(const double *__restrict__ r, int
 }
 
 // The step's substream bases: base[0] = seeded state advanced by step * 2^72 (the
-// step's relaxation pairs), base[1] = base[0] + 2^70 (its orbit slots).  A block of
-// RB_T threads (rng_jump_block); the offset's bits 72..127 are the step's bits 0..55.
-constexpr int RB_T = 128;
+// step's relaxation pairs), base[1] = base[0] + 2^70 (its orbit slots), base[2] = base[1] +
+// 2^20 (orbit slot 1, the sampler's first).  One wave.
+constexpr int RB_T = 64;
 constexpr int DT_SLOTS = 64;     // the step's time-step minimum: slots of sigma_dt_kernel (<= RB_T)
-__device__ __forceinline__ void rng_bases(const RngTable *__restrict__ T, DevScalars *s, const Rng *__restrict__ seeded,
+__device__ __forceinline__ void rng_bases(const JumpLevel *__restrict__ J, DevScalars *s, const Rng *__restrict__ seeded,
                                           Rng *__restrict__ base, int64_t step_override)
 {
-    __shared__ uint32_t cols[56 * 128];
-    __shared__ Rng res;
     const uint64_t step = step_override >= 0 ? (uint64_t)step_override : s->step;
-    Rng b = rng_jump_block(T, *seeded, step, 72, 56, cols, &res);
-    if (threadIdx.x == 0) base[0] = b;
-    b = rng_jump_block(T, b, 1ull, 70, 1, cols, &res);
-    if (threadIdx.x == 0) base[1] = b;
+    const Rng a = jump_uniform(J + JL_STEP, JL_STEP_N, rng_uniform(*seeded), step & 0xffffffffffffffull);
+    const Rng b = jump_wave(J[JL_PHASE], a, 16);
+    const Rng c = jump_wave(J[JL_SLOT], b, 1);
+    if (threadIdx.x == 0) {
+        base[0] = a;
+        base[1] = b;
+        base[2] = c;
+    }
 }
 struct rng_bases_kernel {
     static constexpr int LB = RB_T, MB = 0;
-    static __device__ __forceinline__ void run(KGrid kg_, const RngTable *__restrict__ T, DevScalars *s,
+    static __device__ __forceinline__ void run(KGrid kg_, const JumpLevel *__restrict__ J, DevScalars *s,
                                                          const Rng *__restrict__ seeded, Rng *__restrict__ base,
                                                          int64_t step_override)
 {
-    rng_bases(T, s, seeded, base, step_override);
-}
-};
-
-// state at the first pair (phase 0: offset 3 * 64 w) or slot (phase 1: offset
-// (1 + 64 w) 2^20) of wave w.  With w = 256 b + t (block b, thread t) the offset
-// splits into a block part, jumped once per block from the global tables, and
-// 3 t 2^6 (phase 0) or t 2^26 (phase 1), jumped through LDS nibble tables of
-// WB_NB consecutive powers; jumps by powers of one matrix commute.
-constexpr int WB_T = 256, WB_NB = RNG_WB_POWERS;
-struct rng_wave_bases_kernel {
-    static constexpr int LB = WB_T, MB = 0;
-    static __device__ __forceinline__ void run(KGrid kg_, const RngTable *__restrict__ T,
-                                                              const Rng *__restrict__ base, int phase,
-                                                              int64_t nwaves, Rng *__restrict__ out, int jb1,
-                                                              const NibbleTables<WB_NB> *__restrict__ nib)
-{
-    __shared__ NibbleTables<WB_NB> lt;
-    __shared__ uint32_t cols[64 * 128];
-    __shared__ Rng res;
-    const int t = threadIdx.x;
-    const uint64_t b = kg_.bid;
-    copy_nibble_tables<WB_NB>(nib, lt);     // powers 2^6.. (phase 0) or 2^26.. (phase 1), built on the host
-    const Rng bb = phase == 0 ? rng_jump_block(T, base[0], 49152ull * b, 0, jb1, cols, &res)
-                              : rng_jump_block(T, base[1], 1ull + (b << 14), 20, jb1 - 20, cols, &res);
-    const int64_t w = (int64_t)b * WB_T + t;
-    if (w >= nwaves) return;
-    out[w] = rng_jump_lds<WB_NB>(lt, bb, phase == 0 ? 3u * (uint32_t)t : (uint32_t)t);
+    rng_bases(J, s, seeded, base, step_override);
 }
 };
 
@@ -191,34 +166,28 @@ struct timestep_finalize_kernel { static constexpr int LB = 1024, MB = 0; static
 // are reset for the next step, when dt_part is given), then its RNG substream bases
 struct timestep_rng_bases_kernel {
     static constexpr int LB = RB_T, MB = 0;
-    static __device__ __forceinline__ void run(KGrid kg_, const RngTable *__restrict__ T, DevScalars *s,
+    static __device__ __forceinline__ void run(KGrid kg_, const JumpLevel *__restrict__ J, DevScalars *s,
                                                                   const Rng *__restrict__ seeded,
                                                                   Rng *__restrict__ base,
                                                                   unsigned long long *__restrict__ dt_part)
 {
-    __shared__ unsigned long long wmin[RB_T / 64];
     if (dt_part) {
-        unsigned long long mine = 0x7ff0000000000000ull;
-        if (threadIdx.x < DT_SLOTS) {
-            const unsigned long long c = ~dt_part[threadIdx.x * 16];
-            dt_part[threadIdx.x * 16] = 0ull;
-            mine = c < mine ? c : mine;
-        }
+        unsigned long long mine = ~dt_part[threadIdx.x * 16];
+        dt_part[threadIdx.x * 16] = 0ull;
+        const unsigned long long inf = 0x7ff0000000000000ull;
+        mine = mine < inf ? mine : inf;
 #pragma unroll
         for (int o = 32; o >= 1; o >>= 1) {
             const unsigned long long other = __shfl_xor(mine, o, 64);
             mine = other < mine ? other : mine;
         }
-        if ((threadIdx.x & 63) == 0) wmin[threadIdx.x >> 6] = mine;
-        __syncthreads();
         if (threadIdx.x == 0) {
-            for (int q = 1; q < RB_T / 64; q++) mine = wmin[q] < mine ? wmin[q] : mine;
             const unsigned long long cur = (unsigned long long)__double_as_longlong(s->dtrel);
             s->dtrel = __longlong_as_double((long long)(mine < cur ? mine : cur));
         }
     }
     if (threadIdx.x == 0) timestep_finalize(s);
-    rng_bases(T, s, seeded, base, -1);
+    rng_bases(J, s, seeded, base, -1);
 }
 };
 
@@ -371,8 +340,7 @@ struct sigma_dt_kernel {
 }
 };
 
-// Pair pr draws from offset 3 pr; a wave's first pair starts at the per-wave state
-// and lane l jumps 3 l < 2^8 steps through the LDS tables.
+// Pair pr draws from offset 3 pr (jump_lanes).
 // energy_conservation1 (cmc_utils.c:227-236) for star i from its values after the
 // relaxation: vtold, vrold and Uoldrold = phi + MPI_PHI_S(r, i)
 __device__ __forceinline__ void ec1_star(DevFields &f, const KParams &P, int64_t i, double r, double m, double phi,
@@ -390,13 +358,12 @@ template <bool EC1, int T>
 struct relax_kernel {
     static constexpr int LB = T, MB = 0;
     static __device__ __forceinline__ void run(KGrid kg_, DevFields f, DevScalars *s, KParams P,
-                                                    const Rng *__restrict__ wave_base,
-                                                    const NibbleTables<8> *__restrict__ nib)
+                                                    const Rng *__restrict__ base,
+                                                    const JumpLevel *__restrict__ J)
 {
-    __shared__ NibbleTables<8> lt;
-    copy_nibble_tables<8>(nib, lt);
     int64_t pr = (int64_t)kg_.bid * blockDim.x + threadIdx.x;
     int64_t N = s->n_max;
+    Rng rng = jump_lanes(J + JL_PAIR, JL_PAIR_N, base[0], (uint32_t)(pr >> 6));    // before any lane leaves
     if (EC1 && pr == N / 2 && (N & 1)) {    // the unpaired last star keeps its velocities
         ec1_star(f, P, N, f.r[N], f.m[N], f.phi[N], f.vr[N], f.vt[N]);
         return;
@@ -404,7 +371,6 @@ struct relax_kernel {
     if (pr >= N / 2) return;            // pairs while si <= N - N%2 - 1 (cmc_dynamics.c:203)
     const int64_t k = 2 * pr + 1, kp = k + 1;
     const double dt = s->Dt;
-    Rng rng = rng_jump_lds<8>(lt, wave_base[pr >> 6], 3u * (uint32_t)(pr & 63));
 
     // calc_encounter_dyns (cmc_dynamics_helper.c:831-871)
     double Y = rng_dbl(rng);
@@ -473,27 +439,15 @@ int bits_needed(uint64_t x)
 }
 } // namespace
 
-hipError_t launch_rng_bases(const RngTable *T, DevScalars *s, const Scratch &sc, hipStream_t st)
+hipError_t launch_rng_bases(DevScalars *s, const Scratch &sc, hipStream_t st)
 {
-    kl<rng_bases_kernel>(dim3(1), dim3(RB_T), 0, st, T, s, sc.rng_seeded, sc.rng_base, (int64_t)-1);
+    kl<rng_bases_kernel>(dim3(1), dim3(RB_T), 0, st, (const JumpLevel *)sc.jump->level, s, sc.rng_seeded, sc.rng_base, (int64_t)-1);
     return hipGetLastError();
 }
 
-hipError_t launch_rng_bases_step(const RngTable *T, DevScalars *s, const Scratch &sc, int64_t step, hipStream_t st)
+hipError_t launch_rng_bases_step(DevScalars *s, const Scratch &sc, int64_t step, hipStream_t st)
 {
-    kl<rng_bases_kernel>(dim3(1), dim3(RB_T), 0, st, T, s, sc.rng_seeded, sc.rng_base, step);
-    return hipGetLastError();
-}
-
-hipError_t launch_rng_wave_bases(const RngTable *T, const Scratch &sc, int phase, int64_t count, hipStream_t st)
-{
-    int64_t nwaves = (count + 63) / 64;
-    if (nwaves <= 0) return hipSuccess;
-    if (nwaves > sc.max_waves) return hipErrorInvalidValue;
-    int jb1 = phase == 0 ? bits_needed(192ull * (uint64_t)nwaves) : 20 + bits_needed((uint64_t)(64 * nwaves + 1));
-    const NibbleTables<WB_NB> *nib = (const NibbleTables<WB_NB> *)sc.wb_nib + (phase == 0 ? 0 : 1);
-    kl<rng_wave_bases_kernel>(dim3((unsigned)((nwaves + WB_T - 1) / WB_T)), dim3(WB_T), 0, st, T,
-                       (const Rng *)sc.rng_base, phase, nwaves, sc.rng_wave, jb1, nib);
+    kl<rng_bases_kernel>(dim3(1), dim3(RB_T), 0, st, (const JumpLevel *)sc.jump->level, s, sc.rng_seeded, sc.rng_base, step);
     return hipGetLastError();
 }
 
@@ -554,28 +508,28 @@ hipError_t launch_simul_relax(const DevFields &f, DevScalars *s, const KParams &
     return hipGetLastError();
 }
 
-hipError_t launch_timestep_rng_bases(const RngTable *T, DevScalars *s, const Scratch &sc, hipStream_t st)
+hipError_t launch_timestep_rng_bases(DevScalars *s, const Scratch &sc, hipStream_t st)
 {
-    kl<timestep_rng_bases_kernel>(dim3(1), dim3(RB_T), 0, st, T, s, sc.rng_seeded, sc.rng_base,
+    kl<timestep_rng_bases_kernel>(dim3(1), dim3(RB_T), 0, st, (const JumpLevel *)sc.jump->level, s, sc.rng_seeded, sc.rng_base,
                        (unsigned long long *)nullptr);
     return hipGetLastError();
 }
 
 // The step's time-step phase: calc_sigma_r and simul_relax_new in one pass (or, for a
 // window longer than the pass stages, their own kernels), then Dt and the RNG bases.
-hipError_t launch_timestep_sigma(const DevFields &f, DevScalars *s, const KParams &P, const RngTable *T,
-                                 const Scratch &sc, int64_t n_ub, hipStream_t st)
+hipError_t launch_timestep_sigma(const DevFields &f, DevScalars *s, const KParams &P, const Scratch &sc,
+                                 int64_t n_ub, hipStream_t st)
 {
     if (P.avekernel > SIG_MAXP || n_ub <= 0) {
         if (hipError_t e = launch_simul_relax(f, s, P, n_ub, st, false)) return e;
         if (hipError_t e = launch_sigma(f, s, P, n_ub, st)) return e;
-        return launch_timestep_rng_bases(T, s, sc, st);
+        return launch_timestep_rng_bases(s, sc, st);
     }
     const int64_t nb = (n_ub + SIG_T - 1) / SIG_T;
     if (nb > sc.max_blocks) return hipErrorInvalidValue;
     kl<sigma_dt_kernel>(dim3((unsigned)nb), dim3(SIG_T), 0, st, f.r, f.m, f.vr, f.vt, f.sigma, s, P,
                        sc.dt_part);
-    kl<timestep_rng_bases_kernel>(dim3(1), dim3(RB_T), 0, st, T, s, sc.rng_seeded, sc.rng_base,
+    kl<timestep_rng_bases_kernel>(dim3(1), dim3(RB_T), 0, st, (const JumpLevel *)sc.jump->level, s, sc.rng_seeded, sc.rng_base,
                        sc.dt_part);
     return hipGetLastError();
 }
@@ -589,7 +543,7 @@ template <bool EC1, int TH>
 void relax_launch(int64_t nth, hipStream_t st, const DevFields &f, DevScalars *s, const KParams &P, const Scratch &sc)
 {
     kl<relax_kernel<EC1, TH>>(dim3((unsigned)((nth + TH - 1) / TH)), dim3(TH), 0, st, f, s, P,
-                              (const Rng *)sc.rng_wave, (const NibbleTables<8> *)sc.relax_nib);
+                              (const Rng *)sc.rng_base, (const JumpLevel *)sc.jump->level);
 }
 
 template <bool EC1>
@@ -606,19 +560,16 @@ hipError_t relax_launch_shape(int threads, int64_t nth, hipStream_t st, const De
     return hipGetLastError();
 }
 
-hipError_t launch_relax(const DevFields &f, DevScalars *s, const KParams &P, const RngTable *T,
-                        const Scratch &sc, int64_t n_ub, hipStream_t st, bool with_ec1, int threads)
+hipError_t launch_relax(const DevFields &f, DevScalars *s, const KParams &P, const Scratch &sc,
+                        int64_t n_ub, hipStream_t st, bool with_ec1, int threads)
 {
     int64_t npairs = n_ub / 2;
     if (with_ec1) {
         // one thread more for an unpaired last star
         const int64_t nth = (n_ub + 1) / 2;
         if (nth <= 0) return hipSuccess;
-        if (npairs > 0)
-            if (hipError_t e = launch_rng_wave_bases(T, sc, 0, npairs, st)) return e;
         return relax_launch_shape<true>(threads, nth, st, f, s, P, sc);
     }
     if (npairs <= 0) return hipSuccess;
-    if (hipError_t e = launch_rng_wave_bases(T, sc, 0, npairs, st)) return e;
     return relax_launch_shape<false>(threads, npairs, st, f, s, P, sc);
 }

@@ -7,8 +7,7 @@
 #include "cmcg_internal.hpp"
 #include "mlp.hpp"
 
-// orbit sampler: most LDS samples of any launch variant; lane jumps l 2^20 by nibble
-// tables of the powers 2^ORB_NIB_B0 .. 2^(ORB_NIB_B0 + ORB_NIB_POWERS - 1)
+// orbit sampler: most LDS samples of any launch variant
 constexpr int ORB_MAX_COARSE = 2048;
 // sort payload records: at most 16 words (128 B, one cache line) per star
 constexpr int SORT_AOS_WORDS = 16;
@@ -33,9 +32,7 @@ inline SortShape sort_shape(int64_t n_ub)
     return sh;
 }
 constexpr int RED2_BLOCKS = 64;
-constexpr int ORB_NIB_B0 = 20, ORB_NIB_POWERS = 6;
 
-constexpr int RNG_WB_POWERS = 10;   // nibble-table powers of the wave-base jumps
 constexpr int RIDX_TILE = 4096;     // buckets per block of the radial index's scan
 __host__ __device__ constexpr int64_t ridx_entries(int bits) { return ((int64_t)1 << bits) + 2; }
 __host__ __device__ constexpr int64_t ridx_tiles(int bits) { return (ridx_entries(bits) + RIDX_TILE - 1) / RIDX_TILE; }
@@ -83,9 +80,7 @@ struct Scratch {
     double *sv3_dpre;           // D = vold^2 + 2(1-q)(Uoldrold - Uoldrnew) per star, in the order before the step's sort
     unsigned long long *dt_part;  // the step's time step: 64 slots, 128 bytes apart, of complemented dt minima
     double2 *coarse;            // orbit sampler's (r, phi) samples, copied into LDS by every block
-    void *orb_nib;              // orbit sampler's GF(2) nibble tables (constant per context)
-    void *relax_nib;            // relaxation's nibble tables, powers 2^0 .. 2^7 (constant per context)
-    void *wb_nib;               // wave-base nibble tables: powers 2^6 .. 2^15 and 2^26 .. 2^35
+    const JumpTables *jump;     // the device's jump tables, shared by its contexts
     double *red2;               // second level of the block-partial reductions (RED2_BLOCKS x 16)
     int64_t sort_aos_cap;
     // set_velocities3 excess chain: per-star excess, ordered event list, per-event
@@ -100,11 +95,9 @@ struct Scratch {
     int32_t *strip_done;
     // orbit stars deferred to the linear-scan path (65536 slots)
     int64_t *defer_list, *defer_kfirst;   // KParams::defer_cap entries
-    // RNG bases of the current step: [0] relaxation, [1] orbits; seeded state
+    // RNG bases of the current step: [0] relaxation, [1] orbits, [2] orbit slot 1; seeded state
     Rng *rng_base;
     Rng *rng_seeded;
-    Rng *rng_wave;              // per-wave substream starts (relaxation pairs / orbit slots)
-    int64_t max_waves;
 };
 
 hipError_t launch_potential(const DevFields &f, DevScalars *s, const KParams &P, int64_t n_ub,
@@ -122,22 +115,19 @@ hipError_t launch_potential_at(const DevFields &f, DevScalars *s, const KParams 
 hipError_t launch_sigma(const DevFields &f, DevScalars *s, const KParams &P, int64_t n_ub, hipStream_t st);
 hipError_t launch_simul_relax(const DevFields &f, DevScalars *s, const KParams &P, int64_t n_ub, hipStream_t st,
                               bool init_min = true);
-hipError_t launch_timestep_rng_bases(const RngTable *T, DevScalars *s, const Scratch &sc, hipStream_t st);
-hipError_t launch_timestep_sigma(const DevFields &f, DevScalars *s, const KParams &P, const RngTable *T,
-                                 const Scratch &sc, int64_t n_ub, hipStream_t st);
+hipError_t launch_timestep_rng_bases(DevScalars *s, const Scratch &sc, hipStream_t st);
+hipError_t launch_timestep_sigma(const DevFields &f, DevScalars *s, const KParams &P, const Scratch &sc,
+                                 int64_t n_ub, hipStream_t st);
 hipError_t launch_timestep_finalize(DevScalars *s, hipStream_t st);
 // threads: block size of the relaxation kernel, one of RELAX_SHAPES (an autotuned
 // launch shape; results do not depend on it)
 constexpr int RELAX_SHAPES[] = {256, 128, 512, 1024};
 constexpr int RELAX_NSHAPES = 4;
-hipError_t launch_relax(const DevFields &f, DevScalars *s, const KParams &P, const RngTable *T,
-                        const Scratch &sc, int64_t n_ub, hipStream_t st,
+hipError_t launch_relax(const DevFields &f, DevScalars *s, const KParams &P, const Scratch &sc,
+                        int64_t n_ub, hipStream_t st,
                         bool with_ec1 = false, int threads = 256);
-hipError_t launch_rng_bases(const RngTable *T, DevScalars *s, const Scratch &sc, hipStream_t st);
-hipError_t launch_rng_bases_step(const RngTable *T, DevScalars *s, const Scratch &sc, int64_t step, hipStream_t st);
-// substream start of every 64-lane wave: relaxation (phase 0, pairs 64w..) or orbits
-// (phase 1, slots 1 + 64w..), for `count` pairs / slots
-hipError_t launch_rng_wave_bases(const RngTable *T, const Scratch &sc, int phase, int64_t count, hipStream_t st);
+hipError_t launch_rng_bases(DevScalars *s, const Scratch &sc, hipStream_t st);
+hipError_t launch_rng_bases_step(DevScalars *s, const Scratch &sc, int64_t step, hipStream_t st);
 // the packed node table and the radial index in one pass over r and phi
 hipError_t launch_node_index(const DevFields &f, DevScalars *s, const Scratch &sc, int64_t n_ub, hipStream_t st);
 // middle level of the (r, phi) search tables, from the current arrays
