@@ -435,10 +435,13 @@ const JumpTables *jump_acquire(int device, const RngTable &T)
     fill_jump_level(T.col[66], h->level, JL_PHASE);
     for (int k = 0; k < JL_STEP_N; k++)
         if (72 + 6 * k < 128) fill_jump_level(T.col[72 + 6 * k], h->level, JL_STEP + k);
-    for (int b = 0; b < ORB_NIB_POWERS; b++)
+    for (int d = 0; d < 8; d++)                 // d slots and 8 d slots, from the level's own table
         for (int c = 0; c < 4; c++)
             for (int q = 0; q < 8; q++)
-                for (int v = 0; v < 16; v++) h->orbit.t[b][c][q][v] = host_matvec(T.col[ORB_NIB_B0 + b][c], (uint32_t)v << (4 * q));
+                for (int v = 0; v < 16; v++) {
+                    h->orbit.lo.t[c][q][v][d] = h->level[JL_SLOT].t[jump_index(false, c, q, v, d)];
+                    h->orbit.hi.t[c][q][v][d] = h->level[JL_SLOT].t[jump_index(false, c, q, v, 8 * d)];
+                }
     void *ptr = nullptr;
     if (hipMalloc(&ptr, sizeof(JumpTables)) != hipSuccess) return nullptr;
     if (hipMemcpy(ptr, h.get(), sizeof(JumpTables), hipMemcpyHostToDevice) != hipSuccess) {

@@ -177,34 +177,39 @@ __device__ __forceinline__ Rng jump_uniform(const JumpLevel *__restrict__ L, int
     }
     return z;
 }
-// The orbit sampler's lanes jump through LDS instead: for the matrix powers 2^20 .. 2^25
-// and each state word, t[b][c][q][v] is the product of the matrix with the value v of the
-// word's 4-bit piece q, so a 32x32 GF(2) product is 8 lookups.  The sampler waits on
-// gathers, not on these, while the table loads above evict its nodes from the L1 (1071 ->
-// 1172 us at N = 4e6), and as a pass before it they took 58 us.
-constexpr int ORB_NIB_B0 = 20, ORB_NIB_POWERS = 6;
-struct NibbleTables { uint32_t t[ORB_NIB_POWERS][4][8][16]; };
-__device__ __forceinline__ Rng rng_jump_lds(const NibbleTables &lt, Rng s, uint32_t off)
+// The orbit sampler's lanes jump through LDS instead, in two digits of 8, lane = 8 h + l: the
+// products for h 8 units are looked up by the wave together (lane 8 h + q takes piece q of
+// each word), those for l by each lane in LDS, 32 lookups.  t[c][q][v][d]: the product of
+// d U (d 8 U) with value v of piece q of word c.  (Lane tables as above evict the sampler's
+// nodes from the L1: 1071 -> 1172 us at N = 4e6; as a pass before it they took 58 us; single
+// powers of two, 192 LDS lookups, took about 700 of its 5700 vector instructions a wave.)
+struct LaneDigit { uint32_t t[4][8][16][8]; };
+struct LaneDigits { LaneDigit lo, hi; };
+__device__ __forceinline__ uint32_t xor_over_8_lanes(uint32_t x)
 {
-    auto matvec = [](const uint32_t (&tab)[8][16], uint32_t v) {
+    x ^= (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0xB1, 0xf, 0xf, true);      // quad_perm [1, 0, 3, 2]
+    x ^= (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x4E, 0xf, 0xf, true);      // quad_perm [2, 3, 0, 1]
+    x ^= (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x141, 0xf, 0xf, true);     // row_half_mirror
+    return x;
+}
+// z uniform over the wave, every lane active; lo in LDS
+__device__ __forceinline__ Rng jump_lane_digits(const LaneDigit &hi, const LaneDigit &lo, const Rng &z)
+{
+    const int lane = threadIdx.x & 63, g = lane >> 3, l = lane & 7;
+    auto upper = [&](int c, uint32_t x) { return xor_over_8_lanes(hi.t[c][l][(x >> (4 * l)) & 15u][g]); };
+    const Rng s{upper(0, z.z0), upper(1, z.z1), upper(2, z.z2), upper(3, z.z3)};
+    auto lower = [&](int c, uint32_t x) {
         uint32_t o = 0;
 #pragma unroll
-        for (int q = 0; q < 8; q++) o ^= tab[q][(v >> (4 * q)) & 15u];
+        for (int q = 0; q < 8; q++) o ^= lo.t[c][q][(x >> (4 * q)) & 15u][l];
         return o;
     };
-    for (int b = 0; b < ORB_NIB_POWERS; b++) {
-        if (!((off >> b) & 1u)) continue;
-        s.z0 = matvec(lt.t[b][0], s.z0);
-        s.z1 = matvec(lt.t[b][1], s.z1);
-        s.z2 = matvec(lt.t[b][2], s.z2);
-        s.z3 = matvec(lt.t[b][3], s.z3);
-    }
-    return s;
+    return Rng{lower(0, s.z0), lower(1, s.z1), lower(2, s.z2), lower(3, s.z3)};
 }
 // what a device holds of them
 struct JumpTables {
     JumpLevel level[JL_COUNT];
-    NibbleTables orbit;
+    LaneDigits orbit;
 };
 
 // The state of the lane's pair: the wave's first is number 64 w after base.  Every lane of
@@ -234,7 +239,7 @@ __device__ __forceinline__ double phi_s(const double *__restrict__ r, const doub
 }
 __device__ __forceinline__ double phi_s_own(double rj, double mj, double inv_nstar, double rad)
 {
-    return (rad >= rj ? mj / rad : mj / rj) * inv_nstar;
+    return mj / (rad >= rj ? rad : rj) * inv_nstar;
 }
 
 // cmc_utils.c:1654-1662 function_q evaluated in double (the reference uses x87
@@ -248,28 +253,40 @@ __device__ __forceinline__ double function_q(double rj, double mj, double inv_ns
     return 2.0 * (E - (pot + phis)) - Jr;
 }
 
-// Sign of function_q(rj, mj, inv_nstar, r, pot, E, J) as that function computes it
-// in double: -1 (Q < 0), 0 (Q == 0), 1 (Q > 0), 2 (NaN).  A division-free value q~
-// (1/r from the hardware reciprocal refined by two Newton steps, accurate to 2^-45
-// for any seed accurate to 12 bits) differs from the computed Q by less than
-// (2 2^-45 + 10 2^-53) S, S = 2(|E| + |pot| + |phis|) + (J/r)^2, since each of the two
-// evaluations rounds at most six times; when |q~| exceeds 2^-42 S the signs agree,
-// otherwise function_q itself decides.  qa receives q~ (a guide for searches only).
-__device__ __forceinline__ int q_sign(double rj, double mj, double inv_nstar, double r, double pot, double E,
-                                      double J, double *qa = nullptr)
+// What the sign of a star's function_q needs at every node: s0 = (m_j / r_j) / N and
+// s1 = m_j / N, the star's own term below and (times 1 / r) above its radius.
+struct QStar {
+    double rj, mj, inv, E, J;
+    double s0, s1, J2, c1, k;
+};
+__device__ __forceinline__ QStar q_star(double rj, double mj, double inv_nstar, double E, double J)
 {
-    double y = __builtin_amdgcn_rcp(r);
-    double e = __builtin_fma(-r, y, 1.0);
-    y = __builtin_fma(y, e, y);
-    e = __builtin_fma(-r, y, 1.0);
-    y = __builtin_fma(y, e, y);
-    const double a = J * y, T = a * a;
-    const double ph = (r >= rj ? mj * y : mj / rj) * inv_nstar;
-    const double q = 2.0 * (E - (pot + ph)) - T;
-    if (qa) *qa = q;
-    const double S = 2.0 * (__builtin_fabs(E) + __builtin_fabs(pot) + __builtin_fabs(ph)) + T;
-    if (__builtin_fabs(q) > 0x1p-42 * S) return q < 0.0 ? -1 : 1;
-    const double qe = function_q(rj, mj, inv_nstar, r, pot, E, J);
+    QStar q;
+    q.rj = rj; q.mj = mj; q.inv = inv_nstar; q.E = E; q.J = J;
+    q.s0 = mj / rj * inv_nstar;
+    q.s1 = mj * inv_nstar;
+    q.J2 = J * J;
+    q.c1 = __builtin_fabs(E) + __builtin_fabs(q.s0);
+    q.k = __builtin_fma(0x1p-42, q.J2, 1e-290);
+    return q;
+}
+
+// Sign of function_q(rj, mj, inv_nstar, r, pot, E, J) as that function computes it in
+// double: -1 (Q < 0), 0 (Q == 0), 1 (Q > 0), 2 (NaN).  Without a division: g = Q r^2 =
+// 2 ((E - pot) r - s) r - J^2, s = s0 r below r_j and s1 above, and each of g and the
+// computed Q r^2 differs from the exact value by less than 10 2^-53 S r^2, S = 2 (|E| +
+// |pot| + |s0|) + (J / r)^2, since each evaluation rounds at most ten times; when |g| exceeds
+// 2^-42 S r^2 (plus 1e-290, for products that underflow) the signs agree, otherwise
+// function_q itself decides.  (With the reciprocal of r by two Newton steps, as before, a
+// sign took about 45 vector instructions, now 20; the samples' two bisections alone take 20 signs.)
+__device__ __forceinline__ int q_sign(const QStar &q, double r, double pot)
+{
+    const double t = q.E - pot, r2 = r + r;
+    const double s = r >= q.rj ? q.s1 : q.s0 * r;
+    const double g = __builtin_fma(__builtin_fma(t, r, -s), r2, -q.J2);
+    const double thr = __builtin_fma((q.c1 + __builtin_fabs(pot)) * r, r2 * 0x1p-42, q.k);
+    if (__builtin_fabs(g) > thr) return g < 0.0 ? -1 : 1;
+    const double qe = function_q(q.rj, q.mj, q.inv, r, pot, q.E, q.J);
     return qe < 0.0 ? -1 : (qe > 0.0 ? 1 : (qe == 0.0 ? 0 : 2));
 }
 __device__ __forceinline__ bool q_lt0(int sg) { return sg == -1; }
@@ -353,11 +370,12 @@ template <class N>
 __device__ __forceinline__ int64_t find_zero_Q_n(const N &nd, double rj, double mj, double inv_nstar,
                                                  int64_t kmin, int64_t kmax, double E, double J)
 {
+    const QStar q = q_star(rj, mj, inv_nstar, E, J);
     double a, b, a2, b2;
     nd.RP(kmin, a, b);
     nd.RP(kmax, a2, b2);
     // the direction test qmin < qmax: decided by the signs when they differ
-    const int smin = q_sign(rj, mj, inv_nstar, a, b, E, J), smax = q_sign(rj, mj, inv_nstar, a2, b2, E, J);
+    const int smin = q_sign(q, a, b), smax = q_sign(q, a2, b2);
     bool up;
     if ((smin == -1 || smin == 1) && (smax == -1 || smax == 1) && smin != smax) up = smin < smax;
     else up = function_q(rj, mj, inv_nstar, a, b, E, J) < function_q(rj, mj, inv_nstar, a2, b2, E, J);
@@ -366,14 +384,14 @@ __device__ __forceinline__ int64_t find_zero_Q_n(const N &nd, double rj, double 
         do {
             int64_t ktry = (kmin + kmax + 1) / 2;
             nd.RP(ktry, a, b);
-            if (q_lt0(q_sign(rj, mj, inv_nstar, a, b, E, J))) kmin = ktry;
+            if (q_lt0(q_sign(q, a, b))) kmin = ktry;
             else kmax = ktry - 1;
         } while (kmax != kmin && ++guard < 96);
     } else {
         do {
             int64_t ktry = (kmin + kmax + 1) / 2;
             nd.RP(ktry, a, b);
-            if (q_gt0(q_sign(rj, mj, inv_nstar, a, b, E, J))) kmin = ktry;
+            if (q_gt0(q_sign(q, a, b))) kmin = ktry;
             else kmax = ktry - 1;
         } while (kmax != kmin && ++guard < 96);
     }
@@ -442,9 +460,10 @@ __device__ __forceinline__ bool interval_converged(double lo, double hi, double 
 
 // cmc_nr.c:500-603 find_root_vr by the Brent-Dekker method (Brent 1973, ch. 4),
 // the same iteration as the CPU oracle's.  Rare fallback path; scalar arguments and a
-// returned pair keep its caller's objects out of private memory.
+// returned pair keep its caller's objects out of private memory.  (Not a call: around one
+// the sampler spilled 30 registers, 128 B a star.)
 struct RootVr { double root; int bad; };
-__device__ __noinline__ RootVr find_root_vr(const double *__restrict__ r, const double *__restrict__ phi,
+__device__ __forceinline__ RootVr find_root_vr(const double *__restrict__ r, const double *__restrict__ phi,
                                             double rj, double mj, double inv_nstar, double cen, int64_t k,
                                             double E, double J)
 {
@@ -549,6 +568,7 @@ __device__ __forceinline__ void ridx_bracket(const RIdx &x, double r, int32_t &l
 struct Coarse {
     const double *cr, *cphi;
     int64_t stride, n1;          // stride is a multiple of MID_STEP
+    uint32_t inv_stride;         // 2^32 / stride, for coarse_s
     int cs;
     // middle level in global memory (L2-resident): (r, phi) at every MID_STEP-th node
     const double2 *mid;
@@ -572,6 +592,17 @@ __device__ __forceinline__ int64_t coarse_k(const Coarse &c, int s)
 {
     int64_t k = (int64_t)s * c.stride;
     return k < c.n1 ? k : c.n1;
+}
+__device__ __forceinline__ int32_t coarse_k32(const Coarse &c, int s)
+{
+    const int32_t k = s * (int32_t)c.stride;       // at most n + 1 + the stride
+    return k < (int32_t)c.n1 ? k : (int32_t)c.n1;
+}
+// k / stride: the truncated reciprocal gives the quotient or one less
+__device__ __forceinline__ int coarse_s(const Coarse &c, int32_t k)
+{
+    const uint32_t q = __umulhi((uint32_t)k, c.inv_stride), st = (uint32_t)c.stride;
+    return (int)(q + ((uint32_t)k - q * st >= st ? 1u : 0u));
 }
 
 // Largest t in [t0, t1] with eval(mid[t]) true, or t0 - 1 if there is none, for a
@@ -707,27 +738,28 @@ __device__ __forceinline__ double potential_at_ridx(const double2 *__restrict__ 
 // the two nodes (exactly the reference's interpolation when they are adjacent) plus
 // the star's own term (m_j/r_j below r_j, m_j/r above; judged at ra), so that
 // Q r^2 = 2(E - B - s0) r^2 - 2(A + s1) r - J^2.  The smaller positive root for the
-// pericentre, the larger for the apocentre; -1 when there is none.  Only a guess:
-// every index it leads to is verified by the signs of Q.
-__device__ __forceinline__ double interp_root(double ra, double pa, double rb, double pb, double rj, double mj,
-                                              double inv, double E, double J, bool peri)
+// pericentre, the larger for the apocentre; negative or NaN when there is none.  Only a
+// guess: every index it leads to is verified by the signs of Q.  So its reciprocals and root
+// are the hardware's estimates and one Newton step: where that is not enough, the guess is a
+// node or two off, or outside the bracket, and costs a probe.
+__device__ __forceinline__ double rcp_guess(double x)
 {
-    const double ia = 1.0 / ra, ib = 1.0 / rb;
-    const double A = (pb - pa) / (ib - ia), B = pa - A * ia;
-    double s0 = 0.0, s1 = 0.0;
-    if (ra >= rj) s1 = mj * inv;
-    else s0 = mj * inv / rj;
-    const double a2 = 2.0 * (E - B - s0), a1 = -2.0 * (A + s1), a0 = -J * J;
-    const double disc = a1 * a1 - 4.0 * a2 * a0;
-    if (!(disc >= 0.0) || a2 == 0.0) return -1.0;
-    const double sq = sqrt(disc);
-    const double q = -0.5 * (a1 + (a1 >= 0.0 ? sq : -sq));
-    if (q == 0.0) return -1.0;
-    double x1 = q / a2, x2 = a0 / q;
-    if (x1 > x2) { const double t = x1; x1 = x2; x2 = t; }
-    if (x2 <= 0.0) return -1.0;
-    if (x1 <= 0.0) return x2;
-    return peri ? x1 : x2;
+    const double y = __builtin_amdgcn_rcp(x);
+    return __builtin_fma(y, __builtin_fma(-x, y, 1.0), y);
+}
+__device__ __forceinline__ double interp_root(const QStar &q, double ra, double pa, double rb, double pb, bool peri)
+{
+    const double A = (pb - pa) * ra * (rb * rcp_guess(ra - rb)), B = pa - A * rcp_guess(ra);
+    const bool out = ra >= q.rj;
+    const double h2 = q.E - B - (out ? 0.0 : q.s0), h1 = A + (out ? q.s1 : 0.0);
+    const double disc = __builtin_fma(h1, h1, 2.0 * h2 * q.J2);         // roots of 2 h2 r^2 - 2 h1 r - J^2
+    const double y = __builtin_amdgcn_rsq(disc);
+    double sq = disc * y;
+    sq = __builtin_fma(__builtin_fma(-sq, sq, disc), 0.5 * y, sq);
+    const double w = h1 + (h1 >= 0.0 ? sq : -sq);
+    const double x1 = 0.5 * w * rcp_guess(h2), x2 = -q.J2 * rcp_guess(w);
+    const double lo = x1 < x2 ? x1 : x2, hi = x1 < x2 ? x2 : x1;
+    return peri && lo > 0.0 ? lo : hi;
 }
 
 // find_zero_Q's answer on a bracket [lo, hi] whose ends have the bisection's
@@ -742,21 +774,20 @@ __device__ __forceinline__ double interp_root(double ra, double pa, double rb, d
 // load; probing the two ends of the index's bracket, with its ends and the answer's nodes
 // read for themselves, took about 12 a search, this about 5.)
 template <bool POSITIVE>
-__device__ __forceinline__ int64_t ridx_zero_Q(const double2 *__restrict__ nodes, const RIdx &ri, double rj, double mj,
-                                               double inv, double E, double J, int64_t lo, int64_t hi, double &rl,
-                                               double &pl, double &rh, double &ph)
+__device__ __forceinline__ int32_t ridx_zero_Q(const double2 *__restrict__ nodes, const RIdx &ri, const QStar &q,
+                                               int32_t lo, int32_t hi, double &rl, double &pl, double &rh, double &ph)
 {
-    int32_t l = (int32_t)lo, h = (int32_t)hi;
+    int32_t l = lo, h = hi;
     // node k probed: true when the bracket's lower end moved to it
     auto probe = [&](int32_t k, const double2 &v) {
-        const int sg = q_sign(rj, mj, inv, v.x, v.y, E, J);
+        const int sg = q_sign(q, v.x, v.y);
         const bool in = POSITIVE ? q_gt0(sg) : q_lt0(sg);
         if (in) { l = k; rl = v.x; pl = v.y; }
         else { h = k; rh = v.x; ph = v.y; }
         return in;
     };
     for (int it = 0; it < 3 && h - l > 1; it++) {
-        const double rg = interp_root(rl, pl, rh, ph, rj, mj, inv, E, J, !POSITIVE);
+        const double rg = interp_root(q, rl, pl, rh, ph, !POSITIVE);
         int32_t a = l + ((h - l) >> 1);            // no usable guess: a bisection step
         if (rg > rl && rg < rh) {
             const int32_t g = (int32_t)ri.t[ridx_bucket(ri, rg)];
@@ -778,14 +809,14 @@ struct OrbitRS { double rp, ra, dQdrp, dQdra; int64_t kmin, kmax; int circular; 
 // cmc_orbit.c:413-540 calc_orbit_new after get_positive_Q_index has produced ktemp
 // (an index with Q > 0; ktemp < 0 means "no positive Q": circular orbit).
 // HAS_C: the LDS samples, radial index and learned proposal of Cr are available, and pj is
-// phi at j.  (A template flag rather than a null test of a pointer: comparing the address
+// phi at j, q the star's QStar.  (A template flag rather than a null test of a pointer: comparing the address
 // of a private object with null is not folded on this target and keeps the object in
 // scratch memory.)
 template <class N, bool HAS_C>
 __device__ __forceinline__ OrbitRS calc_orbit_core(const N &nd, const double *__restrict__ r,
                                                    const double *__restrict__ phi, int64_t n_max, int64_t j,
                                                    double rj, double mj, const KParams &P, double E, double J,
-                                                   int64_t ktemp, const Coarse &Cr, double pj = 0.0)
+                                                   int64_t ktemp, const Coarse &Cr, const QStar &q, double pj = 0.0)
 {
     OrbitRS o;
     o.brent = 0; o.linscan = 0; o.err = 0; o.hint_hits = 0; o.hint_misses = 0;
@@ -801,8 +832,8 @@ __device__ __forceinline__ OrbitRS calc_orbit_core(const N &nd, const double *__
         // negative far out (r^3 dPhi/dr = r M(r) increases), so the index bisection's result
         // is the unique sign change of its bracket; the LDS samples narrow both brackets
         // to one sample interval before the interpolation search in global memory.
-        const double inv = P.inv_nstar;
-        int64_t kp_lo = 0, kp_hi = ktemp, ka_lo = ktemp, ka_hi = n_max + 1;
+        const int32_t kt = (int32_t)ktemp, n1 = (int32_t)n_max + 1;
+        int32_t kp_lo = 0, kp_hi = kt, ka_lo = kt, ka_hi = n1;
         bool got_p = false, got_a = false;
         bool vp = false, va = false;   // bracket ends checked: Q(lo), Q(hi) have the bisection's signs
         rp1 = ra0 = rj;
@@ -813,39 +844,39 @@ __device__ __forceinline__ OrbitRS calc_orbit_core(const N &nd, const double *__
             const float ep = __expf(Cr.margin);
             int32_t a, b;
             ridx_bracket(Cr.ri, (double)(__expf(Cr.lrp) / ep), a, b);
-            int64_t lo = a < 0 ? 0 : a;
+            int32_t lo = a < 0 ? 0 : a;
             ridx_bracket(Cr.ri, (double)(__expf(Cr.lrp) * ep), a, b);
-            int64_t hi = b > ktemp ? ktemp : b;
-            if (lo < hi && q_lt0(q_sign(rj, mj, inv, nd.R(lo), nd.P(lo), E, J)) &&
-                (hi == ktemp || q_ge0(q_sign(rj, mj, inv, nd.R(hi), nd.P(hi), E, J)))) {
+            int32_t hi = b > kt ? kt : b;
+            if (lo < hi && q_lt0(q_sign(q, nd.R(lo), nd.P(lo))) &&
+                (hi == kt || q_ge0(q_sign(q, nd.R(hi), nd.P(hi))))) {
                 kp_lo = lo; kp_hi = hi; got_p = vp = true; o.hint_hits++;
             } else {
                 o.hint_misses++;
             }
             ridx_bracket(Cr.ri, (double)(__expf(Cr.lra) / ep), a, b);
-            lo = a < ktemp ? ktemp : a;
+            lo = a < kt ? kt : a;
             ridx_bracket(Cr.ri, (double)(__expf(Cr.lra) * ep), a, b);
-            hi = b > n_max + 1 ? n_max + 1 : b;
-            if (lo < hi && (lo == ktemp || q_gt0(q_sign(rj, mj, inv, nd.R(lo), nd.P(lo), E, J))) &&
-                !q_gt0(q_sign(rj, mj, inv, nd.R(hi), nd.P(hi), E, J))) {
+            hi = b > n1 ? n1 : b;
+            if (lo < hi && (lo == kt || q_gt0(q_sign(q, nd.R(lo), nd.P(lo)))) &&
+                !q_gt0(q_sign(q, nd.R(hi), nd.P(hi)))) {
                 ka_lo = lo; ka_hi = hi; got_a = va = true; o.hint_hits++;
             } else {
                 o.hint_misses++;
             }
             // a verified learned bracket is narrowed by the LDS samples inside it: the
             // sample bisection runs over those samples only
-            auto narrow = [&](int64_t &lo, int64_t &hi, bool positive) {
-                const int s0 = (int)(lo / Cr.stride) + 1, s1 = (int)((hi - 1) / Cr.stride);
+            auto narrow = [&](int32_t &lo, int32_t &hi, bool positive) {
+                const int s0 = coarse_s(Cr, lo) + 1, s1 = coarse_s(Cr, hi - 1);
                 if (s0 > s1 || s1 > Cr.cs) return;
                 int a = s0 - 1, b = s1;                    // sample a: predicate true (a = s0 - 1: node lo)
                 while (a < b) {
                     const int m = (a + b + 1) >> 1;
-                    const int sg = q_sign(rj, mj, inv, Cr.cr[m], Cr.cphi[m], E, J);
+                    const int sg = q_sign(q, Cr.cr[m], Cr.cphi[m]);
                     if (positive ? q_gt0(sg) : q_lt0(sg)) a = m;
                     else b = m - 1;
                 }
-                if (a >= s0) lo = coarse_k(Cr, a);
-                if (a < s1) hi = coarse_k(Cr, a + 1);
+                if (a >= s0) lo = coarse_k32(Cr, a);
+                if (a < s1) hi = coarse_k32(Cr, a + 1);
             };
             if (got_p) {
                 narrow(kp_lo, kp_hi, false);
@@ -858,39 +889,39 @@ __device__ __forceinline__ OrbitRS calc_orbit_core(const N &nd, const double *__
                 nd.RP(ka_hi, ra1, pa1);
             }
         }
-        if (!got_p && ktemp >= 1 && q_lt0(q_sign(rj, mj, inv, Cr.cr[0], Cr.cphi[0], E, J))) {
-            int a = 0, b = (int)((ktemp - 1) / Cr.stride);
+        if (!got_p && kt >= 1 && q_lt0(q_sign(q, Cr.cr[0], Cr.cphi[0]))) {
+            int a = 0, b = coarse_s(Cr, kt - 1);
             const int top = b;
             while (a < b) {
                 int m = (a + b + 1) >> 1;
-                if (q_lt0(q_sign(rj, mj, inv, Cr.cr[m], Cr.cphi[m], E, J))) a = m;
+                if (q_lt0(q_sign(q, Cr.cr[m], Cr.cphi[m]))) a = m;
                 else b = m - 1;
             }
-            kp_lo = coarse_k(Cr, a);
+            kp_lo = coarse_k32(Cr, a);
             rp0 = Cr.cr[a];
             pp0 = Cr.cphi[a];
             if (a < top) {
-                kp_hi = coarse_k(Cr, a + 1);
+                kp_hi = coarse_k32(Cr, a + 1);
                 rp1 = Cr.cr[a + 1];
                 pp1 = Cr.cphi[a + 1];
             }
             vp = true;
         }
-        const int sb = (int)(ktemp / Cr.stride) + 1;
-        if (!got_a && sb <= Cr.cs && !q_gt0(q_sign(rj, mj, inv, Cr.cr[Cr.cs], Cr.cphi[Cr.cs], E, J))) {
+        const int sb = coarse_s(Cr, kt) + 1;
+        if (!got_a && sb <= Cr.cs && !q_gt0(q_sign(q, Cr.cr[Cr.cs], Cr.cphi[Cr.cs]))) {
             va = true;
             int a = sb - 1, b = Cr.cs - 1;                 // sample a: Q > 0 (a = sb - 1: node ktemp)
             while (a < b) {
                 int m = (a + b + 1) >> 1;
-                if (q_gt0(q_sign(rj, mj, inv, Cr.cr[m], Cr.cphi[m], E, J))) a = m;
+                if (q_gt0(q_sign(q, Cr.cr[m], Cr.cphi[m]))) a = m;
                 else b = m - 1;
             }
             if (a >= sb) {
-                ka_lo = coarse_k(Cr, a);
+                ka_lo = coarse_k32(Cr, a);
                 ra0 = Cr.cr[a];
                 pa0 = Cr.cphi[a];
             }
-            ka_hi = coarse_k(Cr, a + 1);
+            ka_hi = coarse_k32(Cr, a + 1);
             ra1 = Cr.cr[a + 1];
             pa1 = Cr.cphi[a + 1];
         }
@@ -898,18 +929,18 @@ __device__ __forceinline__ OrbitRS calc_orbit_core(const N &nd, const double *__
         // full-range bisection (which also settles the direction itself)
         const double2 *nodes = nd.rp;
         if (vp) {
-            kmin = ridx_zero_Q<false>(nodes, Cr.ri, rj, mj, inv, E, J, kp_lo, kp_hi, rp0, pp0, rp1, pp1);
+            kmin = ridx_zero_Q<false>(nodes, Cr.ri, q, kp_lo, kp_hi, rp0, pp0, rp1, pp1);
         } else {
-            kmin = find_zero_Q_n(nd, rj, mj, inv, kp_lo, kp_hi, E, J);
+            kmin = find_zero_Q_n(nd, rj, mj, P.inv_nstar, kp_lo, kp_hi, E, J);
             if (kmin >= 0) {
                 nd.RP(kmin, rp0, pp0);
                 nd.RP(kmin + 1, rp1, pp1);
             }
         }
         if (va) {
-            kmax = ridx_zero_Q<true>(nodes, Cr.ri, rj, mj, inv, E, J, ka_lo, ka_hi, ra0, pa0, ra1, pa1);
+            kmax = ridx_zero_Q<true>(nodes, Cr.ri, q, ka_lo, ka_hi, ra0, pa0, ra1, pa1);
         } else {
-            kmax = find_zero_Q_n(nd, rj, mj, inv, ka_lo, ka_hi, E, J);
+            kmax = find_zero_Q_n(nd, rj, mj, P.inv_nstar, ka_lo, ka_hi, E, J);
             if (kmax >= 0) {
                 nd.RP(kmax, ra0, pa0);
                 nd.RP(kmax + 1, ra1, pa1);
@@ -930,39 +961,32 @@ __device__ __forceinline__ OrbitRS calc_orbit_core(const N &nd, const double *__
         o.rp = o.ra = rj; o.kmin = o.kmax = j; o.dQdrp = o.dQdra = 0.0; o.circular = 1;
         return o;
     }
-    double a, b, rmin, rmax, inside_sqrt;
-    bool bad = false;
-    if (kmin == 0) set_a_b_n(nd, rj, mj, P, 0, &a, &b);
-    else set_a_b_nodes(rj, mj, P, rp0, pp0, rp1, pp1, &a, &b);
-    inside_sqrt = a * a - 2.0 * J * J * (b - E);
-    if (inside_sqrt < 0.0) {
-        rmin = -1.0 * J * J / a;
-        if ((rmin < rp0) || (rmin > rp1)) {
-            const RootVr rv = find_root_vr(r, phi, rj, mj, P.inv_nstar, P.cenma_m * P.madhoc, kmin, E, J);
-            rmin = rv.root;
-            bad |= rv.bad != 0;
-            o.brent = 1;
+    double ap, aa, b, rmin, rmax;
+    if (kmin == 0) set_a_b_n(nd, rj, mj, P, 0, &ap, &b);
+    else set_a_b_nodes(rj, mj, P, rp0, pp0, rp1, pp1, &ap, &b);
+    double inside_sqrt = ap * ap - 2.0 * J * J * (b - E);
+    if (inside_sqrt < 0.0) rmin = -1.0 * J * J / ap;
+    else rmin = J * J / (-ap + sqrt(inside_sqrt));
+    const bool brent_p = inside_sqrt < 0.0 && ((rmin < rp0) || (rmin > rp1));
+    if (kmax == 0) set_a_b_n(nd, rj, mj, P, 0, &aa, &b);
+    else set_a_b_nodes(rj, mj, P, ra0, pa0, ra1, pa1, &aa, &b);
+    inside_sqrt = aa * aa - 2.0 * J * J * (b - E);
+    if (inside_sqrt < 0.0) rmax = -aa / (2.0 * (b - E));
+    else rmax = (-aa + sqrt(inside_sqrt)) / (2.0 * (b - E));
+    const bool brent_a = inside_sqrt < 0.0 && ((rmax < ra0) || (rmax > ra1));
+    if (brent_p || brent_a) {
+        o.brent = 1;
+#pragma unroll 1
+        for (int side = 0; side < 2; side++) {
+            if (!(side ? brent_a : brent_p)) continue;
+            const RootVr rv = find_root_vr(r, phi, rj, mj, P.inv_nstar, P.cenma_m * P.madhoc, side ? kmax : kmin, E, J);
+            if (rv.bad) o.err = CMCG_E_BRENT;
+            if (side) rmax = rv.root;
+            else rmin = rv.root;
         }
-    } else {
-        rmin = J * J / (-a + sqrt(inside_sqrt));
     }
-    double dQdr_min = 2.0 * J * J / (rmin * rmin * rmin) + 2.0 * a / (rmin * rmin);
-    if (kmax == 0) set_a_b_n(nd, rj, mj, P, 0, &a, &b);
-    else set_a_b_nodes(rj, mj, P, ra0, pa0, ra1, pa1, &a, &b);
-    inside_sqrt = a * a - 2.0 * J * J * (b - E);
-    if (inside_sqrt < 0.0) {
-        rmax = -a / (2.0 * (b - E));
-        if ((rmax < ra0) || (rmax > ra1)) {
-            const RootVr rv = find_root_vr(r, phi, rj, mj, P.inv_nstar, P.cenma_m * P.madhoc, kmax, E, J);
-            rmax = rv.root;
-            bad |= rv.bad != 0;
-            o.brent = 1;
-        }
-    } else {
-        rmax = (-a + sqrt(inside_sqrt)) / (2.0 * (b - E));
-    }
-    double dQdr_max = 2.0 * J * J / (rmax * rmax * rmax) + 2.0 * a / (rmax * rmax);
-    if (bad) o.err = CMCG_E_BRENT;
+    const double dQdr_min = 2.0 * J * J / (rmin * rmin * rmin) + 2.0 * ap / (rmin * rmin);
+    const double dQdr_max = 2.0 * J * J / (rmax * rmax * rmax) + 2.0 * aa / (rmax * rmax);
     if ((rmin > rmax) || (dQdr_min <= 0.) || (dQdr_max >= 0.)) {
         o.rp = o.ra = rj; o.kmin = o.kmax = j; o.dQdrp = o.dQdra = 0.0; o.circular = 1;
     } else {
@@ -979,7 +1003,8 @@ __device__ __forceinline__ OrbitRS calc_orbit_from_n(const N &nd, const double *
                                                      int64_t ktemp)
 {
     const Coarse none{};
-    return calc_orbit_core<N, false>(nd, r, phi, n_max, j, rj, mj, P, E, J, ktemp, none);
+    const QStar unused{};
+    return calc_orbit_core<N, false>(nd, r, phi, n_max, j, rj, mj, P, E, J, ktemp, none, unused);
 }
 
 __device__ __forceinline__ OrbitRS calc_orbit_from(const double *__restrict__ r, const double *__restrict__ phi,

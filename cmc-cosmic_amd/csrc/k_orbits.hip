@@ -12,11 +12,12 @@
 // thread would stall the whole phase, so such stars are deferred: a grid-wide
 // search finds the same first positive index, and a tail kernel finishes them.
 //
-// The phase is bound by the rate of gathers into the sorted (r, phi) table (16 B a node,
-// a line each: about 5 a search and 4 a try), which at N = 4e6 is 64 MB and lives in
-// L2/MALL, by their latency and by the FP64 work of the exact apsides and tries; the
-// compulsory HBM traffic is 96 B/star.  Sampler at N = 4e6: 1071 us with about 12 gathers
-// a search and 6 a try (71 load instructions a wave), 873 now.
+// The phase is bound about equally by vector instructions (4000 a wave, 56% of the sampler's
+// time at N = 4e6), by the rate of gathers into the sorted (r, phi) table (16 B a node, a line
+// each: about 5 a search and 4 a try), which at N = 4e6 is 64 MB and lives in L2/MALL, and by
+// the gathers' latency; the compulsory HBM traffic is 96 B/star.  Sampler at N = 4e6: 1071 us
+// with about 12 gathers a search and 6 a try, 873 with these, 787 with division-free signs,
+// two-digit jumps and the tries' results through LDS instead of 5700 instructions a wave.
 #include "kernels.hpp"
 
 namespace {
@@ -32,18 +33,42 @@ constexpr int ORB_COARSE = 1024;     // LDS samples of the (r, phi) table per bl
 constexpr int NRED = 15, RED_STRIDE = 16;
 __device__ __forceinline__ bool red_is_max(int i) { return i == 0 || i == 12; }
 
+// The counts come from ballots and the removed stars' sums are formed only in waves that
+// have some (zeros add nothing), so a wave shuffles one value, not fifteen.
 template <int THREADS>
-__device__ void block_reduce_store(double (&v)[NRED], double *__restrict__ out)
+__device__ void block_reduce_store(double max_r, double Em, double Jm, double mm, int flags, int ntry, int hits, int misses,
+                                   double *__restrict__ out)
 {
     __shared__ double wsum[THREADS / 64][NRED];
-    for (int off = 32; off > 0; off >>= 1)
-        for (int i = 0; i < NRED; i++) {
-            double o = __shfl_xor(v[i], off);
-            v[i] = red_is_max(i) ? (v[i] >= o ? v[i] : o) : v[i] + o;
-        }
     const int w = threadIdx.x >> 6;
-    if ((threadIdx.x & 63) == 0)
-        for (int i = 0; i < NRED; i++) wsum[w][i] = v[i];
+    const bool first = (threadIdx.x & 63) == 0;
+    auto count = [](bool b) { return (int)__popcll(__ballot(b)); };
+    for (int off = 32; off > 0; off >>= 1) {
+        const double o = __shfl_xor(max_r, off);
+        max_r = max_r >= o ? max_r : o;
+    }
+    if (__ballot(flags & (CMCG_SF_REMOVED_E | CMCG_SF_REMOVED_RT)))
+        for (int off = 32; off > 0; off >>= 1) {
+            Em += __shfl_xor(Em, off);
+            Jm += __shfl_xor(Jm, off);
+            mm += __shfl_xor(mm, off);
+        }
+    int sum = 0, top = 0, bits = 0;            // tries: sum and maximum over the wave, bit by bit
+    for (; __ballot((ntry >> bits) != 0); bits++) sum += count((ntry >> bits) & 1) << bits;
+    uint64_t at_top = ~0ull;
+    while (bits-- > 0) {
+        const uint64_t m = at_top & __ballot((ntry >> bits) & 1);
+        if (m) { at_top = m; top |= 1 << bits; }
+    }
+    const int c[NRED - 5] = {count(flags & CMCG_SF_CIRCULAR),   count(flags & CMCG_SF_REMOVED_E),
+                             count(flags & CMCG_SF_REMOVED_RT), count(flags & CMCG_SF_DESTROYED),
+                             count(flags & CMCG_SF_BRENT),      count(flags & CMCG_SF_LINSCAN),
+                             sum, top, count(hits & 1) + 2 * count(hits & 2), count(misses & 1) + 2 * count(misses & 2)};
+    if (first) {
+        wsum[w][0] = max_r;
+        wsum[w][1] = Em; wsum[w][2] = Jm; wsum[w][3] = mm; wsum[w][4] = Em;
+        for (int i = 5; i < NRED; i++) wsum[w][i] = (double)c[i - 5];
+    }
     __syncthreads();
     if (threadIdx.x < NRED) {
         const int i = threadIdx.x;
@@ -53,16 +78,14 @@ __device__ void block_reduce_store(double (&v)[NRED], double *__restrict__ out)
     }
 }
 
-// outcome counters of one star into the partials
-__device__ __forceinline__ void count_star(double (&red)[NRED], int flags, int ntry, int hits, int misses,
-                                           bool count_linscan)
+// outcome counters of one deferred star into its record (its scan is counted where it was deferred)
+__device__ __forceinline__ void count_star(double (&red)[NRED], int flags, int ntry, int hits, int misses)
 {
     red[5] += (flags & CMCG_SF_CIRCULAR) ? 1.0 : 0.0;
     red[6] += (flags & CMCG_SF_REMOVED_E) ? 1.0 : 0.0;
     red[7] += (flags & CMCG_SF_REMOVED_RT) ? 1.0 : 0.0;
     red[8] += (flags & CMCG_SF_DESTROYED) ? 1.0 : 0.0;
     red[9] += (flags & CMCG_SF_BRENT) ? 1.0 : 0.0;
-    red[10] += (count_linscan && (flags & CMCG_SF_LINSCAN)) ? 1.0 : 0.0;
     red[11] += (double)ntry;
     red[12] = red[12] >= (double)ntry ? red[12] : (double)ntry;
     red[13] += (double)hits;
@@ -177,43 +200,35 @@ __device__ void sample_star(const N &nd, const DevFields &f, DevScalars *s, cons
 // accepted try).  A star's result is its lowest-numbered terminating try, exactly as
 // the sequential loop, so outputs do not depend on the grouping.
 
-// what a star's tries need (set by prepare_star)
+// What a star's tries need (set by prepare_star), and in its place their result, written by
+// the lane that ran the last one.
 struct TryCtx {
-    double rmin, rmax, F, E, J, rj, mj;
+    double rmin, rmax, F, E, rj, mj, J;
 };
-
-// result of a star's tries
 struct TryOut {
     double X, rr, vr, potr;
     int32_t kn;        // index of rr among the nodes
-    int k;             // tries taken; CMCG_N_TRY + 1 when none was accepted
-    bool bad, nan;
+    int32_t k;         // tries taken; CMCG_N_TRY + 1 when none was accepted
+    int32_t nan, pad;
+    double J;          // TryCtx::J
 };
-
-// q-th (from 0) set bit of m
-__device__ __forceinline__ int nth_set_bit(uint64_t m, int q)
-{
-    int pos = 0;
-#pragma unroll
-    for (int w = 32; w >= 1; w >>= 1) {
-        const uint64_t low = m & ((1ull << w) - 1ull);
-        const int c = __popcll(low);
-        if (q >= c) { q -= c; m >>= w; pos += w; }
-        else m = low;
-    }
-    return pos;
-}
+union TrySlot {
+    Rng rng;           // while the star's apsides are sought: its substream state, out of the registers
+    TryCtx in;
+    TryOut out;
+};
+static_assert(sizeof(TryCtx) == sizeof(TryOut) && offsetof(TryCtx, J) == offsetof(TryOut, J), "J is common to both");
 
 // The part of get_positions_loop between the positive-Q index and the rejection loop
 // (cmc_evolution_thr.c:832-857): apsides, removal at r_apo >= Rtidal, circular
 // orbits, and the loop's constants.  Returns true if the star samples a new radius.
 template <class N>
 __device__ __forceinline__ bool prepare_star(const N &nd, const DevFields &f, DevScalars *s, const KParams &P,
-                                             const Coarse &C, int64_t n, int64_t j, double rj, double mj,
-                                             double E, double J, double pj, int &flags, int &hits, int &misses,
-                                             TryCtx &tc)
+                                             const Coarse &C, int64_t n, int64_t j, const QStar &q, double pj, int &flags, int &hits, int &misses,
+                                             TrySlot &slot, Rng &rng)
 {
-    OrbitRS o = calc_orbit_core<N, true>(nd, f.r, f.phi, n, j, rj, mj, P, E, J, j, C, pj);
+    const double rj = q.rj;
+    OrbitRS o = calc_orbit_core<N, true>(nd, f.r, f.phi, n, j, rj, q.mj, P, q.E, q.J, j, C, q, pj);
     if (o.err) dev_set_error(s, o.err, j);
     hits = o.hint_hits;
     misses = o.hint_misses;
@@ -231,12 +246,15 @@ __device__ __forceinline__ bool prepare_star(const N &nd, const DevFields &f, De
         flags |= CMCG_SF_REMOVED_RT;      // its removal sums are added by the caller
         return false;
     }
-    tc.rmin = o.rp;
-    tc.rmax = o.ra;
-    const double g1 = sqrt(3.0 * (tc.rmax - tc.rmin) / o.dQdrp);
-    const double g2 = sqrt(-3.0 * (tc.rmax - tc.rmin) / o.dQdra);
+    f.r_peri[j] = o.rp;
+    f.r_apo[j] = o.ra;
+    const double g1 = sqrt(3.0 * (o.ra - o.rp) / o.dQdrp);
+    const double g2 = sqrt(-3.0 * (o.ra - o.rp) / o.dQdra);
+    rng = slot.rng;
+    TryCtx &tc = slot.in;
+    tc.rmin = o.rp; tc.rmax = o.ra;
     tc.F = 1.2 * (g1 >= g2 ? g1 : g2);
-    tc.E = E; tc.J = J; tc.rj = rj; tc.mj = mj;
+    tc.E = q.E; tc.J = q.J; tc.rj = rj; tc.mj = q.mj;
     return true;
 }
 
@@ -264,33 +282,47 @@ __device__ __forceinline__ bool one_try(const double2 *__restrict__ nodes, const
     return g0 < 1.0 / vr * drds;
 }
 
+__device__ __forceinline__ uint32_t from_lane(uint32_t x, int lane4)
+{
+    return (uint32_t)__builtin_amdgcn_ds_bpermute(lane4, (int)x);
+}
+
 // All lanes of the wave call this together (convergent).  need: this lane's star
-// samples; wctx: the wave's 64 try constants in LDS (slot = lane, written before a
-// block barrier); rng: this lane's substream state before its star's first try.
+// samples; slots: the wave's 64 try constants in LDS (slot = lane, written before a
+// block barrier), which hold the results on return; rng: this lane's substream state before
+// its star's first try.  Returns whether a try up to the star's last found no interval.
+// A round has R stars: c = 64 / R lanes each, one more for the first 64 - c R of them, but at
+// most CAP (then the rest idle): fewer wasted tries.  About 3.4 rounds a wave at CAP = 4.
 template <int CAP>
-__device__ void wave_tries(const double2 *__restrict__ nodes, const RIdx &ri, const KParams &P, int64_t n, bool need,
-                           const TryCtx *__restrict__ wctx, Rng rng, TryOut &out)
+__device__ bool wave_tries(const double2 *__restrict__ nodes, const RIdx &ri, const KParams &P, int64_t n, bool need,
+                           TrySlot *__restrict__ slots, Rng rng)
 {
     const int lane = threadIdx.x & 63;
     int next = 1;                         // owner: first try not yet evaluated
     bool bad_acc = false;
-    out.k = 0; out.bad = false; out.nan = false; out.kn = 0;
-    out.X = out.rr = out.vr = out.potr = 0.0;
     const double r1 = nodes[1].x;
+    auto rank_in = [](uint64_t m) {       // set bits of m below the lane
+        return (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
+    };
+    // quotients of integers up to 64 by the reciprocal's estimate: a half keeps them off the integers
+    auto over = [](float a, int b) { return (int)((a + 0.5f) * __builtin_amdgcn_rcpf((float)b)); };
     uint64_t pending = __ballot(need);
     while (pending) {
-        const int R = __popcll(pending);
-        int c = 64 / R, rem = 64 - c * R;
-        if (c >= CAP) { c = CAP; rem = 0; }              // at most CAP lanes per star: fewer wasted tries
-        const bool idle = lane >= c * R + rem;
-        int q, o, cs;
-        if (lane < (c + 1) * rem) { q = lane / (c + 1); o = lane % (c + 1); cs = c + 1; }
-        else { const int l2 = lane - (c + 1) * rem; q = rem + l2 / c; o = l2 % c; cs = c; }
-        const int sl = idle ? nth_set_bit(pending, 0) : nth_set_bit(pending, q);   // owner lane of the star helped
-        const TryCtx t = wctx[sl];
-        Rng st;
-        st.z0 = __shfl(rng.z0, sl); st.z1 = __shfl(rng.z1, sl); st.z2 = __shfl(rng.z2, sl); st.z3 = __shfl(rng.z3, sl);
-        const int k = __shfl(next, sl) + o;
+        const int R = (int)__popcll(pending), c64 = over(64.f, R);
+        const int c = c64 >= CAP ? CAP : c64, rem = c64 >= CAP ? 0 : 64 - c64 * R;
+        const bool owner = (pending >> lane) & 1ull;
+        const int my_q = rank_in(pending);
+        // lane q learns which lane owns the q-th star (the others fill the lanes after R)
+        const int own = __builtin_amdgcn_ds_permute((owner ? my_q : R + lane - my_q) << 2, lane);
+        const int big = (c + 1) * rem;
+        const bool in_big = lane < big;
+        const int cs = in_big ? c + 1 : c, l2 = in_big ? lane : lane - big;
+        const int g = over((float)l2, cs), o = l2 - g * cs, q = in_big ? g : rem + g;
+        const bool idle = q >= R;
+        const int sl = (int)from_lane((uint32_t)own, idle ? 0 : q << 2), sl4 = sl << 2;   // owner of the star helped
+        const TryCtx t = slots[sl].in;
+        Rng st{from_lane(rng.z0, sl4), from_lane(rng.z1, sl4), from_lane(rng.z2, sl4), from_lane(rng.z3, sl4)};
+        const int k = (int)from_lane((uint32_t)next, sl4) + o;
         const bool eval = !idle && k <= CMCG_N_TRY;
         if (!idle)
             for (int d = 0; d < 2 * o; d++) (void)rng_int(st);
@@ -299,58 +331,54 @@ __device__ void wave_tries(const double2 *__restrict__ nodes, const RIdx &ri, co
         bool bad = false, nan = false, term = false;
         if (eval) {
             term = one_try(nodes, ri, r1, P, n, t, st, X, rr, vr, potr, kn, bad, nan);
-            Rng sg = st;
-            if (term && !nan && rng_dbl(sg) < 0.5) vr = -vr;    // sign draw after the accepted try
-        }
-        // the last try of a round that ends without acceptance also signs its v_r:
-        // it is the final try when the star runs out of tries
-        if (eval && !term && k == CMCG_N_TRY) {
-            Rng sg = st;
-            if (rng_dbl(sg) < 0.5) vr = -vr;
-        }
-        const uint64_t tmask = __ballot(eval && term), bmask = __ballot(eval && bad);
-        // owners collect their star's lanes [base, base + cs)
-        const int my_q = __popcll(pending & ((1ull << lane) - 1ull));
-        const bool owner = (pending >> lane) & 1ull;
-        const int my_cs = my_q < rem ? c + 1 : c;
-        const int base = my_q < rem ? my_q * (c + 1) : rem * (c + 1) + (my_q - rem) * c;
-        const uint64_t span = (my_cs >= 64 ? ~0ull : ((1ull << my_cs) - 1ull)) << base;
-        const uint64_t tw = tmask & span;
-        const int last_k = next + my_cs - 1;               // owner: its last try this round
-        int src = -1;
-        bool done = false;
-        if (owner) {
-            if (tw) { src = __ffsll((unsigned long long)tw) - 1; done = true; }
-            else if (last_k >= CMCG_N_TRY) { src = base + (CMCG_N_TRY - next); done = true; }
-            else src = base + my_cs - 1;        // continue from the round's last try
-        }
-        const int srcl = src < 0 ? lane : src;
-        const double sX = __shfl(X, srcl), srr = __shfl(rr, srcl), svr = __shfl(vr, srcl), spot = __shfl(potr, srcl);
-        const int snan = __shfl((int)nan, srcl), skn = __shfl(kn, srcl);
-        Rng ns;
-        ns.z0 = __shfl(st.z0, srcl); ns.z1 = __shfl(st.z1, srcl); ns.z2 = __shfl(st.z2, srcl); ns.z3 = __shfl(st.z3, srcl);
-        if (owner) {
-            // bad of the tries up to the final one (or all of this round's if none ended)
-            const uint64_t upto = (src >= 63 ? ~0ull : ((1ull << (src + 1)) - 1ull)) & span;
-            bad_acc |= (bmask & upto) != 0ull;
-            if (done) {
-                out.X = sX; out.rr = srr; out.vr = svr; out.potr = spot; out.nan = snan != 0; out.kn = skn;
-                out.k = tw ? next + (src - base) : CMCG_N_TRY + 1;
-                out.bad = bad_acc;
-            } else {
-                next += my_cs;
-                rng = ns;
+            // the sign draw follows the accepted try, or the last one if the star runs out of them
+            if ((term && !nan) || k == CMCG_N_TRY) {
+                Rng sg = st;
+                if (rng_dbl(sg) < 0.5) vr = -vr;
             }
         }
-        pending &= ~__ballot(owner && done);
+        // the star's lanes are [lane - o, lane - o + cs); its result is their first that ends
+        const uint64_t tmask = __ballot(eval && term), bmask = __ballot(eval && bad);
+        const uint64_t ones = cs >= 64 ? ~0ull : (1ull << cs) - 1ull;
+        const uint64_t mine = (tmask >> (lane - o)) & ones;
+        const bool win = eval && (term ? (mine & ((1ull << o) - 1ull)) == 0ull : (k == CMCG_N_TRY && mine == 0ull));
+        if (win) {
+            TryOut &r = slots[sl].out;
+            r.X = X; r.rr = rr; r.vr = vr; r.potr = potr; r.kn = kn;
+            r.k = term ? k : CMCG_N_TRY + 1;
+            r.nan = nan;
+        }
+        const uint64_t wmask = __ballot(win);
+        // owners: the star's lanes are [base, base + my_cs)
+        const int my_cs = my_q < rem ? c + 1 : c;
+        const int base = owner ? my_q * c + (my_q < rem ? my_q : rem) : 0;
+        const uint64_t my_ones = my_cs >= 64 ? ~0ull : (1ull << my_cs) - 1ull;
+        const uint64_t won = (wmask >> base) & my_ones;
+        const bool done = owner && won != 0ull;
+        if (bmask && owner) {              // up to the final try, or all of this round's
+            const uint64_t upto = done ? ((won << 1) - 1ull) : my_ones;
+            bad_acc |= ((bmask >> base) & my_ones & upto) != 0ull;
+        }
+        const int last4 = (base + my_cs - 1) << 2;
+        const Rng ns{from_lane(st.z0, last4), from_lane(st.z1, last4), from_lane(st.z2, last4), from_lane(st.z3, last4)};
+        if (owner && !done) {              // go on from the round's last try
+            next += my_cs;
+            rng = ns;
+        }
+        pending &= ~__ballot(done);
     }
+    // the results come from other lanes of the wave
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    return bad_acc;
 }
 
 // Slot j draws from offset j 2^20 (base[2]: the state of slot 1): the wave jumps to its
 // first slot, its lanes on through the LDS tables.  With learned brackets the network's
 // prediction proposes both find_zero_Q brackets.
 // MINB: blocks per CU the register allocation must allow (1: no constraint; 5 blocks of 256
-// threads: five waves per SIMD, 96 registers)
+// threads: five waves per SIMD, at most 102 registers)
 template <int THREADS, int COARSE, int CAP, int MINB>
 struct orbits_kernel {
     static constexpr int LB = THREADS, MB = MINB;
@@ -365,46 +393,60 @@ struct orbits_kernel {
                                                              const double2 *__restrict__ coarse,
                                                              const uint32_t *__restrict__ ridx, int ridx_bits)
 {
-    // the jump tables are needed only for the lanes' first states, the try constants
-    // only after the apsides: one LDS area serves both
+    // the jump table is needed only for the lanes' first states: the samples wait in
+    // registers and take its place (31 KB in all: five blocks share a CU's 160 KB)
     __shared__ union alignas(16) Share {
-        NibbleTables lt;
-        TryCtx ctx[THREADS];
+        LaneDigit lt;
+        struct { double cr[COARSE + 1], cphi[COARSE + 1]; } c;
     } sh;
-    TryCtx *const ctx = sh.ctx;
-    __shared__ double cr[COARSE + 1], cphi[COARSE + 1];
+    __shared__ TrySlot slot[THREADS];
+    double *const cr = sh.c.cr, *const cphi = sh.c.cphi;
     const int64_t n = s->n_max;
     Coarse C;
     C.cr = cr; C.cphi = cphi; C.cs = COARSE; C.n1 = n + 1;
     C.stride = coarse_stride(n, COARSE);
+    C.inv_stride = 0xffffffffu / (uint32_t)C.stride;
     C.hint = false; C.lrp = C.lra = 0.f; C.margin = margin;
     C.mid = mid;
     C.ri.t = nullptr;
     if (n >= 1) C.ri = ridx_of(ridx, nodes, n, ridx_bits);
-    // built once per phase: a contiguous copy
-    for (int sI = threadIdx.x; sI <= COARSE; sI += blockDim.x) {
-        const double2 v = coarse[sI];
-        cr[sI] = v.x;
-        cphi[sI] = v.y;
-    }
+    constexpr int NC = COARSE / THREADS;
+    static_assert(COARSE % THREADS == 0, "the samples are dealt out evenly, and one more");
+    double2 sample[NC];                        // built once per phase
+#pragma unroll
+    for (int u = 0; u < NC; u++) sample[u] = coarse[threadIdx.x + u * THREADS];
     {
-        constexpr int NQ = (int)(sizeof(NibbleTables) / sizeof(uint4));
-        const uint4 *src = reinterpret_cast<const uint4 *>(&jump->orbit);
+        constexpr int NQ = (int)(sizeof(LaneDigit) / sizeof(uint4));
+        const uint4 *src = reinterpret_cast<const uint4 *>(&jump->orbit.lo);
         uint4 *dst = reinterpret_cast<uint4 *>(&sh.lt);
-        for (int q = threadIdx.x; q < NQ; q += blockDim.x) dst[q] = src[q];
+        for (int q = threadIdx.x; q < NQ; q += THREADS) dst[q] = src[q];
     }
     const int64_t j = 1 + xcd_block(kg_) * blockDim.x + threadIdx.x;
     Rng rng = jump_uniform(jump->level + JL_SLOT + 1, JL_SLOT_N - 1, rng_uniform(base[2]),
                            (uint32_t)__builtin_amdgcn_readfirstlane((int)((j - 1) >> 6)));
     __syncthreads();
-    rng = rng_jump_lds(sh.lt, rng, (uint32_t)((j - 1) & 63));
-    __syncthreads();                           // the tables are dead from here
+    rng = jump_lane_digits(jump->orbit.hi, sh.lt, rng);
+    slot[threadIdx.x].rng = rng;
+    asm volatile("" ::: "memory");             // ... so that it is read again there
+    __syncthreads();                           // the table is dead from here
+#pragma unroll
+    for (int u = 0; u < NC; u++) {
+        cr[threadIdx.x + u * THREADS] = sample[u].x;
+        cphi[threadIdx.x + u * THREADS] = sample[u].y;
+    }
+    if (threadIdx.x == 0) {
+        const double2 last = coarse[COARSE];
+        cr[COARSE] = last.x;
+        cphi[COARSE] = last.y;
+    }
+    __syncthreads();
     bool need = false;
     int flags = 0, ntry = 0, hits = 0, misses = 0;
     if (j <= n) {
         const double rj = f.r[j], mj = f.m[j];
         const double Ej = f.E[j], J = f.J[j];
         const double E = Ej + phi_s_own(rj, mj, P.inv_nstar, rj);    // cmc_evolution_thr.c:806
+        const QStar q = q_star(rj, mj, P.inv_nstar, E, J);
         if (mj < CMCG_ZERO) {
             // destroy_obj (cmc_dynamics_helper.c:131-153) + remove_star_center
             f.vr[j] = 0.0; f.vt[j] = 0.0; f.E[j] = 0.0; f.J[j] = 0.0; f.id[j] = 0;
@@ -417,7 +459,7 @@ struct orbits_kernel {
             flags = CMCG_SF_REMOVED_E;
         } else {
             const double pj = f.phi[j];
-            if (q_le0(q_sign(rj, mj, P.inv_nstar, rj, pj, E, J))) {
+            if (q_le0(q_sign(q, rj, pj))) {
                 // linear-scan case: finished by the deferred path
                 flags = CMCG_SF_LINSCAN;
                 unsigned long long slot = atomicAdd((unsigned long long *)&s->n_defer, 1ull);
@@ -430,42 +472,40 @@ struct orbits_kernel {
                     C.lrp = y.x;
                     C.lra = y.y;
                 }
-                need = prepare_star(PackedNodes{nodes}, f, s, P, C, n, j, rj, mj, E, J, pj, flags, hits, misses,
-                                    ctx[threadIdx.x]);
+                need = prepare_star(PackedNodes{nodes}, f, s, P, C, n, j, q, pj, flags, hits, misses,
+                                    slot[threadIdx.x], rng);
             }
         }
     }
     __syncthreads();                           // try constants visible to the wave
     // every lane of the wave takes part, stars or not
-    TryOut to;
-    wave_tries<CAP>(nodes, C.ri, P, n, need, ctx + (threadIdx.x & ~63), rng, to);
-    double red[NRED];
-    for (int i = 0; i < NRED; i++) red[i] = 0.0;
+    const bool bad = wave_tries<CAP>(nodes, C.ri, P, n, need, slot + (threadIdx.x & ~63), rng);
+    double max_r = 0.0, Em = 0.0, Jm = 0.0, mm = 0.0;
     if (j <= n) {
         if (need) {
-            const TryCtx &tc = ctx[threadIdx.x];
-            if (to.bad) dev_set_error(s, CMCG_E_BRACKET, j);
+            const TryOut to = slot[threadIdx.x].out;
+            if (bad) dev_set_error(s, CMCG_E_BRACKET, j);
             if (to.nan) dev_set_error(s, CMCG_E_NAN, j);
             else if (to.k == CMCG_N_TRY + 1) dev_set_error(s, CMCG_E_NTRY, j);
             ntry = to.k;
             f.X[j] = to.X;
-            f.r_peri[j] = tc.rmin;
-            f.r_apo[j] = tc.rmax;
             f.rnew[j] = to.rr;
             f.knew[j] = knew_of(to.kn, to.rr);
             f.vrnew[j] = to.vr;
-            f.vtnew[j] = tc.J / to.rr;
+            f.vtnew[j] = to.J / to.rr;
             f.pot_rnew[j] = to.potr;
             flags |= 256;      // sampled: pot_rnew holds potential(rnew)
-            red[0] = to.rr;
+            max_r = to.rr;
         }
-        if (flags & (CMCG_SF_REMOVED_E | CMCG_SF_REMOVED_RT))
-            removed(red, f.E[j], f.J[j], f.m[j], P);     // fields the removal left unchanged
+        if (flags & (CMCG_SF_REMOVED_E | CMCG_SF_REMOVED_RT)) {      // fields the removal left unchanged
+            double red[NRED];
+            removed(red, f.E[j], f.J[j], f.m[j], P);
+            Em = red[1]; Jm = red[2]; mm = red[3];
+        }
         f.flags[j] = flags;
         f.ntry[j] = ntry;
-        count_star(red, flags, ntry, hits, misses, true);
     }
-    block_reduce_store<THREADS>(red, partials + RED_STRIDE * xcd_block(kg_));
+    block_reduce_store<THREADS>(max_r, Em, Jm, mm, flags, ntry, hits, misses, partials + RED_STRIDE * xcd_block(kg_));
 }
 };
 
@@ -579,7 +619,7 @@ struct defer_tail_kernel {
                         rj, mj, E, Ej, J, kt, flags, ntry, hits, misses, red);
             f.flags[j] = flags;
             f.ntry[j] = ntry;
-            count_star(red, flags, ntry, hits, misses, false);
+            count_star(red, flags, ntry, hits, misses);
             for (int i = 0; i < NRED; i++) part[t][i] = red[i];
         }
         __syncthreads();
@@ -871,8 +911,9 @@ struct OrbVariant { OrbFn fn; int threads, coarse, cap, minb; };
 #define ORB_V(T, C, K, M) {orbits_launch<T, C, K, M>, T, C, K, M}
 const OrbVariant kOrbVariants[] = {
     // the first is the default: five waves per SIMD hide the gathers best and at most four
-    // lanes per star waste few tries.  Sampler time, default / the same unconstrained / with
-    // 64 lanes: N = 4e6 873 / 972 / 1020 us, 1e6 225 / 246 / 262, 3e5 75 / 87 / 99, 1e4 40 / 41 / 46.
+    // lanes per star waste few tries.  Sampler time, default / with 64 lanes / 128 threads (whose
+    // LDS allows fewer waves): N = 4e6 787 / 861 / 1006 us, 1e6 192 / 211 / 257, 3e5 60 / 71 / 87,
+    // 1e4 33 / 40 / 39.
     ORB_V(256, 1024, 4, 5),  ORB_V(256, 512, 64, 1), ORB_V(256, 2048, 64, 1), ORB_V(128, 1024, 64, 1),
     ORB_V(512, 1024, 64, 1), ORB_V(128, 512, 64, 1), ORB_V(256, 1024, 2, 1),  ORB_V(256, 1024, 4, 1),
     ORB_V(256, 1024, 8, 1),  ORB_V(256, 512, 4, 1),  ORB_V(256, 1024, 64, 1), ORB_V(256, 512, 4, 5),
