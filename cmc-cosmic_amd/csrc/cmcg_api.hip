@@ -239,7 +239,6 @@ struct set_dt_step_kernel {
     if (step >= 0) s->step = (uint64_t)step;
 }
 };
-struct step_end_kernel { static constexpr int LB = 1024, MB = 0; static __device__ __forceinline__ void run(KGrid kg_, DevScalars *s) { s->step += 1; } };
 
 // payload field lists for the sort
 struct SortSpec {
@@ -499,7 +498,6 @@ int cmcg_create(cmcg_ctx **out, int device, int64_t n_cap, const cmcg_params *pa
     if (sc.max_blocks < 1024) sc.max_blocks = 1024;   // the stripping passes' fixed grid
     const SortShape sort_max = sort_shape(n_cap);
     sc.sort_mat_cap = (size_t)sort_max.tiles * sort_max.buckets;
-    sc.merge_ends_cap = 2 * (n_cap / 256 + 4);       // two per merge block of set_velocities3 (>= 256 stars)
     sc.sort_aos_cap = n_cap + 4;
     // about two radial-index buckets per star: 2^10 .. 2^23 buckets (at N = 4e6 one per
     // star makes the orbit sampler 3% slower; four per star cost more to build than the
@@ -515,14 +513,14 @@ int cmcg_create(cmcg_ctx **out, int device, int64_t n_cap, const cmcg_params *pa
         (e = dalloc(c, &sc.sort_first, SB_MAX_BUCKETS + 1)) ||
         (e = dalloc(c, &sc.sort_order, 2 * (size_t)sc.sort_aos_cap)) ||
         (e = dalloc(c, &sc.mid, (size_t)(n_cap + 2) / MID_STEP + 4)) || (e = dalloc(c, &sc.nodes, (size_t)n_cap + 8)) || (e = dalloc(c, &sc.u_old, 2 * ((size_t)n_cap + 8))) ||
-        (e = dalloc(c, &sc.merge_ends, (size_t)sc.merge_ends_cap)) || (e = dalloc(c, &sc.sv3_dpre, (size_t)n_cap + 6)) || (e = dalloc(c, &sc.dt_part, (size_t)64 * 16)) || (e = dalloc(c, &sc.coarse, (size_t)ORB_MAX_COARSE + 8)) || (e = dalloc(c, &sc.red2, (size_t)RED2_BLOCKS * 16)) ||
+        (e = dalloc(c, &sc.sv3_dpre, (size_t)n_cap + 6)) || (e = dalloc(c, &sc.dt_part, (size_t)64 * 16)) || (e = dalloc(c, &sc.coarse, (size_t)ORB_MAX_COARSE + 8)) || (e = dalloc(c, &sc.red2, (size_t)RED2_BLOCKS * 16)) ||
         (e = dalloc(c, &sc.vals_a, (size_t)n_cap + 4)) ||
         (e = dalloc(c, &sc.excess_c, (size_t)n_cap + 6)) || (e = dalloc(c, &sc.excess_list, (size_t)n_cap + 2)) ||
         (e = dalloc(c, &sc.sv3_wend, (size_t)n_cap + 2)) || (e = dalloc(c, &sc.sv3_merged, (size_t)n_cap + 2)) ||
         (e = dalloc(c, &sc.sv3_blk, (size_t)sc.max_blocks)) || (e = dalloc(c, &sc.sv3_fallback, 1)) ||
         (e = dalloc(c, &sc.strip_done, 1)) || (e = dalloc(c, &sc.chain_x, (size_t)n_cap + 8)) ||
         (e = dalloc(c, &sc.chain_g, (size_t)n_cap + 8)) ||
-        (e = dalloc(c, &sc.defer_list, (size_t)P.defer_cap)) || (e = dalloc(c, &sc.defer_kfirst, (size_t)P.defer_cap)) ||
+        (e = dalloc(c, &sc.defer_list, (size_t)P.defer_cap)) || (e = dalloc(c, &sc.defer_kfirst, (size_t)P.defer_cap)) || (e = dalloc(c, &sc.defer_order, (size_t)P.defer_cap)) ||
         (e = dalloc(c, &sc.chain_scal, 4)) || (e = dalloc(c, &sc.chain_len, 4)) || (e = dalloc(c, &sc.chain_fbad, 8)) ||
         (e = dalloc(c, &sc.esa_idx, (size_t)sc.esa_max)) || (e = dalloc(c, &sc.esa_racc, (size_t)sc.esa_max)) ||
         (e = dalloc(c, &sc.esa_v, (size_t)sc.esa_max)) || (e = dalloc(c, &sc.esa_n, 8)) ||
@@ -1094,41 +1092,43 @@ int cmcg_init_cluster(cmcg_ctx *c)
 // stripping loop is a few guarded grid passes and a one-block tail that finishes a
 // longer loop (no host round trip), so the whole step can be captured; nub bounds
 // the grids (the kernels read N_MAX on the device).
-constexpr int STRIP_GRAPH_PASSES = 3;     // grid passes; a one-block tail kernel finishes rarer longer loops
-
 static int enqueue_step(cmcg_ctx *c, int64_t nub, bool graph)
 {
+    const bool one_strip = strip_one_block(nub);
+    // bounds of r_apo per block for the stripping passes, in scratch that is free until set_velocities3
+    double *apo_max = c->params.tidal_strip ? reinterpret_cast<double *>(c->sc.sv3_blk) : nullptr;
     {
         PhaseTimer t(c, "timestep");
-        LAUNCH(launch_step_begin(c->s, c->stream));                 // also starts the time step's minimum
-        // calc_sigma_r with simul_relax_new, then Dt and the RNG bases
+        // the step's begin, calc_sigma_r with simul_relax_new, then Dt and the RNG bases
         LAUNCH(launch_timestep_sigma(c->f, c->s, c->kp, c->sc, nub, c->stream));
     }
     {
         // relaxation with energy_conservation1 fused in
         PhaseTimer t(c, "relax");
         LAUNCH(launch_relax(c->f, c->s, c->kp, c->sc, nub, c->stream, true, c->relax_threads));
-        LAUNCH(launch_after_dynamics(c->s, c->stream));
     }
     {
         PhaseTimer t(c, "orbits");
         hipEvent_t ka = nullptr, kb = nullptr;
         kernel_events(c, "orbits_kernel", ka, kb);
         LAUNCH(launch_orbits(c->f, c->s, c->kp, c->T, c->sc, nub, c->stream, c->learned ? &c->mlp : nullptr,
-                             c->margin, ka, kb, c->orb_variant, c->pred_fixed));
+                             c->margin, ka, kb, c->orb_variant, c->pred_fixed, true));
         if (c->harvest) LAUNCH(launch_mlp_harvest(c->f, c->s, c->kp, c->mlp, nub, c->stream));
     }
     {
-        // energy_conservation2 with ComputeIntermediateEnergy's EI fused in
+        // energy_conservation2 with ComputeIntermediateEnergy's EI and the stripping's begin fused in
         PhaseTimer t(c, "glue_pre_sort");
-        LAUNCH(launch_energy_conservation2(c->f, c->s, c->kp, nub, c->stream, true, c->sc.sv3_dpre));
-        if (c->params.tidal_strip)
-            LAUNCH(launch_strip(c->f, c->s, c->kp, c->sc, c->sc.strip_done, nub, graph ? STRIP_GRAPH_PASSES : 2, true,
-                                c->stream));
+        LAUNCH(launch_energy_conservation2(c->f, c->s, c->kp, nub, c->stream, true, c->sc.sv3_dpre,
+                                           c->params.tidal_strip ? c->sc.strip_done : nullptr, apo_max));
+        if (c->params.tidal_strip) {
+            if (one_strip) LAUNCH(launch_strip_loop(c->f, c->s, c->kp, c->sc, graph, c->stream, apo_max));
+            else LAUNCH(launch_strip(c->f, c->s, c->kp, c->sc, c->sc.strip_done, nub, graph ? STRIP_GRAPH_PASSES : 2, false,
+                                     c->stream, apo_max));
+        }
     }
-    if (c->params.tidal_strip) {
+    if (c->params.tidal_strip && !one_strip) {
         if (graph) {
-            LAUNCH(launch_strip_tail(c->f, c->s, c->kp, c->sc, c->stream));
+            LAUNCH(launch_strip_tail(c->f, c->s, c->kp, c->sc, c->stream, apo_max));
         } else {
             // the stripping loop normally ends within two passes; otherwise continue it here
             for (int guard = 0; guard < 100000; guard++) {
@@ -1136,7 +1136,7 @@ static int enqueue_step(cmcg_ctx *c, int64_t nub, bool graph)
                 if (sync(c) != hipSuccess) return CMCG_E_HIP;
                 if (hipMemcpy(&done, c->sc.strip_done, 4, hipMemcpyDeviceToHost) != hipSuccess) return CMCG_E_HIP;
                 if (done) break;
-                LAUNCH(launch_strip(c->f, c->s, c->kp, c->sc, c->sc.strip_done, nub, 1, false, c->stream));
+                LAUNCH(launch_strip(c->f, c->s, c->kp, c->sc, c->sc.strip_done, nub, 1, false, c->stream, apo_max));
             }
         }
     }
@@ -1157,8 +1157,7 @@ static int enqueue_step(cmcg_ctx *c, int64_t nub, bool graph)
         PhaseTimer t(c, "glue_post_sort");
         // the sort above read the old sorted radii from what is now the alternate r
         LAUNCH(launch_set_velocities3(c->f, c->s, c->kp, c->sc, nub, c->stream, c->alt.r, c->sc.sv3_dpre));
-        LAUNCH(launch_compute_energy(c->f, c->s, c->kp, c->sc, nub, c->stream));
-        kl<step_end_kernel>(dim3(1), dim3(1), 0, c->stream, c->s);
+        LAUNCH(launch_compute_energy(c->f, c->s, c->kp, c->sc, nub, c->stream, true));
     }
     c->parity ^= 1;
     return CMCG_OK;

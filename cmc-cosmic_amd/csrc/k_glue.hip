@@ -9,58 +9,42 @@ namespace {
 constexpr int GT = 256;
 __device__ __forceinline__ double sqr(double x) { return x * x; }
 
+// Sums over GT threads by halving (off = GT / 2 .. 1: thread t < off adds thread t + off's), in
+// v of thread 0: the first two halvings through LDS, the rest by shuffles of the first wave (one
+// barrier, not nine).  t: the thread's index among the GT.
+template <int NV>
+__device__ __forceinline__ void tree_sum(double (&v)[NV], double (*lds)[GT], int t)
+{
+    static_assert(GT == 256, "two halvings down to a wave");
+    for (int i = 0; i < NV; i++) lds[i][t] = v[i];
+    __syncthreads();
+    if (t < 64) {
+        for (int i = 0; i < NV; i++) v[i] = (lds[i][t] + lds[i][t + 128]) + (lds[i][t + 64] + lds[i][t + 192]);
+        for (int off = 32; off > 0; off >>= 1)
+            for (int i = 0; i < NV; i++) v[i] += __shfl_down(v[i], off, 64);
+    }
+}
+
 template <int NV>
 __device__ void block_sum_store(double (&v)[NV], double *__restrict__ out)
 {
     __shared__ double lds[NV][GT];
-    const int t = threadIdx.x;
-    for (int i = 0; i < NV; i++) lds[i][t] = v[i];
-    __syncthreads();
-    for (int off = GT / 2; off > 0; off >>= 1) {
-        if (t < off)
-            for (int i = 0; i < NV; i++) lds[i][t] += lds[i][t + off];
-        __syncthreads();
-    }
-    if (t == 0)
-        for (int i = 0; i < NV; i++) out[i] = lds[i][0];
+    tree_sum<NV>(v, lds, threadIdx.x);
+    if (threadIdx.x == 0)
+        for (int i = 0; i < NV; i++) out[i] = v[i];
 }
 
+// the sum of block partials, in res of thread 0
 template <int NV>
 __device__ void final_sum(const double *__restrict__ partials, int64_t nblocks, double (&res)[NV])
 {
     __shared__ double lds[NV][GT];
-    const int t = threadIdx.x;
-    double acc[NV];
-    for (int i = 0; i < NV; i++) acc[i] = 0.0;
+    for (int i = 0; i < NV; i++) res[i] = 0.0;
 #pragma unroll 8
-    for (int64_t b = t; b < nblocks; b += GT)      // unrolled: independent loads in flight
-        for (int i = 0; i < NV; i++) acc[i] += partials[8 * b + i];
-    for (int i = 0; i < NV; i++) lds[i][t] = acc[i];
-    __syncthreads();
-    for (int off = GT / 2; off > 0; off >>= 1) {
-        if (t < off)
-            for (int i = 0; i < NV; i++) lds[i][t] += lds[i][t + off];
-        __syncthreads();
-    }
-    for (int i = 0; i < NV; i++) res[i] = lds[i][0];
+    for (int64_t b = threadIdx.x; b < nblocks; b += GT)      // unrolled: independent loads in flight
+        for (int i = 0; i < NV; i++) res[i] += partials[8 * b + i];
+    tree_sum<NV>(res, lds, threadIdx.x);
 }
-
-// cmc.c:246-258, 278: per-step resets
-struct step_begin_kernel {
-    static constexpr int LB = 1024, MB = 0;
-    static __device__ __forceinline__ void run(KGrid kg_, DevScalars *s)
-{
-    s->Eescaped_old = s->Eescaped;
-    s->Jescaped_old = s->Jescaped;
-    s->TidalMassLoss_old = s->TidalMassLoss;
-    s->Etidal_old = s->Etidal;
-    s->Eescaped = 0.0; s->Jescaped = 0.0; s->TidalMassLoss = 0.0; s->Etidal = 0.0;
-    s->n_max_new = s->n_max;
-    s->dtrel = __longlong_as_double(0x7ff0000000000000ll);     // the time step's minimum starts at +inf
-}
-};
-
-struct after_dynamics_kernel { static constexpr int LB = 1024, MB = 0; static __device__ __forceinline__ void run(KGrid kg_, DevScalars *s) { s->Prev_Dt = s->Dt; } };   // cmc.c:297
 
 struct ec1_kernel {
     static constexpr int LB = 1024, MB = 0;
@@ -108,32 +92,56 @@ struct ec2_kernel {
 // It also forms D = vold^2 + 2 (1 - q) (Uoldrold - Uoldrnew), the part of
 // set_velocities3's vnew^2 (cmc_utils.c:242-247) that reaches it through the permutation
 // in place of its four inputs: the same operations in the same order, so the same double.
+// With strip_done it also begins the stripping loop that follows, and leaves every block's
+// largest r_apo of the stars that loop may strip: a pass then reads the stars of the blocks
+// that reach beyond the tidal radius only (16 -> 6 us at N = 4e6, 20 -> 3 in one block at 6e4).
 struct ec2_ie_kernel {
-    static constexpr int LB = 1024, MB = 0;
-    static __device__ __forceinline__ void run(KGrid kg_, DevFields f, DevScalars *s, KParams P, double *__restrict__ dpre)
+    static constexpr int LB = GT, MB = 0;
+    static __device__ __forceinline__ void run(KGrid kg_, DevFields f, DevScalars *s, KParams P, double *__restrict__ dpre,
+                                               int32_t *strip_done, double *__restrict__ apo_max)
 {
-    int64_t i = 1 + (int64_t)kg_.bid * blockDim.x + threadIdx.x;
-    int64_t n = s->n_max;
-    if (i > n) return;
-    const double x = f.rnew[i];
-    double pot;
-    const int fl = f.flags[i];
-    if (fl & 256) {
-        pot = f.pot_rnew[i];
-    } else {
-        bool bad = false;
-        pot = potential_at(f.r, f.phi, n, x, 1, n + 1, &bad);
-        if (bad) dev_set_error(s, CMCG_E_BRACKET, i);
-        f.pot_rnew[i] = pot;
-        f.flags[i] = fl | 256;
+    __shared__ double wmax[GT / 64];
+    const int64_t i = 1 + (int64_t)kg_.bid * GT + threadIdx.x;
+    const int64_t n = s->n_max;
+    if (i == 1 && strip_done) {
+        s->Etidal = 0.0;        // cmc_evolution_thr.c:449
+        *strip_done = 0;
     }
-    const double Uoldrnew = pot + phi_s_own(f.r[i], f.m[i], P.inv_nstar, x);
-    f.Uoldrnew[i] = Uoldrnew;
-    if (x < 1.0e6) f.EI[i] = sqr(f.vr[i]) + sqr(f.vt[i]) + f.phi[i] - pot;
-    const double q = 0.5;
-    const double vtold = f.vtold[i], vrold = f.vrold[i];
-    const double vold2 = vtold * vtold + vrold * vrold;
-    dpre[i] = vold2 + 2.0 * (1.0 - q) * (f.Uoldrold[i] - Uoldrnew);
+    double apo = 0.0;
+    if (i <= n) {
+        const double x = f.rnew[i];
+        double pot;
+        const int fl = f.flags[i];
+        if (fl & 256) {
+            pot = f.pot_rnew[i];
+        } else {
+            bool bad = false;
+            pot = potential_at(f.r, f.phi, n, x, 1, n + 1, &bad);
+            if (bad) dev_set_error(s, CMCG_E_BRACKET, i);
+            f.pot_rnew[i] = pot;
+            f.flags[i] = fl | 256;
+        }
+        const double Uoldrnew = pot + phi_s_own(f.r[i], f.m[i], P.inv_nstar, x);
+        f.Uoldrnew[i] = Uoldrnew;
+        if (x < 1.0e6) f.EI[i] = sqr(f.vr[i]) + sqr(f.vt[i]) + f.phi[i] - pot;
+        const double q = 0.5;
+        const double vtold = f.vtold[i], vrold = f.vrold[i];
+        const double vold2 = vtold * vtold + vrold * vrold;
+        dpre[i] = vold2 + 2.0 * (1.0 - q) * (f.Uoldrold[i] - Uoldrnew);
+        if (apo_max && x < 1000000) apo = f.r_apo[i];
+    }
+    if (!apo_max) return;
+#pragma unroll
+    for (int o = 32; o >= 1; o >>= 1) {
+        const double other = __shfl_xor(apo, o, 64);
+        apo = other > apo ? other : apo;               // NaN: not beyond any radius, as in the pass
+    }
+    if ((threadIdx.x & 63) == 0) wmax[threadIdx.x >> 6] = apo;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        for (int w = 1; w < GT / 64; w++) apo = wmax[w] > apo ? wmax[w] : apo;
+        apo_max[kg_.bid] = apo;
+    }
 }
 };
 
@@ -153,38 +161,56 @@ struct strip_begin_kernel {
 // loop ends.  Passes after the end return at once, so a fixed number of passes can be
 // enqueued (or captured in a graph) without a host round trip.
 constexpr int STRIP_BLOCKS = 1024;
-constexpr int STRIP_TAIL_PASSES = 64;
+constexpr int STRIP_TAIL_PASSES = 64;     // after STRIP_GRAPH_PASSES grid passes of a captured step
+
+// Star i in one pass: strip it if it is due and add its share to (Eescaped, Jescaped,
+// DTidalMassLoss, Etidal).
+__device__ __forceinline__ void strip_star(DevFields &f, const KParams &P, double Rt, int64_t n, int64_t i, double (&v)[4])
+{
+    if (i <= n && f.r_apo[i] > Rt && f.rnew[i] < 1000000) {
+        double m = f.m[i], E = f.E[i], J = f.J[i];
+        f.rnew[i] = CMCG_SF_INFINITY; f.vrnew[i] = 0.0; f.vtnew[i] = 0.0;
+        f.knew[i] = -1;
+        v[0] += E * m / (double)P.n_star;   // Eescaped
+        v[1] += J * m / (double)P.n_star;   // Jescaped
+        v[2] += m / (double)P.n_star;       // DTidalMassLoss
+        v[3] += E * m / (double)P.n_star;   // Etidal
+        // destroy_obj
+        f.vr[i] = 0.0; f.vt[i] = 0.0; f.E[i] = 0.0; f.J[i] = 0.0; f.id[i] = 0;
+        f.X[i] = 0.0; f.Y[i] = 0.0; f.r_peri[i] = 0.0; f.r_apo[i] = 0.0;
+        f.rOld[i] = 0.0; f.Uoldrold[i] = 0.0; f.Uoldrnew[i] = 0.0; f.vrold[i] = 0.0; f.vtold[i] = 0.0;
+        f.EI[i] = 0.0;
+        f.m[i] = 2.2250738585072014e-308;
+        f.flags[i] |= CMCG_SF_STRIPPED;
+    }
+}
 
 // Block bi's share of one pass (stars 1 + bi*GT + t, stride nb*GT): strip them and
-// store the block's partial sums (Eescaped, Jescaped, DTidalMassLoss, Etidal).
+// store the block's partial sums.  apo_max (or null): bounds of r_apo per GT stars.
 __device__ void strip_block(DevFields &f, const KParams &P, double Rt, int64_t n, double *__restrict__ partials,
-                            unsigned nb, unsigned bi)
+                            unsigned nb, unsigned bi, const double *__restrict__ apo_max)
 {
     double v[4] = {0.0, 0.0, 0.0, 0.0};
-    for (int64_t i = 1 + (int64_t)bi * blockDim.x + threadIdx.x; i <= n; i += (int64_t)nb * blockDim.x) {
-        if (f.r_apo[i] > Rt && f.rnew[i] < 1000000) {
-            double m = f.m[i], E = f.E[i], J = f.J[i];
-            f.rnew[i] = CMCG_SF_INFINITY; f.vrnew[i] = 0.0; f.vtnew[i] = 0.0;
-            f.knew[i] = -1;
-            v[0] += E * m / (double)P.n_star;   // Eescaped
-            v[1] += J * m / (double)P.n_star;   // Jescaped
-            v[2] += m / (double)P.n_star;       // DTidalMassLoss
-            v[3] += E * m / (double)P.n_star;   // Etidal
-            // destroy_obj
-            f.vr[i] = 0.0; f.vt[i] = 0.0; f.E[i] = 0.0; f.J[i] = 0.0; f.id[i] = 0;
-            f.X[i] = 0.0; f.Y[i] = 0.0; f.r_peri[i] = 0.0; f.r_apo[i] = 0.0;
-            f.rOld[i] = 0.0; f.Uoldrold[i] = 0.0; f.Uoldrnew[i] = 0.0; f.vrold[i] = 0.0; f.vtold[i] = 0.0;
-            f.EI[i] = 0.0;
-            f.m[i] = 2.2250738585072014e-308;
-            f.flags[i] |= CMCG_SF_STRIPPED;
-        }
-    }
+    for (int64_t b = bi; b * GT < n; b += nb)
+        if (!apo_max || apo_max[b] > Rt) strip_star(f, P, Rt, n, 1 + b * GT + threadIdx.x, v);
     block_sum_store<4>(v, partials + 8 * bi);
 }
 
 __device__ __forceinline__ double strip_rtidal(const DevScalars *s, const KParams &P)
 {
     return P.orbit_r * pow(s->Mtotal - (s->TidalMassLoss - s->OldTidalMassLoss), 1.0 / 3.0);
+}
+
+// The scalars at the end of a pass with sums res (one thread), and the loop's exit
+__device__ void strip_update(DevScalars *s, double Rt, const double (&res)[4], int32_t *done)
+{
+    s->Rtidal = Rt;
+    s->Eescaped += res[0];
+    s->Jescaped += res[1];
+    s->Etidal += res[3];
+    s->TidalMassLoss += res[2];
+    s->DTidalMassLoss = res[2];
+    if (!(res[2] > 0)) *done = 1;
 }
 
 // The end of a pass: the block partials summed in block order, the scalars updated,
@@ -194,24 +220,16 @@ __device__ void strip_finish(DevScalars *s, double Rt, int32_t *done, const doub
 {
     double res[4];
     final_sum<4>(partials, nb, res);
-    if (threadIdx.x == 0) {
-        s->Rtidal = Rt;
-        s->Eescaped += res[0];
-        s->Jescaped += res[1];
-        s->Etidal += res[3];
-        s->TidalMassLoss += res[2];
-        s->DTidalMassLoss = res[2];
-        if (!(res[2] > 0)) *done = 1;
-    }
+    if (threadIdx.x == 0) strip_update(s, Rt, res, done);
 }
 
 struct strip_pass_kernel {
     static constexpr int LB = GT, MB = 0;
     static __device__ __forceinline__ void run(KGrid kg_, DevFields f, DevScalars *s, KParams P, const int32_t *done,
-                                               double *__restrict__ partials)
+                                               double *__restrict__ partials, const double *__restrict__ apo_max)
     {
         if (*done) return;
-        strip_block(f, P, strip_rtidal(s, P), s->n_max, partials, kg_.nb, kg_.bid);
+        strip_block(f, P, strip_rtidal(s, P), s->n_max, partials, kg_.nb, kg_.bid, apo_max);
     }
 };
 
@@ -233,7 +251,8 @@ struct strip_end_kernel {
 struct strip_tail_kernel {
     static constexpr int LB = GT, MB = 0;
     static __device__ __forceinline__ void run(KGrid kg_, DevFields f, DevScalars *s, KParams P, int32_t *done,
-                                                        double *__restrict__ partials, unsigned nb)
+                                                        double *__restrict__ partials, unsigned nb,
+                                                        const double *__restrict__ apo_max)
 {
     __shared__ int32_t sdone;
     for (int pass = 0; pass < STRIP_TAIL_PASSES; pass++) {
@@ -243,7 +262,10 @@ struct strip_tail_kernel {
         const double Rt = strip_rtidal(s, P);
         const int64_t n = s->n_max;
         __syncthreads();
-        for (unsigned bi = 0; bi < nb; bi++) strip_block(f, P, Rt, n, partials, nb, bi);
+        for (unsigned bi = 0; bi < nb; bi++) {
+            strip_block(f, P, Rt, n, partials, nb, bi, apo_max);
+            __syncthreads();               // its LDS is reused
+        }
         __threadfence_block();
         __syncthreads();
         strip_finish(s, Rt, done, partials, nb);
@@ -251,6 +273,67 @@ struct strip_tail_kernel {
         __syncthreads();
     }
     if (threadIdx.x == 0 && !*(volatile int32_t *)done) dev_set_error(s, CMCG_E_STRIP, 0);
+}
+};
+
+// The whole loop in one block for a cluster of at most STRIP_ONE stars: a pass strips and sums
+// only the groups of four blocks of the grid pass that may have something to strip, by the 256
+// threads that play each of their blocks with the same tree; the other blocks' sums are zero.
+// So the sums are those of the grid passes.  (A pass and its end took 9 us in two launches,
+// however few the stars, and a step has two passes at least, or in a captured step three and
+// the tail, 31 us; here all passes take 6 us at 1e4 stars, 23 at 6e4 of a King cluster at its tidal
+// radius.)
+constexpr int64_t STRIP_ONE = 65536;
+constexpr int STRIP_ONE_T = 1024;
+struct strip_one_kernel {
+    static constexpr int LB = STRIP_ONE_T, MB = 0;
+    static __device__ __forceinline__ void run(KGrid kg_, DevFields f, DevScalars *s, KParams P, int32_t *done,
+                                               int max_passes, bool report, const double *__restrict__ apo_max)
+{
+    __shared__ double lds[4][4][GT];
+    __shared__ double blk[4][STRIP_ONE / GT];      // the grid pass's block sums
+    __shared__ uint32_t found[STRIP_ONE / STRIP_ONE_T];
+    __shared__ bool more;
+    const int t = threadIdx.x, vt = t & (GT - 1), sub = t >> 8;
+    const int64_t n = s->n_max;
+    const int groups = (int)((n + STRIP_ONE_T - 1) / STRIP_ONE_T);
+    for (int pass = 0; pass < max_passes; pass++) {
+        const double Rt = strip_rtidal(s, P);
+        if (t < groups) {
+            bool b = false;
+            for (int q = 0; q < 4; q++) b |= (int64_t)(4 * t + q) * GT < n && apo_max[4 * t + q] > Rt;
+            found[t] = b;
+        }
+        if (t < STRIP_ONE / GT)
+            for (int q = 0; q < 4; q++) blk[q][t] = 0.0;
+        __syncthreads();
+        bool any = false;
+        for (int g = 0; g < groups; g++) {
+            if (!found[g]) continue;
+            any = true;
+            double v[4] = {0.0, 0.0, 0.0, 0.0};
+            strip_star(f, P, Rt, n, 1 + (int64_t)g * STRIP_ONE_T + t, v);
+            tree_sum<4>(v, lds[sub], vt);
+            if (vt == 0)
+                for (int q = 0; q < 4; q++) blk[q][4 * g + sub] = v[q];
+            __syncthreads();
+        }
+        // final_sum over the grid pass's block sums: its thread b holds block b alone here
+        double res[4] = {0.0, 0.0, 0.0, 0.0};
+        if (any) {
+            if (sub == 0)
+                for (int q = 0; q < 4; q++) res[q] = blk[q][vt];
+            tree_sum<4>(res, lds[sub], vt);
+        }
+        if (t == 0) {
+            strip_update(s, Rt, res, done);
+            more = res[2] > 0;
+        }
+        __threadfence_block();
+        __syncthreads();
+        if (!more) return;
+    }
+    if (t == 0 && report) dev_set_error(s, CMCG_E_STRIP, 0);
 }
 };
 
@@ -296,7 +379,7 @@ struct ie_transfer_kernel {
 // potential(r) of the new potential at every old node.  The old radii (the array the
 // sort read, left intact in the alternate buffer) are sorted, so a block's MERGE_BLK
 // consecutive old radii [x_first, x_last] fall into one contiguous run of new nodes:
-// two lanes find its ends by bisection, the block stages the run in LDS (coalesced)
+// two waves find its ends, the block stages the run in LDS (coalesced)
 // and every radius is placed by bisection in LDS.  A run longer than MERGE_LDS nodes
 // is searched in global memory within the same ends.  The interval is the largest
 // k with r_k < x, as in potential_at (the search predicate is monotone, so any bracket
@@ -304,36 +387,31 @@ struct ie_transfer_kernel {
 // the values equal potential_at(x) bit for bit.
 constexpr int MERGE_T = 256, MERGE_PER = 2, MERGE_BLK = MERGE_T * MERGE_PER, MERGE_LDS = 1024;
 
-// The node index of both ends of every merge block (slot 2b: the block's first old
-// radius, 2b + 1: its last), one search per thread, so the merge blocks start from
-// their brackets instead of each waiting on two full-range searches.
-struct merge_ends_kernel {
-    static constexpr int LB = 256, MB = 0;
-    static __device__ __forceinline__ void run(KGrid kg_, const double *__restrict__ r_old,
-                                               const double2 *__restrict__ nodes, const DevScalars *s,
-                                               int64_t *__restrict__ ends)
-    {
-        const int64_t q = (int64_t)kg_.bid * 256 + threadIdx.x;       // 2 b + (0: first, 1: last)
-        const int64_t n_old = s->sort_in, n = s->n_max;
-        const int64_t first = 1 + (q >> 1) * MERGE_BLK;
-        if (first > n_old) return;
-        const int64_t last = first + MERGE_BLK - 1 <= n_old ? first + MERGE_BLK - 1 : n_old;
-        const PackedNodes nd{nodes};
-        const double x = r_old[(q & 1) ? last : first];
-        // largest k in [1, n+1] with r_k < x (1 if none); monotone in x
-        ends[q] = (x == 0.0 || x < nd.R(1)) ? 1 : find_zero_r_n(nd, 1, n + 1, x);
+// Largest k in [1, n + 1] with r_k < x (1 if none) by a whole wave: 64 probes split the range
+// into 65, four rounds at N = 4e6 where a bisection takes 22.  Uniform over the wave.
+__device__ __forceinline__ int64_t wave_find_zero_r(const PackedNodes &nd, int64_t n, double x)
+{
+    const int lane = threadIdx.x & 63;
+    int64_t lo = 1, hi = n + 1;
+    while (lo < hi) {
+        const int64_t step = (hi - lo) / 65 + 1, p = lo + (lane + 1) * step;     // lo + 65 step > hi
+        const int c = (int)__popcll(__ballot(p <= hi && nd.R(p) < x));
+        const int64_t top = lo + (c + 1) * step - 1;
+        lo += c * step;
+        hi = top < hi ? top : hi;
     }
-};
+    return lo;
+}
 
 struct old_node_potential_kernel {
     static constexpr int LB = MERGE_T, MB = 0;
     static __device__ __forceinline__ void run(KGrid kg_, const double *__restrict__ r_old,
                                                                      const double2 *__restrict__ nodes,
                                                                      DevScalars *s, double2 *__restrict__ u_old,
-                                                                     const int64_t *__restrict__ ends,
                                                                      const double *__restrict__ dpre)
 {
     __shared__ double2 L[MERGE_LDS];
+    __shared__ int64_t ends[2];
     const int64_t n_old = s->sort_in, n = s->n_max;
     const int64_t first = 1 + (int64_t)kg_.bid * MERGE_BLK;
     if (first > n_old) return;
@@ -341,8 +419,14 @@ struct old_node_potential_kernel {
     const PackedNodes nd{nodes};
     const double r1 = nd.R(1);
     const int t = threadIdx.x;
-    const int64_t lo = ends[2 * (int64_t)kg_.bid], hi = ends[2 * (int64_t)kg_.bid + 1];
     const double xf = r_old[first], xl = r_old[last];
+    if (t < 128) {                                 // wave 0: the first's, wave 1: the last's
+        const double x = t < 64 ? xf : xl;
+        const int64_t k = x == 0.0 || x < r1 ? 1 : wave_find_zero_r(nd, n, x);
+        if ((t & 63) == 0) ends[t >> 6] = k;
+    }
+    __syncthreads();
+    const int64_t lo = ends[0], hi = ends[1];
     const int64_t span = hi + 2 - lo;             // nodes lo .. hi+1
     const bool staged = span <= MERGE_LDS && hi + 1 <= n + 1;
     if (staged)
@@ -455,7 +539,8 @@ struct sv3_kernel {
 constexpr int SV3_CHUNK = 16;
 struct sv3_scan_kernel {
     static constexpr int LB = 1024, MB = 0;
-    static __device__ __forceinline__ void run(KGrid kg_, DevScalars *s, int64_t *__restrict__ blk_cnt, int64_t nb)
+    static __device__ __forceinline__ void run(KGrid kg_, DevScalars *s, int64_t *__restrict__ blk_cnt, int64_t nb,
+                                               int64_t *__restrict__ relink)
 {
     __shared__ int64_t wtot[16];
     const int t = threadIdx.x, lane = t & 63, w = t >> 6;
@@ -486,7 +571,10 @@ struct sv3_scan_kernel {
         if (q < w) run += wtot[q];
         tot += wtot[q];
     }
-    if (t == 1023) s->n_excess = tot;
+    if (t == 1023) {
+        s->n_excess = tot;
+        *relink = INT64_MAX;                   // sv3_verify_kernel takes the minimum
+    }
     if (regs) {
 #pragma unroll
         for (int q = 0; q < SV3_CHUNK; q++)
@@ -562,18 +650,23 @@ __device__ int64_t excess_walk(const DevFields &f, const double *__restrict__ ex
 // Fresh (no carried excess) bounded walk of every event.  joins[d] = 1 when that
 // walk reaches event d + 1 or was cut off, so event d + 1 is presumed to lie inside
 // the same episode.  An episode starting at a true head is exactly its fresh walk.
+__device__ __forceinline__ void sv3_spec(const DevFields &f, const double *__restrict__ excess_c, const int64_t *events,
+                                         int64_t *wend, int32_t *joins, int64_t n, int64_t ne, int64_t d0, int64_t stride)
+{
+    for (int64_t d = d0; d < ne; d += stride) {
+        int64_t e = excess_walk(f, excess_c, events[d], n, false, SPEC_WALK_MAX);
+        wend[d] = e;
+        joins[d] = (e < 0) || (d + 1 < ne && e >= events[d + 1]);
+    }
+}
 struct sv3_spec_kernel {
     static constexpr int LB = 1024, MB = 0;
     static __device__ __forceinline__ void run(KGrid kg_, DevFields f, DevScalars *s, const double *__restrict__ excess_c,
                                 const int64_t *__restrict__ events, int64_t *__restrict__ wend,
                                 int32_t *__restrict__ joins)
 {
-    const int64_t ne = s->n_excess;
-    for (int64_t d = (int64_t)kg_.bid * blockDim.x + threadIdx.x; d < ne; d += (int64_t)kg_.nb * blockDim.x) {
-        int64_t e = excess_walk(f, excess_c, events[d], s->n_max, false, SPEC_WALK_MAX);
-        wend[d] = e;
-        joins[d] = (e < 0) || (d + 1 < ne && e >= events[d + 1]);
-    }
+    sv3_spec(f, excess_c, events, wend, joins, s->n_max, s->n_excess, (int64_t)kg_.bid * blockDim.x + threadIdx.x,
+             (int64_t)kg_.nb * blockDim.x);
 }
 };
 
@@ -582,14 +675,10 @@ struct sv3_spec_kernel {
 // ends inside its group's span [events[q], events[q+1]), then by induction from
 // event 0 (which starts with no carried excess) each presumed head is a true head
 // and its walk is the true episode.  Otherwise the heads are relinked exactly.
-struct sv3_verify_kernel {
-    static constexpr int LB = 1024, MB = 0;
-    static __device__ __forceinline__ void run(KGrid kg_, DevScalars *s, const int64_t *__restrict__ events,
-                                  const int32_t *__restrict__ joins, const int64_t *__restrict__ wend,
-                                  int64_t *__restrict__ relink)
+__device__ __forceinline__ void sv3_verify(const int64_t *events, const int32_t *joins, const int64_t *wend, int64_t *relink,
+                                           int64_t ne, int64_t d0, int64_t stride)
 {
-    const int64_t ne = s->n_excess;
-    for (int64_t d = (int64_t)kg_.bid * blockDim.x + threadIdx.x; d < ne; d += (int64_t)kg_.nb * blockDim.x) {
+    for (int64_t d = d0; d < ne; d += stride) {
         if (d > 0 && joins[d - 1]) continue;
         int64_t q = d;
         while (q + 1 < ne && joins[q]) q++;
@@ -598,22 +687,24 @@ struct sv3_verify_kernel {
             atomicMin((unsigned long long *)relink, (unsigned long long)d);
     }
 }
+struct sv3_verify_kernel {
+    static constexpr int LB = 1024, MB = 0;
+    static __device__ __forceinline__ void run(KGrid kg_, DevScalars *s, const int64_t *__restrict__ events,
+                                  const int32_t *__restrict__ joins, const int64_t *__restrict__ wend,
+                                  int64_t *__restrict__ relink)
+{
+    sv3_verify(events, joins, wend, relink, s->n_excess, (int64_t)kg_.bid * blockDim.x + threadIdx.x,
+               (int64_t)kg_.nb * blockDim.x);
+}
 };
 
 // Exact head chain in event order: the next head is the first event after the end
 // of the current episode.  Runs only when a presumed head failed the check, and
 // starts at the first one that did: every presumed head before it passed, so by
 // induction it is a true head and the groups before it are exact.
-struct sv3_relink_kernel {
-    static constexpr int LB = 1024, MB = 0;
-    static __device__ __forceinline__ void run(KGrid kg_, DevFields f, DevScalars *s, const double *__restrict__ excess_c,
-                                  const int64_t *__restrict__ events, const int64_t *__restrict__ wend,
-                                  int32_t *__restrict__ joins, const int64_t *__restrict__ relink)
+__device__ __forceinline__ void sv3_relink(const DevFields &f, const double *__restrict__ excess_c, const int64_t *events,
+                                           const int64_t *wend, int32_t *joins, int64_t d, int64_t n, int64_t ne)
 {
-    if (threadIdx.x != 0 || kg_.bid != 0) return;
-    int64_t n = s->n_max, ne = s->n_excess;
-    int64_t d = *relink;
-    if (d >= ne) return;
     while (d < ne) {
         int64_t end = wend[d];
         if (end < 0) end = excess_walk(f, excess_c, events[d], n, false, INT64_MAX);
@@ -623,21 +714,97 @@ struct sv3_relink_kernel {
         d = d2;
     }
 }
+struct sv3_relink_kernel {
+    static constexpr int LB = 1024, MB = 0;
+    static __device__ __forceinline__ void run(KGrid kg_, DevFields f, DevScalars *s, const double *__restrict__ excess_c,
+                                  const int64_t *__restrict__ events, const int64_t *__restrict__ wend,
+                                  int32_t *__restrict__ joins, const int64_t *__restrict__ relink)
+{
+    if (threadIdx.x != 0 || kg_.bid != 0) return;
+    sv3_relink(f, excess_c, events, wend, joins, *relink, s->n_max, s->n_excess);
+}
 };
 
 // every head walks its episode and writes the dumped velocities
+__device__ __forceinline__ void sv3_heads(const DevFields &f, const double *__restrict__ excess_c, const int64_t *events,
+                                          const int32_t *joins, int64_t n, int64_t ne, int64_t d0, int64_t stride)
+{
+    for (int64_t d = d0; d < ne; d += stride)
+        if (d == 0 || !joins[d - 1]) excess_walk(f, excess_c, events[d], n, true, INT64_MAX);
+}
 struct sv3_heads_kernel {
     static constexpr int LB = 1024, MB = 0;
     static __device__ __forceinline__ void run(KGrid kg_, DevFields f, DevScalars *s, const double *__restrict__ excess_c,
                                  const int64_t *__restrict__ events, const int32_t *__restrict__ joins)
 {
-    const int64_t ne = s->n_excess;
-    for (int64_t d = (int64_t)kg_.bid * blockDim.x + threadIdx.x; d < ne; d += (int64_t)kg_.nb * blockDim.x)
-        if (d == 0 || !joins[d - 1]) excess_walk(f, excess_c, events[d], s->n_max, true, INT64_MAX);
+    sv3_heads(f, excess_c, events, joins, s->n_max, s->n_excess, (int64_t)kg_.bid * blockDim.x + threadIdx.x,
+              (int64_t)kg_.nb * blockDim.x);
 }
 };
 
-struct sv3_begin_kernel { static constexpr int LB = 1024, MB = 0; static __device__ __forceinline__ void run(KGrid kg_, DevScalars *s, int64_t *relink) { s->n_excess = 0; *relink = INT64_MAX; } };
+// The excess chain after sv3_kernel (the count of events, their ordered list, and the four
+// kernels on it above) in one block for a cluster of at most SV3_ONE stars: six launches of
+// 1 to 4 us with gaps as long.  Wave w lists the events of sv3_kernel's blocks w, w + 16, ...
+constexpr int64_t SV3_ONE = 65536;
+struct sv3_one_kernel {
+    static constexpr int LB = 1024, MB = 0;
+    static __device__ __forceinline__ void run(KGrid kg_, DevFields f, DevScalars *s, const double *__restrict__ excess_c,
+                                               const int64_t *__restrict__ blk_cnt, int nb, int64_t *events, int64_t *wend,
+                                               int32_t *joins)
+{
+    constexpr int NB = SV3_ONE / GT, NW = NB / 64;     // as many waves scan the counts
+    __shared__ int off[NB + 1], wtot[NW];
+    __shared__ int64_t relink;
+    const int t = threadIdx.x, lane = t & 63, w = t >> 6;
+    const int64_t n = s->n_max;
+    if (t < NB) {
+        const int c = t < nb ? (int)blk_cnt[t] : 0;
+        int inc = c;
+#pragma unroll
+        for (int d = 1; d < 64; d <<= 1) {
+            const int o = __shfl_up(inc, d, 64);
+            if (lane >= d) inc += o;
+        }
+        off[t] = inc - c;
+        if (lane == 63) wtot[w] = inc;
+    }
+    __syncthreads();
+    int ne = 0;
+    for (int q = 0; q < NW; q++) {
+        if (q == w && t < NB) off[t] += ne;
+        ne += wtot[q];
+    }
+    if (t == 0) {
+        off[NB] = ne;
+        s->n_excess = ne;
+        relink = INT64_MAX;
+    }
+    if (ne == 0) return;
+    __syncthreads();
+    for (int b = w; b < nb; b += 16) {
+        int pos = off[b];
+        if (pos == off[b + 1]) continue;
+        for (int q = 0; q < GT; q += 64) {
+            const int64_t i = 1 + (int64_t)b * GT + q + lane;
+            const bool ev = i <= n && excess_c[i] >= 0.0;
+            const uint64_t bal = __ballot(ev);
+            if (ev) events[pos + __popcll(bal & ((1ull << lane) - 1ull))] = i;
+            pos += (int)__popcll(bal);
+        }
+    }
+    __threadfence_block();
+    __syncthreads();
+    sv3_spec(f, excess_c, events, wend, joins, n, ne, t, 1024);
+    __threadfence_block();
+    __syncthreads();
+    sv3_verify(events, joins, wend, &relink, ne, t, 1024);
+    __syncthreads();
+    if (t == 0) sv3_relink(f, excess_c, events, wend, joins, relink, n, ne);
+    __threadfence_block();
+    __syncthreads();
+    sv3_heads(f, excess_c, events, joins, n, ne, t, 1024);
+}
+};
 
 struct energy_kernel {
     static constexpr int LB = GT, MB = 0;
@@ -658,10 +825,11 @@ struct energy_kernel {
 }
 };
 
-// compute_energy_new (cmc_utils.c:2017-2028) + the totals of ComputeEnergy
+// compute_energy_new (cmc_utils.c:2017-2028) + the totals of ComputeEnergy (and the step's end)
 struct energy_end_kernel {
     static constexpr int LB = 1024, MB = 0;
-    static __device__ __forceinline__ void run(KGrid kg_, DevScalars *s, const double *__restrict__ partials, int64_t nblocks)
+    static __device__ __forceinline__ void run(KGrid kg_, DevScalars *s, const double *__restrict__ partials, int64_t nblocks,
+                                               bool end_step)
 {
     double res[2];
     final_sum<2>(partials, nblocks, res);
@@ -674,6 +842,7 @@ struct energy_end_kernel {
         s->Epot = Pt;
         s->Etot = K + Pt + 0.0 + 0.0;
         s->Etot += 0.0 + s->Eescaped + 0.0 + 0.0;
+        if (end_step) s->step += 1;
     }
 }
 };
@@ -681,16 +850,6 @@ struct energy_end_kernel {
 unsigned grid_for(int64_t n) { return (unsigned)((n + GT - 1) / GT > 0 ? (n + GT - 1) / GT : 1); }
 } // namespace
 
-hipError_t launch_step_begin(DevScalars *s, hipStream_t st)
-{
-    kl<step_begin_kernel>(dim3(1), dim3(1), 0, st, s);
-    return hipGetLastError();
-}
-hipError_t launch_after_dynamics(DevScalars *s, hipStream_t st)
-{
-    kl<after_dynamics_kernel>(dim3(1), dim3(1), 0, st, s);
-    return hipGetLastError();
-}
 hipError_t launch_energy_conservation1(const DevFields &f, DevScalars *s, const KParams &P, int64_t n_ub,
                                        hipStream_t st)
 {
@@ -698,15 +857,15 @@ hipError_t launch_energy_conservation1(const DevFields &f, DevScalars *s, const 
     return hipGetLastError();
 }
 hipError_t launch_energy_conservation2(const DevFields &f, DevScalars *s, const KParams &P, int64_t n_ub,
-                                       hipStream_t st, bool with_ie, double *dpre)
+                                       hipStream_t st, bool with_ie, double *dpre, int32_t *strip_done, double *apo_max)
 {
     if (with_ie && !dpre) return hipErrorInvalidValue;
-    if (with_ie) kl<ec2_ie_kernel>(dim3(grid_for(n_ub)), dim3(GT), 0, st, f, s, P, dpre);
+    if (with_ie) kl<ec2_ie_kernel>(dim3(grid_for(n_ub)), dim3(GT), 0, st, f, s, P, dpre, strip_done, apo_max);
     else kl<ec2_kernel>(dim3(grid_for(n_ub)), dim3(GT), 0, st, f, s, P);
     return hipGetLastError();
 }
 hipError_t launch_strip(const DevFields &f, DevScalars *s, const KParams &P, const Scratch &sc, int32_t *done,
-                        int64_t n_ub, int passes, bool begin, hipStream_t st)
+                        int64_t n_ub, int passes, bool begin, hipStream_t st, const double *apo_max)
 {
     (void)n_ub;
     // a fixed grid (grid-stride over the stars) that the per-block partials hold
@@ -714,17 +873,30 @@ hipError_t launch_strip(const DevFields &f, DevScalars *s, const KParams &P, con
     if (sc.max_blocks < STRIP_BLOCKS) return hipErrorInvalidValue;
     if (begin) kl<strip_begin_kernel>(dim3(1), dim3(1), 0, st, s, done);
     for (int it = 0; it < passes; it++) {
-        kl<strip_pass_kernel>(dim3(nb), dim3(GT), 0, st, f, s, P, (const int32_t *)done, sc.partials);
+        kl<strip_pass_kernel>(dim3(nb), dim3(GT), 0, st, f, s, P, (const int32_t *)done, sc.partials, apo_max);
         kl<strip_end_kernel>(dim3(1), dim3(GT), 0, st, s, P, done, (const double *)sc.partials, nb);
     }
     return hipGetLastError();
 }
 
-hipError_t launch_strip_tail(const DevFields &f, DevScalars *s, const KParams &P, const Scratch &sc, hipStream_t st)
+bool strip_one_block(int64_t n_ub) { return n_ub <= STRIP_ONE; }
+
+// The loop whose begin energy_conservation2 has done, in one block: as many passes as the grid
+// passes and the tail of a captured step have, or the eager loop.
+hipError_t launch_strip_loop(const DevFields &f, DevScalars *s, const KParams &P, const Scratch &sc, bool graph, hipStream_t st,
+                             const double *apo_max)
+{
+    kl<strip_one_kernel>(dim3(1), dim3(STRIP_ONE_T), 0, st, f, s, P, sc.strip_done,
+                         graph ? STRIP_GRAPH_PASSES + STRIP_TAIL_PASSES : 100002, graph, apo_max);
+    return hipGetLastError();
+}
+
+hipError_t launch_strip_tail(const DevFields &f, DevScalars *s, const KParams &P, const Scratch &sc, hipStream_t st,
+                             const double *apo_max)
 {
     if (sc.max_blocks < STRIP_BLOCKS) return hipErrorInvalidValue;
     kl<strip_tail_kernel>(dim3(1), dim3(GT), 0, st, f, s, P, sc.strip_done, sc.partials,
-                       (unsigned)STRIP_BLOCKS);
+                       (unsigned)STRIP_BLOCKS, apo_max);
     return hipGetLastError();
 }
 hipError_t launch_intermediate_energy(const DevFields &f, DevScalars *s, const KParams &P, int64_t n_ub,
@@ -747,22 +919,23 @@ hipError_t launch_set_velocities3(const DevFields &f, DevScalars *s, const KPara
     if (nb > sc.max_blocks) return hipErrorInvalidValue;
     unsigned ge = grid_for(n_ub);
     if (ge > 256) ge = 256;            // the excess-list kernels stride over the list
-    kl<sv3_begin_kernel>(dim3(1), dim3(1), 0, st, s, sc.sv3_fallback);
     // the step calls this right after the potential, which left the node table current
     if (!dpre)
         if (hipError_t e = launch_mid_build(f, s, sc, n_ub, st)) return e;
     if (r_old_sorted) {
         const int64_t mb = (n_ub + MERGE_BLK - 1) / MERGE_BLK;
-        if (2 * mb > sc.merge_ends_cap) return hipErrorInvalidValue;
-        kl<merge_ends_kernel>(dim3((unsigned)((2 * mb + 255) / 256)), dim3(256), 0, st, r_old_sorted,
-                              (const double2 *)sc.nodes, (const DevScalars *)s, sc.merge_ends);
         kl<old_node_potential_kernel>(dim3((unsigned)mb), dim3(MERGE_T), 0, st, r_old_sorted,
-                                      (const double2 *)sc.nodes, s, sc.u_old, (const int64_t *)sc.merge_ends, dpre);
+                                      (const double2 *)sc.nodes, s, sc.u_old, dpre);
     }
     kl<sv3_kernel>(dim3((unsigned)nb), dim3(GT), 0, st, f, s, P, sc.excess_c, sc.sv3_blk,
                        (const double2 *)sc.mid, (const double2 *)sc.nodes,
                        r_old_sorted ? (const double2 *)sc.u_old : nullptr, (const uint32_t *)sc.vals_a);
-    kl<sv3_scan_kernel>(dim3(1), dim3(1024), 0, st, s, sc.sv3_blk, nb);
+    if (n_ub <= SV3_ONE) {
+        kl<sv3_one_kernel>(dim3(1), dim3(1024), 0, st, f, s, (const double *)sc.excess_c, (const int64_t *)sc.sv3_blk, (int)nb,
+                           sc.excess_list, sc.sv3_wend, sc.sv3_merged);
+        return hipGetLastError();
+    }
+    kl<sv3_scan_kernel>(dim3(1), dim3(1024), 0, st, s, sc.sv3_blk, nb, sc.sv3_fallback);
     kl<sv3_compact_kernel>(dim3((unsigned)nb), dim3(GT), 0, st, s, (const double *)sc.excess_c,
                        (const int64_t *)sc.sv3_blk, sc.excess_list);
     kl<sv3_spec_kernel>(dim3(ge), dim3(GT), 0, st, f, s, (const double *)sc.excess_c,
@@ -777,11 +950,11 @@ hipError_t launch_set_velocities3(const DevFields &f, DevScalars *s, const KPara
     return hipGetLastError();
 }
 hipError_t launch_compute_energy(const DevFields &f, DevScalars *s, const KParams &P, const Scratch &sc,
-                                 int64_t n_ub, hipStream_t st)
+                                 int64_t n_ub, hipStream_t st, bool end_step)
 {
     int64_t nb = grid_for(n_ub);
     if (nb > sc.max_blocks) return hipErrorInvalidValue;
     kl<energy_kernel>(dim3((unsigned)nb), dim3(GT), 0, st, f, s, P, sc.partials);
-    kl<energy_end_kernel>(dim3(1), dim3(GT), 0, st, s, (const double *)sc.partials, nb);
+    kl<energy_end_kernel>(dim3(1), dim3(GT), 0, st, s, (const double *)sc.partials, nb, end_step);
     return hipGetLastError();
 }

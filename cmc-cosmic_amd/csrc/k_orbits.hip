@@ -387,6 +387,7 @@ struct orbits_kernel {
                                                              const Rng *__restrict__ base,
                                                              double *__restrict__ partials,
                                                              int64_t *__restrict__ defer_list,
+                                                             int64_t *__restrict__ defer_kfirst,
                                                              const float2 *__restrict__ pred, float margin,
                                                              const double2 *__restrict__ mid,
                                                              const double2 *__restrict__ nodes,
@@ -463,8 +464,12 @@ struct orbits_kernel {
                 // linear-scan case: finished by the deferred path
                 flags = CMCG_SF_LINSCAN;
                 unsigned long long slot = atomicAdd((unsigned long long *)&s->n_defer, 1ull);
-                if ((int64_t)slot < P.defer_cap) defer_list[slot] = j;
-                else dev_set_error(s, CMCG_E_STATE, j);
+                if ((int64_t)slot < P.defer_cap) {
+                    defer_list[slot] = j;
+                    defer_kfirst[slot] = n + 2;          // the search takes the minimum
+                } else {
+                    dev_set_error(s, CMCG_E_STATE, j);
+                }
             } else {
                 if (pred) {
                     const float2 y = pred[j];
@@ -509,71 +514,106 @@ struct orbits_kernel {
 }
 };
 
-// Deferred stars (one block of DEFER_T threads): order the list by star index, so
-// the reduction of their sums does not depend on the order in which they were
-// appended, and reset the first-positive-index slots.  A short list is sorted by one
-// thread; a longer one by a bitonic sort over the next power of two (the list's
-// capacity is one, above the number of stars), padded with INT64_MAX, in global memory.
+// The deferred stars in star order, so that the reduction of their sums does not depend on the
+// order in which they were appended (one block): order[] is their stars and slots packed into
+// one word, sorted.  A short list is sorted by one thread; a longer one by a bitonic sort over
+// the next power of two (the list's capacity is one, above the number of stars), padded with
+// INT64_MAX, in global memory.
 constexpr int DEFER_T = 1024;
-struct defer_prepare_kernel {
-    static constexpr int LB = DEFER_T, MB = 0;
-    static __device__ __forceinline__ void run(KGrid kg_, DevScalars *s, int64_t *__restrict__ list,
-                                                                int64_t *__restrict__ kfirst, int64_t cap)
+constexpr int DEFER_SLOT_BITS = 31;            // star and slot indices are below 2^31
+__device__ __forceinline__ int64_t deferred(const DevScalars *s, const KParams &P)
+{
+    return s->n_defer < P.defer_cap ? s->n_defer : P.defer_cap;
+}
+__device__ void defer_sort(const int64_t *__restrict__ list, int64_t *__restrict__ order, int64_t nd)
 {
     const int t = threadIdx.x;
-    const int64_t nd = s->n_defer < cap ? s->n_defer : cap;
+    auto word = [&](int64_t d) { return (list[d] << DEFER_SLOT_BITS) | d; };
     if (nd <= 64) {
         if (t == 0)
-            for (int64_t a = 1; a < nd; a++) {
-                const int64_t v = list[a];
+            for (int64_t a = 0; a < nd; a++) {
+                const int64_t v = word(a);
                 int64_t b = a - 1;
-                while (b >= 0 && list[b] > v) { list[b + 1] = list[b]; b--; }
-                list[b + 1] = v;
+                while (b >= 0 && order[b] > v) { order[b + 1] = order[b]; b--; }
+                order[b + 1] = v;
             }
-    } else {
-        int64_t P = 1;
-        while (P < nd) P <<= 1;
-        for (int64_t i = nd + t; i < P; i += DEFER_T) list[i] = INT64_MAX;
-        __syncthreads();
-        for (int64_t k = 2; k <= P; k <<= 1)
-            for (int64_t j = k >> 1; j > 0; j >>= 1) {
-                for (int64_t i = t; i < P; i += DEFER_T) {
-                    const int64_t l = i ^ j;
-                    if (l > i) {
-                        const int64_t a = list[i], b = list[l];
-                        if ((a > b) == ((i & k) == 0)) { list[i] = b; list[l] = a; }
-                    }
-                }
-                __syncthreads();
-            }
+        return;
     }
-    const int64_t kf = s->n_max + 2;
-    for (int64_t d = t; d < nd; d += DEFER_T) kfirst[d] = kf;
+    int64_t P = 1;
+    while (P < nd) P <<= 1;
+    for (int64_t i = t; i < P; i += DEFER_T) order[i] = i < nd ? word(i) : INT64_MAX;
+    __syncthreads();
+    for (int64_t k = 2; k <= P; k <<= 1)
+        for (int64_t j = k >> 1; j > 0; j >>= 1) {
+            for (int64_t i = t; i < P; i += DEFER_T) {
+                const int64_t l = i ^ j;
+                if (l > i) {
+                    const int64_t a = order[i], b = order[l];
+                    if ((a > b) == ((i & k) == 0)) { order[i] = b; order[l] = a; }
+                }
+            }
+            __syncthreads();
+        }
 }
-};
 
-// Grid-wide equivalent of the linear scan: the first k in [0, N_MAX+1] with Q > 0.
-struct defer_search_kernel {
-    static constexpr int LB = 256, MB = 0;
-    static __device__ __forceinline__ void run(KGrid kg_, DevFields f, DevScalars *s, KParams P,
-                                                           const int64_t *__restrict__ list,
-                                                           int64_t *__restrict__ kfirst)
+// Grid-wide equivalent of the linear scan: the first k in [0, N_MAX+1] with Q > 0 of every
+// deferred star, four stars at a time, each by a quarter of the nb blocks.
+__device__ void defer_search(const DevFields &f, const KParams &P, const int64_t *__restrict__ list,
+                             int64_t *__restrict__ kfirst, int64_t nd, int64_t n, int b, int nb)
 {
-    const int64_t nd = s->n_defer < P.defer_cap ? s->n_defer : P.defer_cap;
-    if (nd == 0) return;
-    const int64_t n = s->n_max;
-    const int64_t stride = (int64_t)kg_.nb * blockDim.x;
-    for (int64_t d = kg_.by; d < nd; d += kg_.nby) {
+    const int64_t stride = (int64_t)(nb / 4) * DEFER_T;
+    for (int64_t d = b & 3; d < nd; d += 4) {
         const int64_t j = list[d];
         const double rj = f.r[j], mj = f.m[j];
         const double E = f.E[j] + phi_s_own(rj, mj, P.inv_nstar, rj);
         const double J = f.J[j];
-        for (int64_t k = (int64_t)kg_.bid * blockDim.x + threadIdx.x; k <= n + 1; k += stride) {
-            if (k > (int64_t)kfirst[d]) break;
+        for (int64_t k = (int64_t)(b >> 2) * DEFER_T + threadIdx.x; k <= n + 1; k += stride) {
+            if (k > kfirst[d]) break;
             if (function_q(rj, mj, P.inv_nstar, f.r[k], f.phi[k], E, J) > 0.0)
                 atomicMin((unsigned long long *)&kfirst[d], (unsigned long long)k);
         }
     }
+}
+
+// First level of the orbit phase's reduction: block B of RED2_BLOCKS sums the partial
+// records of sampler blocks [B C, (B + 1) C), C = ceil(nblocks / RED2_BLOCKS); 16
+// consecutive threads read one record (coalesced), its 64 groups take records
+// g, g + 64, ... of the range, and the groups are combined in group order.
+__device__ void orbits_part(const double *__restrict__ partials, int64_t nblocks, double *__restrict__ out, int B)
+{
+    __shared__ double gsum[64][RED_STRIDE];
+    const int t = threadIdx.x, i = t & 15, g = t >> 4;
+    const int64_t C = (nblocks + RED2_BLOCKS - 1) / RED2_BLOCKS;
+    const int64_t b0 = (int64_t)B * C, b1 = b0 + C < nblocks ? b0 + C : nblocks;
+    double acc = 0.0;
+    if (i < NRED)
+        for (int64_t b = b0 + g; b < b1; b += 64) {
+            double p = partials[RED_STRIDE * b + i];
+            acc = red_is_max(i) ? (acc >= p ? acc : p) : acc + p;
+        }
+    gsum[g][i] = acc;
+    __syncthreads();
+    if (t < NRED) {
+        double a = gsum[0][t];
+        for (int g2 = 1; g2 < 64; g2++) a = red_is_max(t) ? (a >= gsum[g2][t] ? a : gsum[g2][t]) : a + gsum[g2][t];
+        out[RED_STRIDE * B + t] = a;
+    }
+}
+
+// After the sampler, in one launch (three kernels of 4 to 12 us before): its reduction's first
+// level, the order of the deferred stars, and their linear scans.
+constexpr int DEFER_BLOCKS = 256;
+struct after_orbits_kernel {
+    static constexpr int LB = DEFER_T, MB = 0;
+    static __device__ __forceinline__ void run(KGrid kg_, DevFields f, DevScalars *s, KParams P,
+                                                           const double *__restrict__ partials, int64_t nblocks,
+                                                           double *__restrict__ red2, const int64_t *__restrict__ list,
+                                                           int64_t *__restrict__ kfirst, int64_t *__restrict__ order)
+{
+    const int b = (int)kg_.bid - RED2_BLOCKS - 1;
+    if (b < -1) orbits_part(partials, nblocks, red2, (int)kg_.bid);
+    else if (b == -1) defer_sort(list, order, deferred(s, P));
+    else defer_search(f, P, list, kfirst, deferred(s, P), s->n_max, b, DEFER_BLOCKS);
 }
 };
 
@@ -586,7 +626,7 @@ struct defer_tail_kernel {
     static __device__ __forceinline__ void run(KGrid kg_, DevFields f, DevScalars *s, KParams P,
                                                                  const RngTable *__restrict__ T,
                                                                  const Rng *__restrict__ base, int jb1,
-                                                                 const int64_t *__restrict__ list,
+                                                                 const int64_t *__restrict__ order,
                                                                  const int64_t *__restrict__ kfirst,
                                                                  const double *__restrict__ red2)
 {
@@ -601,16 +641,16 @@ struct defer_tail_kernel {
         }
         acc[t] = a;
     }
-    const int64_t nd = s->n_defer < P.defer_cap ? s->n_defer : P.defer_cap;
+    const int64_t nd = deferred(s, P);
     const int64_t n = s->n_max;
     for (int64_t c0 = 0; c0 < nd; c0 += ORB_THREADS) {          // block-uniform
         const int64_t d = c0 + t;
         if (d < nd) {
-            const int64_t j = list[d];
+            const int64_t j = order[d] >> DEFER_SLOT_BITS;
             const double rj = f.r[j], mj = f.m[j];
             const double Ej = f.E[j], J = f.J[j];
             const double E = Ej + phi_s_own(rj, mj, P.inv_nstar, rj);
-            int64_t kt = kfirst[d];
+            int64_t kt = kfirst[order[d] & ((1ll << DEFER_SLOT_BITS) - 1)];
             if (kt >= n) kt = -1;                      // cmc_orbit.c:52-56: circular
             double red[NRED];
             for (int i = 0; i < NRED; i++) red[i] = 0.0;
@@ -652,35 +692,6 @@ struct defer_tail_kernel {
         s->tries_max = (int64_t)acc[12];
         s->n_bracket_hit = (int64_t)acc[13];
         s->n_bracket_fallback = (int64_t)acc[14];
-    }
-}
-};
-
-// First level of the orbit phase's reduction: block B of RED2_BLOCKS sums the partial
-// records of sampler blocks [B C, (B + 1) C), C = ceil(nblocks / RED2_BLOCKS); 16
-// consecutive threads read one record (coalesced), its 64 groups take records
-// g, g + 64, ... of the range, and the groups are combined in group order.
-struct orbits_part_kernel {
-    static constexpr int LB = 1024, MB = 0;
-    static __device__ __forceinline__ void run(KGrid kg_, const double *__restrict__ partials, int64_t nblocks,
-                                                           double *__restrict__ out)
-{
-    __shared__ double gsum[64][RED_STRIDE];
-    const int t = threadIdx.x, i = t & 15, g = t >> 4;
-    const int64_t C = (nblocks + RED2_BLOCKS - 1) / RED2_BLOCKS;
-    const int64_t b0 = (int64_t)kg_.bid * C, b1 = b0 + C < nblocks ? b0 + C : nblocks;
-    double acc = 0.0;
-    if (i < NRED)
-        for (int64_t b = b0 + g; b < b1; b += 64) {
-            double p = partials[RED_STRIDE * b + i];
-            acc = red_is_max(i) ? (acc >= p ? acc : p) : acc + p;
-        }
-    gsum[g][i] = acc;
-    __syncthreads();
-    if (t < NRED) {
-        double a = gsum[0][t];
-        for (int g2 = 1; g2 < 64; g2++) a = red_is_max(t) ? (a >= gsum[g2][t] ? a : gsum[g2][t]) : a + gsum[g2][t];
-        out[RED_STRIDE * kg_.bid + t] = a;
     }
 }
 };
@@ -811,16 +822,37 @@ struct node_index_kernel {
 }
 };
 
+// The LDS samples of the (r, phi) table for a COARSE-sample launch: node
+// min(s * stride, n + 1) for s = 0..cs, from the packed nodes.
+__device__ void coarse_build(const double2 *__restrict__ nodes, DevScalars *s, int cs, double2 *__restrict__ out, int i)
+{
+    if (i == 0) {
+        // new_orbits_calculate (cmc_utils.c:2198) and the counters of this call
+        s->OldTidalMassLoss = s->TidalMassLoss_old;
+        s->n_defer = 0;
+    }
+    if (i > cs) return;
+    const int64_t n = s->n_max;
+    const int64_t k = (int64_t)i * coarse_stride(n, cs);
+    out[i] = nodes[k < n + 1 ? k : n + 1];
+}
+
 // t[b] = the largest marked index below b in its tile, or the tile's entry value:
 // an exclusive running maximum, in place.  16 buckets per thread (four 16-byte loads),
 // the threads' maxima scanned by wave shuffles and the four wave totals through LDS.
+// The blocks after the tiles build the sampler's LDS samples.
 struct ridx_scan_kernel {
     static constexpr int LB = 256, MB = 0;
     static __device__ __forceinline__ void run(KGrid kg_, uint32_t *__restrict__ t, const uint32_t *__restrict__ tb,
-                                                        int bits)
+                                                        int bits, const double2 *__restrict__ nodes, DevScalars *s, int cs,
+                                                        double2 *__restrict__ coarse)
 {
     __shared__ uint32_t wtot[4];
     const int64_t entries = ridx_entries(bits);
+    if (kg_.bid >= ridx_tiles(bits)) {
+        coarse_build(nodes, s, cs, coarse, (int)(kg_.bid - ridx_tiles(bits)) * 256 + threadIdx.x);
+        return;
+    }
     const int64_t i0 = (int64_t)kg_.bid * RIDX_TILE + 16 * threadIdx.x;
     const bool whole = i0 + 16 <= entries;
     uint32_t v[16];
@@ -870,41 +902,20 @@ struct ridx_scan_kernel {
 }
 };
 
-// The LDS samples of the (r, phi) table for a COARSE-sample launch: node
-// min(s * stride, n + 1) for s = 0..cs, from the packed nodes.
-struct coarse_build_kernel {
-    static constexpr int LB = 1024, MB = 0;
-    static __device__ __forceinline__ void run(KGrid kg_, const double2 *__restrict__ nodes, DevScalars *s, int cs,
-                                    double2 *__restrict__ out)
-{
-    const int i = kg_.bid * blockDim.x + threadIdx.x;
-    if (i == 0) {
-        // new_orbits_calculate (cmc_utils.c:2198) and the counters of this call
-        s->OldTidalMassLoss = s->TidalMassLoss_old;
-        s->n_defer = 0;
-    }
-    if (i > cs) return;
-    const int64_t n = s->n_max;
-    const int64_t st = coarse_stride(n, cs);
-    const int64_t k = (int64_t)i * st;
-    out[i] = nodes[k < n + 1 ? k : n + 1];
-}
-};
-
 // Launch shapes of the orbit sampler that the autotuner chooses from: threads per
 // block, LDS samples of the (r, phi) table, and the most lanes one star's tries get
 // in a round (64: all idle lanes; fewer: less speculative work).  Every variant gives
 // the same stars; only the block order of the escape sums differs.
 using OrbFn = void (*)(dim3, dim3, hipStream_t, DevFields, DevScalars *, KParams, const JumpTables *,
-                       const Rng *, double *, int64_t *, const float2 *, float, const double2 *, const double2 *, const double2 *,
+                       const Rng *, double *, int64_t *, int64_t *, const float2 *, float, const double2 *, const double2 *, const double2 *,
                        const uint32_t *, int);
 template <int THREADS, int COARSE, int CAP, int MINB>
 void orbits_launch(dim3 g, dim3 b, hipStream_t st, DevFields f, DevScalars *s, KParams P, const JumpTables *jump,
-                   const Rng *base, double *partials, int64_t *defer, const float2 *pred, float margin,
+                   const Rng *base, double *partials, int64_t *defer, int64_t *kfirst, const float2 *pred, float margin,
                    const double2 *mid, const double2 *nodes, const double2 *coarse,
                    const uint32_t *ridx, int ridx_bits)
 {
-    kl<orbits_kernel<THREADS, COARSE, CAP, MINB>>(g, b, 0, st, f, s, P, jump, base, partials, defer, pred, margin, mid, nodes,
+    kl<orbits_kernel<THREADS, COARSE, CAP, MINB>>(g, b, 0, st, f, s, P, jump, base, partials, defer, kfirst, pred, margin, mid, nodes,
                                                   coarse, ridx, ridx_bits);
 }
 struct OrbVariant { OrbFn fn; int threads, coarse, cap, minb; };
@@ -931,17 +942,15 @@ int bits_needed(uint64_t x)
 
 hipError_t launch_orbits(const DevFields &f, DevScalars *s, const KParams &P, const RngTable *T,
                          const Scratch &sc, int64_t n_ub, hipStream_t st, const MlpState *mlp,
-                         float margin, hipEvent_t ev_a, hipEvent_t ev_b, int variant, bool pred_fixed)
+                         float margin, hipEvent_t ev_a, hipEvent_t ev_b, int variant, bool pred_fixed, bool index_clear)
 {
     const OrbVariant &V = kOrbVariants[variant >= 0 && variant < ORB_NVARIANTS ? variant : 0];
     int64_t nblocks = (n_ub + V.threads - 1) / V.threads;
     if (nblocks < 1) nblocks = 1;
     if (nblocks > sc.max_blocks) return hipErrorInvalidValue;
     int jb1 = 20 + bits_needed((uint64_t)n_ub);
-    if (hipError_t e = launch_node_index(f, s, sc, n_ub, st)) return e;
     if (V.coarse > ORB_MAX_COARSE) return hipErrorInvalidValue;
-    kl<coarse_build_kernel>(dim3((unsigned)((V.coarse + 256) / 256)), dim3(256), 0, st,
-                       (const double2 *)sc.nodes, s, V.coarse, sc.coarse);
+    if (hipError_t e = launch_node_index(f, s, sc, n_ub, V.coarse, index_clear, st)) return e;
     const float2 *pred = nullptr;
     if (mlp) {
         if (!sc.pred) return hipErrorInvalidValue;
@@ -951,17 +960,14 @@ hipError_t launch_orbits(const DevFields &f, DevScalars *s, const KParams &P, co
     }
     if (ev_a) hipEventRecord(ev_a, st);
     V.fn(dim3((unsigned)nblocks), dim3(V.threads), st, f, s, P, sc.jump, (const Rng *)sc.rng_base,
-                       sc.partials, sc.defer_list, pred, margin, (const double2 *)sc.mid,
+                       sc.partials, sc.defer_list, sc.defer_kfirst, pred, margin, (const double2 *)sc.mid,
                        (const double2 *)sc.nodes, (const double2 *)sc.coarse,
                        (const uint32_t *)sc.ridx, sc.ridx_bits);
     if (ev_b) hipEventRecord(ev_b, st);
-    kl<defer_prepare_kernel>(dim3(1), dim3(DEFER_T), 0, st, s, sc.defer_list, sc.defer_kfirst, P.defer_cap);
-    kl<defer_search_kernel>(dim3(256, 4), dim3(256), 0, st, f, s, P, (const int64_t *)sc.defer_list,
-                       sc.defer_kfirst);
-    kl<orbits_part_kernel>(dim3(RED2_BLOCKS), dim3(1024), 0, st, (const double *)sc.partials, nblocks,
-                       sc.red2);
+    kl<after_orbits_kernel>(dim3(RED2_BLOCKS + 1 + DEFER_BLOCKS), dim3(DEFER_T), 0, st, f, s, P, (const double *)sc.partials,
+                       nblocks, sc.red2, (const int64_t *)sc.defer_list, sc.defer_kfirst, sc.defer_order);
     kl<defer_tail_kernel>(dim3(1), dim3(ORB_THREADS), 0, st, f, s, P, T, sc.rng_base, jb1,
-                       (const int64_t *)sc.defer_list, (const int64_t *)sc.defer_kfirst, (const double *)sc.red2);
+                       (const int64_t *)sc.defer_order, (const int64_t *)sc.defer_kfirst, (const double *)sc.red2);
     return hipGetLastError();
 }
 
@@ -975,14 +981,15 @@ hipError_t launch_pred_from_apsides(const DevFields &f, DevScalars *s, const Scr
     return hipGetLastError();
 }
 
-hipError_t launch_node_index(const DevFields &f, DevScalars *s, const Scratch &sc, int64_t n_ub, hipStream_t st)
+hipError_t launch_node_index(const DevFields &f, DevScalars *s, const Scratch &sc, int64_t n_ub, int coarse, bool clear,
+                             hipStream_t st)
 {
     const int64_t entries = ridx_entries(sc.ridx_bits);
-    kl<ridx_clear_kernel>(dim3(512), dim3(256), 0, st, sc.ridx, entries);
+    if (!clear) kl<ridx_clear_kernel>(dim3(512), dim3(256), 0, st, sc.ridx, entries);
     kl<node_index_kernel>(dim3((unsigned)((n_ub + 2 + 255) / 256)), dim3(256), 0, st, f.r, f.phi, s,
                        (double2 *)sc.nodes, (double2 *)sc.mid, sc.ridx, sc.ridx_tb, sc.ridx_bits, sc.sort_bad);
-    kl<ridx_scan_kernel>(dim3((unsigned)ridx_tiles(sc.ridx_bits)), dim3(256), 0, st, sc.ridx,
-                       (const uint32_t *)sc.ridx_tb, sc.ridx_bits);
+    kl<ridx_scan_kernel>(dim3((unsigned)(ridx_tiles(sc.ridx_bits) + (coarse + 256) / 256)), dim3(256), 0, st, sc.ridx,
+                       (const uint32_t *)sc.ridx_tb, sc.ridx_bits, (const double2 *)sc.nodes, s, coarse, sc.coarse);
     return hipGetLastError();
 }
 

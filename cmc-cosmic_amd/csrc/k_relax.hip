@@ -162,15 +162,44 @@ __device__ __forceinline__ void timestep_finalize(DevScalars *s)
     s->TotalTime += Dt;
 }
 struct timestep_finalize_kernel { static constexpr int LB = 1024, MB = 0; static __device__ __forceinline__ void run(KGrid kg_, DevScalars *s) { timestep_finalize(s); } };
-// the step's time step (thread 0; first the minimum over sigma_dt_kernel's slots, which
-// are reset for the next step, when dt_part is given), then its RNG substream bases
+// Begin of a step (cmc.c:246-258, 278): the per-step resets.
+__device__ __forceinline__ void step_begin(DevScalars *s)
+{
+    s->Eescaped_old = s->Eescaped;
+    s->Jescaped_old = s->Jescaped;
+    s->TidalMassLoss_old = s->TidalMassLoss;
+    s->Etidal_old = s->Etidal;
+    s->Eescaped = 0.0; s->Jescaped = 0.0; s->TidalMassLoss = 0.0; s->Etidal = 0.0;
+    s->n_max_new = s->n_max;
+    s->dtrel = __longlong_as_double(0x7ff0000000000000ll);     // the time step's minimum starts at +inf
+}
+struct step_begin_kernel { static constexpr int LB = 1024, MB = 0; static __device__ __forceinline__ void run(KGrid kg_, DevScalars *s) { step_begin(s); } };
+
+// Block 0: the begin of the step and the minimum over sigma_dt_kernel's slots, which are reset
+// for the next step (when dt_part is given; sigma_dt_kernel touches nothing the begin sets),
+// the time step (thread 0) with Prev_Dt for the next one (cmc.c:297: only the time step reads
+// it), then the step's RNG substream bases.  The other blocks clear the radial index for the
+// orbit phase.  (Four launches of 4 to 5 us each that had no work of their own.)
+constexpr int64_t CLEAR_BLK = RB_T * 16;           // index entries per block
 struct timestep_rng_bases_kernel {
     static constexpr int LB = RB_T, MB = 0;
     static __device__ __forceinline__ void run(KGrid kg_, const JumpLevel *__restrict__ J, DevScalars *s,
                                                                   const Rng *__restrict__ seeded,
                                                                   Rng *__restrict__ base,
-                                                                  unsigned long long *__restrict__ dt_part)
+                                                                  unsigned long long *__restrict__ dt_part,
+                                                                  uint32_t *__restrict__ ridx, int64_t entries)
 {
+    if (kg_.bid > 0) {
+        const int64_t b0 = (int64_t)(kg_.bid - 1) * CLEAR_BLK;
+#pragma unroll
+        for (int q = 0; q < 4; q++) {
+            const int64_t i = b0 + 4 * (q * RB_T + threadIdx.x);
+            if (i + 4 <= entries) *reinterpret_cast<uint4 *>(ridx + i) = make_uint4(0, 0, 0, 0);
+            else
+                for (int64_t k = i; k < entries; k++) ridx[k] = 0;
+        }
+        return;
+    }
     if (dt_part) {
         unsigned long long mine = ~dt_part[threadIdx.x * 16];
         dt_part[threadIdx.x * 16] = 0ull;
@@ -182,11 +211,14 @@ struct timestep_rng_bases_kernel {
             mine = other < mine ? other : mine;
         }
         if (threadIdx.x == 0) {
-            const unsigned long long cur = (unsigned long long)__double_as_longlong(s->dtrel);
-            s->dtrel = __longlong_as_double((long long)(mine < cur ? mine : cur));
+            step_begin(s);
+            s->dtrel = __longlong_as_double((long long)mine);
         }
     }
-    if (threadIdx.x == 0) timestep_finalize(s);
+    if (threadIdx.x == 0) {
+        timestep_finalize(s);
+        s->Prev_Dt = s->Dt;
+    }
     rng_bases(J, s, seeded, base, -1);
 }
 };
@@ -508,29 +540,27 @@ hipError_t launch_simul_relax(const DevFields &f, DevScalars *s, const KParams &
     return hipGetLastError();
 }
 
-hipError_t launch_timestep_rng_bases(DevScalars *s, const Scratch &sc, hipStream_t st)
-{
-    kl<timestep_rng_bases_kernel>(dim3(1), dim3(RB_T), 0, st, (const JumpLevel *)sc.jump->level, s, sc.rng_seeded, sc.rng_base,
-                       (unsigned long long *)nullptr);
-    return hipGetLastError();
-}
-
-// The step's time-step phase: calc_sigma_r and simul_relax_new in one pass (or, for a
-// window longer than the pass stages, their own kernels), then Dt and the RNG bases.
+// The step's begin and time-step phase: calc_sigma_r and simul_relax_new in one pass (or, for
+// a window longer than the pass stages, their own kernels), then Dt, the RNG bases and the
+// cleared radial index of the orbit phase.
 hipError_t launch_timestep_sigma(const DevFields &f, DevScalars *s, const KParams &P, const Scratch &sc,
                                  int64_t n_ub, hipStream_t st)
 {
-    if (P.avekernel > SIG_MAXP || n_ub <= 0) {
+    const bool one_pass = P.avekernel <= SIG_MAXP && n_ub > 0;
+    if (one_pass) {
+        const int64_t nb = (n_ub + SIG_T - 1) / SIG_T;
+        if (nb > sc.max_blocks) return hipErrorInvalidValue;
+        kl<sigma_dt_kernel>(dim3((unsigned)nb), dim3(SIG_T), 0, st, f.r, f.m, f.vr, f.vt, f.sigma, s, P,
+                           sc.dt_part);
+    } else {
+        kl<step_begin_kernel>(dim3(1), dim3(1), 0, st, s);
         if (hipError_t e = launch_simul_relax(f, s, P, n_ub, st, false)) return e;
         if (hipError_t e = launch_sigma(f, s, P, n_ub, st)) return e;
-        return launch_timestep_rng_bases(s, sc, st);
     }
-    const int64_t nb = (n_ub + SIG_T - 1) / SIG_T;
-    if (nb > sc.max_blocks) return hipErrorInvalidValue;
-    kl<sigma_dt_kernel>(dim3((unsigned)nb), dim3(SIG_T), 0, st, f.r, f.m, f.vr, f.vt, f.sigma, s, P,
-                       sc.dt_part);
-    kl<timestep_rng_bases_kernel>(dim3(1), dim3(RB_T), 0, st, (const JumpLevel *)sc.jump->level, s, sc.rng_seeded, sc.rng_base,
-                       sc.dt_part);
+    const int64_t entries = ridx_entries(sc.ridx_bits);
+    kl<timestep_rng_bases_kernel>(dim3(1 + (unsigned)((entries + CLEAR_BLK - 1) / CLEAR_BLK)), dim3(RB_T), 0, st,
+                       (const JumpLevel *)sc.jump->level, s, sc.rng_seeded, sc.rng_base,
+                       one_pass ? sc.dt_part : (unsigned long long *)nullptr, sc.ridx, entries);
     return hipGetLastError();
 }
 hipError_t launch_timestep_finalize(DevScalars *s, hipStream_t st)

@@ -75,8 +75,6 @@ struct Scratch {
     uint32_t *ridx_tb;          // its value at every RIDX_TILE-th bucket
     int ridx_bits;              // log2 of the bucket count
     double2 *u_old;             // (new potential, radius), (D, -) at each old sorted radius (set_velocities3)
-    int64_t *merge_ends;        // set_velocities3: node index of both ends of each merge block
-    int64_t merge_ends_cap;
     double *sv3_dpre;           // D = vold^2 + 2(1-q)(Uoldrold - Uoldrnew) per star, in the order before the step's sort
     unsigned long long *dt_part;  // the step's time step: 64 slots, 128 bytes apart, of complemented dt minima
     double2 *coarse;            // orbit sampler's (r, phi) samples, copied into LDS by every block
@@ -94,7 +92,7 @@ struct Scratch {
     // tidal stripping loop flag
     int32_t *strip_done;
     // orbit stars deferred to the linear-scan path (65536 slots)
-    int64_t *defer_list, *defer_kfirst;   // KParams::defer_cap entries
+    int64_t *defer_list, *defer_kfirst, *defer_order;   // KParams::defer_cap entries
     // RNG bases of the current step: [0] relaxation, [1] orbits, [2] orbit slot 1; seeded state
     Rng *rng_base;
     Rng *rng_seeded;
@@ -115,7 +113,6 @@ hipError_t launch_potential_at(const DevFields &f, DevScalars *s, const KParams 
 hipError_t launch_sigma(const DevFields &f, DevScalars *s, const KParams &P, int64_t n_ub, hipStream_t st);
 hipError_t launch_simul_relax(const DevFields &f, DevScalars *s, const KParams &P, int64_t n_ub, hipStream_t st,
                               bool init_min = true);
-hipError_t launch_timestep_rng_bases(DevScalars *s, const Scratch &sc, hipStream_t st);
 hipError_t launch_timestep_sigma(const DevFields &f, DevScalars *s, const KParams &P, const Scratch &sc,
                                  int64_t n_ub, hipStream_t st);
 hipError_t launch_timestep_finalize(DevScalars *s, hipStream_t st);
@@ -129,7 +126,8 @@ hipError_t launch_relax(const DevFields &f, DevScalars *s, const KParams &P, con
 hipError_t launch_rng_bases(DevScalars *s, const Scratch &sc, hipStream_t st);
 hipError_t launch_rng_bases_step(DevScalars *s, const Scratch &sc, int64_t step, hipStream_t st);
 // the packed node table and the radial index in one pass over r and phi
-hipError_t launch_node_index(const DevFields &f, DevScalars *s, const Scratch &sc, int64_t n_ub, hipStream_t st);
+hipError_t launch_node_index(const DevFields &f, DevScalars *s, const Scratch &sc, int64_t n_ub, int coarse, bool clear,
+                             hipStream_t st);
 // middle level of the (r, phi) search tables, from the current arrays
 hipError_t launch_mid_build(const DevFields &f, DevScalars *s, const Scratch &sc, int64_t n_ub, hipStream_t st);
 hipError_t launch_rng_draws(const RngTable *T, const Rng *base, int phase, int64_t first, int64_t count,
@@ -140,7 +138,7 @@ hipError_t launch_rng_draws(const RngTable *T, const Rng *base, int phase, int64
 hipError_t launch_orbits(const DevFields &f, DevScalars *s, const KParams &P, const RngTable *T,
                          const Scratch &sc, int64_t n_ub, hipStream_t st, const MlpState *mlp = nullptr,
                          float margin = 0.f, hipEvent_t ev_a = nullptr, hipEvent_t ev_b = nullptr, int variant = 0,
-                         bool pred_fixed = false);
+                         bool pred_fixed = false, bool index_clear = false);
 // proposals equal to the apsides the last orbit phase wrote (log r_peri, log r_apo): a
 // perfect predictor, for measuring what any learned proposal could save
 hipError_t launch_pred_from_apsides(const DevFields &f, DevScalars *s, const Scratch &sc, int64_t n_ub,
@@ -169,14 +167,19 @@ hipError_t launch_sort_fields(const double *key_src, double *r_dst, int nf, cons
                               uint64_t *const *dst, DevScalars *s, const Scratch &sc, int64_t n_ub,
                               const int32_t *knew, hipStream_t st);
 
-hipError_t launch_step_begin(DevScalars *s, hipStream_t st);
-hipError_t launch_after_dynamics(DevScalars *s, hipStream_t st);
 hipError_t launch_energy_conservation1(const DevFields &f, DevScalars *s, const KParams &P, int64_t n_ub, hipStream_t st);
 hipError_t launch_energy_conservation2(const DevFields &f, DevScalars *s, const KParams &P, int64_t n_ub, hipStream_t st,
-                                       bool with_ie = false, double *dpre = nullptr);
+                                       bool with_ie = false, double *dpre = nullptr, int32_t *strip_done = nullptr,
+                                       double *apo_max = nullptr);
+constexpr int STRIP_GRAPH_PASSES = 3;     // grid passes of a captured step; a one-block tail kernel finishes rarer longer loops
+// the tidal stripping loop: whether one block runs it to its end for a cluster of n_ub stars
+bool strip_one_block(int64_t n_ub);
+hipError_t launch_strip_loop(const DevFields &f, DevScalars *s, const KParams &P, const Scratch &sc, bool graph, hipStream_t st,
+                             const double *apo_max);
 hipError_t launch_strip(const DevFields &f, DevScalars *s, const KParams &P, const Scratch &sc, int32_t *done,
-                        int64_t n_ub, int passes, bool begin, hipStream_t st);
-hipError_t launch_strip_tail(const DevFields &f, DevScalars *s, const KParams &P, const Scratch &sc, hipStream_t st);
+                        int64_t n_ub, int passes, bool begin, hipStream_t st, const double *apo_max = nullptr);
+hipError_t launch_strip_tail(const DevFields &f, DevScalars *s, const KParams &P, const Scratch &sc, hipStream_t st,
+                             const double *apo_max);
 hipError_t launch_intermediate_energy(const DevFields &f, DevScalars *s, const KParams &P, int64_t n_ub, hipStream_t st);
 hipError_t launch_ie_transfer(const DevFields &f, DevScalars *s, int64_t n_ub, hipStream_t st);
 // r_old_sorted: the radii the sort of this step read (old sorted order), or nullptr
@@ -184,7 +187,7 @@ hipError_t launch_set_velocities3(const DevFields &f, DevScalars *s, const KPara
                                   int64_t n_ub, hipStream_t st, const double *r_old_sorted = nullptr,
                                   const double *dpre = nullptr);
 hipError_t launch_compute_energy(const DevFields &f, DevScalars *s, const KParams &P, const Scratch &sc,
-                                 int64_t n_ub, hipStream_t st);
+                                 int64_t n_ub, hipStream_t st, bool end_step = false);
 
 // learned apsides brackets (k_mlp.hip)
 int mlp_grid_blocks(int64_t batch);
