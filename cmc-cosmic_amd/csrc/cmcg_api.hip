@@ -45,6 +45,9 @@ struct cmcg_ctx {
     int64_t adam_t = 0;
     float *io = nullptr;
     int64_t io_cap = 0;          // floats
+    double *query = nullptr;     // inputs and outputs of a batch of queries, kept between calls
+    int64_t query_cap = 0;       // doubles
+    std::mutex query_mu;         // a query holds it: queries may come from several threads
     // step graphs: the fused sort swaps buffer pointers, so steps alternate between
     // two pointer states; graph[p] is the step captured in state p
     hipGraphExec_t graph[2] = {nullptr, nullptr};
@@ -555,9 +558,11 @@ int cmcg_destroy(cmcg_ctx *c)
     for (auto e : c->event_pool) hipEventDestroy(e);
     for (void *p : c->allocs) hipFree(p);
     if (c->io) hipFree(c->io);
+    if (c->query) hipFree(c->query);
     if (c->flush_buf) hipFree(c->flush_buf);
     if (c->mpc_buf) hipFree(c->mpc_buf);
     if (c->cen_buf) hipFree(c->cen_buf);
+    if (c->rep_buf) hipFree(c->rep_buf);
     if (c->sc.jump) jump_release(c->device);
     if (c->stream) hipStreamDestroy(c->stream);
     delete c;
@@ -811,22 +816,30 @@ int cmcg_potential(cmcg_ctx *c, int64_t *n_max, double *mtotal, double *rtidal)
     return h.error;
 }
 
+static int query_reserve(cmcg_ctx *c, int64_t doubles)
+{
+    if (doubles <= c->query_cap) return CMCG_OK;
+    if (c->query) { hipFree(c->query); c->query = nullptr; c->query_cap = 0; }
+    if (hipMalloc((void **)&c->query, (size_t)doubles * sizeof(double)) != hipSuccess) {
+        c->query = nullptr;
+        return CMCG_E_NOMEM;
+    }
+    c->query_cap = doubles;
+    return CMCG_OK;
+}
+
 int cmcg_potential_at(cmcg_ctx *c, int64_t count, const double *r, double *out)
 {
     if (!c || count < 0 || (count > 0 && (!r || !out))) return CMCG_E_ARG;
     if (count == 0) return CMCG_OK;
-    double *dx = nullptr, *dy = nullptr;
-    if (hipMalloc(&dx, count * sizeof(double)) != hipSuccess) return CMCG_E_NOMEM;
-    if (hipMalloc(&dy, count * sizeof(double)) != hipSuccess) { hipFree(dx); return CMCG_E_NOMEM; }
-    int rc = CMCG_OK;
+    std::lock_guard<std::mutex> lk(c->query_mu);
+    if (int e = query_reserve(c, 2 * count)) return e;
+    double *dx = c->query, *dy = dx + count;
     if (hipMemcpyAsync(dx, r, count * sizeof(double), hipMemcpyHostToDevice, c->stream) != hipSuccess ||
         launch_potential_at(c->f, c->s, c->kp, dx, dy, count, c->stream) != hipSuccess ||
         hipMemcpyAsync(out, dy, count * sizeof(double), hipMemcpyDeviceToHost, c->stream) != hipSuccess ||
         sync(c) != hipSuccess)
-        rc = CMCG_E_HIP;
-    hipFree(dx);
-    hipFree(dy);
-    if (rc) return rc;
+        return CMCG_E_HIP;
     return check_error(c);
 }
 
@@ -908,34 +921,33 @@ int cmcg_calc_pericenter_and_apocenter(cmcg_ctx *c, int64_t first, int64_t count
     if (!c || count < 0 || !E || !J) return CMCG_E_ARG;
     if (count == 0) return CMCG_OK;
     if (first < 1 || first + count - 1 > c->n_ub) return CMCG_E_ARG;
-    double *dE, *dJ, *d4;
-    int64_t *dk;
-    int32_t *dc;
-    if (hipMalloc(&dE, count * 8) || hipMalloc(&dJ, count * 8) || hipMalloc(&d4, count * 32) ||
-        hipMalloc(&dk, count * 16) || hipMalloc(&dc, count * 4))
-        return CMCG_E_NOMEM;
-    std::vector<double> h4(4 * count);
-    std::vector<int64_t> hk(2 * count);
-    std::vector<int32_t> hc(count);
-    int rc = CMCG_OK;
-    if (hipMemcpyAsync(dE, E, count * 8, hipMemcpyHostToDevice, c->stream) ||
-        hipMemcpyAsync(dJ, J, count * 8, hipMemcpyHostToDevice, c->stream) ||
-        launch_apsides(c->f, c->s, c->kp, first, count, dE, dJ, d4, dk, dc, c->stream) ||
-        hipMemcpyAsync(h4.data(), d4, count * 32, hipMemcpyDeviceToHost, c->stream) ||
-        hipMemcpyAsync(hk.data(), dk, count * 16, hipMemcpyDeviceToHost, c->stream) ||
-        hipMemcpyAsync(hc.data(), dc, count * 4, hipMemcpyDeviceToHost, c->stream) || sync(c))
-        rc = CMCG_E_HIP;
-    hipFree(dE); hipFree(dJ); hipFree(d4); hipFree(dk); hipFree(dc);
-    if (rc) return rc;
-    for (int64_t i = 0; i < count; i++) {
-        if (rp) rp[i] = h4[4 * i];
-        if (ra) ra[i] = h4[4 * i + 1];
-        if (dQdrp) dQdrp[i] = h4[4 * i + 2];
-        if (dQdra) dQdra[i] = h4[4 * i + 3];
-        if (kmin) kmin[i] = hk[2 * i];
-        if (kmax) kmax[i] = hk[2 * i + 1];
-        if (circular) circular[i] = hc[i];
-    }
+    // eight 8-byte arrays and one of 4 bytes in the context's query buffer, each copied
+    // straight to and from the caller's (five allocations and frees, and outputs interleaved
+    // and sorted out on the host: 900 us for 1e5 stars)
+    std::lock_guard<std::mutex> lk(c->query_mu);
+    if (int e = query_reserve(c, 9 * count)) return e;
+    double *d = c->query;
+    ApsidesOut o;
+    o.rp = d + 2 * count;
+    o.ra = d + 3 * count;
+    o.dQdrp = d + 4 * count;
+    o.dQdra = d + 5 * count;
+    o.kmin = (int64_t *)(d + 6 * count);
+    o.kmax = (int64_t *)(d + 7 * count);
+    o.circular = (int32_t *)(d + 8 * count);
+    const size_t b8 = (size_t)count * 8;
+    hipStream_t st = c->stream;
+    bool bad = hipMemcpyAsync(d, E, b8, hipMemcpyHostToDevice, st) ||
+               hipMemcpyAsync(d + count, J, b8, hipMemcpyHostToDevice, st) ||
+               launch_apsides_soa(c->f, c->s, c->kp, first, count, d, d + count, o, st);
+    if (!bad && rp) bad = hipMemcpyAsync(rp, o.rp, b8, hipMemcpyDeviceToHost, st);
+    if (!bad && ra) bad = hipMemcpyAsync(ra, o.ra, b8, hipMemcpyDeviceToHost, st);
+    if (!bad && dQdrp) bad = hipMemcpyAsync(dQdrp, o.dQdrp, b8, hipMemcpyDeviceToHost, st);
+    if (!bad && dQdra) bad = hipMemcpyAsync(dQdra, o.dQdra, b8, hipMemcpyDeviceToHost, st);
+    if (!bad && kmin) bad = hipMemcpyAsync(kmin, o.kmin, b8, hipMemcpyDeviceToHost, st);
+    if (!bad && kmax) bad = hipMemcpyAsync(kmax, o.kmax, b8, hipMemcpyDeviceToHost, st);
+    if (!bad && circular) bad = hipMemcpyAsync(circular, o.circular, (size_t)count * 4, hipMemcpyDeviceToHost, st);
+    if (sync(c) || bad) return CMCG_E_HIP;
     return check_error(c);
 }
 

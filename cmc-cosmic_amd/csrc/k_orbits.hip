@@ -696,25 +696,7 @@ struct defer_tail_kernel {
 }
 };
 
-struct apsides_kernel {
-    static constexpr int LB = 1024, MB = 0;
-    static __device__ __forceinline__ void run(KGrid kg_, DevFields f, DevScalars *s, KParams P, int64_t first, int64_t count,
-                               const double *__restrict__ E, const double *__restrict__ J,
-                               double *__restrict__ out4, int64_t *__restrict__ kout, int32_t *__restrict__ circ)
-{
-    int64_t i = (int64_t)kg_.bid * blockDim.x + threadIdx.x;
-    if (i >= count) return;
-    int64_t j = first + i, n = s->n_max;
-    OrbitRS o = calc_orbit(f.r, f.phi, n, j, f.r[j], f.m[j], P, E[i], J[i]);
-    if (o.err) dev_set_error(s, o.err, j);
-    out4[4 * i + 0] = o.rp; out4[4 * i + 1] = o.ra; out4[4 * i + 2] = o.dQdrp; out4[4 * i + 3] = o.dQdra;
-    kout[2 * i + 0] = o.kmin; kout[2 * i + 1] = o.kmax;
-    circ[i] = o.circular;
-}
-};
-
-// The same per-star apsides written to one array per output (for callers that copy
-// each output straight into its own host array).
+// calc_orbit_new of a batch, one array per output (callers copy each straight into their own).
 struct apsides_soa_kernel {
     static constexpr int LB = 1024, MB = 0;
     static __device__ __forceinline__ void run(KGrid kg_, DevFields f, DevScalars *s, KParams P, int64_t first, int64_t count,
@@ -1000,16 +982,6 @@ void orbit_variant_shape(int v, int *threads, int *coarse, int *cap, int *minb)
     *coarse = kOrbVariants[v].coarse;
     if (cap) *cap = kOrbVariants[v].cap;
     if (minb) *minb = kOrbVariants[v].minb;
-}
-
-hipError_t launch_apsides(const DevFields &f, DevScalars *s, const KParams &P, int64_t first, int64_t count,
-                          const double *E, const double *J, double *out4, int64_t *kout, int32_t *circ,
-                          hipStream_t st)
-{
-    if (count <= 0) return hipSuccess;
-    kl<apsides_kernel>(dim3((unsigned)((count + 255) / 256)), dim3(256), 0, st, f, s, P, first,
-                       count, E, J, out4, kout, circ);
-    return hipGetLastError();
 }
 
 hipError_t launch_apsides_soa(const DevFields &f, DevScalars *s, const KParams &P, int64_t first, int64_t count,
