@@ -61,6 +61,7 @@ struct cmcg_ctx {
     size_t flush_words = 0;
     void *mpc_buf = nullptr;     // cmcg_comp_mass_percent results (allocated on first use)
     void *cen_buf = nullptr;     // cmcg_central_calculate results (allocated on first use)
+    void *rep_buf = nullptr;     // the chain lists of both (allocated on first use)
 };
 
 static void invalidate_graphs(cmcg_ctx *c)
@@ -522,9 +523,8 @@ int cmcg_create(cmcg_ctx **out, int device, int64_t n_cap, const cmcg_params *pa
         (e = dalloc(c, &sc.sv3_wend, (size_t)n_cap + 2)) || (e = dalloc(c, &sc.sv3_merged, (size_t)n_cap + 2)) ||
         (e = dalloc(c, &sc.sv3_blk, (size_t)sc.max_blocks)) || (e = dalloc(c, &sc.sv3_fallback, 1)) ||
         (e = dalloc(c, &sc.strip_done, 1)) || (e = dalloc(c, &sc.chain_x, (size_t)n_cap + 8)) ||
-        (e = dalloc(c, &sc.chain_g, (size_t)n_cap + 8)) ||
         (e = dalloc(c, &sc.defer_list, (size_t)P.defer_cap)) || (e = dalloc(c, &sc.defer_kfirst, (size_t)P.defer_cap)) || (e = dalloc(c, &sc.defer_order, (size_t)P.defer_cap)) ||
-        (e = dalloc(c, &sc.chain_scal, 4)) || (e = dalloc(c, &sc.chain_len, 4)) || (e = dalloc(c, &sc.chain_fbad, 8)) ||
+        (e = dalloc(c, &sc.chain_scal, 4)) || (e = dalloc(c, &sc.chain_fbad, 8)) ||
         (e = dalloc(c, &sc.esa_idx, (size_t)sc.esa_max)) || (e = dalloc(c, &sc.esa_racc, (size_t)sc.esa_max)) ||
         (e = dalloc(c, &sc.esa_v, (size_t)sc.esa_max)) || (e = dalloc(c, &sc.esa_n, 8)) ||
         (e = dalloc(c, &sc.esa_raw_idx, 2 * 2048)) || (e = dalloc(c, &sc.esa_raw_part, 2 * 3 * 2048)) ||
@@ -1853,6 +1853,15 @@ int cmcg_autotune(cmcg_ctx *c, int reps, int32_t *variant, int32_t *threads, int
     return CMCG_OK;
 }
 
+// the reports' chain lists (9.5 MB and 0.2 words per star), allocated by the first of them
+static int report_reserve(cmcg_ctx *c)
+{
+    if (c->rep_buf) return CMCG_OK;
+    if (hipMalloc(&c->rep_buf, report_work_bytes(c->sc)) == hipSuccess) return CMCG_OK;
+    c->rep_buf = nullptr;
+    return CMCG_E_NOMEM;
+}
+
 int cmcg_comp_mass_percent(cmcg_ctx *c, const double *mass_pc, int32_t count, int32_t bh_include,
                            double initial_total_mass, double minimum_r, cmcg_mass_pc *out)
 {
@@ -1865,13 +1874,14 @@ int cmcg_comp_mass_percent(cmcg_ctx *c, const double *mass_pc, int32_t count, in
             return CMCG_E_NOMEM;
         }
     }
+    if (int e = report_reserve(c)) return e;
     char *dev = (char *)c->mpc_buf;
     double *dpc = (double *)(dev + mass_percent_out_bytes());
     if (count > 0 && hipMemcpyAsync(dpc, mass_pc, count * sizeof(double), hipMemcpyHostToDevice, c->stream) != hipSuccess)
         return CMCG_E_HIP;
     if (hipMemsetAsync(dev, 0, mass_percent_out_bytes(), c->stream) != hipSuccess) return CMCG_E_HIP;
     LAUNCH(launch_mass_percent(c->f, c->s, c->kp, c->n_ub, c->sc, dpc, count, bh_include, initial_total_mass,
-                               minimum_r, dev, c->stream));
+                               minimum_r, dev, c->rep_buf, c->stream));
     std::vector<char> host(mass_percent_out_bytes());
     if (hipMemcpyAsync(host.data(), dev, host.size(), hipMemcpyDeviceToHost, c->stream) != hipSuccess ||
         sync(c) != hipSuccess)
@@ -1900,7 +1910,8 @@ int cmcg_central_calculate(cmcg_ctx *c, cmcg_central *out)
             return CMCG_E_NOMEM;
         }
     }
-    LAUNCH(launch_central(c->f, c->s, c->kp, c->n_ub, c->sc, c->cen_buf, c->stream));
+    if (int e = report_reserve(c)) return e;
+    LAUNCH(launch_central(c->f, c->s, c->kp, c->n_ub, c->sc, c->cen_buf, c->rep_buf, c->stream));
     // layout: int64 nave, int32 error, int32 pad, then 13 doubles in cmcg_central's order
     std::vector<char> host(central_out_bytes());
     if (hipMemcpyAsync(host.data(), c->cen_buf, host.size(), hipMemcpyDeviceToHost, c->stream) != hipSuccess ||

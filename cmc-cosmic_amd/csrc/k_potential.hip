@@ -1201,21 +1201,95 @@ struct pot_at_kernel {
 }
 };
 
-// The chain's increments must be in e.x; `summed`: their tile sums are already formed
-// (by a producer that calls esa_tile_sums over the same grid).
-hipError_t run_chain(const EsaArgs &e, int64_t n_ub, hipStream_t st, bool summed = false)
+// Independent chains side by side: the buffers of chain c lie c words (xs for the increments
+// and values) after those of chain 0.
+__device__ __forceinline__ EsaArgs esa_chain(EsaArgs e, int64_t c, int64_t words, int64_t xs)
+{
+    const int64_t w = c * words;
+    e.x += c * xs; e.g += c * xs;
+    e.v0p += w; e.first_bad += w; e.Lp += w;
+    e.tsumP += w; e.tpreP += w; e.tcnt += w; e.ttail += w; e.toff += w; e.tcarry += w;
+    e.s_idx += w; e.s_pre += w; e.s_v += w; e.s_n += w;
+    e.raw_n += w; e.raw_idx += w; e.raw_part += w; e.raw_bp += 2 * w; e.raw_sx += w;
+    return e;
+}
+// kernel K of every chain in one launch, `per` blocks each
+template <class K>
+struct esa_each {
+    static constexpr int LB = K::LB, MB = 0;
+    static __device__ __forceinline__ void run(KGrid kg_, EsaArgs e, int64_t words, int64_t xs, unsigned per)
+    {
+        const unsigned c = kg_.bid / per;
+        K::run(KGrid{kg_.bid - c * per, per, 0, 1}, esa_chain(e, c, words, xs));
+    }
+};
+template <class K>
+struct esa_each1 {
+    static constexpr int LB = K::LB, MB = 0;
+    static __device__ __forceinline__ void run(KGrid kg_, EsaArgs e, int64_t words, int64_t xs, unsigned per, int64_t arg)
+    {
+        const unsigned c = kg_.bid / per;
+        K::run(KGrid{kg_.bid - c * per, per, 0, 1}, esa_chain(e, c, words, xs), arg);
+    }
+};
+
+// The increments must be in every chain's x.  (One after another, the five chains of
+// comp_mass_percent and the seven of central_calculate took 30 and 50 launches, each too
+// small to fill the chip: 380 and 350 us at N = 1e6.)
+hipError_t run_chains(const EsaArgs &e, int64_t words, int64_t xs, int chains, int64_t n_ub, hipStream_t st)
 {
     int64_t ntiles = (n_ub + CTILE - 1) / CTILE;
     if (ntiles < 1) ntiles = 1;
-    dim3 gt((unsigned)ntiles), bt(CT);
-    if (!summed) kl<esa_sum_kernel>(gt, bt, 0, st, e);
+    const unsigned per = (unsigned)ntiles;
+    const dim3 gt(per * chains), gc((unsigned)chains), bt(CT);
+    kl<esa_each<esa_sum_kernel>>(gt, bt, 0, st, e, words, xs, per);
     const bool self_prefix = ntiles <= SELF_PREFIX_MAX;
-    if (!self_prefix) kl<esa_tile_scan_kernel>(dim3(1), dim3(WALK_T), 0, st, e, ntiles);
-    kl<esa_classify_kernel>(gt, bt, 0, st, e, (int)self_prefix);
-    kl<esa_walk_kernel>(dim3(1), dim3(CT), 0, st, e);
-    kl<esa_rebuild_kernel>(gt, bt, 0, st, e);
-    kl<chain_finish_kernel>(dim3(1), dim3(WALK_T), 0, st, e);
+    if (!self_prefix) kl<esa_each1<esa_tile_scan_kernel>>(gc, dim3(WALK_T), 0, st, e, words, xs, 1u, ntiles);
+    kl<esa_each1<esa_classify_kernel>>(gt, bt, 0, st, e, words, xs, per, (int64_t)self_prefix);
+    kl<esa_each<esa_walk_kernel>>(gc, bt, 0, st, e, words, xs, 1u);
+    kl<esa_each<esa_rebuild_kernel>>(gt, bt, 0, st, e, words, xs, per);
+    kl<esa_each<chain_finish_kernel>>(gc, dim3(WALK_T), 0, st, e, words, xs, 1u);
     return hipGetLastError();
+}
+
+// The buffers of up to REPORT_CHAINS chains: the lists and tile sums in the report workspace,
+// the increments and values in the sort's record scratch (16 words per star, free between
+// sorts; 12 are used).
+constexpr int REPORT_CHAINS = 6;
+constexpr int64_t REPORT_LIST = 1 << 16;
+int64_t report_words(int64_t T) { return 6 * T + 3 * REPORT_LIST + 8 + 4 * RAW_CAP; }
+EsaArgs report_chain0(const Scratch &sc, int slack, void *work, int64_t xs)
+{
+    const int64_t T = sc.max_tiles;
+    double *w = (double *)work;
+    EsaArgs e{};
+    e.slack = slack;
+    e.sign = 1.0;
+    e.x = (const double *)sc.sort_aos;
+    e.g = (double *)sc.sort_aos + REPORT_CHAINS * xs;
+    e.tsumP = w;
+    e.tpreP = w + T;
+    e.tcnt = (int64_t *)(w + 2 * T);
+    e.ttail = (int64_t *)(w + 3 * T);
+    e.toff = (int64_t *)(w + 4 * T);
+    e.tcarry = (int64_t *)(w + 5 * T);
+    w += 6 * T;
+    e.s_idx = (int64_t *)w;
+    e.s_pre = w + REPORT_LIST;
+    e.s_v = w + 2 * REPORT_LIST;
+    e.smax = REPORT_LIST;
+    w += 3 * REPORT_LIST;
+    e.s_n = (int64_t *)w;
+    e.raw_n = (int64_t *)(w + 1);
+    e.first_bad = (int64_t *)(w + 2);
+    e.Lp = (const int64_t *)(w + 4);
+    e.v0p = w + 5;
+    w += 8;
+    e.raw_idx = (int64_t *)w;
+    e.raw_part = (int64_t *)(w + RAW_CAP);
+    e.raw_bp = (int32_t *)(e.raw_part + RAW_CAP);
+    e.raw_sx = (double *)(e.raw_part + 2 * RAW_CAP);
+    return e;
 }
 
 // The chains' per-tile and list buffers in the context's scratch (tile_sums: six
@@ -1260,37 +1334,28 @@ struct MassPcOut {
     int64_t reached;             // fractions assigned
 };
 
-struct mpc_prep_m_kernel {
+// Chain 0: star_m[k] / clus.N_STAR; 1 to 4: 0.5 m madhoc vr vr, 0.5 m madhoc vt vt, vr vr,
+// vt vt (left to right), k = j + 1; and the chains' lengths and start values.
+struct mpc_prep_kernel {
     static constexpr int LB = 1024, MB = 0;
-    static __device__ __forceinline__ void run(KGrid kg_, const double *__restrict__ m, const DevScalars *s, double nstar,
-                                  double *__restrict__ x, int64_t *__restrict__ len)
+    static __device__ __forceinline__ void run(KGrid kg_, const DevFields f, const DevScalars *s, double nstar, double madhoc,
+                                  double mprev0, EsaArgs e, int64_t words, int64_t xs)
 {
-    const int64_t j = (int64_t)kg_.bid * blockDim.x + threadIdx.x;
-    const int64_t n = s->n_max;
-    if (j == 0) len[3] = n;
-    if (j < n) x[j] = m[j + 1] / nstar;                   // star_m[k] / clus.N_STAR, k = j + 1
-}
-};
-
-// term 0: 0.5 m madhoc vr vr, 1: 0.5 m madhoc vt vt, 2: vr vr, 3: vt vt (left to right)
-struct mpc_prep_v_kernel {
-    static constexpr int LB = 1024, MB = 0;
-    static __device__ __forceinline__ void run(KGrid kg_, const DevFields f, const DevScalars *s, double madhoc, int term,
-                                  double *__restrict__ x, int64_t *__restrict__ len)
-{
-    const int64_t j = (int64_t)kg_.bid * blockDim.x + threadIdx.x;
-    const int64_t n = s->n_max_new;
-    if (j == 0) len[3] = n;
-    if (j >= n) return;
-    const int64_t k = j + 1;
-    double v;
-    switch (term) {
-    case 0: v = 0.5 * f.m[k] * madhoc * f.vr[k] * f.vr[k]; break;
-    case 1: v = 0.5 * f.m[k] * madhoc * f.vt[k] * f.vt[k]; break;
-    case 2: v = f.vr[k] * f.vr[k]; break;
-    default: v = f.vt[k] * f.vt[k]; break;
+    const int64_t j = (int64_t)kg_.bid * blockDim.x + threadIdx.x, k = j + 1;
+    const int64_t n = s->n_max, nn = s->n_max_new;
+    double *x = const_cast<double *>(e.x);
+    if (j < 5) {
+        const_cast<int64_t *>(e.Lp)[j * words] = j == 0 ? n : nn;
+        const_cast<double *>(e.v0p)[j * words] = j == 0 ? mprev0 : 0.0;
     }
-    x[j] = v;
+    if (j < n) x[j] = f.m[k] / nstar;
+    if (j < nn) {
+        const double m = f.m[k], vr = f.vr[k], vt = f.vt[k];
+        x[xs + j] = 0.5 * m * madhoc * vr * vr;
+        x[2 * xs + j] = 0.5 * m * madhoc * vt * vt;
+        x[3 * xs + j] = vr * vr;
+        x[4 * xs + j] = vt * vt;
+    }
 }
 };
 
@@ -1303,65 +1368,61 @@ __device__ __forceinline__ double cube_rn(double x)
     return q + (f1 + e * x);
 }
 
-// the fractions' indices (one fraction per star at most, as the reference's loop),
-// from the enclosed-mass chain g[k-1] = mprev after star k
-struct mpc_assign_kernel {
-    static constexpr int LB = 1024, MB = 0;
-    static __device__ __forceinline__ void run(KGrid kg_, const double *__restrict__ r, const DevScalars *s, const double *__restrict__ g,
-                                  const double *__restrict__ pc, int count, int bh_include, double mprev0,
-                                  double itm, double minimum_r, MassPcOut *o)
+// The fractions' indices (one fraction per star at most, as the reference's loop) from the
+// enclosed-mass chain g[k-1] = mprev after star k, which does not decrease: a thread finds
+// each fraction's first k with g[k-1] > pc Mtotal, one thread then moves them past the
+// fraction before, and the threads take the values there.  (One thread searching for one
+// fraction after another waited on 20 loads for each.)
+struct mpc_finish_kernel {
+    static constexpr int LB = MPC_MAX, MB = 0;
+    static __device__ __forceinline__ void run(KGrid kg_, const double *__restrict__ r, const DevScalars *s,
+                                  const double *__restrict__ g, int64_t xs, const double *__restrict__ pc, int count,
+                                  int bh_include, double mprev0, double itm, double minimum_r, MassPcOut *o)
 {
-    if (threadIdx.x != 0 || kg_.bid != 0) return;
+    __shared__ int64_t ks[MPC_MAX];
+    __shared__ int reached;
     const double PI = 3.14159265358979323;                  // include/cmc/cmc.h:62
     const double Mtotal = s->Mtotal;
     const int64_t n = s->n_max;
-    int mc = 0;
-    if (bh_include)
-        for (; mc < count && mprev0 / Mtotal > pc[mc]; mc++) {
-            o->v[0][mc] = minimum_r;
-            for (int q = 1; q < 7; q++) o->v[q][mc] = 0.0;
-            o->k[mc] = 0;
-        }
-    int64_t kprev = 0;
-    for (; mc < count; mc++) {
-        const double thr = pc[mc] * Mtotal;
-        // smallest k in (kprev, n] with g[k-1] > thr; g is non-decreasing
-        int64_t lo = kprev + 1, hi = n + 1;
+    const int i = threadIdx.x;
+    if (i < count) {
+        const double thr = pc[i] * Mtotal;
+        int64_t lo = 1, hi = n + 1;
         while (lo < hi) {
             const int64_t mid = lo + (hi - lo) / 2;
             if (g[mid - 1] > thr) hi = mid;
             else lo = mid + 1;
         }
-        if (lo > n) break;
-        const int64_t k = lo;
-        const double mprev = g[k - 1];
-        o->v[0][mc] = r[k];
-        o->v[1][mc] = mprev / Mtotal / k * itm;
-        o->v[2][mc] = mprev / (4.0 / 3.0 * PI * cube_rn(r[k]));
-        o->k[mc] = k;
-        kprev = k;
+        ks[i] = lo;
     }
-    o->reached = mc;
-}
-};
-
-struct mpc_init_kernel {
-    static constexpr int LB = 1024, MB = 0;
-    static __device__ __forceinline__ void run(KGrid kg_, double *v0, double mprev0)
-{
-    v0[0] = mprev0;
-    v0[1] = 0.0;
-}
-};
-
-struct mpc_take_kernel {
-    static constexpr int LB = 1024, MB = 0;
-    static __device__ __forceinline__ void run(KGrid kg_, const double *__restrict__ g, MassPcOut *o, int term, int count)
-{
-    const int i = threadIdx.x;
-    if (i >= count || i >= o->reached) return;
-    const int64_t k = o->k[i];
-    o->v[3 + term][i] = k > 0 ? g[k - 1] : 0.0;
+    __syncthreads();
+    if (i == 0) {
+        int mc = 0;
+        if (bh_include)
+            for (; mc < count && mprev0 / Mtotal > pc[mc]; mc++) ks[mc] = 0;
+        int64_t kprev = 0;
+        for (; mc < count; mc++) {
+            const int64_t k = ks[mc] > kprev ? ks[mc] : kprev + 1;
+            if (k > n) break;
+            ks[mc] = kprev = k;
+        }
+        reached = mc;
+        o->reached = mc;
+    }
+    __syncthreads();
+    if (i >= reached) return;
+    const int64_t k = ks[i];
+    o->k[i] = k;
+    if (k > 0) {
+        const double mprev = g[k - 1];
+        o->v[0][i] = r[k];
+        o->v[1][i] = mprev / Mtotal / k * itm;
+        o->v[2][i] = mprev / (4.0 / 3.0 * PI * cube_rn(r[k]));
+        for (int t = 0; t < 4; t++) o->v[3 + t][i] = g[(t + 1) * xs + k - 1];
+    } else {                                                // the central mass alone
+        o->v[0][i] = minimum_r;
+        for (int q = 1; q < 7; q++) o->v[q][i] = 0.0;
+    }
 }
 };
 
@@ -1420,39 +1481,25 @@ hipError_t launch_potential_at(const DevFields &f, DevScalars *s, const KParams 
     return hipGetLastError();
 }
 
-// comp_mass_percent: pc (device, count <= MPC_MAX, ascending), results into out
+size_t report_work_bytes(const Scratch &sc) { return (size_t)REPORT_CHAINS * report_words(sc.max_tiles) * 8; }
+
+// comp_mass_percent: pc (device, count <= MPC_MAX, ascending), results into out; work: the
+// report workspace
 hipError_t launch_mass_percent(const DevFields &f, DevScalars *s, const KParams &P, int64_t n_ub, const Scratch &sc,
                                const double *pc, int count, int bh_include, double itm, double minimum_r,
-                               void *out, hipStream_t st)
+                               void *out, void *work, hipStream_t st)
 {
     if (count < 0 || count > MPC_MAX) return hipErrorInvalidValue;
     int64_t ntiles = (n_ub + CTILE - 1) / CTILE + 1;
     if (ntiles > sc.max_tiles) return hipErrorInvalidValue;
-    EsaArgs e = esa_args(sc, P.chain_k_drop);
-    e.x = sc.chain_x; e.g = sc.chain_g; e.sign = 1.0; e.first_bad = sc.chain_fbad + 6;
-    e.Lp = sc.chain_len + 3;
-    double *v0 = sc.chain_scal + 2;              // start values: [2] mprev0, [3] 0
+    const int64_t xs = n_ub + 4, words = report_words(sc.max_tiles);
+    const EsaArgs e = report_chain0(sc, P.chain_k_drop, work, xs);
     const double mprev0 = bh_include ? P.cenma_m * P.madhoc : 0.0;   // cmc_utils.c:878
-    kl<mpc_init_kernel>(dim3(1), dim3(1), 0, st, v0, mprev0);
-    MassPcOut *o = (MassPcOut *)out;
-    unsigned g1 = (unsigned)((n_ub + 256) / 256);
-    // chain M
-    kl<mpc_prep_m_kernel>(dim3(g1), dim3(256), 0, st, f.m, (const DevScalars *)s, (double)P.n_star,
-                       sc.chain_x, sc.chain_len);
-    EsaArgs em = e;
-    em.v0p = v0;
-    if (hipError_t err = run_chain(em, n_ub, st)) return err;
-    kl<mpc_assign_kernel>(dim3(1), dim3(1), 0, st, (const double *)f.r, (const DevScalars *)s,
-                       (const double *)sc.chain_g, pc, count, bh_include, mprev0, itm, minimum_r, o);
-    // the four running sums
-    for (int term = 0; term < 4; term++) {
-        kl<mpc_prep_v_kernel>(dim3(g1), dim3(256), 0, st, f, (const DevScalars *)s, P.madhoc, term,
-                           sc.chain_x, sc.chain_len);
-        EsaArgs ev = e;
-        ev.v0p = v0 + 1;
-        if (hipError_t err = run_chain(ev, n_ub, st)) return err;
-        kl<mpc_take_kernel>(dim3(1), dim3(MPC_MAX), 0, st, (const double *)sc.chain_g, o, term, count);
-    }
+    kl<mpc_prep_kernel>(dim3((unsigned)((n_ub + 256) / 256)), dim3(256), 0, st, f, (const DevScalars *)s, (double)P.n_star,
+                       P.madhoc, mprev0, e, words, xs);
+    if (hipError_t err = run_chains(e, words, xs, 5, n_ub, st)) return err;
+    kl<mpc_finish_kernel>(dim3(1), dim3(MPC_MAX), 0, st, (const double *)f.r, (const DevScalars *)s, (const double *)e.g, xs,
+                       pc, count, bh_include, mprev0, itm, minimum_r, (MassPcOut *)out);
     return hipGetLastError();
 }
 
@@ -1493,78 +1540,95 @@ __device__ __forceinline__ double cen_rhoj(const double *__restrict__ r, const d
     return mrho / Vrj;
 }
 
-__device__ __forceinline__ double cen_term(const DevFields &f, double madhoc, int64_t i, int t)
+__device__ __forceinline__ void cen_terms(const DevFields &f, double madhoc, int64_t i, double (&v)[CEN_TERMS])
 {
-    const double rj = cen_rhoj(f.r, f.m, madhoc, i);
-    switch (t) {
-    case 0: return rj;
-    case 1: return rj * rj;
-    case 2: return rj * (f.vr[i] * f.vr[i] + f.vt[i] * f.vt[i]);
-    case 3: return rj * f.r[i];
-    case 4: { const double q = rj * f.r[i]; return q * q; }
-    default: return rj * f.m[i] * madhoc;
-    }
+    const double rj = cen_rhoj(f.r, f.m, madhoc, i), r = f.r[i], vr = f.vr[i], vt = f.vt[i], q = rj * r;
+    v[0] = rj;
+    v[1] = rj * rj;
+    v[2] = rj * (vr * vr + vt * vt);
+    v[3] = q;
+    v[4] = q * q;
+    v[5] = rj * f.m[i] * madhoc;
 }
 
-struct cen_init_kernel {
+// The enclosed-mass chain's increments star_m[k] / N_STAR from 0, the results and the
+// start values cleared.
+struct cen_begin_kernel {
     static constexpr int LB = 1024, MB = 0;
-    static __device__ __forceinline__ void run(KGrid kg_, CentralOut *o, double *v0)
+    static __device__ __forceinline__ void run(KGrid kg_, const double *__restrict__ m, const DevScalars *s, double nstar,
+                                  CentralOut *o, EsaArgs e, int64_t words)
 {
-    if (threadIdx.x != 0 || kg_.bid != 0) return;
-    o->nave = 0;
-    o->error = CEN_OK;
-    for (int t = 0; t < CEN_TERMS; t++) {
-        o->mx[t] = 0ull;
-        o->S[t] = 0.0;
-        o->scale[t] = o->unscale[t] = 1.0;
-    }
-    v0[0] = 0.0;
-    v0[1] = 0.0;
-}
-};
-
-// nave and rh from the chain g[k-1] = m after star k (cmc_utils.c:1247-1257, 1620-1623);
-// the chain length for the sums becomes nave
-struct cen_nave_kernel {
-    static constexpr int LB = 1024, MB = 0;
-    static __device__ __forceinline__ void run(KGrid kg_, const double *__restrict__ r, const DevScalars *s, const double *__restrict__ g,
-                                int64_t n_star, CentralOut *o, int64_t *len)
-{
-    if (threadIdx.x != 0 || kg_.bid != 0) return;
+    const int64_t j = (int64_t)kg_.bid * blockDim.x + threadIdx.x;
     const int64_t n = s->n_max;
-    const double thr = 0.5 * s->Mtotal;
-    int64_t lo = 1, hi = n + 1;                 // smallest k with !(g[k-1] < thr); g non-decreasing
-    while (lo < hi) {
-        const int64_t mid = lo + (hi - lo) / 2;
-        if (!(g[mid - 1] < thr)) hi = mid;
-        else lo = mid + 1;
-    }
-    const int64_t nave = lo + 1;
-    const int64_t jmax_last = (nave - 3 > 1 ? nave - 3 : 1) + 6;
-    if (lo > n || n_star <= 12 || nave >= n_star - 6 || jmax_last > n + 1) {
-        o->error = CEN_E_STATE;
+    if (j == 0) {
         o->nave = 0;
-        len[3] = 1;                             // the sums then run over one zero term
-        return;
+        o->error = CEN_OK;
+        *const_cast<int64_t *>(e.Lp) = n;
     }
-    o->nave = nave;
-    o->rh = r[nave];
-    len[3] = nave;
+    if (j < CEN_TERMS) {
+        o->mx[j] = 0ull;
+        o->S[j] = 0.0;
+        o->scale[j] = o->unscale[j] = 1.0;
+        const_cast<double *>(e.v0p)[j * words] = 0.0;
+    }
+    if (j < n) const_cast<double *>(e.x)[j] = m[j + 1] / nstar;
 }
 };
 
+// Smallest k in [lo, hi) for which pred (true, then false) fails, or hi, by a whole wave: 64
+// probes split the range into 65.
+template <class Pred>
+__device__ __forceinline__ int64_t wave_first_false(int64_t lo, int64_t hi, Pred pred)
+{
+    const int lane = threadIdx.x & 63;
+    while (lo < hi) {
+        const int64_t step = (hi - lo) / 65 + 1, p = lo + (lane + 1) * step - 1;       // lo + 65 step > hi
+        const int c = (int)__popcll(__ballot(p < hi && pred(p)));
+        const int64_t top = lo + (c + 1) * step - 1;
+        lo += c * step;
+        hi = top < hi ? top : hi;
+    }
+    return lo;
+}
+
+// nave and rh from the chain g[k-1] = m after star k (cmc_utils.c:1247-1257, 1620-1623), by
+// every block for itself: nave is the sums' length; then the terms' maxima.
 struct cen_max_kernel {
     static constexpr int LB = 256, MB = 0;
-    static __device__ __forceinline__ void run(KGrid kg_, const DevFields f, double madhoc, CentralOut *o)
+    static __device__ __forceinline__ void run(KGrid kg_, const DevFields f, const DevScalars *s, const double *__restrict__ g,
+                                  int64_t n_star, double madhoc, CentralOut *o, EsaArgs e, int64_t words)
 {
     __shared__ unsigned long long red[CEN_TERMS][256 / 64];
-    const int64_t nave = o->nave;
+    __shared__ int64_t found;
+    const int64_t n = s->n_max;
+    const double thr = 0.5 * s->Mtotal;
+    if (threadIdx.x < 64) {
+        // smallest k with !(g[k-1] < thr); g does not decrease
+        const int64_t k = wave_first_false(1, n + 1, [&](int64_t q) { return g[q - 1] < thr; });
+        if (threadIdx.x == 0) found = k;
+    }
+    __syncthreads();
+    const int64_t k = found;
+    const int64_t jmax_last = (k + 1 - 3 > 1 ? k + 1 - 3 : 1) + 6;
+    const bool bad = k > n || n_star <= 12 || k + 1 >= n_star - 6 || jmax_last > n + 1;
+    const int64_t nave = bad ? 0 : k + 1;
+    if (kg_.bid == 0 && threadIdx.x < CEN_TERMS) {
+        const_cast<int64_t *>(e.Lp)[threadIdx.x * words] = bad ? 1 : nave;    // bad: the sums run over one zero term
+        if (threadIdx.x == 0) {
+            o->nave = nave;
+            if (bad) o->error = CEN_E_STATE;
+            else o->rh = f.r[nave];
+        }
+    }
     unsigned long long mx[CEN_TERMS] = {0, 0, 0, 0, 0, 0};
-    for (int64_t j = (int64_t)kg_.bid * blockDim.x + threadIdx.x; j < nave; j += (int64_t)kg_.nb * blockDim.x)
+    for (int64_t j = (int64_t)kg_.bid * blockDim.x + threadIdx.x; j < nave; j += (int64_t)kg_.nb * blockDim.x) {
+        double v[CEN_TERMS];
+        cen_terms(f, madhoc, j + 1, v);
         for (int t = 0; t < CEN_TERMS; t++) {
-            const unsigned long long b = (unsigned long long)__double_as_longlong(cen_term(f, madhoc, j + 1, t));
+            const unsigned long long b = (unsigned long long)__double_as_longlong(v[t]);
             mx[t] = b > mx[t] ? b : mx[t];      // a negative or NaN term has the largest patterns
         }
+    }
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
     for (int t = 0; t < CEN_TERMS; t++) {
         unsigned long long v = mx[t];
@@ -1583,59 +1647,65 @@ struct cen_max_kernel {
 }
 };
 
-struct cen_scale_kernel {
-    static constexpr int LB = 1024, MB = 0;
-    static __device__ __forceinline__ void run(KGrid kg_, CentralOut *o)
-{
-    if (threadIdx.x != 0 || kg_.bid != 0 || o->error) return;
-    for (int t = 0; t < CEN_TERMS; t++) {
-        if (o->mx[t] >= 0x7ff0000000000000ull) {   // infinite, NaN or negative
-            o->error = CEN_E_RANGE;
-            return;
-        }
-        const double bound = (double)o->nave * __longlong_as_double((long long)o->mx[t]);
-        if (bound > 0.0) {
-            int e;
-            frexp(bound, &e);                      // bound <= 2^e
-            o->scale[t] = ldexp(1.0, -e);
-            o->unscale[t] = ldexp(1.0, e);
-        }
-    }
-}
-};
-
+// The scales (by every block for itself; block 0 keeps them) and the scaled terms.
 struct cen_prep_kernel {
     static constexpr int LB = 1024, MB = 0;
-    static __device__ __forceinline__ void run(KGrid kg_, const DevFields f, double madhoc, int t, CentralOut *o, double *__restrict__ x)
+    static __device__ __forceinline__ void run(KGrid kg_, const DevFields f, double madhoc, CentralOut *o, EsaArgs e, int64_t xs)
 {
-    const int64_t j = (int64_t)kg_.bid * blockDim.x + threadIdx.x;
-    const int64_t nave = o->nave;
-    if (o->error) {
-        if (j == 0) x[0] = 0.0;
+    __shared__ double scale[CEN_TERMS];
+    __shared__ int range;
+    const int t = threadIdx.x;
+    const int64_t j = (int64_t)kg_.bid * blockDim.x + t, nave = o->nave;
+    if (t == 0) range = 0;
+    __syncthreads();
+    if (t < CEN_TERMS) {
+        const unsigned long long mx = o->mx[t];
+        double up = 1.0, down = 1.0;
+        if (mx >= 0x7ff0000000000000ull) {         // infinite, NaN or negative
+            range = 1;
+        } else {
+            const double bound = (double)nave * __longlong_as_double((long long)mx);
+            if (bound > 0.0) {
+                int x;
+                frexp(bound, &x);                  // bound <= 2^x
+                down = ldexp(1.0, -x);
+                up = ldexp(1.0, x);
+            }
+        }
+        scale[t] = down;
+        if (kg_.bid == 0) {
+            o->scale[t] = down;
+            o->unscale[t] = up;
+        }
+    }
+    __syncthreads();
+    if (range && kg_.bid == 0 && t == 0) o->error = CEN_E_RANGE;
+    double *x = const_cast<double *>(e.x);
+    if (nave == 0 || range) {                      // one zero term, or sums that are not used
+        if (j < (nave > 0 ? nave : 1))
+            for (int q = 0; q < CEN_TERMS; q++) x[q * xs + j] = 0.0;
         return;
     }
     if (j >= nave) return;
-    const double v = cen_term(f, madhoc, j + 1, t) * o->scale[t];
-    if (v != 0.0 && v < 2.2250738585072014e-308) o->error = CEN_E_RANGE;   // scaled into subnormals
-    x[j] = v;
-}
-};
-
-struct cen_take_kernel {
-    static constexpr int LB = 1024, MB = 0;
-    static __device__ __forceinline__ void run(KGrid kg_, const double *__restrict__ g, CentralOut *o, int t)
-{
-    if (threadIdx.x != 0 || kg_.bid != 0 || o->error) return;
-    o->S[t] = g[o->nave - 1] * o->unscale[t];
+    double v[CEN_TERMS];
+    cen_terms(f, madhoc, j + 1, v);
+    for (int q = 0; q < CEN_TERMS; q++) {
+        const double w = v[q] * scale[q];
+        if (w != 0.0 && w < 2.2250738585072014e-308) o->error = CEN_E_RANGE;   // scaled into subnormals
+        x[q * xs + j] = w;
+    }
 }
 };
 
 // the averages and derived quantities, cmc_utils.c:1323-1345
 struct cen_final_kernel {
-    static constexpr int LB = 1024, MB = 0;
-    static __device__ __forceinline__ void run(KGrid kg_, CentralOut *o)
+    static constexpr int LB = 64, MB = 0;
+    static __device__ __forceinline__ void run(KGrid kg_, const double *__restrict__ g, int64_t xs, CentralOut *o)
 {
-    if (threadIdx.x != 0 || kg_.bid != 0 || o->error) return;
+    if (o->error) return;
+    if (threadIdx.x < CEN_TERMS) o->S[threadIdx.x] = g[threadIdx.x * xs + o->nave - 1] * o->unscale[threadIdx.x];
+    __syncthreads();
+    if (threadIdx.x != 0) return;
     const double PI = 3.14159265358979323;
     const double rhojsum = o->S[0], rhoj2sum = o->S[1];
     double rho = o->S[1], v_rms = o->S[2], rc = o->S[3], rc_nb = o->S[4], m_ave = o->S[5];
@@ -1664,36 +1734,22 @@ struct cen_final_kernel {
 };
 
 hipError_t launch_central(const DevFields &f, DevScalars *s, const KParams &P, int64_t n_ub, const Scratch &sc,
-                          void *out, hipStream_t st)
+                          void *out, void *work, hipStream_t st)
 {
     int64_t ntiles = (n_ub + CTILE - 1) / CTILE + 1;
     if (ntiles > sc.max_tiles) return hipErrorInvalidValue;
-    EsaArgs e = esa_args(sc, P.chain_k_drop);
-    e.x = sc.chain_x; e.g = sc.chain_g; e.sign = 1.0; e.first_bad = sc.chain_fbad + 6;
-    e.Lp = sc.chain_len + 3;
-    double *v0 = sc.chain_scal + 2;              // both start values 0
+    const int64_t xs = n_ub + 4, words = report_words(sc.max_tiles);
+    const EsaArgs e = report_chain0(sc, P.chain_k_drop, work, xs);
     CentralOut *o = (CentralOut *)out;
     const unsigned g1 = (unsigned)((n_ub + 256) / 256);
-    kl<cen_init_kernel>(dim3(1), dim3(1), 0, st, o, v0);
-    // enclosed mass, star_m[k] / N_STAR from 0
-    kl<mpc_prep_m_kernel>(dim3(g1), dim3(256), 0, st, f.m, (const DevScalars *)s, (double)P.n_star,
-                       sc.chain_x, sc.chain_len);
-    EsaArgs em = e;
-    em.v0p = v0;
-    if (hipError_t err = run_chain(em, n_ub, st)) return err;
-    kl<cen_nave_kernel>(dim3(1), dim3(1), 0, st, (const double *)f.r, (const DevScalars *)s,
-                       (const double *)sc.chain_g, (int64_t)P.n_star, o, sc.chain_len);
+    kl<cen_begin_kernel>(dim3(g1), dim3(256), 0, st, (const double *)f.m, (const DevScalars *)s, (double)P.n_star, o, e, words);
+    if (hipError_t err = run_chains(e, words, xs, 1, n_ub, st)) return err;
     const unsigned gmax = g1 < 1024u ? g1 : 1024u;
-    kl<cen_max_kernel>(dim3(gmax), dim3(256), 0, st, f, P.madhoc, o);
-    kl<cen_scale_kernel>(dim3(1), dim3(1), 0, st, o);
-    for (int t = 0; t < CEN_TERMS; t++) {
-        kl<cen_prep_kernel>(dim3(g1), dim3(256), 0, st, f, P.madhoc, t, o, sc.chain_x);
-        EsaArgs es = e;
-        es.v0p = v0 + 1;
-        if (hipError_t err = run_chain(es, n_ub, st)) return err;
-        kl<cen_take_kernel>(dim3(1), dim3(1), 0, st, (const double *)sc.chain_g, o, t);
-    }
-    kl<cen_final_kernel>(dim3(1), dim3(1), 0, st, o);
+    kl<cen_max_kernel>(dim3(gmax), dim3(256), 0, st, f, (const DevScalars *)s, (const double *)e.g, (int64_t)P.n_star,
+                       P.madhoc, o, e, words);
+    kl<cen_prep_kernel>(dim3(g1), dim3(256), 0, st, f, P.madhoc, o, e, xs);
+    if (hipError_t err = run_chains(e, words, xs, CEN_TERMS, n_ub, st)) return err;
+    kl<cen_final_kernel>(dim3(1), dim3(64), 0, st, (const double *)e.g, xs, o);
     return hipGetLastError();
 }
 

@@ -42,9 +42,8 @@ struct Scratch {
     // (48 B per tile), chain increments / iterates / enclosed masses per star
     double *tile_sums;         // two sets of 6 words per tile (potential chains)
     int64_t max_tiles;
-    double *chain_x, *chain_g;
+    double *chain_x;
     double *chain_scal;         // 4 doubles
-    int64_t *chain_len;         // 4
     int64_t *chain_fbad;        // 6
     // potential chains: list of sensitive elements (index, int128 prefix, value)
     int64_t *esa_idx;
@@ -102,10 +101,11 @@ hipError_t launch_potential(const DevFields &f, DevScalars *s, const KParams &P,
                             const Scratch &sc, hipStream_t st, bool count = true);
 hipError_t launch_mass_percent(const DevFields &f, DevScalars *s, const KParams &P, int64_t n_ub, const Scratch &sc,
                                const double *pc, int count, int bh_include, double itm, double minimum_r,
-                               void *out, hipStream_t st);
+                               void *out, void *work, hipStream_t st);
 size_t mass_percent_out_bytes();
 hipError_t launch_central(const DevFields &f, DevScalars *s, const KParams &P, int64_t n_ub, const Scratch &sc,
-                          void *out, hipStream_t st);
+                          void *out, void *work, hipStream_t st);
+size_t report_work_bytes(const Scratch &sc);     // what both need as `work`
 size_t central_out_bytes();
 hipError_t launch_potential_at(const DevFields &f, DevScalars *s, const KParams &P,
                                const double *x, double *out, int64_t count, hipStream_t st);
