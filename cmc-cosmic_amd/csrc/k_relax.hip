@@ -289,7 +289,7 @@ struct sigma_kernel {
 };
 
 // calc_sigma_r and simul_relax_new in one pass (the step's form): each block stages
-// m*madhoc and m*madhoc*(vr^2 + vt^2) for its SIG_T stars and 2p on either side (the
+// m*madhoc and m*madhoc*(vr^2 + vt^2) for its SD_N stars and 2p on either side (the
 // roundings of both references' loops, as sigma_lds_kernel and simul_relax_kernel
 // take them), writes sigma of its stars, evaluates the relaxation-time windows that
 // start among its stars (window w = [1 + 2pw, 1 + 2p(w+1)), the sums in the
@@ -298,48 +298,85 @@ struct sigma_kernel {
 // doubles order like their patterns; 0 is the identity, so the slots start and are
 // left at 0); the one-block time-step kernel takes the minimum over the slots.  Needs
 // p <= SIG_MAXP.
+// Bound by LDS reads, 80 a star for p = 20, when a thread has one star, and by the launch for
+// few stars.  For many (SD_MANY) a thread takes SD_PER = 5 neighbours, whose windows share all
+// but SD_PER - 1 elements at either end, and reads each element once (18 a star); an odd number
+// keeps the lanes' reads off each other's banks.  Each star's sums are still formed one element
+// after another.
+template <int SD_T, int SD_PER>
 struct sigma_dt_kernel {
-    static constexpr int LB = SIG_T, MB = 0;
+    static constexpr int LB = SD_T, MB = 0;
+    static constexpr int SD_N = SD_T * SD_PER, SD_LDS = SD_N + 4 * SIG_MAXP + 1;
     static __device__ __forceinline__ void run(KGrid kg_, const double *__restrict__ r, const double *__restrict__ m,
                                                          const double *__restrict__ vr, const double *__restrict__ vt,
                                                          double *__restrict__ sigma, DevScalars *s, KParams P,
                                                          unsigned long long *__restrict__ dt_part)
 {
-    __shared__ double a[SIG_LDS], b[SIG_LDS];
-    __shared__ unsigned long long wmin[SIG_T / 64];
+    __shared__ double a[SD_LDS], b[SD_LDS];
+    __shared__ unsigned long long wmin[SD_T / 64];
     const unsigned long long kInf = 0x7ff0000000000000ull;
     const int64_t N = s->n_max, p = P.avekernel, len = 2 * p;
-    const int64_t first = 1 + (int64_t)kg_.bid * SIG_T;
-    const int64_t last = first + SIG_T - 1 < N ? first + SIG_T - 1 : N;
+    const int64_t first = 1 + (int64_t)kg_.bid * SD_N;
+    const int64_t last = first + SD_N - 1 < N ? first + SD_N - 1 : N;
     const int64_t lo = first - 2 * p > 1 ? first - 2 * p : 1;
     const int64_t hi = last + 2 * p < N ? last + 2 * p : N;
     if (first <= N)
-        for (int64_t k = lo + threadIdx.x; k <= hi; k += SIG_T) {
+        for (int64_t k = lo + threadIdx.x; k <= hi; k += SD_T) {
             const double mk = m[k] * P.madhoc;
             a[k - lo] = mk;
             b[k - lo] = mk * (sqr(vr[k]) + sqr(vt[k]));
         }
     __syncthreads();
     unsigned long long mine = kInf;
+    double sg[SD_PER];
     if (first <= N) {
-        const int64_t si = first + threadIdx.x;
-        if (si <= N) {
-            int64_t simin = si - p, simax = simin + (2 * p - 1);
-            if (simin < 1) { simin = 1; simax = simin + (2 * p - 1); }
-            else if (simax > N) { simax = N; simin = simax - (2 * p - 1); }
-            if (simin < 1) simin = 1;
-            if (simax > N) simax = N;
-            double Mv2ave = 0.0, Mave = 0.0;
-            for (int64_t k = simin; k <= simax; k++) {
-                Mv2ave += b[k - lo];
-                Mave += a[k - lo];
+        const int64_t s0 = first + (int64_t)threadIdx.x * SD_PER;
+        double Mv2[SD_PER], M[SD_PER];
+#pragma unroll
+        for (int u = 0; u < SD_PER; u++) Mv2[u] = M[u] = 0.0;
+        if (p >= SD_PER && s0 - p >= 1 && s0 + SD_PER - 1 + p - 1 <= N) {
+            // no window of the SD_PER is shifted: star u's is elements u .. u + 2p - 1 from s0 - p
+            const double *ea = a + (s0 - p - lo), *eb = b + (s0 - p - lo);
+            const int n2 = 2 * (int)p;
+#pragma unroll
+            for (int k = 0; k < SD_PER - 1; k++)
+#pragma unroll
+                for (int u = 0; u <= k; u++) { Mv2[u] += eb[k]; M[u] += ea[k]; }
+#pragma unroll 4
+            for (int k = SD_PER - 1; k < n2; k++) {
+                const double x = ea[k], y = eb[k];
+#pragma unroll
+                for (int u = 0; u < SD_PER; u++) { Mv2[u] += y; M[u] += x; }
             }
-            sigma[si] = sqrt(Mv2ave / Mave);
+#pragma unroll
+            for (int k = 0; k < SD_PER - 1; k++)
+#pragma unroll
+                for (int u = k + 1; u < SD_PER; u++) { Mv2[u] += eb[n2 + k]; M[u] += ea[n2 + k]; }
+        } else {
+            for (int u = 0; u < SD_PER; u++) {
+                const int64_t si = s0 + u;
+                if (si > N) break;
+                int64_t simin = si - p, simax = simin + (2 * p - 1);
+                if (simin < 1) { simin = 1; simax = simin + (2 * p - 1); }
+                else if (simax > N) { simax = N; simin = simax - (2 * p - 1); }
+                if (simin < 1) simin = 1;
+                if (simax > N) simax = N;
+                double x = 0.0, y = 0.0;
+                for (int64_t k = simin; k <= simax; k++) {
+                    y += b[k - lo];
+                    x += a[k - lo];
+                }
+                Mv2[u] = y;
+                M[u] = x;
+            }
         }
+#pragma unroll
+        for (int u = 0; u < SD_PER; u++) sg[u] = sqrt(Mv2[u] / M[u]);
         // the windows starting at 1 + 2pw in [first, last]; each lies inside [lo, hi]
-        const int64_t w = (first - 1 + len - 1) / len + threadIdx.x;
-        const int64_t wstart = 1 + w * len, wsi = wstart + p;
-        if (wstart <= last && wsi < N - p) {
+        const int64_t w0 = (first - 1 + len - 1) / len;
+        for (int64_t w = w0 + threadIdx.x; 1 + w * len <= last; w += SD_T) {
+            const int64_t wstart = 1 + w * len, wsi = wstart + p;
+            if (wsi >= N - p) break;
             double Mv2ave = 0.0, Mave = 0.0, M2ave = 0.0;
             for (int64_t k = wstart; k < wstart + len; k++) {
                 const double tmp = a[k - lo];
@@ -350,14 +387,21 @@ struct sigma_dt_kernel {
             Mv2ave /= (double)(2 * p);
             Mave /= (double)(2 * p);
             M2ave /= (double)(2 * p);
-            const double sg = sqrt(Mv2ave / Mave);
-            const double W = 4.0 * sg / sqrt(3.0 * CMCG_PI);
+            const double sw = sqrt(Mv2ave / Mave);
+            const double W = 4.0 * sw / sqrt(3.0 * CMCG_PI);
             const double n_local = calc_n_local(r, wsi, p, N);
             const double dt = sqr(2.0 * P.theta_se_max / CMCG_PI) * (CMCG_PI / 32.0) * cub(W) /
                               (((double)P.n_star) * n_local * (4.0 * M2ave));
-            if (dt >= 0.0) mine = (unsigned long long)__double_as_longlong(dt);
+            if (dt >= 0.0) {
+                const unsigned long long bits = (unsigned long long)__double_as_longlong(dt);
+                mine = bits < mine ? bits : mine;
+            }
         }
     }
+    __syncthreads();                           // the sums are done: sigma leaves through a, coalesced
+    if (first <= N)
+#pragma unroll
+        for (int u = 0; u < SD_PER; u++) a[threadIdx.x * SD_PER + u] = sg[u];
 #pragma unroll
     for (int o = 32; o >= 1; o >>= 1) {
         const unsigned long long other = __shfl_xor(mine, o, 64);
@@ -365,8 +409,9 @@ struct sigma_dt_kernel {
     }
     if ((threadIdx.x & 63) == 0) wmin[threadIdx.x >> 6] = mine;
     __syncthreads();
+    for (int64_t k = first + threadIdx.x; k <= last; k += SD_T) sigma[k] = a[k - first];
     if (threadIdx.x == 0) {
-        for (int q = 1; q < SIG_T / 64; q++) mine = wmin[q] < mine ? wmin[q] : mine;
+        for (int q = 1; q < SD_T / 64; q++) mine = wmin[q] < mine ? wmin[q] : mine;
         if (mine != kInf) atomicMax(&dt_part[(kg_.bid % DT_SLOTS) * 16], ~mine);
     }
 }
@@ -540,6 +585,16 @@ hipError_t launch_simul_relax(const DevFields &f, DevScalars *s, const KParams &
     return hipGetLastError();
 }
 
+template <int T, int PER>
+void sigma_dt_launch(const DevFields &f, DevScalars *s, const KParams &P, const Scratch &sc, int64_t n_ub, hipStream_t st)
+{
+    kl<sigma_dt_kernel<T, PER>>(dim3((unsigned)((n_ub + T * PER - 1) / (T * PER))), dim3(T), 0, st, f.r, f.m, f.vr, f.vt,
+                                f.sigma, s, P, sc.dt_part);
+}
+// One star a thread fills the chip from fewer stars: 12 / 17 us at 3e5 (one / five a thread),
+// 24 / 24 at 1e6, 41 / 33 at 2e6, 72 / 48 at 4e6.
+constexpr int64_t SD_MANY = 1500000;
+
 // The step's begin and time-step phase: calc_sigma_r and simul_relax_new in one pass (or, for
 // a window longer than the pass stages, their own kernels), then Dt, the RNG bases and the
 // cleared radial index of the orbit phase.
@@ -548,10 +603,8 @@ hipError_t launch_timestep_sigma(const DevFields &f, DevScalars *s, const KParam
 {
     const bool one_pass = P.avekernel <= SIG_MAXP && n_ub > 0;
     if (one_pass) {
-        const int64_t nb = (n_ub + SIG_T - 1) / SIG_T;
-        if (nb > sc.max_blocks) return hipErrorInvalidValue;
-        kl<sigma_dt_kernel>(dim3((unsigned)nb), dim3(SIG_T), 0, st, f.r, f.m, f.vr, f.vt, f.sigma, s, P,
-                           sc.dt_part);
+        if (n_ub > SD_MANY) sigma_dt_launch<128, 5>(f, s, P, sc, n_ub, st);
+        else sigma_dt_launch<512, 1>(f, s, P, sc, n_ub, st);
     } else {
         kl<step_begin_kernel>(dim3(1), dim3(1), 0, st, s);
         if (hipError_t e = launch_simul_relax(f, s, P, n_ub, st, false)) return e;

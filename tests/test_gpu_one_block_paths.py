@@ -94,3 +94,25 @@ def test_gpu_old_potential_search_splits(gpu, O, n):
     idx = _order(d, o)
     for k in FIELDS:
         assert np.array_equal(d[k][idx], o[k][1:o.N + 1]), k
+
+
+@pytest.mark.parametrize("n,ave", [(1500000, 20), (1500001, 20), (1500640, 5), (1501283, 4), (1500003, 64), (1600637, 1)])
+def test_gpu_step_sigma_of_many_stars(gpu, n, ave):
+    """The step's sigma and time step on both sides of 1.5e6 stars and for windows shorter and
+    longer than a thread's share of stars, against the phase call's kernels."""
+    cm = gpu
+    print("[gpu-test] step sigma", n, ave, flush=True)
+    cl = cm.make_plummer(n, seed=3, kroupa=True)
+    got = []
+    for step in (False, True):
+        with cm.Context(cl.n, cm.default_params(cl.n, orbit_r=cl.rtid, avekernel=ave)) as ctx:
+            ctx.upload(cl)
+            ctx.init_cluster()
+            dt = None if step else ctx.calc_timestep()
+            if step:
+                ctx.step()
+                dt = ctx.scalars()["Dt"]
+            got.append((dt, ctx.download(fields=["sigma"])["sigma"][1:n + 1].copy()))
+    assert got[0][0] == got[1][0]
+    kept = got[1][1].size                             # stars that leave in the step are not downloaded
+    assert kept > 0.99 * n and np.array_equal(got[0][1][:kept], got[1][1])
