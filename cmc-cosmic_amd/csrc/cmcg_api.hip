@@ -408,26 +408,18 @@ void fill_jump_level(const uint32_t m[4][32], JumpLevel *levels, int level)
     for (int d = 0; d < 64; d++)
         for (int c = 0; c < 4; c++) {
             for (int q = 0; q < 8; q++)
-                for (int v = 0; v < 16; v++) {
-                    uint32_t o = 0;
-                    for (int i = 0; i < 4; i++)
-                        if ((v >> i) & 1) o ^= col[c][4 * q + i];
-                    L.t[jump_index(lanes, c, q, v, d)] = o;
-                }
+                for (int v = 0; v < 16; v++)
+                    L.t[jump_index(lanes, c, q, v, d)] = v ? L.t[jump_index(lanes, c, q, v & (v - 1), d)] ^
+                                                                 col[c][4 * q + __builtin_ctz(v)]
+                                                           : 0u;
             for (int i = 0; i < 32; i++) col[c][i] = host_matvec(m[c], col[c][i]);
         }
 }
 
-// With `device` current: its jump tables, filled for the first user (null: failed).
-const JumpTables *jump_acquire(int device, const RngTable &T)
+// The host's copy, made once (the generator's matrices are constants).
+const JumpTables *jump_host(const RngTable &T)
 {
-    if (device < 0 || device >= NOALLOC_MAX_DEVICES) return nullptr;
-    std::lock_guard<std::mutex> lk(g_scratch_mu);
-    if (g_jump_ptr[device]) {
-        g_jump_users[device]++;
-        return g_jump_ptr[device];
-    }
-    auto h = std::make_unique<JumpTables>();
+    auto *h = new JumpTables();
     uint32_t m[4][32];
     for (int k = 0; k < JL_PAIR_N; k++) {       // 3 64^k = 2^(6k) + 2^(6k + 1)
         for (int c = 0; c < 4; c++)
@@ -445,9 +437,22 @@ const JumpTables *jump_acquire(int device, const RngTable &T)
                     h->orbit.lo.t[c][q][v][d] = h->level[JL_SLOT].t[jump_index(false, c, q, v, d)];
                     h->orbit.hi.t[c][q][v][d] = h->level[JL_SLOT].t[jump_index(false, c, q, v, 8 * d)];
                 }
+    return h;
+}
+
+// With `device` current: its jump tables, copied for the first user (null: failed).
+const JumpTables *jump_acquire(int device, const RngTable &T)
+{
+    if (device < 0 || device >= NOALLOC_MAX_DEVICES) return nullptr;
+    static const JumpTables *host = jump_host(T);
+    std::lock_guard<std::mutex> lk(g_scratch_mu);
+    if (g_jump_ptr[device]) {
+        g_jump_users[device]++;
+        return g_jump_ptr[device];
+    }
     void *ptr = nullptr;
     if (hipMalloc(&ptr, sizeof(JumpTables)) != hipSuccess) return nullptr;
-    if (hipMemcpy(ptr, h.get(), sizeof(JumpTables), hipMemcpyHostToDevice) != hipSuccess) {
+    if (hipMemcpy(ptr, host, sizeof(JumpTables), hipMemcpyHostToDevice) != hipSuccess) {
         hipFree(ptr);
         return nullptr;
     }
@@ -816,6 +821,10 @@ int cmcg_potential(cmcg_ctx *c, int64_t *n_max, double *mtotal, double *rtidal)
     return h.error;
 }
 
+// Batches of apsides up to this go through one host buffer and two copies; the nine copies of
+// larger ones cost less than moving their data twice: 61 us packed, 156 copied apart at 100 to
+// 4000 stars, 154 / 209 at 20000, 237 / 247 at 32000, 343 / 297 at 50000.
+constexpr int64_t QUERY_PACKED = 32768;
 static int query_reserve(cmcg_ctx *c, int64_t doubles)
 {
     if (doubles <= c->query_cap) return CMCG_OK;
@@ -937,6 +946,20 @@ int cmcg_calc_pericenter_and_apocenter(cmcg_ctx *c, int64_t first, int64_t count
     o.circular = (int32_t *)(d + 8 * count);
     const size_t b8 = (size_t)count * 8;
     hipStream_t st = c->stream;
+    if (count <= QUERY_PACKED) {
+        std::vector<double> h(9 * count);
+        std::memcpy(h.data(), E, b8);
+        std::memcpy(h.data() + count, J, b8);
+        if (hipMemcpyAsync(d, h.data(), 2 * b8, hipMemcpyHostToDevice, st) ||
+            launch_apsides_soa(c->f, c->s, c->kp, first, count, d, d + count, o, st) ||
+            hipMemcpyAsync(h.data() + 2 * count, d + 2 * count, 6 * b8 + (size_t)count * 4, hipMemcpyDeviceToHost, st) ||
+            sync(c))
+            return CMCG_E_HIP;
+        void *const dst[7] = {rp, ra, dQdrp, dQdra, kmin, kmax, circular};
+        for (int q = 0; q < 7; q++)
+            if (dst[q]) std::memcpy(dst[q], h.data() + (2 + q) * count, q < 6 ? b8 : (size_t)count * 4);
+        return check_error(c);
+    }
     bool bad = hipMemcpyAsync(d, E, b8, hipMemcpyHostToDevice, st) ||
                hipMemcpyAsync(d + count, J, b8, hipMemcpyHostToDevice, st) ||
                launch_apsides_soa(c->f, c->s, c->kp, first, count, d, d + count, o, st);

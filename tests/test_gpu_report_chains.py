@@ -94,3 +94,21 @@ def test_gpu_queries_from_threads_and_growing_batches(gpu, O):
         for t in threads:
             t.join()
     assert not bad
+
+
+@pytest.mark.parametrize("count", [32767, 32768, 32769])
+def test_gpu_apsides_batches_packed_and_apart(gpu, count):
+    cm = gpu
+    print("[gpu-test] apsides batch", count, flush=True)
+    cl = cm.make_plummer(40000, seed=5, kroupa=True)
+    with cm.Context(cl.n, cm.default_params(cl.n, orbit_r=cl.rtid)) as ctx:
+        ctx.upload(cl)
+        ctx.init_cluster()
+        d = ctx.download()
+        s = slice(7, 7 + count)
+        E, J = d["E"][s] + d["m"][s] / d["r"][s] / cl.n, d["J"][s]
+        got = ctx.apsides(7, E, J)
+        for a in range(0, count, 20000):
+            part = ctx.apsides(7 + a, E[a:a + 20000], J[a:a + 20000], noalloc=True)
+            for k, v in part.items():
+                assert np.array_equal(got[k][a:a + 20000], v), k
