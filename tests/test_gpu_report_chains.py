@@ -112,3 +112,24 @@ def test_gpu_apsides_batches_packed_and_apart(gpu, count):
             part = ctx.apsides(7 + a, E[a:a + 20000], J[a:a + 20000], noalloc=True)
             for k, v in part.items():
                 assert np.array_equal(got[k][a:a + 20000], v), k
+
+
+@pytest.mark.parametrize("n", [1, 3, 63, 64, 65, 127, 129, 1000, 80000, 80001])
+def test_gpu_network_predictions_at_block_edges(gpu, n):
+    """Every row's prediction is its own: a batch of any size gives what rows one by one give,
+    and the float64 oracle within 1e-4 of the outputs' scale (FP32 sums of 64 terms)."""
+    print("[gpu-test] predictions", n, flush=True)
+    rng = np.random.default_rng(n)
+    x = rng.normal(size=(n, 6)).astype(np.float32)
+    nr = np.concatenate([rng.normal(size=6), rng.uniform(0.5, 2.0, 6), rng.normal(size=2),
+                         rng.uniform(0.5, 2.0, 2)]).astype(np.float32)
+    with gpu.Context(1000, gpu.default_params(1000)) as ctx:
+        ctx.mlp_init(seed=5, max_rows=1024)
+        th, _ = ctx.mlp_params()
+        ctx.mlp_set_params(th, nr)
+        y = ctx.mlp_predict(x)
+        for k in {0, n // 2, n - 1}:
+            assert np.array_equal(ctx.mlp_predict(x[k:k + 1])[0], y[k])
+    yo, _ = M.forward(th.astype(np.float64), (x.astype(np.float64) - nr[:6]) / nr[6:12])
+    yo = yo * nr[14:16] + nr[12:14]
+    assert np.max(np.abs(y - yo)) <= 1e-4 * (1 + np.max(np.abs(yo)))
