@@ -42,9 +42,12 @@ def test_gpu_strip_and_excess_vs_oracle(gpu, O, n, cut, graph):
         assert sc[k] == pytest.approx(o.sc(k), rel=1e-12, abs=1e-300), k
 
 
-@pytest.mark.parametrize("n", [2, 255, 256, 257, 4097, 65535, 65536])
-@pytest.mark.parametrize("p_ev,scale", [(0.0, 1.0), (0.01, 2.0), (0.3, 1.5), (2e-3, 2e3)])
-def test_gpu_excess_chain_one_block(gpu, O, n, p_ev, scale):
+EVENTS = [(0.0, 1.0), (0.01, 2.0), (0.3, 1.5), (2e-3, 2e3)]
+
+
+@pytest.mark.parametrize("n,p_ev,scale", [(n, *e) for n in (2, 255, 256, 257, 4097, 65535, 65536, 65537, 262145, 278784)
+                                          for e in EVENTS] + [(4194304, 0.01, 2.0), (4200000, 0.01, 2.0)])
+def test_gpu_excess_chain_sizes(gpu, O, n, p_ev, scale):
     cm = gpu
     print("[gpu-test] excess chain", n, p_ev, scale, flush=True)
     cl = cm.make_plummer(n, seed=11)
