@@ -128,13 +128,13 @@ struct ec2_ie_kernel {
         const double vtold = f.vtold[i], vrold = f.vrold[i];
         const double vold2 = vtold * vtold + vrold * vrold;
         dpre[i] = vold2 + 2.0 * (1.0 - q) * (f.Uoldrold[i] - Uoldrnew);
-        if (apo_max && x < 1000000) apo = f.r_apo[i];
+        if (apo_max && x < 1000000) apo = fmax(f.r_apo[i], 0.0);      // NaN: 0, beyond no radius, as in the pass
     }
     if (!apo_max) return;
 #pragma unroll
     for (int o = 32; o >= 1; o >>= 1) {
         const double other = __shfl_xor(apo, o, 64);
-        apo = other > apo ? other : apo;               // NaN: not beyond any radius, as in the pass
+        apo = other > apo ? other : apo;
     }
     if ((threadIdx.x & 63) == 0) wmax[threadIdx.x >> 6] = apo;
     __syncthreads();
