@@ -45,7 +45,7 @@ struct cmcg_ctx {
     int64_t adam_t = 0;
     float *io = nullptr;
     int64_t io_cap = 0;          // floats
-    double *query = nullptr;     // inputs and outputs of a batch of queries, kept between calls
+    double *query = nullptr;     // inputs and outputs of a batch of queries (QueryBuffer)
     int64_t query_cap = 0;       // doubles
     std::mutex query_mu;         // a query holds it: queries may come from several threads
     // step graphs: the fused sort swaps buffer pointers, so steps alternate between
@@ -825,30 +825,53 @@ int cmcg_potential(cmcg_ctx *c, int64_t *n_max, double *mtotal, double *rtidal)
 // larger ones cost less than moving their data twice: 61 us packed, 156 copied apart at 100 to
 // 4000 stars, 154 / 209 at 20000, 237 / 247 at 32000, 343 / 297 at 50000.
 constexpr int64_t QUERY_PACKED = 32768;
-static int query_reserve(cmcg_ctx *c, int64_t doubles)
-{
-    if (doubles <= c->query_cap) return CMCG_OK;
-    if (c->query) { hipFree(c->query); c->query = nullptr; c->query_cap = 0; }
-    if (hipMalloc((void **)&c->query, (size_t)doubles * sizeof(double)) != hipSuccess) {
-        c->query = nullptr;
-        return CMCG_E_NOMEM;
+
+// A batch of queries: the context's buffer, held by one thread at a time, of `arrays` 8-byte
+// arrays of `count`.  Up to QUERY_KEEP doubles stay with the context for the next batch; a
+// larger buffer goes back when the batch ends (64 MB take 5 ms to copy each way, and the
+// allocation and the free about 0.2).
+constexpr int64_t QUERY_KEEP = (int64_t)1 << 23;
+struct QueryBuffer {
+    cmcg_ctx *c;
+    std::lock_guard<std::mutex> lk;
+    int rc = CMCG_OK;
+    QueryBuffer(cmcg_ctx *c_, int64_t arrays, int64_t count) : c(c_), lk(c_->query_mu)
+    {
+        if (count > INT64_MAX / (int64_t)sizeof(double) / arrays) { rc = CMCG_E_NOMEM; return; }
+        const int64_t doubles = arrays * count;
+        if (doubles <= c->query_cap) return;
+        release();
+        if (hipMalloc((void **)&c->query, (size_t)doubles * sizeof(double)) != hipSuccess) {
+            c->query = nullptr;
+            rc = CMCG_E_NOMEM;
+            return;
+        }
+        c->query_cap = doubles;
     }
-    c->query_cap = doubles;
-    return CMCG_OK;
-}
+    ~QueryBuffer()
+    {
+        if (c->query_cap > QUERY_KEEP) release();
+    }
+    void release()
+    {
+        if (c->query) hipFree(c->query);
+        c->query = nullptr;
+        c->query_cap = 0;
+    }
+};
 
 int cmcg_potential_at(cmcg_ctx *c, int64_t count, const double *r, double *out)
 {
     if (!c || count < 0 || (count > 0 && (!r || !out))) return CMCG_E_ARG;
     if (count == 0) return CMCG_OK;
-    std::lock_guard<std::mutex> lk(c->query_mu);
-    if (int e = query_reserve(c, 2 * count)) return e;
+    QueryBuffer q(c, 2, count);
+    if (q.rc) return q.rc;
     double *dx = c->query, *dy = dx + count;
-    if (hipMemcpyAsync(dx, r, count * sizeof(double), hipMemcpyHostToDevice, c->stream) != hipSuccess ||
+    const bool bad =
+        hipMemcpyAsync(dx, r, count * sizeof(double), hipMemcpyHostToDevice, c->stream) != hipSuccess ||
         launch_potential_at(c->f, c->s, c->kp, dx, dy, count, c->stream) != hipSuccess ||
-        hipMemcpyAsync(out, dy, count * sizeof(double), hipMemcpyDeviceToHost, c->stream) != hipSuccess ||
-        sync(c) != hipSuccess)
-        return CMCG_E_HIP;
+        hipMemcpyAsync(out, dy, count * sizeof(double), hipMemcpyDeviceToHost, c->stream) != hipSuccess;
+    if (sync(c) != hipSuccess || bad) return CMCG_E_HIP;      // the copies use the caller's memory: always waited for
     return check_error(c);
 }
 
@@ -933,8 +956,8 @@ int cmcg_calc_pericenter_and_apocenter(cmcg_ctx *c, int64_t first, int64_t count
     // eight 8-byte arrays and one of 4 bytes in the context's query buffer, each copied
     // straight to and from the caller's (five allocations and frees, and outputs interleaved
     // and sorted out on the host: 900 us for 1e5 stars)
-    std::lock_guard<std::mutex> lk(c->query_mu);
-    if (int e = query_reserve(c, 9 * count)) return e;
+    QueryBuffer q(c, 9, count);
+    if (q.rc) return q.rc;
     double *d = c->query;
     ApsidesOut o;
     o.rp = d + 2 * count;
@@ -950,14 +973,14 @@ int cmcg_calc_pericenter_and_apocenter(cmcg_ctx *c, int64_t first, int64_t count
         std::vector<double> h(9 * count);
         std::memcpy(h.data(), E, b8);
         std::memcpy(h.data() + count, J, b8);
-        if (hipMemcpyAsync(d, h.data(), 2 * b8, hipMemcpyHostToDevice, st) ||
+        const bool bad =
+            hipMemcpyAsync(d, h.data(), 2 * b8, hipMemcpyHostToDevice, st) ||
             launch_apsides_soa(c->f, c->s, c->kp, first, count, d, d + count, o, st) ||
-            hipMemcpyAsync(h.data() + 2 * count, d + 2 * count, 6 * b8 + (size_t)count * 4, hipMemcpyDeviceToHost, st) ||
-            sync(c))
-            return CMCG_E_HIP;
+            hipMemcpyAsync(h.data() + 2 * count, d + 2 * count, 6 * b8 + (size_t)count * 4, hipMemcpyDeviceToHost, st);
+        if (sync(c) || bad) return CMCG_E_HIP;
         void *const dst[7] = {rp, ra, dQdrp, dQdra, kmin, kmax, circular};
-        for (int q = 0; q < 7; q++)
-            if (dst[q]) std::memcpy(dst[q], h.data() + (2 + q) * count, q < 6 ? b8 : (size_t)count * 4);
+        for (int a = 0; a < 7; a++)
+            if (dst[a]) std::memcpy(dst[a], h.data() + (2 + a) * count, a < 6 ? b8 : (size_t)count * 4);
         return check_error(c);
     }
     bool bad = hipMemcpyAsync(d, E, b8, hipMemcpyHostToDevice, st) ||
