@@ -178,7 +178,7 @@ struct sb_sample_kernel {
 
 // The step's bucket of a star: its index among the old nodes, cut into B equal parts
 // (monotone in the new radius while the old radii ascend; when they do not, every star
-// goes to the last bucket, which the merge sort orders).
+// goes to the last bucket, which its block splits).
 struct StepBucket {
     double f;
     int B;
@@ -431,19 +431,41 @@ __device__ __forceinline__ bool rec_less(const uint64_t *__restrict__ rec, uint3
     return ia < ib || (ia == ib && x[2] < y[2]);
 }
 
-// the same with the keys known
+// word w of record a as an unsigned key: the order (r, id, slot) word by word
 template <int W>
-__device__ __forceinline__ bool key_less(const uint64_t *__restrict__ rec, uint64_t ka, uint32_t a, uint64_t kb, uint32_t b)
+__device__ __forceinline__ uint64_t rec_key(const uint64_t *__restrict__ rec, uint32_t a, int w)
 {
-    return ka < kb || (ka == kb && a != b && rec_less<W>(rec, a, b));
+    const uint64_t x = rec[(int64_t)W * a + w];
+    return w == 0 ? sortable(__longlong_as_double((long long)x)) : w == 1 ? x ^ 0x8000000000000000ull : x;
 }
 
-constexpr int BS_T = 512, BS_BINS = 2048, BS_RANK = 48;
+// Some records of a bucket: those that a list names, or (no list) all of them.
+struct Records {
+    const uint32_t *list;
+    __device__ __forceinline__ uint32_t operator()(uint32_t e) const { return list ? list[e] : e; }
+};
 
-// Bitonic sort in LDS of the first cnt entries (cnt <= CAP, a power of two), idx indexing
-// the records; the rest of the next power of two is padded with keys above every live one.
+constexpr int BS_T = 512, BS_BINS = 2048, BS_RANK = 48;
+constexpr int SPLIT_BINS = 1024;        // parts of one split of a bucket beyond the LDS capacity
+
 template <int W, int CAP>
-__device__ void bitonic(const uint64_t *__restrict__ rec, uint64_t *key, uint16_t *idx, int cnt)
+struct BucketLds {
+    static constexpr int PC = W / 2, SN = 256 * 8 / W;              // records staged at a time: 16 KB
+    static constexpr int STAGE = SN * PC + SN * PC / 32;            // 16-byte pieces, one pad per 32
+    static constexpr int BUF = 2 * STAGE > CAP ? 2 * STAGE : CAP;
+    static_assert(CAP % BS_T == 0 && (CAP & (CAP - 1)) == 0, "LDS capacity");
+    __align__(16) uint64_t buf[BUF];                                // keys, later the staged records
+    uint16_t idx[CAP], fin[CAP];
+    uint32_t bin[BS_BINS + 1], sub[SPLIT_BINS];
+    uint32_t scan[BS_T / 64];
+    uint64_t red[2][BS_T / 64];
+    uint32_t worst;
+};
+
+// Bitonic sort in LDS of the first cnt entries (cnt <= CAP, a power of two), idx numbering
+// the records of `of`; the rest of the next power of two is padded with entries above every record.
+template <int W>
+__device__ void bitonic(const uint64_t *__restrict__ rec, const Records &of, uint64_t *key, uint16_t *idx, int cnt)
 {
     int P = 1;
     while (P < cnt) P <<= 1;
@@ -457,7 +479,7 @@ __device__ void bitonic(const uint64_t *__restrict__ rec, uint64_t *key, uint16_
                     const uint64_t ka = key[q], kb = key[x];
                     const uint16_t a = idx[q], b = idx[x];
                     const bool up = (q & kk) == 0;
-                    const bool gt = ka == ~0ull || kb == ~0ull ? kb < ka : key_less<W>(rec, kb, b, ka, a);
+                    const bool gt = kb < ka || (kb == ka && b != 0xffff && (a == 0xffff || rec_less<W>(rec, of(b), of(a))));
                     if (gt == up) { key[q] = kb; key[x] = ka; idx[q] = b; idx[x] = a; }
                 }
             }
@@ -465,79 +487,252 @@ __device__ void bitonic(const uint64_t *__restrict__ rec, uint64_t *key, uint16_
         }
 }
 
-// A bucket beyond the LDS capacity: pieces of CAP sorted in LDS, then bottom-up merges of
-// record numbers between two global arrays (ord and tmp), each merge split among the
-// threads along its merge path.  The order ends in the returned array.
-template <int W, int CAP>
-__device__ uint32_t *merge_bucket(const uint64_t *__restrict__ rec, uint64_t *key, uint16_t *idx, int64_t cnt,
-                                  uint32_t *ord, uint32_t *tmp)
+// values that every lane of the block holds, as the scalars they are
+__device__ __forceinline__ uint32_t uniform(uint32_t x) { return (uint32_t)__builtin_amdgcn_readfirstlane((int)x); }
+__device__ __forceinline__ uint64_t uniform(uint64_t x) { return (uint64_t)uniform((uint32_t)(x >> 32)) << 32 | uniform((uint32_t)x); }
+
+// sh.red's wave values folded: the least and the greatest key over the block
+template <class Lds>
+__device__ __forceinline__ void block_range(Lds &sh, uint64_t &lo, uint64_t &hi)
 {
-    const int t = threadIdx.x;
-    for (int64_t c = 0; c < cnt; c += CAP) {
-        const int m = (int)(cnt - c < CAP ? cnt - c : CAP);
-        for (int q = t; q < m; q += BS_T) {
-            key[q] = sortable(__longlong_as_double((long long)rec[W * (c + q)]));
-            idx[q] = (uint16_t)q;
-        }
-        __syncthreads();
-        bitonic<W, CAP>(rec + W * c, key, idx, m);
-        for (int q = t; q < m; q += BS_T) ord[c + q] = (uint32_t)(c + idx[q]);
-        __syncthreads();
+    for (int o = 32; o > 0; o >>= 1) {
+        const uint64_t x = __shfl_xor(lo, o, 64), y = __shfl_xor(hi, o, 64);
+        lo = x < lo ? x : lo;
+        hi = y > hi ? y : hi;
     }
-    for (int64_t w = CAP; w < cnt; w <<= 1) {
-        for (int64_t p = 0; p < cnt; p += 2 * w) {
-            const int64_t la = cnt - p < w ? cnt - p : w;
-            const int64_t lb = cnt - p - la < w ? cnt - p - la : w;
-            const uint32_t *A = ord + p, *B = ord + p + la;
-            const int64_t L = la + lb;
-            const int64_t d0 = L * t / BS_T, d1 = L * (t + 1) / BS_T;
-            // the first d0 outputs hold A[0, ia) and B[0, d0 - ia); A[m] is among them
-            // iff it does not follow B[d0 - 1 - m]
-            int64_t a_lo = d0 > lb ? d0 - lb : 0, a_hi = d0 < la ? d0 : la;
-            while (a_lo < a_hi) {
-                const int64_t m = (a_lo + a_hi) >> 1;
-                if (!rec_less<W>(rec, B[d0 - 1 - m], A[m])) a_lo = m + 1;
-                else a_hi = m;
-            }
-            int64_t ia = a_lo, ib = d0 - a_lo;
-            for (int64_t d = d0; d < d1; d++) {
-                const bool takeA = ib >= lb || (ia < la && !rec_less<W>(rec, B[ib], A[ia]));
-                tmp[p + d] = takeA ? A[ia++] : B[ib++];
-            }
-        }
-        __syncthreads();
-        uint32_t *x = ord; ord = tmp; tmp = x;
+    if ((threadIdx.x & 63) == 0) { sh.red[0][threadIdx.x >> 6] = lo; sh.red[1][threadIdx.x >> 6] = hi; }
+    __syncthreads();
+    for (int q = 0; q < BS_T / 64; q++) {
+        lo = sh.red[0][q] < lo ? sh.red[0][q] : lo;
+        hi = sh.red[1][q] > hi ? sh.red[1][q] : hi;
     }
-    return ord;
+    lo = uniform(lo);
+    hi = uniform(hi);
 }
 
-// Block b orders bucket b and writes its stars' fields.  In LDS: the keys are counted
-// into BS_BINS equal parts of the bucket's key range, placed part by part, and each takes
-// its rank among the few keys of its part; a part of more than BS_RANK keys (many equal
-// radii, a very uneven bucket) sends the bucket through the bitonic sort instead.  The
-// sorted records are then read back in output order, W/2 lanes per record, and leave
-// through LDS with one coalesced store per field.  Bound by HBM (528 MB in 129 us at
-// N = 4e6); holding the records in registers between the two reads, or 256 threads a
-// block, changed nothing.
+// The order of cnt <= CAP records of a bucket in LDS: sh.fin[rank] = e for record of(e).
+// They agree in the words before w.  The keys are counted into BS_BINS equal parts of their
+// range, placed part by part, and each takes its rank among the few keys of its part; a part
+// of more than BS_RANK keys (many equal radii, a very uneven bucket) sends them through the
+// bitonic sort instead.
+template <int W, int CAP>
+__device__ __forceinline__ void order_records(const uint64_t *__restrict__ rec, const Records &of, int cnt, int w,
+                                              BucketLds<W, CAP> &sh)
+{
+    constexpr int ITEMS = CAP / BS_T;
+    int t = threadIdx.x;
+    asm volatile("" : "+v"(t));
+    uint64_t k[ITEMS], lo = ~0ull, hi = 0ull;
+    uint32_t at[ITEMS];
+#pragma unroll
+    for (int u = 0; u < ITEMS; u++) {
+        const int e = u * BS_T + t;
+        k[u] = 0;
+        if (e < cnt) {
+            k[u] = rec_key<W>(rec, of(e), w);
+            lo = k[u] < lo ? k[u] : lo;
+            hi = k[u] > hi ? k[u] : hi;
+        }
+    }
+    for (int q = t; q <= BS_BINS; q += BS_T) sh.bin[q] = 0;
+    if (t == 0) sh.worst = 0;
+    block_range(sh, lo, hi);
+    const Binning bin_of(lo, hi, BS_BINS);
+#pragma unroll
+    for (int u = 0; u < ITEMS; u++)
+        if (u * BS_T + t < cnt) at[u] = atomicAdd(&sh.bin[bin_of(k[u])], 1u);
+    __syncthreads();
+    constexpr int PER = BS_BINS / BS_T;
+    uint32_t c[PER], sum = 0, mx = 0, dummy;
+#pragma unroll
+    for (int q = 0; q < PER; q++) {
+        c[q] = sh.bin[t * PER + q];
+        sum += c[q];
+        mx = c[q] > mx ? c[q] : mx;
+    }
+    if (mx > BS_RANK) sh.worst = mx;                       // any value above BS_RANK will do
+    uint32_t run = block_excl(sum, sh.scan, &dummy);
+#pragma unroll
+    for (int q = 0; q < PER; q++) { sh.bin[t * PER + q] = run; run += c[q]; }
+    if (t == 0) sh.bin[BS_BINS] = (uint32_t)cnt;
+    __syncthreads();
+    const bool uneven = uniform(sh.worst) > BS_RANK;
+#pragma unroll
+    for (int u = 0; u < ITEMS; u++) {
+        const int e = u * BS_T + t;
+        if (e < cnt) {
+            const uint32_t p = uneven ? (uint32_t)e : sh.bin[bin_of(k[u])] + at[u];
+            sh.buf[p] = k[u];
+            sh.idx[p] = (uint16_t)e;
+            at[u] = p;
+        }
+    }
+    __syncthreads();
+    if (uneven) {
+        bitonic<W>(rec, of, sh.buf, sh.idx, cnt);
+        for (int q = t; q < cnt; q += BS_T) sh.fin[q] = sh.idx[q];
+    } else {
+#pragma unroll
+        for (int u = 0; u < ITEMS; u++) {
+            const int e = u * BS_T + t;
+            if (e < cnt) {
+                const uint32_t bn = bin_of(k[u]), e0 = sh.bin[bn], e1 = sh.bin[bn + 1];
+                uint32_t rank = e0;
+                for (uint32_t q = e0; q < e1; q++)
+                    if (q != at[u])
+                        rank += sh.buf[q] < k[u] || (sh.buf[q] == k[u] && rec_less<W>(rec, of(sh.idx[q]), of((uint32_t)e)));
+                sh.fin[rank] = (uint16_t)e;
+            }
+        }
+    }
+    __syncthreads();
+}
+
+// A bucket beyond the LDS capacity is ordered by its block in time proportional to its
+// records, whatever their radii: their numbers are split into SPLIT_BINS equal parts of their
+// key range, in key order; runs of parts that fit are ordered in LDS, and a part that does
+// not is split again, by its narrower range or, all its keys equal, by the next word (ids, then
+// slots, which differ).
+// A part that waits has its numbers in one of (ord, tmp) and a note at the same place of the
+// other one: the part that waits after it (place and array), its length and its word.
+// (Buckets grow beyond their 1024 records where the cluster is far from equilibrium, where
+// radii are tied, and all of them from 8.4e6 stars on, when there are as many as there may be.)
+struct Part {
+    uint32_t start, len;
+    int w, in;                                             // numbers: 0 in ord, 1 in tmp, 2 all records
+};
+// The numbers of part p to the other array, part by part; sh.sub[b] is the end of its part b.
+template <int W, class Lds>
+__device__ __forceinline__ void split_part(const uint64_t *__restrict__ rec, Part &p, uint32_t *ord, uint32_t *tmp, Lds &sh)
+{
+    int t = threadIdx.x;
+    asm volatile("" : "+v"(t));
+    const Records of{p.in == 2 ? nullptr : (p.in ? tmp : ord) + p.start};
+    uint64_t lo, hi;
+    for (;; p.w++) {
+        lo = ~0ull;
+        hi = 0ull;
+#pragma unroll 4
+        for (uint32_t e = t; e < p.len; e += BS_T) {
+            const uint64_t k = rec_key<W>(rec, of(e), p.w);
+            lo = k < lo ? k : lo;
+            hi = k > hi ? k : hi;
+        }
+        for (int q = t; q < SPLIT_BINS; q += BS_T) sh.sub[q] = 0;
+        block_range(sh, lo, hi);
+        if (lo < hi || p.w == 2) break;
+        __syncthreads();
+    }
+    const Binning bin_of(lo, hi, SPLIT_BINS);
+#pragma unroll 4
+    for (uint32_t e = t; e < p.len; e += BS_T) atomicAdd(&sh.sub[bin_of(rec_key<W>(rec, of(e), p.w))], 1u);
+    __syncthreads();
+    constexpr int PER = SPLIT_BINS / BS_T;
+    uint32_t c[PER], sum = 0, dummy;
+#pragma unroll
+    for (int q = 0; q < PER; q++) { c[q] = sh.sub[t * PER + q]; sum += c[q]; }
+    uint32_t run = block_excl(sum, sh.scan, &dummy);
+#pragma unroll
+    for (int q = 0; q < PER; q++) { sh.sub[t * PER + q] = run; run += c[q]; }
+    __syncthreads();
+    p.in = p.in == 0 ? 1 : 0;
+    uint32_t *to = (p.in ? tmp : ord) + p.start;
+#pragma unroll 4
+    for (uint32_t e = t; e < p.len; e += BS_T) {
+        const uint32_t a = of(e);
+        to[atomicAdd(&sh.sub[bin_of(rec_key<W>(rec, a, p.w))], 1u)] = a;
+    }
+    __syncthreads();
+}
+
+// The order of a bucket's cnt records: in sh.fin up to CAP of them, else in ord.
+template <int W, int CAP>
+__device__ __forceinline__ void order_bucket(const uint64_t *__restrict__ rec, uint32_t cnt, uint32_t *ord, uint32_t *tmp,
+                                             BucketLds<W, CAP> &sh)
+{
+    constexpr uint64_t NONE = ~0ull;
+    const int t = threadIdx.x;
+    Part p{0, cnt, 0, 2};
+    uint64_t waiting = NONE;                               // 2 place + array
+    uint32_t s = 0, e = cnt;                               // the run of p in hand
+    int b = SPLIT_BINS;
+    const bool fits = cnt <= CAP;
+    if (!fits) {
+        split_part<W>(rec, p, ord, tmp, sh);
+        e = b = 0;
+    }
+    for (;;) {
+        if (!fits) {
+            // the next run: parts b .. b1 - 1 fit together
+            s = e;
+            if (s == p.len) {
+                if (waiting == NONE) return;
+                __syncthreads();
+                p.in = (int)(waiting & 1);
+                p.start = (uint32_t)(waiting >> 1);
+                const uint32_t *note = (p.in ? ord : tmp) + p.start;
+                waiting = uniform(note[0]) | (uint64_t)uniform(note[1]) << 32;
+                p.len = uniform(note[2]);
+                p.w = (int)uniform(note[3]);
+                __syncthreads();                           // the split writes where the note is
+                split_part<W>(rec, p, ord, tmp, sh);
+                s = 0;
+                b = 0;
+            }
+            int b1 = b, top = SPLIT_BINS;
+            while (b1 < top) {
+                const int m = (b1 + top) >> 1;
+                if (uniform(sh.sub[m]) - s <= CAP) b1 = m + 1;
+                else top = m;
+            }
+            if (b1 == b) {                                 // part b alone is too long: it waits
+                e = uniform(sh.sub[b]);
+                if (t == 0) {
+                    uint32_t *note = (p.in ? ord : tmp) + p.start + s;
+                    note[0] = (uint32_t)waiting;
+                    note[1] = (uint32_t)(waiting >> 32);
+                    note[2] = e - s;
+                    note[3] = (uint32_t)p.w;
+                }
+                waiting = 2 * (uint64_t)(p.start + s) + p.in;
+                b++;
+                continue;
+            }
+            e = uniform(sh.sub[b1 - 1]);
+            b = b1;
+            if (e == s) continue;
+        }
+        const int m = (int)(e - s);
+        const Records of{fits ? nullptr : (p.in ? tmp : ord) + p.start + s};
+        order_records<W, CAP>(rec, of, m, p.w, sh);
+        if (fits) return;
+        uint32_t v[CAP / BS_T];
+#pragma unroll
+        for (int u = 0; u < CAP / BS_T; u++)
+            if (u * BS_T + t < m) v[u] = of(sh.fin[u * BS_T + t]);
+        __syncthreads();                                   // the numbers may be in ord
+#pragma unroll
+        for (int u = 0; u < CAP / BS_T; u++)
+            if (u * BS_T + t < m) ord[p.start + s + u * BS_T + t] = v[u];
+        __syncthreads();
+    }
+}
+
+// Block b orders bucket b and writes its stars' fields: the sorted records are read back in
+// output order, W/2 lanes per record, and leave through LDS with one coalesced store per
+// field.  Bound by HBM (N = 4e6, 8 words: 129 us); holding the records in registers
+// between the two reads, or 256 threads a block, changed nothing.
 template <int W, int CAP>
 struct sb_sort_kernel {
     static constexpr int LB = BS_T, MB = 0;
     static __device__ __forceinline__ void run(KGrid kg_, DevScalars *s, const uint32_t *__restrict__ place, int32_t *bad,
-                                               const uint64_t *__restrict__ aos, uint32_t *__restrict__ order, int64_t n_cap,
+                                               const uint64_t *__restrict__ aos, uint32_t *order, int64_t n_cap,
                                                double *__restrict__ r_out, uint64_t *__restrict__ id_out,
                                                uint32_t *__restrict__ perm, GatherList g)
 {
-    constexpr int NF = W - 3, PC = W / 2, ITEMS = CAP / BS_T;
-    constexpr int SN = 256 * 8 / W;                                 // records staged at a time: 16 KB
-    constexpr int STAGE = SN * PC + SN * PC / 32;                   // 16-byte pieces, one pad per 32
-    constexpr int BUF = 2 * STAGE > CAP ? 2 * STAGE : CAP;
-    static_assert(CAP % BS_T == 0 && (CAP & (CAP - 1)) == 0, "LDS capacity");
-    __shared__ __align__(16) uint64_t buf[BUF];                     // keys, later the staged records
-    __shared__ uint16_t idx[CAP], fin[CAP];
-    __shared__ uint32_t bin[BS_BINS + 1];
-    __shared__ uint32_t lds[BS_T / 64];
-    __shared__ uint64_t red[2][BS_T / 64];
-    __shared__ uint32_t worst;
+    using Lds = BucketLds<W, CAP>;
+    constexpr int NF = W - 3, PC = Lds::PC, SN = Lds::SN;
+    __shared__ Lds sh;
     const int t = threadIdx.x, nb = kg_.nb, b = kg_.bid;
     const uint32_t first = place[b], mine = place[b + 1] - first;
     if (b == 0 && t == 0) {
@@ -551,92 +746,16 @@ struct sb_sort_kernel {
     if (!mine) return;
     const int64_t cnt = mine;
     const uint64_t *rec = aos + (int64_t)W * first;
-    const uint32_t *ord = nullptr;                         // global order of a bucket beyond CAP
-    if (cnt > CAP) {
-        ord = merge_bucket<W, CAP>(rec, buf, idx, cnt, order + first, order + n_cap + first);
-    } else {
-        uint64_t k[ITEMS], lo = ~0ull, hi = 0ull;
-        uint32_t at[ITEMS];
-#pragma unroll
-        for (int u = 0; u < ITEMS; u++) {
-            const int e = u * BS_T + t;
-            k[u] = 0;
-            if (e < cnt) {
-                k[u] = sortable(__longlong_as_double((long long)rec[(int64_t)W * e]));
-                lo = k[u] < lo ? k[u] : lo;
-                hi = k[u] > hi ? k[u] : hi;
-            }
-        }
-        for (int o = 32; o > 0; o >>= 1) {
-            const uint64_t x = __shfl_xor(lo, o, 64), y = __shfl_xor(hi, o, 64);
-            lo = x < lo ? x : lo;
-            hi = y > hi ? y : hi;
-        }
-        if ((t & 63) == 0) { red[0][t >> 6] = lo; red[1][t >> 6] = hi; }
-        for (int q = t; q <= BS_BINS; q += BS_T) bin[q] = 0;
-        if (t == 0) worst = 0;
-        __syncthreads();
-        for (int q = 0; q < BS_T / 64; q++) {
-            lo = red[0][q] < lo ? red[0][q] : lo;
-            hi = red[1][q] > hi ? red[1][q] : hi;
-        }
-        const Binning bin_of(lo, hi, BS_BINS);
-#pragma unroll
-        for (int u = 0; u < ITEMS; u++)
-            if (u * BS_T + t < cnt) at[u] = atomicAdd(&bin[bin_of(k[u])], 1u);
-        __syncthreads();
-        constexpr int PER = BS_BINS / BS_T;
-        uint32_t c[PER], sum = 0, mx = 0, dummy;
-#pragma unroll
-        for (int q = 0; q < PER; q++) {
-            c[q] = bin[t * PER + q];
-            sum += c[q];
-            mx = c[q] > mx ? c[q] : mx;
-        }
-        if (mx > BS_RANK) worst = mx;                      // any value above BS_RANK will do
-        uint32_t run = block_excl(sum, lds, &dummy);
-#pragma unroll
-        for (int q = 0; q < PER; q++) { bin[t * PER + q] = run; run += c[q]; }
-        if (t == 0) bin[BS_BINS] = (uint32_t)cnt;
-        __syncthreads();
-        const bool uneven = worst > BS_RANK;
-#pragma unroll
-        for (int u = 0; u < ITEMS; u++) {
-            const int e = u * BS_T + t;
-            if (e < cnt) {
-                const uint32_t p = uneven ? (uint32_t)e : bin[bin_of(k[u])] + at[u];
-                buf[p] = k[u];
-                idx[p] = (uint16_t)e;
-                at[u] = p;
-            }
-        }
-        __syncthreads();
-        if (uneven) {
-            bitonic<W, CAP>(rec, buf, idx, (int)cnt);
-            for (int q = t; q < cnt; q += BS_T) fin[q] = idx[q];
-        } else {
-#pragma unroll
-            for (int u = 0; u < ITEMS; u++) {
-                const int e = u * BS_T + t;
-                if (e < cnt) {
-                    const uint32_t bn = bin_of(k[u]), e0 = bin[bn], e1 = bin[bn + 1];
-                    uint32_t rank = e0;
-                    for (uint32_t q = e0; q < e1; q++)
-                        if (q != at[u]) rank += key_less<W>(rec, buf[q], idx[q], k[u], (uint32_t)e);
-                    fin[rank] = (uint16_t)e;
-                }
-            }
-        }
-    }
-    __syncthreads();
-    ulonglong2 *stage = (ulonglong2 *)buf;
+    const uint32_t *ord = cnt > CAP ? order + first : nullptr;
+    order_bucket<W, CAP>(rec, mine, order + first, order + n_cap + first, sh);
+    ulonglong2 *stage = (ulonglong2 *)sh.buf;
     for (int64_t c0 = 0; c0 < cnt; c0 += SN) {
         const int live = (int)(cnt - c0 < SN ? cnt - c0 : SN);
 #pragma unroll
         for (int u = 0; u < SN * PC / BS_T; u++) {
             const int task = u * BS_T + t, sl = task / PC, pc = task % PC;
             if (sl < live) {
-                const uint32_t e = ord ? ord[c0 + sl] : fin[c0 + sl];
+                const uint32_t e = ord ? ord[c0 + sl] : sh.fin[c0 + sl];
                 stage[task + task / 32] = *(const ulonglong2 *)(rec + (int64_t)W * e + 2 * pc);
             }
         }
@@ -723,12 +842,14 @@ hipError_t launch_sort_fields(const double *key_src, double *r_dst, int nf, cons
     if ((size_t)sh.tiles * sh.buckets > sc.sort_mat_cap) return hipErrorInvalidValue;
     const uint64_t *id_src = src[nf - 1];
     uint64_t *id_dst = dst[nf - 1];
-    const bool small = sh.small;
     // Records: 8 words hold r, id, slot and five fields (the step's sort); a wider payload
-    // takes 16 words, and its buckets, cut from a sample, get twice the LDS capacity.
-    if (g.nf <= 5)
-        return small ? sort_launch<8, SB_SMALL_BUCKETS, 2048>(key_src, r_dst, id_src, id_dst, g, s, sc, sh, n_ub, knew, st)
-                     : sort_launch<8, SB_MAX_BUCKETS, 2048>(key_src, r_dst, id_src, id_dst, g, s, sc, sh, n_ub, knew, st);
-    return small ? sort_launch<16, SB_SMALL_BUCKETS, 4096>(key_src, r_dst, id_src, id_dst, g, s, sc, sh, n_ub, knew, st)
-                 : sort_launch<16, SB_MAX_BUCKETS, 4096>(key_src, r_dst, id_src, id_dst, g, s, sc, sh, n_ub, knew, st);
+    // takes 16 words, and its buckets, cut from a sample, get twice the LDS capacity.  So do
+    // the step's where SB_MAX_BUCKETS of SB_AVG stars are not enough: its sort at 1.8e7 stars
+    // 1.70 ms with 2048 records in LDS, 1.28 with 4096; 3.90 and 3.44 at 3.6e7, 8.6 and 7.9 at
+    // 7e7 (below, fewer blocks share a compute unit for nothing).
+    const bool small = sh.small, wide = n_ub > (int64_t)SB_MAX_BUCKETS * SB_AVG;
+    auto launch = g.nf <= 5 ? (small ? sort_launch<8, SB_SMALL_BUCKETS, 2048>
+                               : wide ? sort_launch<8, SB_MAX_BUCKETS, 4096> : sort_launch<8, SB_MAX_BUCKETS, 2048>)
+                            : (small ? sort_launch<16, SB_SMALL_BUCKETS, 4096> : sort_launch<16, SB_MAX_BUCKETS, 4096>);
+    return launch(key_src, r_dst, id_src, id_dst, g, s, sc, sh, n_ub, knew, st);
 }

@@ -1,0 +1,108 @@
+"""Buckets of the sort beyond the LDS capacity, which one block splits: ties in radius and id,
+clumps within clumps, steps that crowd most stars into one bucket, and cluster sizes at which
+every bucket is that long."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+KEYS = ("m", "vr", "vt", "E", "J", "rnew", "vrnew", "vtnew", "X", "Y", "r_peri", "r_apo", "rOld", "Uoldrold", "Uoldrnew",
+        "vrold", "vtold", "EI")
+
+
+def _case(kind, n, rng):
+    """radii and ids of n stars"""
+    r, i = np.full(n, 0.75), rng.permutation(n) - n // 2
+    if kind == "tied":                         # few radii and few ids: slots decide
+        r = rng.choice([0.25, 0.5, 0.5 + 2.0 ** -53], n)
+        i = rng.integers(-2, 3, n) * 2 ** 62 // 2
+    elif kind == "extreme ids":                # equal radii, ids at the ends of their type
+        i = rng.choice([-2 ** 63, -1, 0, 2 ** 63 - 1], n)
+    elif kind == "nested":                     # clumps within clumps, and two stars that stretch the range
+        depth = rng.integers(1, 7, n)
+        r = 1.0 + 2.0 ** (-8.0 * depth) * (1.0 + rng.random(n))
+        r[0], r[-1] = 1e-9, 9e9
+    elif kind == "most":                       # one part just at the capacity, the rest in another
+        r = np.where(np.arange(n) < n - 2048, 1.0 + 1e-12 * rng.random(n), 2.0 + rng.random(n))
+    p = rng.permutation(n)
+    return r[p], i.astype(np.int64)[p]
+
+
+@pytest.mark.parametrize("kind", ["equal", "tied", "extreme ids", "nested", "most"])
+@pytest.mark.parametrize("n", [2048, 4096, 4097, 8193, 12289, 70000])
+def test_gpu_sort_of_long_buckets(gpu, n, kind):
+    cm = gpu
+    print("[gpu-test] long buckets", n, kind, flush=True)
+    rng = np.random.default_rng(n)
+    cl = cm.Cluster(n)
+    cl["r"][1:n + 1], cl["id"][1:n + 1] = _case(kind, n, rng)
+    for k in KEYS:
+        cl[k][1:n + 1] = rng.random(n)
+    order = 1 + np.lexsort((cl["id"][1:n + 1], cl["r"][1:n + 1]))        # stable: slots decide last
+    with cm.Context(n, cm.default_params(n)) as ctx:
+        ctx.upload(cl)
+        assert ctx.sort_by_r() == n
+        d = ctx.download()
+    for k in ("r", "id") + KEYS:
+        assert np.array_equal(d[k][1:n + 1], cl[k][order]), k
+
+
+def _shell(cm, n):
+    """A thin shell: half of its stars go inside every radius of before, into the first bucket."""
+    cl = cm.make_plummer(n, seed=n, kroupa=True)
+    cl["r"][1:n + 1] = np.sort(0.8 + 1e-3 * np.random.default_rng(n).random(n))
+    return cl
+
+
+@pytest.mark.parametrize("n", [3000, 20000, 140000])
+@pytest.mark.parametrize("graph", [False, True])
+def test_gpu_step_of_a_shell(gpu, O, n, graph):
+    cm = gpu
+    print("[gpu-test] shell", n, graph, flush=True)
+    cl = _shell(cm, n)
+    o = O.Oracle(cl.a, n, orbit_r=1e3, rng_mode=O.RNG_PER_STAR, q_mode=O.Q_FP64, libm_mode=O.LIBM_DD)
+    o.init()
+    with cm.Context(n, cm.default_params(n, orbit_r=1e3)) as ctx:
+        ctx.upload(cl)
+        ctx.init_cluster()
+        for _ in range(2):
+            (ctx.step_graph if graph else ctx.step)()
+            assert o.step() == 0
+        d = ctx.download()
+    N = o.N
+    assert d.n == N
+    for k in ("r", "id", "vr", "vt", "m", "phi"):
+        assert np.array_equal(d[k][1:N + 1], o[k][1:N + 1]), k
+
+
+def _sort_ms(cm, n):
+    """The sort's time in a step of an even cluster, the least of three."""
+    cl = cm.Cluster(n, fields=["r", "m", "vr", "vt", "id"])
+    rng = np.random.default_rng(1)
+    a = 3 * np.pi / 16
+    r = np.sort(a / np.sqrt((rng.random(n) * 0.999998 + 1e-6) ** (-2 / 3) - 1))
+    v = 0.6 * np.sqrt(2) * (r * r + a * a) ** -0.25
+    c = 1 - 2 * rng.random(n)
+    cl["r"][0], cl["r"][n + 1] = 1e-20, 1e10
+    for k, x in (("r", r), ("m", np.ones(n)), ("vr", c * v), ("vt", v * np.sqrt(1 - c * c)), ("id", np.arange(1, n + 1))):
+        cl[k][1:n + 1] = x
+    with cm.Context(n, cm.default_params(n, orbit_r=300 * a)) as ctx:
+        ctx.upload(cl, fields=["r", "m", "vr", "vt", "id"])
+        ctx.init_cluster()
+        ctx.timer_enable(True)
+        ms = []
+        for _ in range(4):
+            ctx.timer_reset()
+            ctx.step()
+            ms.append(ctx.timer_get("sort")[0])
+        d = ctx.download(fields=["r", "id"])
+        assert np.all(d["r"][1:d.n] <= d["r"][2:d.n + 1]) and np.unique(d["id"][1:d.n + 1]).size == d.n
+    return min(ms[1:])
+
+
+def test_gpu_sort_time_stays_in_proportion(gpu):
+    """At 3.5e7 stars every bucket is longer than a block's LDS: the sort's time per star stays
+    within twice that at 4e6 (1.35 times measured)."""
+    small, large = _sort_ms(gpu, 4000000), _sort_ms(gpu, 35000000)
+    print("[gpu-test] sort ms at 4e6 and 3.5e7:", small, large, flush=True)
+    assert large / 35 < 2.0 * small / 4
