@@ -19,7 +19,7 @@
 // and changes the density little, so equal cuts of the old order keep nearly equal counts.
 // The general entry point orders radii it knows nothing about and bisects boundaries taken
 // from a sorted sample.  Counts decide only the speed: a bucket beyond the LDS capacity is
-// merge-sorted in global memory by its block.
+// split further by its block, in time proportional to its stars.
 //
 // Bound: HBM.  The payload (64 B a star) is read and written twice, 256 B a star, plus 4 B
 // of node indices.  It replaced an LSD radix sort of (key, slot) words, which packed the
@@ -98,9 +98,27 @@ struct Binning {
 __device__ __forceinline__ int64_t tile_chunk(int64_t n, int64_t nt) { return (n + nt - 1) / nt; }
 
 // Bucket boundaries from a sample (the general entry point): S keys at even strides,
-// ordered in LDS by a counting sort over sub-ranges and ranks inside them; boundary b is
-// the sample at rank b S / B.
-constexpr int SMP_T = 1024, SMP_MAX = 8192, SMP_BINS = 4096;
+// ordered in LDS by a counting sort over sub-ranges and ranks inside them, or by a bitonic
+// sort where a sub-range holds more than SMP_RANK of them (tied or clumped radii: the ranks
+// among 8192 keys of one sub-range took 3.5 s); boundary b is the sample at rank b S / B.
+constexpr int SMP_T = 1024, SMP_MAX = 8192, SMP_BINS = 4096, SMP_RANK = 64;
+// Bitonic sort of key[0, S) by the whole block; key holds SMP_MAX words.
+__device__ void sample_sort(uint64_t *key, int S)
+{
+    int P = 1;
+    while (P < S) P <<= 1;
+    for (int q = S + threadIdx.x; q < P; q += blockDim.x) key[q] = ~0ull;
+    __syncthreads();
+    for (int kk = 2; kk <= P; kk <<= 1)
+        for (int j = kk >> 1; j > 0; j >>= 1) {
+            for (int p = threadIdx.x; p < P / 2; p += blockDim.x) {
+                const int q = 2 * p - (p & (j - 1)), x = q | j;       // the p-th pair at distance j
+                const uint64_t a = key[q], b = key[x];
+                if ((a > b) == ((q & kk) == 0)) { key[q] = b; key[x] = a; }
+            }
+            __syncthreads();
+        }
+}
 struct sb_sample_kernel {
     static constexpr int LB = SMP_T, MB = 0;
     static __device__ __forceinline__ void run(KGrid kg_, const double *__restrict__ keysrc, const DevScalars *s, int B,
@@ -110,10 +128,12 @@ struct sb_sample_kernel {
     __shared__ uint32_t bin[SMP_BINS + 1];
     __shared__ uint64_t red[2][SMP_T / 64];
     __shared__ uint32_t scan[SMP_T / 64];
+    __shared__ int clumped;
     const int t = threadIdx.x;
     const int64_t n = s->n_max_new;
     const int S = n < SMP_MAX ? (int)n : SMP_MAX;
     for (int q = t; q <= SMP_BINS; q += SMP_T) bin[q] = 0;
+    if (t == 0) clumped = 0;
     uint64_t k[SMP_MAX / SMP_T];
     uint64_t lo = ~0ull, hi = 0ull;
 #pragma unroll
@@ -148,7 +168,11 @@ struct sb_sample_kernel {
     constexpr int PER = SMP_BINS / SMP_T;
     uint32_t c[PER], sum = 0, tot;
 #pragma unroll
-    for (int q = 0; q < PER; q++) { c[q] = bin[t * PER + q]; sum += c[q]; }
+    for (int q = 0; q < PER; q++) {
+        c[q] = bin[t * PER + q];
+        sum += c[q];
+        if (c[q] > SMP_RANK) clumped = 1;
+    }
     uint32_t run = block_excl(sum, scan, &tot);
 #pragma unroll
     for (int q = 0; q < PER; q++) { bin[t * PER + q] = run; run += c[q]; }
@@ -158,6 +182,11 @@ struct sb_sample_kernel {
     for (int u = 0; u < SMP_MAX / SMP_T; u++)
         if (u * SMP_T + t < S) key[bin[bin_of(k[u])] + at[u]] = k[u];
     __syncthreads();
+    if (clumped) {
+        sample_sort(key, S);
+        for (int b = t; b < B; b += SMP_T) split[b] = b > 0 ? key[(int64_t)b * S / B] : 0ull;
+        return;
+    }
     // boundary b: the sample of rank b S / B, found among its bin's keys
     for (int b = t; b < B; b += SMP_T) {
         uint64_t v = 0;

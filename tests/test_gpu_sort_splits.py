@@ -106,3 +106,32 @@ def test_gpu_sort_time_stays_in_proportion(gpu):
     small, large = _sort_ms(gpu, 4000000), _sort_ms(gpu, 35000000)
     print("[gpu-test] sort ms at 4e6 and 3.5e7:", small, large, flush=True)
     assert large / 35 < 2.0 * small / 4
+
+
+@pytest.mark.parametrize("kind", ["equal", "clump"])
+@pytest.mark.parametrize("n", [9000, 140000])
+def test_gpu_sort_of_tied_radii_takes_its_share(gpu, n, kind):
+    """The sampled boundaries of tied or clumped radii: ranks among all samples took seconds,
+    the whole sort now under 10 ms at these sizes (0.1 s leaves room)."""
+    cm = gpu
+    print("[gpu-test] tied radii", n, kind, flush=True)
+    rng = np.random.default_rng(n)
+    r = np.full(n, 0.75)
+    if kind == "clump":
+        r = 1.0 + 1e-9 * rng.random(n)
+        r[0], r[-1] = 1e-6, 1e5
+    cl = cm.Cluster(n, fields=["r", "id"])
+    cl["r"][1:n + 1] = rng.permutation(r)
+    cl["id"][1:n + 1] = rng.permutation(n)
+    order = 1 + np.lexsort((cl["id"][1:n + 1], cl["r"][1:n + 1]))
+    with cm.Context(n, cm.default_params(n)) as ctx:
+        ctx.timer_enable(True)
+        for _ in range(2):                                  # the first loads the kernels
+            ctx.upload(cl)
+            ctx.timer_reset()
+            assert ctx.sort_by_r() == n
+        ms = ctx.timer_get("sort")[0]
+        d = ctx.download(fields=["r", "id"])
+    print("[gpu-test] ms", ms, flush=True)
+    assert np.array_equal(d["r"][1:n + 1], cl["r"][order]) and np.array_equal(d["id"][1:n + 1], cl["id"][order])
+    assert ms < 100.0
