@@ -496,13 +496,14 @@ struct BucketLds {
 template <int W>
 __device__ void bitonic(const uint64_t *__restrict__ rec, const Records &of, uint64_t *key, uint16_t *idx, int cnt)
 {
-    int P = 1;
+    int P = 1, t = threadIdx.x;
+    asm volatile("" : "+v"(t));
     while (P < cnt) P <<= 1;
-    for (int q = cnt + threadIdx.x; q < P; q += BS_T) { key[q] = ~0ull; idx[q] = 0xffff; }
+    for (int q = cnt + t; q < P; q += BS_T) { key[q] = ~0ull; idx[q] = 0xffff; }
     __syncthreads();
     for (int kk = 2; kk <= P; kk <<= 1)
         for (int j = kk >> 1; j > 0; j >>= 1) {
-            for (int q = threadIdx.x; q < P; q += BS_T) {
+            for (int q = t; q < P; q += BS_T) {
                 const int x = q ^ j;
                 if (x > q) {
                     const uint64_t ka = key[q], kb = key[x];
@@ -641,7 +642,7 @@ __device__ __forceinline__ void split_part(const uint64_t *__restrict__ rec, Par
     for (;; p.w++) {
         lo = ~0ull;
         hi = 0ull;
-#pragma unroll 4
+#pragma unroll 2
         for (uint32_t e = t; e < p.len; e += BS_T) {
             const uint64_t k = rec_key<W>(rec, of(e), p.w);
             lo = k < lo ? k : lo;
@@ -653,7 +654,7 @@ __device__ __forceinline__ void split_part(const uint64_t *__restrict__ rec, Par
         __syncthreads();
     }
     const Binning bin_of(lo, hi, SPLIT_BINS);
-#pragma unroll 4
+#pragma unroll 2
     for (uint32_t e = t; e < p.len; e += BS_T) atomicAdd(&sh.sub[bin_of(rec_key<W>(rec, of(e), p.w))], 1u);
     __syncthreads();
     constexpr int PER = SPLIT_BINS / BS_T;
@@ -666,7 +667,7 @@ __device__ __forceinline__ void split_part(const uint64_t *__restrict__ rec, Par
     __syncthreads();
     p.in = p.in == 0 ? 1 : 0;
     uint32_t *to = (p.in ? tmp : ord) + p.start;
-#pragma unroll 4
+#pragma unroll 2
     for (uint32_t e = t; e < p.len; e += BS_T) {
         const uint32_t a = of(e);
         to[atomicAdd(&sh.sub[bin_of(rec_key<W>(rec, a, p.w))], 1u)] = a;
@@ -679,62 +680,77 @@ template <int W, int CAP>
 __device__ __forceinline__ void order_bucket(const uint64_t *__restrict__ rec, uint32_t cnt, uint32_t *ord, uint32_t *tmp,
                                              BucketLds<W, CAP> &sh)
 {
-    constexpr uint64_t NONE = ~0ull;
-    const int t = threadIdx.x;
-    Part p{0, cnt, 0, 2};
-    uint64_t waiting = NONE;                               // 2 place + array
-    uint32_t s = 0, e = cnt;                               // the run of p in hand
-    int b = SPLIT_BINS;
+    constexpr uint64_t NONE = ~0ull, WHOLE = ~1ull;
+    Part p{0, 0, 0, 2};
+    uint64_t waiting = WHOLE;                              // 2 place + array
+    uint32_t s = 0, e = 0;                                 // the run of p in hand
+    int b = 0;
     const bool fits = cnt <= CAP;
-    if (!fits) {
-        split_part<W>(rec, p, ord, tmp, sh);
-        e = b = 0;
+    if (fits) {
+        order_records<W, CAP>(rec, Records{nullptr}, cnt, 0, sh);
+        return;
     }
     for (;;) {
-        if (!fits) {
-            // the next run: parts b .. b1 - 1 fit together
-            s = e;
-            if (s == p.len) {
-                if (waiting == NONE) return;
-                __syncthreads();
+        int t = threadIdx.x;
+        asm volatile("" : "+v"(t));                        // keeps what depends on it out of registers between runs
+        // the next run: parts b .. b1 - 1 fit together
+        s = e;
+        if (s == p.len) {
+            if (waiting == NONE) return;
+            __syncthreads();
+            if (waiting == WHOLE) {
+                waiting = NONE;
+                p.len = cnt;
+            } else {
                 p.in = (int)(waiting & 1);
                 p.start = (uint32_t)(waiting >> 1);
                 const uint32_t *note = (p.in ? ord : tmp) + p.start;
                 waiting = uniform(note[0]) | (uint64_t)uniform(note[1]) << 32;
                 p.len = uniform(note[2]);
                 p.w = (int)uniform(note[3]);
-                __syncthreads();                           // the split writes where the note is
-                split_part<W>(rec, p, ord, tmp, sh);
-                s = 0;
-                b = 0;
+                __syncthreads();                       // the split writes where the note is
             }
-            int b1 = b, top = SPLIT_BINS;
-            while (b1 < top) {
-                const int m = (b1 + top) >> 1;
-                if (uniform(sh.sub[m]) - s <= CAP) b1 = m + 1;
-                else top = m;
-            }
-            if (b1 == b) {                                 // part b alone is too long: it waits
-                e = uniform(sh.sub[b]);
-                if (t == 0) {
-                    uint32_t *note = (p.in ? ord : tmp) + p.start + s;
-                    note[0] = (uint32_t)waiting;
-                    note[1] = (uint32_t)(waiting >> 32);
-                    note[2] = e - s;
-                    note[3] = (uint32_t)p.w;
-                }
-                waiting = 2 * (uint64_t)(p.start + s) + p.in;
-                b++;
-                continue;
-            }
-            e = uniform(sh.sub[b1 - 1]);
-            b = b1;
-            if (e == s) continue;
+            split_part<W>(rec, p, ord, tmp, sh);
+            s = 0;
+            b = 0;
         }
+        int b1 = b, top = SPLIT_BINS;
+        while (b1 < top) {
+            const int m = (b1 + top) >> 1;
+            if (uniform(sh.sub[m]) - s <= CAP) b1 = m + 1;
+            else top = m;
+        }
+        if (b1 == b) {                                 // part b alone is too long: it waits
+            e = uniform(sh.sub[b]);
+            if (t == 0) {
+                uint32_t *note = (p.in ? ord : tmp) + p.start + s;
+                note[0] = (uint32_t)waiting;
+                note[1] = (uint32_t)(waiting >> 32);
+                note[2] = e - s;
+                note[3] = (uint32_t)p.w;
+            }
+            waiting = 2 * (uint64_t)(p.start + s) + p.in;
+            b++;
+            continue;
+        }
+        e = uniform(sh.sub[b1 - 1]);
+        b = b1;
+        if (e == s) continue;
         const int m = (int)(e - s);
-        const Records of{fits ? nullptr : (p.in ? tmp : ord) + p.start + s};
-        order_records<W, CAP>(rec, of, m, p.w, sh);
-        if (fits) return;
+        const Records of{(p.in ? tmp : ord) + p.start + s};
+        // (with 2048 records in LDS four blocks share a compute unit, which leaves 64 registers:
+        // the counting order's keys and places do not fit them inside this loop)
+        if (CAP > 2048) {
+            order_records<W, CAP>(rec, of, m, p.w, sh);
+        } else {
+            for (int q = t; q < m; q += BS_T) {
+                sh.buf[q] = rec_key<W>(rec, of.list[q], p.w);
+                sh.idx[q] = (uint16_t)q;
+            }
+            bitonic<W>(rec, of, sh.buf, sh.idx, m);
+            for (int q = t; q < m; q += BS_T) sh.fin[q] = sh.idx[q];
+            __syncthreads();
+        }
         uint32_t v[CAP / BS_T];
 #pragma unroll
         for (int u = 0; u < CAP / BS_T; u++)
@@ -753,7 +769,7 @@ __device__ __forceinline__ void order_bucket(const uint64_t *__restrict__ rec, u
 // between the two reads, or 256 threads a block, changed nothing.
 template <int W, int CAP>
 struct sb_sort_kernel {
-    static constexpr int LB = BS_T, MB = 0;
+    static constexpr int LB = BS_T, MB = CAP <= 2048 ? 8 : 4;
     static __device__ __forceinline__ void run(KGrid kg_, DevScalars *s, const uint32_t *__restrict__ place, int32_t *bad,
                                                const uint64_t *__restrict__ aos, uint32_t *order, int64_t n_cap,
                                                double *__restrict__ r_out, uint64_t *__restrict__ id_out,
