@@ -757,8 +757,9 @@ struct pred_from_apsides_kernel {
 // ------------------------------------------------------------------ radial index
 struct ridx_clear_kernel {
     static constexpr int LB = 1024, MB = 0;
-    static __device__ __forceinline__ void run(KGrid kg_, uint32_t *__restrict__ t, int64_t count)
+    static __device__ __forceinline__ void run(KGrid kg_, uint32_t *__restrict__ t, int64_t count, int32_t *__restrict__ bad)
 {
+    if (kg_.bid == 0 && threadIdx.x == 0) *bad = 0;
     for (int64_t i = (int64_t)kg_.bid * blockDim.x + threadIdx.x; i < count; i += (int64_t)kg_.nb * blockDim.x)
         t[i] = 0;
 }
@@ -768,7 +769,7 @@ struct ridx_clear_kernel {
 // the radial index's marks (nodes 0..n), in one pass over r and phi: node k (node 0
 // stands for "below every bucket") writes its index at its bucket when it is the
 // bucket's last node, and k at every multiple of RIDX_TILE in (bucket(r_k),
-// bucket(r_{k+1})] of the tile table.  The index array must be cleared before.  *bad is
+// bucket(r_{k+1})] of the tile table.  The index array and *bad must be cleared before; *bad is
 // set where the radii do not ascend (the step's sort then does without their order).
 struct node_index_kernel {
     static constexpr int LB = 1024, MB = 0;
@@ -967,7 +968,7 @@ hipError_t launch_node_index(const DevFields &f, DevScalars *s, const Scratch &s
                              hipStream_t st)
 {
     const int64_t entries = ridx_entries(sc.ridx_bits);
-    if (!clear) kl<ridx_clear_kernel>(dim3(512), dim3(256), 0, st, sc.ridx, entries);
+    if (!clear) kl<ridx_clear_kernel>(dim3(512), dim3(256), 0, st, sc.ridx, entries, sc.sort_bad);
     kl<node_index_kernel>(dim3((unsigned)((n_ub + 2 + 255) / 256)), dim3(256), 0, st, f.r, f.phi, s,
                        (double2 *)sc.nodes, (double2 *)sc.mid, sc.ridx, sc.ridx_tb, sc.ridx_bits, sc.sort_bad);
     kl<ridx_scan_kernel>(dim3((unsigned)(ridx_tiles(sc.ridx_bits) + (coarse + 256) / 256)), dim3(256), 0, st, sc.ridx,

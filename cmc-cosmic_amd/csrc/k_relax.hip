@@ -179,7 +179,8 @@ struct step_begin_kernel { static constexpr int LB = 1024, MB = 0; static __devi
 // for the next step (when dt_part is given; sigma_dt_kernel touches nothing the begin sets),
 // the time step (thread 0) with Prev_Dt for the next one (cmc.c:297: only the time step reads
 // it), then the step's RNG substream bases.  The other blocks clear the radial index for the
-// orbit phase.  (Four launches of 4 to 5 us each that had no work of their own.)
+// orbit phase (its flag of radii out of order: block 0).  (Four launches of 4 to 5 us each that
+// had no work of their own.)
 constexpr int64_t CLEAR_BLK = RB_T * 16;           // index entries per block
 struct timestep_rng_bases_kernel {
     static constexpr int LB = RB_T, MB = 0;
@@ -187,7 +188,8 @@ struct timestep_rng_bases_kernel {
                                                                   const Rng *__restrict__ seeded,
                                                                   Rng *__restrict__ base,
                                                                   unsigned long long *__restrict__ dt_part,
-                                                                  uint32_t *__restrict__ ridx, int64_t entries)
+                                                                  uint32_t *__restrict__ ridx, int64_t entries,
+                                                                  int32_t *__restrict__ bad)
 {
     if (kg_.bid > 0) {
         const int64_t b0 = (int64_t)(kg_.bid - 1) * CLEAR_BLK;
@@ -218,6 +220,7 @@ struct timestep_rng_bases_kernel {
     if (threadIdx.x == 0) {
         timestep_finalize(s);
         s->Prev_Dt = s->Dt;
+        *bad = 0;
     }
     rng_bases(J, s, seeded, base, -1);
 }
@@ -613,7 +616,7 @@ hipError_t launch_timestep_sigma(const DevFields &f, DevScalars *s, const KParam
     const int64_t entries = ridx_entries(sc.ridx_bits);
     kl<timestep_rng_bases_kernel>(dim3(1 + (unsigned)((entries + CLEAR_BLK - 1) / CLEAR_BLK)), dim3(RB_T), 0, st,
                        (const JumpLevel *)sc.jump->level, s, sc.rng_seeded, sc.rng_base,
-                       one_pass ? sc.dt_part : (unsigned long long *)nullptr, sc.ridx, entries);
+                       one_pass ? sc.dt_part : (unsigned long long *)nullptr, sc.ridx, entries, sc.sort_bad);
     return hipGetLastError();
 }
 hipError_t launch_timestep_finalize(DevScalars *s, hipStream_t st)

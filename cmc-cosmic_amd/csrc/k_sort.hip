@@ -770,7 +770,7 @@ __device__ __forceinline__ void order_bucket(const uint64_t *__restrict__ rec, u
 template <int W, int CAP>
 struct sb_sort_kernel {
     static constexpr int LB = BS_T, MB = CAP <= 2048 ? 8 : 4;
-    static __device__ __forceinline__ void run(KGrid kg_, DevScalars *s, const uint32_t *__restrict__ place, int32_t *bad,
+    static __device__ __forceinline__ void run(KGrid kg_, DevScalars *s, const uint32_t *__restrict__ place,
                                                const uint64_t *__restrict__ aos, uint32_t *order, int64_t n_cap,
                                                double *__restrict__ r_out, uint64_t *__restrict__ id_out,
                                                uint32_t *__restrict__ perm, GatherList g)
@@ -782,7 +782,6 @@ struct sb_sort_kernel {
     const uint32_t first = place[b], mine = place[b + 1] - first;
     if (b == 0 && t == 0) {
         const uint32_t tot = place[nb];
-        if (bad) *bad = 0;
         s->sort_n = tot;
         s->n_max = tot;
         s->n_max_new = tot;                                // no block of this launch reads them
@@ -862,8 +861,7 @@ hipError_t sort_launch(const double *key_src, double *r_dst, const uint64_t *id_
                                  (const uint32_t *)sc.sort_mat, (const uint32_t *)sc.sort_tot, sc.sort_first, sh.buckets,
                                  scanned, sc.sort_aos, g);
     kl<sb_sort_kernel<W, CAP>>(dim3((unsigned)sh.buckets), dim3(BS_T), 0, st, s, (const uint32_t *)sc.sort_first,
-                               knew ? sc.sort_bad : (int32_t *)nullptr, (const uint64_t *)sc.sort_aos, sc.sort_order,
-                               sc.sort_aos_cap, r_dst, id_dst, sc.vals_a, g);
+                               (const uint64_t *)sc.sort_aos, sc.sort_order, sc.sort_aos_cap, r_dst, id_dst, sc.vals_a, g);
     if (g.nf > W - 3)
         kl<sb_rest_kernel>(dim3((unsigned)((n_ub + 255) / 256)), dim3(256), 0, st, (const DevScalars *)s,
                            (const uint32_t *)sc.vals_a, W - 3, g);
