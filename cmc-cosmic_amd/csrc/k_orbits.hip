@@ -600,19 +600,59 @@ __device__ void orbits_part(const double *__restrict__ partials, int64_t nblocks
     }
 }
 
+// Whether the new radii's indices cut the stars into even buckets for the step's sort: up to
+// SMP_MAX of them counted (one block).  A bucket is too long at twice its share and 40 more:
+// what a sample can miss, 40 of 8192, costs its block less than 0.4 ms at N = 4e6.  (The
+// deferred stars have the indices of their last orbits; counts decide only the speed.)
+__device__ void sort_balance(const int32_t *__restrict__ knew, int64_t n, int B, int32_t *uneven)
+{
+    __shared__ uint32_t hist[SB_MAX_BUCKETS];
+    const int t = threadIdx.x, S = n < SMP_MAX ? (int)n : SMP_MAX;
+    for (int b = t; b < B; b += DEFER_T) hist[b] = 0;
+    const StepBucket bucket(n, B);
+    const double stride = (double)n / (double)S;           // at least 1
+    uint32_t k[SMP_MAX / DEFER_T];
+#pragma unroll
+    for (int u = 0; u < SMP_MAX / DEFER_T; u++) {
+        const int q = u * DEFER_T + t;
+        k[u] = q < S ? bucket(knew[1 + (int64_t)(q * stride)]) : (uint32_t)SB_TAIL;
+    }
+    __syncthreads();
+    const uint32_t limit = 2 * (uint32_t)S / (uint32_t)B + 40;
+    bool over = false;
+#pragma unroll
+    for (int u = 0; u < SMP_MAX / DEFER_T; u++)
+        if (k[u] != SB_TAIL) over |= atomicAdd(&hist[k[u]], 1u) >= limit;
+    if (over) *uneven = 2;
+}
+// Bucket boundaries from a sample of the new radii, for that case (one block).
+__device__ void step_splits(const double *__restrict__ rnew, int64_t n, int B, uint64_t *__restrict__ split)
+{
+    __shared__ uint64_t key[SMP_MAX];
+    const int t = threadIdx.x, S = n < SMP_MAX ? (int)n : SMP_MAX;
+    for (int q = t; q < S; q += blockDim.x) {
+        const double x = rnew[1 + (int64_t)q * n / S];
+        key[q] = x < CMCG_SF_INFINITY ? sortable(x) : KEY_INF;
+    }
+    sample_sort(key, S);
+    for (int b = t; b < B; b += blockDim.x) split[b] = b > 0 && S > 0 ? key[(int64_t)b * S / B] : 0ull;
+}
+
 // After the sampler, in one launch (three kernels of 4 to 12 us before): its reduction's first
-// level, the order of the deferred stars, and their linear scans.
+// level, the order of the deferred stars, their linear scans, and the buckets' balance.
 constexpr int DEFER_BLOCKS = 256;
 struct after_orbits_kernel {
     static constexpr int LB = DEFER_T, MB = 0;
     static __device__ __forceinline__ void run(KGrid kg_, DevFields f, DevScalars *s, KParams P,
                                                            const double *__restrict__ partials, int64_t nblocks,
                                                            double *__restrict__ red2, const int64_t *__restrict__ list,
-                                                           int64_t *__restrict__ kfirst, int64_t *__restrict__ order)
+                                                           int64_t *__restrict__ kfirst, int64_t *__restrict__ order,
+                                                           int buckets, int32_t *uneven)
 {
     const int b = (int)kg_.bid - RED2_BLOCKS - 1;
     if (b < -1) orbits_part(partials, nblocks, red2, (int)kg_.bid);
     else if (b == -1) defer_sort(list, order, deferred(s, P));
+    else if (b == DEFER_BLOCKS) sort_balance(f.knew, s->n_max, buckets, uneven);
     else defer_search(f, P, list, kfirst, deferred(s, P), s->n_max, b, DEFER_BLOCKS);
 }
 };
@@ -620,7 +660,7 @@ struct after_orbits_kernel {
 // The deferred stars, ORB_THREADS at a time in list order, and the phase's sums: the
 // sampler blocks' records (the first level's RED2_BLOCKS records, in block order), then
 // each deferred star's in list (= star) order, as a single thread would add them; then
-// the end of new_orbits_calculate.
+// the end of new_orbits_calculate.  Block 1: the step's bucket boundaries, where it needs them.
 struct defer_tail_kernel {
     static constexpr int LB = ORB_THREADS, MB = 0;
     static __device__ __forceinline__ void run(KGrid kg_, DevFields f, DevScalars *s, KParams P,
@@ -628,8 +668,14 @@ struct defer_tail_kernel {
                                                                  const Rng *__restrict__ base, int jb1,
                                                                  const int64_t *__restrict__ order,
                                                                  const int64_t *__restrict__ kfirst,
-                                                                 const double *__restrict__ red2)
+                                                                 const double *__restrict__ red2, int buckets,
+                                                                 const int32_t *__restrict__ uneven,
+                                                                 uint64_t *__restrict__ split)
 {
+    if (kg_.bid == 1) {
+        if (*uneven) step_splits(f.rnew, s->n_max, buckets, split);
+        return;
+    }
     __shared__ double part[ORB_THREADS][NRED];
     __shared__ double acc[NRED];
     const int t = threadIdx.x;
@@ -947,10 +993,13 @@ hipError_t launch_orbits(const DevFields &f, DevScalars *s, const KParams &P, co
                        (const double2 *)sc.nodes, (const double2 *)sc.coarse,
                        (const uint32_t *)sc.ridx, sc.ridx_bits);
     if (ev_b) hipEventRecord(ev_b, st);
-    kl<after_orbits_kernel>(dim3(RED2_BLOCKS + 1 + DEFER_BLOCKS), dim3(DEFER_T), 0, st, f, s, P, (const double *)sc.partials,
-                       nblocks, sc.red2, (const int64_t *)sc.defer_list, sc.defer_kfirst, sc.defer_order);
-    kl<defer_tail_kernel>(dim3(1), dim3(ORB_THREADS), 0, st, f, s, P, T, sc.rng_base, jb1,
-                       (const int64_t *)sc.defer_order, (const int64_t *)sc.defer_kfirst, (const double *)sc.red2);
+    const int buckets = sort_shape(n_ub).buckets;
+    kl<after_orbits_kernel>(dim3(RED2_BLOCKS + 1 + DEFER_BLOCKS + 1), dim3(DEFER_T), 0, st, f, s, P, (const double *)sc.partials,
+                       nblocks, sc.red2, (const int64_t *)sc.defer_list, sc.defer_kfirst, sc.defer_order, buckets,
+                       sc.sort_uneven);
+    kl<defer_tail_kernel>(dim3(2), dim3(ORB_THREADS), 0, st, f, s, P, T, sc.rng_base, jb1,
+                       (const int64_t *)sc.defer_order, (const int64_t *)sc.defer_kfirst, (const double *)sc.red2, buckets,
+                       (const int32_t *)sc.sort_uneven, sc.sort_split);
     return hipGetLastError();
 }
 
@@ -968,9 +1017,9 @@ hipError_t launch_node_index(const DevFields &f, DevScalars *s, const Scratch &s
                              hipStream_t st)
 {
     const int64_t entries = ridx_entries(sc.ridx_bits);
-    if (!clear) kl<ridx_clear_kernel>(dim3(512), dim3(256), 0, st, sc.ridx, entries, sc.sort_bad);
+    if (!clear) kl<ridx_clear_kernel>(dim3(512), dim3(256), 0, st, sc.ridx, entries, sc.sort_uneven);
     kl<node_index_kernel>(dim3((unsigned)((n_ub + 2 + 255) / 256)), dim3(256), 0, st, f.r, f.phi, s,
-                       (double2 *)sc.nodes, (double2 *)sc.mid, sc.ridx, sc.ridx_tb, sc.ridx_bits, sc.sort_bad);
+                       (double2 *)sc.nodes, (double2 *)sc.mid, sc.ridx, sc.ridx_tb, sc.ridx_bits, sc.sort_uneven);
     kl<ridx_scan_kernel>(dim3((unsigned)(ridx_tiles(sc.ridx_bits) + (coarse + 256) / 256)), dim3(256), 0, st, sc.ridx,
                        (const uint32_t *)sc.ridx_tb, sc.ridx_bits, (const double2 *)sc.nodes, s, coarse, sc.coarse);
     return hipGetLastError();

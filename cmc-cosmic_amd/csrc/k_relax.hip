@@ -616,7 +616,7 @@ hipError_t launch_timestep_sigma(const DevFields &f, DevScalars *s, const KParam
     const int64_t entries = ridx_entries(sc.ridx_bits);
     kl<timestep_rng_bases_kernel>(dim3(1 + (unsigned)((entries + CLEAR_BLK - 1) / CLEAR_BLK)), dim3(RB_T), 0, st,
                        (const JumpLevel *)sc.jump->level, s, sc.rng_seeded, sc.rng_base,
-                       one_pass ? sc.dt_part : (unsigned long long *)nullptr, sc.ridx, entries, sc.sort_bad);
+                       one_pass ? sc.dt_part : (unsigned long long *)nullptr, sc.ridx, entries, sc.sort_uneven);
     return hipGetLastError();
 }
 hipError_t launch_timestep_finalize(DevScalars *s, hipStream_t st)

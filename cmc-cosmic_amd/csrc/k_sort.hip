@@ -17,8 +17,10 @@
 // In the step the bucket comes from the index of the new radius among the old ones, which
 // the orbit phase found with the potential there: a step moves stars along their orbits
 // and changes the density little, so equal cuts of the old order keep nearly equal counts.
-// The general entry point orders radii it knows nothing about and bisects boundaries taken
-// from a sorted sample.  Counts decide only the speed: a bucket beyond the LDS capacity is
+// Where they would not (a cluster far from equilibrium: of a thin shell half the stars go
+// inside every old radius), or the old radii do not ascend, the orbit phase has sampled the
+// new radii, and the step bisects boundaries as the general entry point does, which orders
+// radii it knows nothing about.  Counts decide only the speed: a bucket beyond the LDS capacity is
 // split further by its block, in time proportional to its stars.
 //
 // Bound: HBM.  The payload (64 B a star) is read and written twice, 256 B a star, plus 4 B
@@ -31,15 +33,6 @@
 
 namespace {
 constexpr int SB_MAX_FIELDS = 20;
-constexpr uint16_t SB_TAIL = 0xffff;               // bucket number of a star of the SF_INFINITY tail
-constexpr uint64_t KEY_INF = 0x8000000000000000ull | 0x4202a05f20000000ull;   // sortable(1.0e10)
-
-__device__ __forceinline__ uint64_t sortable(double x)
-{
-    uint64_t b = (uint64_t)__double_as_longlong(x);
-    return (b >> 63) ? ~b : (b | 0x8000000000000000ull);
-}
-
 // The payload without id: field f goes from src[f] to dst[f].
 struct GatherList {
     int nf;
@@ -101,24 +94,7 @@ __device__ __forceinline__ int64_t tile_chunk(int64_t n, int64_t nt) { return (n
 // ordered in LDS by a counting sort over sub-ranges and ranks inside them, or by a bitonic
 // sort where a sub-range holds more than SMP_RANK of them (tied or clumped radii: the ranks
 // among 8192 keys of one sub-range took 3.5 s); boundary b is the sample at rank b S / B.
-constexpr int SMP_T = 1024, SMP_MAX = 8192, SMP_BINS = 4096, SMP_RANK = 64;
-// Bitonic sort of key[0, S) by the whole block; key holds SMP_MAX words.
-__device__ void sample_sort(uint64_t *key, int S)
-{
-    int P = 1;
-    while (P < S) P <<= 1;
-    for (int q = S + threadIdx.x; q < P; q += blockDim.x) key[q] = ~0ull;
-    __syncthreads();
-    for (int kk = 2; kk <= P; kk <<= 1)
-        for (int j = kk >> 1; j > 0; j >>= 1) {
-            for (int p = threadIdx.x; p < P / 2; p += blockDim.x) {
-                const int q = 2 * p - (p & (j - 1)), x = q | j;       // the p-th pair at distance j
-                const uint64_t a = key[q], b = key[x];
-                if ((a > b) == ((q & kk) == 0)) { key[q] = b; key[x] = a; }
-            }
-            __syncthreads();
-        }
-}
+constexpr int SMP_T = 1024, SMP_BINS = 4096, SMP_RANK = 64;
 struct sb_sample_kernel {
     static constexpr int LB = SMP_T, MB = 0;
     static __device__ __forceinline__ void run(KGrid kg_, const double *__restrict__ keysrc, const DevScalars *s, int B,
@@ -205,48 +181,54 @@ struct sb_sample_kernel {
 }
 };
 
-// The step's bucket of a star: its index among the old nodes, cut into B equal parts
-// (monotone in the new radius while the old radii ascend; when they do not, every star
-// goes to the last bucket, which its block splits).
-struct StepBucket {
-    double f;
-    int B;
-    bool unordered;
-    __device__ __forceinline__ StepBucket(int64_t n, int B_, bool un) : f((double)B_ / (double)(n + 1)), B(B_), unordered(un) {}
-    __device__ __forceinline__ uint32_t operator()(int32_t knew) const
-    {
-        if (knew < 0) return SB_TAIL;
-        const int b = (int)((double)knew * f);
-        return unordered || b >= B ? B - 1 : b;
-    }
-};
-
-// Tile histograms over the buckets (row `tile` of mat), the step's form.
+// Tile histograms over the buckets (row `tile` of mat), the step's form: buckets from the node
+// indices, or, where these would be uneven, from the radii as in sb_count_kernel (the
+// boundaries from memory: LDS for them would halve the blocks of the usual case).
 template <int BM>
 struct sb_count_step_kernel {
     static constexpr int LB = 1024, MB = 0;
     static __device__ __forceinline__ void run(KGrid kg_, const int32_t *__restrict__ knew, DevScalars *s,
-                                               const int32_t *__restrict__ bad, int B, uint32_t *__restrict__ mat)
+                                               const int32_t *__restrict__ uneven, int B, uint32_t *__restrict__ mat,
+                                               const double *__restrict__ keysrc, const uint64_t *__restrict__ split,
+                                               uint16_t *__restrict__ bkt)
 {
     __shared__ uint32_t hist[BM];
     const int t = threadIdx.x;
     const int64_t n = s->n_max_new;
     if (kg_.bid == 0 && t == 0) s->sort_in = n;
-    const StepBucket bucket(n, B, *bad != 0);
+    const StepBucket bucket(n, B);
     for (int b = t; b < B; b += 1024) hist[b] = 0;
     const int64_t chunk = tile_chunk(n, kg_.nb);
     const int64_t i0 = (int64_t)kg_.bid * chunk, i1 = i0 + chunk < n ? i0 + chunk : n;
     __syncthreads();
-    for (int64_t c = i0; c < i1; c += 4 * 1024) {
-        int32_t k[4];
-#pragma unroll
-        for (int u = 0; u < 4; u++) {                     // independent loads in flight
-            const int64_t i = c + u * 1024 + t;
-            k[u] = i < i1 ? knew[i + 1] : -1;
+    if (*uneven) {
+        for (int64_t i = i0 + t; i < i1; i += 1024) {
+            const double x = keysrc[i + 1];
+            const uint64_t k = sortable(x);
+            uint32_t b = SB_TAIL;
+            if (x < CMCG_SF_INFINITY) {                   // as the indices have it: not a NaN
+                b = 0;
+                for (int hi = B - 1; (int)b < hi;) {
+                    const int m = ((int)b + hi + 1) >> 1;
+                    if (split[m] <= k) b = m;
+                    else hi = m - 1;
+                }
+                atomicAdd(&hist[b], 1u);
+            }
+            bkt[i] = (uint16_t)b;
         }
+    } else {
+        for (int64_t c = i0; c < i1; c += 4 * 1024) {
+            int32_t k[4];
 #pragma unroll
-        for (int u = 0; u < 4; u++)
-            if (k[u] >= 0) atomicAdd(&hist[bucket(k[u])], 1u);
+            for (int u = 0; u < 4; u++) {                 // independent loads in flight
+                const int64_t i = c + u * 1024 + t;
+                k[u] = i < i1 ? knew[i + 1] : -1;
+            }
+#pragma unroll
+            for (int u = 0; u < 4; u++)
+                if (k[u] >= 0) atomicAdd(&hist[bucket(k[u])], 1u);
+        }
     }
     __syncthreads();
     for (int b = t; b < B; b += 1024) mat[(int64_t)kg_.bid * B + b] = hist[b];
@@ -343,7 +325,7 @@ struct sb_scan_kernel {
 // Records of W words: r, id, slot, then the first W - 3 payload fields.  A wave packs 64
 // stars at a time through its own LDS patch (odd stride: no bank conflicts), so whole
 // records leave in each store instruction; the next 64 stars' loads are in flight
-// meanwhile.  knew: the step's form (bkt is not read).  scanned: mat holds the tiles'
+// meanwhile.  knew: the step's form (bkt is read only where the indices would be uneven).  scanned: mat holds the tiles'
 // offsets and totals the bucket totals (sb_scan_kernel); otherwise both are formed here
 // from the raw histogram rows.  Bound by HBM: 500 MB in 112 us at N = 4e6.
 constexpr int SC_T = 512, SC_W = SC_T / 64;
@@ -353,7 +335,7 @@ struct sb_scatter_kernel {
     static __device__ __forceinline__ void run(KGrid kg_, const double *__restrict__ keysrc,
                                                const uint64_t *__restrict__ id, const DevScalars *s,
                                                const uint16_t *__restrict__ bkt, const int32_t *__restrict__ knew,
-                                               const int32_t *__restrict__ bad, const uint32_t *__restrict__ mat,
+                                               const int32_t *__restrict__ uneven, const uint32_t *__restrict__ mat,
                                                const uint32_t *__restrict__ totals, uint32_t *__restrict__ first, int B,
                                                int scanned, uint64_t *__restrict__ aos, GatherList g)
 {
@@ -407,13 +389,14 @@ struct sb_scatter_kernel {
     }
     const int64_t chunk = tile_chunk(n, nt);
     const int64_t i0 = (int64_t)tile * chunk, i1 = i0 + chunk < n ? i0 + chunk : n;
-    const StepBucket bucket(n, B, knew && *bad != 0);
+    const StepBucket bucket(n, B);
+    const bool by_index = knew && !*uneven;
     uint64_t v[NF], kr = 0, vid = 0;
     uint32_t bk = SB_TAIL;
     auto load = [&](int64_t i) {
         bk = SB_TAIL;
         if (i < i1) {
-            bk = knew ? bucket(knew[i + 1]) : bkt[i];
+            bk = by_index ? bucket(knew[i + 1]) : bkt[i];
             kr = (uint64_t)__double_as_longlong(keysrc[i + 1]);
             vid = id[i + 1];
 #pragma unroll
@@ -845,8 +828,8 @@ hipError_t sort_launch(const double *key_src, double *r_dst, const uint64_t *id_
                        hipStream_t st)
 {
     if (knew) {
-        kl<sb_count_step_kernel<BM>>(dim3((unsigned)sh.tiles), dim3(1024), 0, st, knew, s, (const int32_t *)sc.sort_bad,
-                                     sh.buckets, sc.sort_mat);
+        kl<sb_count_step_kernel<BM>>(dim3((unsigned)sh.tiles), dim3(1024), 0, st, knew, s, (const int32_t *)sc.sort_uneven,
+                                     sh.buckets, sc.sort_mat, key_src, (const uint64_t *)sc.sort_split, sc.sort_bkt);
     } else {
         kl<sb_sample_kernel>(dim3(1), dim3(SMP_T), 0, st, key_src, (const DevScalars *)s, sh.buckets, sc.sort_split);
         kl<sb_count_kernel<BM>>(dim3((unsigned)sh.tiles), dim3(1024), 0, st, key_src, s, (const uint64_t *)sc.sort_split,
@@ -857,7 +840,7 @@ hipError_t sort_launch(const double *key_src, double *r_dst, const uint64_t *id_
         kl<sb_scan_kernel>(dim3((unsigned)((sh.buckets + 63) / 64)), dim3(1024), 0, st, sc.sort_mat, sc.sort_tot,
                            sh.buckets, sh.tiles);
     kl<sb_scatter_kernel<W, BM>>(dim3((unsigned)sh.tiles), dim3(SC_T), 0, st, key_src, id_src, (const DevScalars *)s,
-                                 (const uint16_t *)sc.sort_bkt, knew, (const int32_t *)sc.sort_bad,
+                                 (const uint16_t *)sc.sort_bkt, knew, (const int32_t *)sc.sort_uneven,
                                  (const uint32_t *)sc.sort_mat, (const uint32_t *)sc.sort_tot, sc.sort_first, sh.buckets,
                                  scanned, sc.sort_aos, g);
     kl<sb_sort_kernel<W, CAP>>(dim3((unsigned)sh.buckets), dim3(BS_T), 0, st, s, (const uint32_t *)sc.sort_first,

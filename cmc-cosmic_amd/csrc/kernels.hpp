@@ -31,6 +31,45 @@ inline SortShape sort_shape(int64_t n_ub)
     sh.tiles = t < 1 ? 1 : t > most ? (int)most : (int)t;
     return sh;
 }
+constexpr uint16_t SB_TAIL = 0xffff;               // bucket number of a star of the SF_INFINITY tail
+constexpr uint64_t KEY_INF = 0x8000000000000000ull | 0x4202a05f20000000ull;   // sortable(1.0e10)
+__device__ __forceinline__ uint64_t sortable(double x)
+{
+    uint64_t b = (uint64_t)__double_as_longlong(x);
+    return (b >> 63) ? ~b : (b | 0x8000000000000000ull);
+}
+// The step's bucket of a star: its index among the old nodes, cut into B equal parts
+// (monotone in the new radius while the old radii ascend).
+struct StepBucket {
+    double f;
+    int B;
+    __device__ __forceinline__ StepBucket(int64_t n, int B_) : f((double)B_ / (double)(n + 1)), B(B_) {}
+    __device__ __forceinline__ uint32_t operator()(int32_t knew) const
+    {
+        if (knew < 0) return SB_TAIL;
+        const int b = (int)((double)knew * f);
+        return b >= B ? B - 1 : b;
+    }
+};
+// Bitonic sort of key[0, S) by the whole block; key holds SMP_MAX words.
+constexpr int SMP_MAX = 8192;          // stars sampled for bucket boundaries
+__device__ __forceinline__ void sample_sort(uint64_t *key, int S)
+{
+    int P = 1;
+    while (P < S) P <<= 1;
+    for (int q = S + threadIdx.x; q < P; q += blockDim.x) key[q] = ~0ull;
+    __syncthreads();
+    for (int kk = 2; kk <= P; kk <<= 1)
+        for (int j = kk >> 1; j > 0; j >>= 1) {
+            for (int p = threadIdx.x; p < P / 2; p += blockDim.x) {
+                const int q = 2 * p - (p & (j - 1)), x = q | j;       // the p-th pair at distance j
+                const uint64_t a = key[q], b = key[x];
+                if ((a > b) == ((q & kk) == 0)) { key[q] = b; key[x] = a; }
+            }
+            __syncthreads();
+        }
+}
+
 constexpr int RED2_BLOCKS = 64;
 
 constexpr int RIDX_TILE = 4096;     // buckets per block of the radial index's scan
@@ -59,7 +98,7 @@ struct Scratch {
     // sort
     uint32_t *vals_a;           // sorted permutation: slot of the star now at each position
     uint64_t *sort_split;       // bucket boundaries (order-preserving keys of r), SB_MAX_BUCKETS
-    int32_t *sort_bad;          // the radii that the orbit phase read do not ascend
+    int32_t *sort_uneven;       // the orbit phase's indices do not cut the stars into even buckets (1: its radii do not ascend, 2: counts)
     uint16_t *sort_bkt;         // bucket of every star
     uint32_t *sort_mat;         // tile histograms over the buckets
     size_t sort_mat_cap;
