@@ -517,7 +517,7 @@ int cmcg_create(cmcg_ctx **out, int device, int64_t n_cap, const cmcg_params *pa
         (e = dalloc(c, &sc.ridx_tb, (size_t)ridx_tiles(sc.ridx_bits) + 1))) { cmcg_destroy(c); return e; }
     if ((e = dalloc(c, &sc.tile_sums, (size_t)sc.max_tiles * 12)) || (e = dalloc(c, &sc.partials, (size_t)sc.max_blocks * 16)) ||
         (e = dalloc(c, &sc.sort_aos, (size_t)(n_cap + 4) * SORT_AOS_WORDS)) || (e = dalloc(c, &sc.sort_split, SB_MAX_BUCKETS)) ||
-        (e = dalloc(c, &sc.sort_uneven, 1)) || (e = dalloc(c, &sc.sort_bkt, (size_t)n_cap + 4)) ||
+        (e = dalloc(c, &sc.sort_uneven, 1)) || (e = dalloc(c, &sc.sort_moved, 1)) || (e = dalloc(c, &sc.sort_bkt, (size_t)n_cap + 4)) ||
         (e = dalloc(c, &sc.sort_mat, sc.sort_mat_cap)) || (e = dalloc(c, &sc.sort_tot, SB_MAX_BUCKETS)) ||
         (e = dalloc(c, &sc.sort_first, SB_MAX_BUCKETS + 1)) ||
         (e = dalloc(c, &sc.sort_order, 2 * (size_t)sc.sort_aos_cap)) ||

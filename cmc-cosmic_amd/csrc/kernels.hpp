@@ -98,6 +98,7 @@ struct Scratch {
     // sort
     uint32_t *vals_a;           // sorted permutation: slot of the star now at each position
     uint64_t *sort_split;       // bucket boundaries (order-preserving keys of r), SB_MAX_BUCKETS
+    int32_t *sort_moved;        // the general entry point: a star is out of order
     int32_t *sort_uneven;       // the orbit phase's indices do not cut the stars into even buckets (1: its radii do not ascend, 2: counts)
     uint16_t *sort_bkt;         // bucket of every star
     uint32_t *sort_mat;         // tile histograms over the buckets

@@ -192,3 +192,64 @@ def test_gpu_uneven_step_sorts_as_fast(gpu, kind):
             assert np.all(d["r"][1:m] <= d["r"][2:m + 1]) and np.unique(d["id"][1:m + 1]).size == m and m > 0.9 * n
     print("[gpu-test] sort ms", kind, ms, flush=True)
     assert ms[1] < 2.0
+
+
+@pytest.mark.parametrize("change", ["none", "tail", "tail inside", "ids", "first", "last", "tiles"])
+@pytest.mark.parametrize("n", [1, 2, 513, 16384, 131073, 700000])
+def test_gpu_sort_of_ordered_radii(gpu, n, change):
+    """Radii in order, which are only copied, and radii in order but for one star."""
+    cm = gpu
+    print("[gpu-test] ordered", n, change, flush=True)
+    rng = np.random.default_rng(n)
+    r = np.sort(np.round(rng.random(n) * n, 1)) + 0.5       # some ties
+    i = np.arange(n) - n // 3
+    if change.startswith("tail"):
+        r[n - n // 5:] = [1e10, np.inf, 2e10][n % 3]
+    if change == "tail inside" and n > 2:
+        r[n // 2] = 1e10
+    if change == "ids":
+        i = i[::-1].copy()
+    if change == "first":
+        r[0] = r[-1] + 1.0
+    if change == "last":
+        r[-1] = 0.25
+    if change == "tiles" and n > 600:                       # neighbours across a tile of 512 stars
+        r[511], r[512] = r[512] + 1e-3, r[511]
+    cl = cm.Cluster(n)
+    cl["r"][1:n + 1], cl["id"][1:n + 1] = r, i
+    for k in KEYS:
+        cl[k][1:n + 1] = rng.random(n)
+    order = 1 + np.lexsort((i, r))
+    order = order[cl["r"][order] < 1e10]
+    with cm.Context(n, cm.default_params(n)) as ctx:
+        ctx.upload(cl)
+        for _ in range(2):                                  # the second time in order
+            assert ctx.sort_by_r() == order.size
+            d = ctx.download()
+            for k in ("r", "id") + KEYS:
+                assert np.array_equal(d[k][1:order.size + 1], cl[k][order]), k
+
+
+def test_gpu_sort_of_ordered_radii_copies(gpu):
+    """Two thirds or less of the time for stars that move by a few places (which was 0.85 to 0.88
+    when the ordered ones went through records too)."""
+    cm = gpu
+    n = 2000000
+    cl = cm.make_plummer(n, seed=5)
+    p = np.argsort(np.arange(n) + 1e-3 * n * np.random.default_rng(2).standard_normal(n), kind="stable")
+    near = cl.copy()
+    for k in ("r", "id"):
+        near[k][1:n + 1] = cl[k][1:n + 1][p]
+    ms = []
+    with cm.Context(n, cm.default_params(n)) as ctx:
+        ctx.timer_enable(True)
+        for c in (cl, near):
+            t = []
+            for _ in range(6):
+                ctx.upload(c)
+                ctx.timer_reset()
+                ctx.sort_by_r()
+                t.append(ctx.timer_get("sort")[0])
+            ms.append(min(t))
+    print("[gpu-test] sort ms: ordered, moved", ms, flush=True)
+    assert ms[0] < 0.75 * ms[1]
