@@ -479,10 +479,11 @@ struct sv3_kernel {
     static __device__ __forceinline__ void run(KGrid kg_, DevFields f, DevScalars *s, KParams P, double *__restrict__ excess_c,
                                                  int64_t *__restrict__ blk_cnt, const double2 *__restrict__ mid,
                                                  const double2 *__restrict__ nodes, const double2 *__restrict__ u_old,
-                                                 const uint32_t *__restrict__ perm)
+                                                 const uint32_t *__restrict__ perm, int64_t *__restrict__ blk_events)
 {
-    __shared__ int cnt;
+    __shared__ int wcnt[GT / 64];
     __shared__ double cr[SV3_COARSE + 1];
+    bool event = false;
     const double q = 0.5;
     int64_t i = 1 + (int64_t)kg_.bid * blockDim.x + threadIdx.x;
     int64_t n = s->n_max;
@@ -492,7 +493,6 @@ struct sv3_kernel {
     C.stride = coarse_stride(n, SV3_COARSE);
     if (!u_old)      // the samples serve only the search for potential(rOld)
         for (int sI = threadIdx.x; sI <= SV3_COARSE; sI += blockDim.x) cr[sI] = f.r[coarse_k(C, sI)];
-    if (threadIdx.x == 0) cnt = 0;
     __syncthreads();
     if (i <= n) {
         double m = f.m[i], ri = f.r[i];
@@ -517,7 +517,7 @@ struct sv3_kernel {
         double vr = f.vr[i], vt = f.vt[i];
         if (vnew2 <= 0.0) {
             excess_c[i] = 0.5 * (sqr(vr) + sqr(vt) - vnew2) * m;
-            atomicAdd(&cnt, 1);
+            event = true;
         } else {
             excess_c[i] = -1.0;
             double alpha = sqrt(vnew2 / (sqr(vr) + sqr(vt)));
@@ -527,8 +527,18 @@ struct sv3_kernel {
             f.vrnew[i] = vr; f.vtnew[i] = vt;      // post-scaling values, read by the chain
         }
     }
+    const uint64_t bal = __ballot(event);
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    if (lane == 0) wcnt[w] = (int)__popcll(bal);
     __syncthreads();
+    int pos = 0, cnt = 0;
+    for (int q = 0; q < GT / 64; q++) {
+        if (q < w) pos += wcnt[q];
+        cnt += wcnt[q];
+    }
     if (threadIdx.x == 0) blk_cnt[kg_.bid] = cnt;
+    if (blk_events && event)               // a block's events from its first star's place on
+        blk_events[(int64_t)kg_.bid * GT + pos + __popcll(bal & ((1ull << lane) - 1ull))] = i;
 }
 };
 
@@ -646,14 +656,64 @@ __device__ int64_t excess_walk(const DevFields &f, const double *__restrict__ ex
     return n + 1;
 }
 
+// The same by a whole wave, unbounded: 64 stars' values at a time in its lanes, so that the
+// chain of additions waits on no memory.  Every lane returns the end.  (With the relinking of
+// 64 heads at a time, set_velocities3 with 1% / 30% of events: 2.15 -> 1.05 / 55 -> 16 ms at
+// N = 1e6, 0.31 -> 0.19 / 15 -> 4.6 at 3e5.)
+__device__ __forceinline__ double wave_value(double x, int lane)
+{
+    const long long b = __double_as_longlong(x);
+    const unsigned lo = __builtin_amdgcn_readlane((unsigned)b, lane), hi = __builtin_amdgcn_readlane((unsigned)(b >> 32), lane);
+    return __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
+}
+__device__ __forceinline__ int64_t wave_value(int64_t x, int lane)
+{
+    return __double_as_longlong(wave_value(__longlong_as_double(x), lane));
+}
+template <bool WRITE>
+__device__ __forceinline__ int64_t excess_walk_wave(const DevFields &f, const double *__restrict__ excess_c, int64_t i, int64_t n)
+{
+    const double E_dump_factor = 0.8;
+    const int lane = threadIdx.x & 63;
+    double Eexcess = 0.0;
+    for (; i <= n; i += 64) {
+        const int cnt = n - i < 63 ? (int)(n - i) + 1 : 64;
+        const int64_t k = i + (lane < cnt ? lane : cnt - 1);
+        const double c = excess_c[k], m = f.m[k], vr = f.vrnew[k], vt = f.vtnew[k];
+        const double v2 = sqr(vr) + sqr(vt);
+        const double capacity = E_dump_factor * 0.5 * m * v2;
+        double dumped = -1.0;                      // this lane's star: what it absorbs
+        int q = 0;
+        for (; q < cnt; q++) {
+            const double cq = wave_value(c, q);
+            if (cq >= 0.0) {
+                Eexcess += cq;
+            } else if (Eexcess > 0) {
+                const double cap = wave_value(capacity, q), E_dump = cap <= Eexcess ? cap : Eexcess;
+                if (lane == q) dumped = E_dump;
+                Eexcess -= E_dump;
+            }
+            if (!(Eexcess > 0)) break;
+        }
+        if (WRITE && dumped >= 0.0) {
+            const double exc_ratio = sqrt((v2 - 2 * dumped / m) / v2);
+            f.vr[k] = vr * exc_ratio;
+            f.vt[k] = vt * exc_ratio;
+        }
+        if (q < cnt) return i + q;
+    }
+    return n + 1;
+}
+
 // Fresh (no carried excess) bounded walk of every event.  joins[d] = 1 when that
 // walk reaches event d + 1 or was cut off, so event d + 1 is presumed to lie inside
 // the same episode.  An episode starting at a true head is exactly its fresh walk.
 __device__ __forceinline__ void sv3_spec(const DevFields &f, const double *__restrict__ excess_c, const int64_t *events,
-                                         int64_t *wend, int32_t *joins, int64_t n, int64_t ne, int64_t d0, int64_t stride)
+                                         int64_t *wend, int32_t *joins, int64_t n, int64_t ne, int64_t d0, int64_t stride,
+                                         int64_t max_steps = SPEC_WALK_MAX)
 {
     for (int64_t d = d0; d < ne; d += stride) {
-        int64_t e = excess_walk(f, excess_c, events[d], n, false, SPEC_WALK_MAX);
+        int64_t e = excess_walk(f, excess_c, events[d], n, false, max_steps);
         wend[d] = e;
         joins[d] = (e < 0) || (d + 1 < ne && e >= events[d + 1]);
     }
@@ -700,56 +760,82 @@ struct sv3_verify_kernel {
 // Exact head chain in event order: the next head is the first event after the end
 // of the current episode.  Runs only when a presumed head failed the check, and
 // starts at the first one that did: every presumed head before it passed, so by
-// induction it is a true head and the groups before it are exact.
+// induction it is a true head and the groups before it are exact.  One whole wave: 64 events
+// and the ends of their own walks in its lanes.
 __device__ __forceinline__ void sv3_relink(const DevFields &f, const double *__restrict__ excess_c, const int64_t *events,
-                                           const int64_t *wend, int32_t *joins, int64_t d, int64_t n, int64_t ne)
+                                           int64_t *wend, int32_t *joins, int64_t first, int64_t n, int64_t ne)
 {
-    while (d < ne) {
-        int64_t end = wend[d];
-        if (end < 0) end = excess_walk(f, excess_c, events[d], n, false, INT64_MAX);
-        int64_t d2 = d + 1;
-        while (d2 < ne && events[d2] <= end) joins[d2 - 1] = 1, d2++;
-        if (d2 < ne) joins[d2 - 1] = 0;
-        d = d2;
+    const int lane = threadIdx.x & 63;
+    int64_t end = -1;                              // of the episode in hand
+    for (int64_t base = first; base < ne; base += 64) {
+        const bool live = base + lane < ne;
+        const int64_t ev = live ? events[base + lane] : INT64_MAX, we = live ? wend[base + lane] : 0;
+        const int cnt = ne - base < 64 ? (int)(ne - base) : 64;
+        uint64_t heads = 0;
+        for (int l = 0;; l++) {
+            l += (int)__popcll(__ballot(lane >= l && ev <= end));      // the next events up to its end
+            if (l >= cnt) break;
+            heads |= 1ull << l;
+            end = wave_value(we, l);
+            if (end < 0) {
+                end = excess_walk_wave<false>(f, excess_c, wave_value(ev, l), n);
+                if (lane == l) wend[base + l] = end;
+            }
+        }
+        if (live && base + lane > first) joins[base + lane - 1] = (heads >> lane) & 1 ? 0 : 1;
     }
 }
 struct sv3_relink_kernel {
     static constexpr int LB = 1024, MB = 0;
     static __device__ __forceinline__ void run(KGrid kg_, DevFields f, DevScalars *s, const double *__restrict__ excess_c,
-                                  const int64_t *__restrict__ events, const int64_t *__restrict__ wend,
+                                  const int64_t *__restrict__ events, int64_t *__restrict__ wend,
                                   int32_t *__restrict__ joins, const int64_t *__restrict__ relink)
 {
-    if (threadIdx.x != 0 || kg_.bid != 0) return;
     sv3_relink(f, excess_c, events, wend, joins, *relink, s->n_max, s->n_excess);
 }
 };
 
-// every head walks its episode and writes the dumped velocities
+// Every head walks its episode and writes the dumped velocities: short episodes a thread
+// each, the long ones a wave (every wave of the block calls; d0: the thread's first event).
+constexpr int64_t LONG_EPISODE = 256;
 __device__ __forceinline__ void sv3_heads(const DevFields &f, const double *__restrict__ excess_c, const int64_t *events,
-                                          const int32_t *joins, int64_t n, int64_t ne, int64_t d0, int64_t stride)
+                                          const int32_t *joins, const int64_t *wend, int64_t n, int64_t ne, int64_t d0,
+                                          int64_t stride)
 {
-    for (int64_t d = d0; d < ne; d += stride)
-        if (d == 0 || !joins[d - 1]) excess_walk(f, excess_c, events[d], n, true, INT64_MAX);
+    const int lane = threadIdx.x & 63;
+    for (int64_t d = d0; d - lane < ne; d += stride) {     // wave-uniform
+        const bool head = d < ne && (d == 0 || !joins[d - 1]);
+        const int64_t i = head ? events[d] : 0;
+        const bool lng = head && (wend[d] < 0 || wend[d] - i >= LONG_EPISODE);
+        if (head && !lng) excess_walk(f, excess_c, i, n, true, INT64_MAX);
+        for (uint64_t todo = __ballot(lng); todo; todo &= todo - 1) {
+            const int src = __ffsll((unsigned long long)todo) - 1;
+            excess_walk_wave<true>(f, excess_c, wave_value(i, src), n);
+        }
+    }
 }
 struct sv3_heads_kernel {
     static constexpr int LB = 1024, MB = 0;
     static __device__ __forceinline__ void run(KGrid kg_, DevFields f, DevScalars *s, const double *__restrict__ excess_c,
-                                 const int64_t *__restrict__ events, const int32_t *__restrict__ joins)
+                                 const int64_t *__restrict__ events, const int32_t *__restrict__ joins,
+                                 const int64_t *__restrict__ wend)
 {
-    sv3_heads(f, excess_c, events, joins, s->n_max, s->n_excess, (int64_t)kg_.bid * blockDim.x + threadIdx.x,
+    sv3_heads(f, excess_c, events, joins, wend, s->n_max, s->n_excess, (int64_t)kg_.bid * blockDim.x + threadIdx.x,
               (int64_t)kg_.nb * blockDim.x);
 }
 };
 
 // The excess chain after sv3_kernel (the count of events, their ordered list, and the four
 // kernels on it above) in one block for a cluster of at most SV3_ONE stars: six launches of
-// 1 to 4 us with gaps as long.  Wave w lists the events of sv3_kernel's blocks w, w + 16, ...
+// 1 to 4 us with gaps as long.  The list comes from those of sv3_kernel's blocks.  (Without
+// events set_velocities3 takes 47 us at N = 6e4, 75 by the launches; with 1% of them 70 / 75,
+// with 30% 7.1 / 7.4 ms.)
 constexpr int64_t SV3_ONE = 65536;
 struct sv3_one_kernel {
     static constexpr int LB = 1024, MB = 0;
     static __device__ __forceinline__ void run(KGrid kg_, DevFields f, DevScalars *s, const double *__restrict__ excess_c,
                                                const int64_t *__restrict__ blk_cnt, int nb, int64_t *events, int64_t *wend,
-                                               int32_t *joins)
+                                               int32_t *joins, const int64_t *__restrict__ blk_events)
 {
     constexpr int NB = SV3_ONE / GT, NW = NB / 64;     // as many waves scan the counts
     __shared__ int off[NB + 1], wtot[NW];
@@ -773,6 +859,7 @@ struct sv3_one_kernel {
         if (q == w && t < NB) off[t] += ne;
         ne += wtot[q];
     }
+    ne = __builtin_amdgcn_readfirstlane(ne);       // scalars: the walks' branches depend on them
     if (t == 0) {
         off[NB] = ne;
         s->n_excess = ne;
@@ -780,28 +867,29 @@ struct sv3_one_kernel {
     }
     if (ne == 0) return;
     __syncthreads();
-    for (int b = w; b < nb; b += 16) {
-        int pos = off[b];
-        if (pos == off[b + 1]) continue;
-        for (int q = 0; q < GT; q += 64) {
-            const int64_t i = 1 + (int64_t)b * GT + q + lane;
-            const bool ev = i <= n && excess_c[i] >= 0.0;
-            const uint64_t bal = __ballot(ev);
-            if (ev) events[pos + __popcll(bal & ((1ull << lane) - 1ull))] = i;
-            pos += (int)__popcll(bal);
+    for (int e = t; e < ne; e += 1024) {           // event e is number e - off[b] of its block b
+        int b = 0, hi = nb - 1;
+        while (b < hi) {
+            const int m = (b + hi + 1) >> 1;
+            if (off[m] <= e) b = m;
+            else hi = m - 1;
         }
+        events[e] = blk_events[(int64_t)b * GT + (e - off[b])];
     }
     __threadfence_block();
     __syncthreads();
-    sv3_spec(f, excess_c, events, wend, joins, n, ne, t, 1024);
+    // one compute unit's walks share its loads: with more events than threads they are cut off
+    // sooner, and the exact chain goes on from there
+    const int per = (ne + 1023) / 1024;
+    sv3_spec(f, excess_c, events, wend, joins, n, ne, t, 1024, per > 1 ? SPEC_WALK_MAX / 8 / per : SPEC_WALK_MAX);
     __threadfence_block();
     __syncthreads();
     sv3_verify(events, joins, wend, &relink, ne, t, 1024);
     __syncthreads();
-    if (t == 0) sv3_relink(f, excess_c, events, wend, joins, relink, n, ne);
+    if (t < 64) sv3_relink(f, excess_c, events, wend, joins, wave_value(relink, 0), n, ne);
     __threadfence_block();
     __syncthreads();
-    sv3_heads(f, excess_c, events, joins, n, ne, t, 1024);
+    sv3_heads(f, excess_c, events, joins, wend, n, ne, t, 1024);
 }
 };
 
@@ -926,12 +1014,15 @@ hipError_t launch_set_velocities3(const DevFields &f, DevScalars *s, const KPara
         kl<old_node_potential_kernel>(dim3((unsigned)mb), dim3(MERGE_T), 0, st, r_old_sorted,
                                       (const double2 *)sc.nodes, s, sc.u_old, dpre);
     }
+    // (the sort's records are free here)
+    int64_t *blk_events = reinterpret_cast<int64_t *>(sc.sort_aos);
     kl<sv3_kernel>(dim3((unsigned)nb), dim3(GT), 0, st, f, s, P, sc.excess_c, sc.sv3_blk,
                        (const double2 *)sc.mid, (const double2 *)sc.nodes,
-                       r_old_sorted ? (const double2 *)sc.u_old : nullptr, (const uint32_t *)sc.vals_a);
+                       r_old_sorted ? (const double2 *)sc.u_old : nullptr, (const uint32_t *)sc.vals_a,
+                       n_ub <= SV3_ONE ? blk_events : (int64_t *)nullptr);
     if (n_ub <= SV3_ONE) {
         kl<sv3_one_kernel>(dim3(1), dim3(1024), 0, st, f, s, (const double *)sc.excess_c, (const int64_t *)sc.sv3_blk, (int)nb,
-                           sc.excess_list, sc.sv3_wend, sc.sv3_merged);
+                           sc.excess_list, sc.sv3_wend, sc.sv3_merged, (const int64_t *)blk_events);
         return hipGetLastError();
     }
     kl<sv3_scan_kernel>(dim3(1), dim3(1024), 0, st, s, sc.sv3_blk, nb, sc.sv3_fallback);
@@ -942,10 +1033,9 @@ hipError_t launch_set_velocities3(const DevFields &f, DevScalars *s, const KPara
     kl<sv3_verify_kernel>(dim3(ge), dim3(GT), 0, st, s, (const int64_t *)sc.excess_list,
                        (const int32_t *)sc.sv3_merged, (const int64_t *)sc.sv3_wend, sc.sv3_fallback);
     kl<sv3_relink_kernel>(dim3(1), dim3(64), 0, st, f, s, (const double *)sc.excess_c,
-                       (const int64_t *)sc.excess_list, (const int64_t *)sc.sv3_wend, sc.sv3_merged,
-                       (const int64_t *)sc.sv3_fallback);
+                       (const int64_t *)sc.excess_list, sc.sv3_wend, sc.sv3_merged, (const int64_t *)sc.sv3_fallback);
     kl<sv3_heads_kernel>(dim3(ge), dim3(GT), 0, st, f, s, (const double *)sc.excess_c,
-                       (const int64_t *)sc.excess_list, (const int32_t *)sc.sv3_merged);
+                       (const int64_t *)sc.excess_list, (const int32_t *)sc.sv3_merged, (const int64_t *)sc.sv3_wend);
     return hipGetLastError();
 }
 hipError_t launch_compute_energy(const DevFields &f, DevScalars *s, const KParams &P, const Scratch &sc,
