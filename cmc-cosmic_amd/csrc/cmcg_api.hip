@@ -502,7 +502,6 @@ int cmcg_create(cmcg_ctx **out, int device, int64_t n_cap, const cmcg_params *pa
     if ((e = dalloc(c, &c->s, 1))) { cmcg_destroy(c); return e; }
     Scratch &sc = c->sc;
     sc.max_tiles = (n_cap + 2047) / 2048 + 1;
-    sc.esa_max = 1 << 16;
     sc.max_blocks = (n_cap + 127) / 128 + 2;      // the smallest block of any launch shape: 128 threads
     if (sc.max_blocks < 1024) sc.max_blocks = 1024;   // the stripping passes' fixed grid
     const SortShape sort_max = sort_shape(n_cap);
@@ -530,9 +529,7 @@ int cmcg_create(cmcg_ctx **out, int device, int64_t n_cap, const cmcg_params *pa
         (e = dalloc(c, &sc.strip_done, 1)) || (e = dalloc(c, &sc.chain_x, (size_t)n_cap + 8)) ||
         (e = dalloc(c, &sc.defer_list, (size_t)P.defer_cap)) || (e = dalloc(c, &sc.defer_kfirst, (size_t)P.defer_cap)) || (e = dalloc(c, &sc.defer_order, (size_t)P.defer_cap)) ||
         (e = dalloc(c, &sc.chain_scal, 4)) || (e = dalloc(c, &sc.chain_fbad, 8)) ||
-        (e = dalloc(c, &sc.esa_idx, (size_t)sc.esa_max)) || (e = dalloc(c, &sc.esa_racc, (size_t)sc.esa_max)) ||
-        (e = dalloc(c, &sc.esa_v, (size_t)sc.esa_max)) || (e = dalloc(c, &sc.esa_n, 8)) ||
-        (e = dalloc(c, &sc.esa_raw_idx, 2 * 2048)) || (e = dalloc(c, &sc.esa_raw_part, 2 * 3 * 2048)) ||
+        (e = dalloc(c, &sc.esa_n, 8)) ||
         (e = dalloc(c, &sc.rng_base, 3)) || (e = dalloc(c, &sc.rng_seeded, 1)) ||
         (e = dalloc(c, &c->T, 1))) {
         cmcg_destroy(c);

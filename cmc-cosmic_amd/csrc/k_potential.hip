@@ -65,12 +65,13 @@ struct EsaArgs {
     double *s_v;                // chain value after the element
     int64_t *s_n;               // count (uncapped)
     int64_t smax;               // capacity
-    // appended by the classification in any order (RAW_CAP entries): index, regular sum
+    // appended by the classification in any order (raw_cap entries): index, regular sum
     // since the previous sensitive element of its tile (or the tile start), binade
-    // before it
+    // before it (raw_bp), its number among the tile's (raw_bp + raw_cap) and its s x
     int64_t *raw_n, *raw_idx, *raw_part;
     int32_t *raw_bp;
-    double *raw_sx;                         // s x of the element
+    double *raw_sx;
+    int64_t raw_cap;
 };
 
 // A run of elements: regular sum after its last sensitive element (all of it when it
@@ -449,17 +450,20 @@ __device__ __forceinline__ bool classify_tile(const EsaArgs &a, const double (&v
         a.ttail[tile] = tot.sum;
     }
     if (!it.sens) return ok;
-    int64_t cur = pre.sum;
+    int64_t cur = pre.sum, k = pre.cnt;
     const int64_t j0 = tile * CTILE + (int64_t)threadIdx.x * CI;
+    int64_t slot = (int64_t)atomicAdd((unsigned long long *)a.raw_n, (unsigned long long)__popc(it.sens));
     for (int u = 0; u < CI; u++) {
         if ((it.sens >> u) & 1) {
-            const unsigned long long slot = atomicAdd((unsigned long long *)a.raw_n, 1ull);
-            if (slot < (unsigned long long)RAW_CAP) {
+            if (slot < a.raw_cap) {
                 a.raw_idx[slot] = j0 + u;
                 a.raw_part[slot] = cur;
                 a.raw_bp[slot] = it.bp[u];
+                a.raw_bp[a.raw_cap + slot] = (int32_t)k;
                 a.raw_sx[slot] = it.sx[u];
             }
+            slot++;
+            k++;
             cur = 0;
         } else {
             cur += it.R[u];
@@ -596,25 +600,20 @@ __device__ Seg walk_scan(const EsaArgs &a, int64_t nt, Seg *lds)
 // LDS of the walk: the appended list put in order
 struct WalkLds {
     Seg s[CT / 64];
-    int64_t idx[RAW_CAP];
     double pre[RAW_CAP], sx[RAW_CAP];
 };
 
-// The appended list (ns <= RAW_CAP entries) put in order by index.
-__device__ void walk_list(const EsaArgs &a, int64_t ns, WalkLds &sh)
+// The appended list (ns entries) put in order, by a group of CT threads: an element's place is
+// its tile's offset and its number there.
+__device__ void walk_list(const EsaArgs &a, int64_t ns, double *pre, double *sx)
 {
-    const int t = threadIdx.x % CT;
-    for (int64_t e = t; e < ns; e += CT) sh.idx[e] = a.raw_idx[e];
-    __syncthreads();
-    for (int64_t e = t; e < ns; e += CT) {
-        const int64_t j = sh.idx[e];
-        int64_t rank = 0;
-        for (int64_t q = 0; q < ns; q++) rank += sh.idx[q] < j;      // the indices are distinct
-        const int64_t tile = j / CTILE;
-        const int64_t pre = a.raw_part[e] + (rank == a.toff[tile] ? a.tcarry[tile] : 0);
-        a.s_idx[rank] = j;
-        sh.pre[rank] = seg_value(pre, a.raw_bp[e]);
-        sh.sx[rank] = a.raw_sx[e];
+    for (int64_t e = threadIdx.x % CT; e < ns; e += CT) {
+        const int64_t j = a.raw_idx[e], tile = j / CTILE;
+        const int32_t k = a.raw_bp[a.raw_cap + e];
+        const int64_t at = a.toff[tile] + k;
+        if (a.s_idx) a.s_idx[at] = j;
+        pre[at] = seg_value(a.raw_part[e] + (k == 0 ? a.tcarry[tile] : 0), a.raw_bp[e]);
+        sx[at] = a.raw_sx[e];
     }
     __syncthreads();
 }
@@ -663,7 +662,7 @@ struct esa_walk_kernel {
         esa_walk_block(a, ns, nullptr, nullptr);
         return;
     }
-    walk_list(a, ns, sh);
+    walk_list(a, ns, sh.pre, sh.sx);
     esa_walk_block(a, ns, sh.pre, sh.sx);
 }
 };
@@ -822,8 +821,7 @@ struct PotArgs {
     double *xc;                 // chain C's increments
     double *scal;               // [0] 0.0 (C's start), [1] Mtotal (B's start), [2] its estimate
     // nonzero: the chains go through the repair.  A kernel reads only the words that earlier
-    // kernels set: [0] classification and [1] lists of A and B, [2] rebuild of B, [3] list
-    // and [4] rebuild of C
+    // kernels set: [0] classification of A and B, [1] rebuild of B, [2] rebuild of C
     int64_t *flag;
     double2 *nodes, *mid;       // packed (r, phi) of every node and of every MID_STEP-th
     int counted;                // N_MAX from the count of radii below SF_INFINITY (pot_count_kernel)
@@ -863,7 +861,7 @@ struct pot_sums_kernel {
     if (kg_.bid == 0 && threadIdx.x == 0) {
         if (p.counted) p.s->n_max = n;               // the other blocks read first_inf
         p.scal[0] = 0.0;
-        for (int q = 0; q < 5; q++) p.flag[q] = 0;
+        for (int q = 0; q < 3; q++) p.flag[q] = 0;
         *p.a.raw_n = 0;
         *p.b.raw_n = 0;
         *p.c.raw_n = 0;
@@ -933,18 +931,29 @@ __device__ __forceinline__ double lane_value(double x, int lane)
 
 // The walk over ns listed elements from v, by one whole wave: 64 elements at a time in
 // its lanes' registers, so that the chain of additions waits on no memory.  s_v (which may
-// be pre or sx) receives the value after each element; every lane returns the last.
+// be pre or sx) receives the value after each element; every lane returns the last.  (Adding a
+// run of nothing, 0.0, changes no value that is not -0.0, and the chains hold none.)
 __device__ __forceinline__ double pot_walk(int64_t ns, double v, const double *pre, const double *sx, double *s_v)
 {
     const int lane = threadIdx.x & 63;
+    double np = lane < ns ? pre[lane] : 0.0, nx = lane < ns ? sx[lane] : 0.0;
     for (int64_t c = 0; c < ns; c += 64) {
         const int cnt = (int)(ns - c < 64 ? ns - c : 64);
-        const double p = lane < cnt ? pre[c + lane] : 0.0, x = lane < cnt ? sx[c + lane] : 0.0;
+        const double p = np, x = nx;
+        if (c + 64 + lane < ns) {                     // the next 64, while these are walked
+            np = pre[c + 64 + lane];
+            nx = sx[c + 64 + lane];
+        }
         double mine = 0.0;
-        for (int k = 0; k < cnt; k++) {
-            const double pk = lane_value(p, k), pred = pk == 0.0 ? v : v + pk;
-            v = pred + lane_value(x, k);
+        auto step = [&](int k) {
+            v = (v + lane_value(p, k)) + lane_value(x, k);
             if (lane == k) mine = v;
+        };
+        if (cnt == 64) {
+#pragma unroll 16
+            for (int k = 0; k < 64; k++) step(k);
+        } else {
+            for (int k = 0; k < cnt; k++) step(k);
         }
         if (lane < cnt) s_v[c + lane] = mine;
     }
@@ -978,16 +987,23 @@ struct pot_walk_ab_kernel {
     const Seg mine = walk_scan(c, nt, sh[h].s);
     if (threadIdx.x % CT == 0) tot[h] = mine;
     __syncthreads();
-    if (tot[0].cnt > RAW_CAP || tot[1].cnt > RAW_CAP) {
-        if (threadIdx.x == 0) p.flag[1] = 1;
-        return;
+    // lists longer than LDS holds go through memory, one after the other
+    const bool lds = tot[0].cnt <= RAW_CAP && tot[1].cnt <= RAW_CAP;
+    double *pa = lds ? sh[0].pre : p.b.s_pre, *xa = lds ? sh[0].sx : p.b.s_v;
+    double *pb = lds ? sh[1].pre : p.b.s_pre, *xb = lds ? sh[1].sx : p.b.s_v;
+    if (lds) walk_list(c, mine.cnt, h ? pb : pa, h ? xb : xa);
+    else walk_list(p.a, h ? 0 : tot[0].cnt, pa, xa);
+    double v = 0.0;                                   // chain A's last value (wave 0)
+    if (threadIdx.x < 64) {
+        v = pot_walk(tot[0].cnt, 0.0, pa, xa, xa);
+        if (tot[0].sum != 0) v += seg_value(tot[0].sum, binade_of(v));   // the run after the last stays in one binade
+        if (threadIdx.x == 0) pot_total(p, P, v);
     }
-    walk_list(c, mine.cnt, sh[h]);
-    if (threadIdx.x >= 64) return;
-    double v = pot_walk(tot[0].cnt, 0.0, sh[0].pre, sh[0].sx, sh[0].pre);
-    if (tot[0].sum != 0) v += seg_value(tot[0].sum, binade_of(v));   // the run after the last stays in one binade
-    if (threadIdx.x == 0) pot_total(p, P, v);
-    pot_walk(tot[1].cnt, pot_mass(P, v), sh[1].pre, sh[1].sx, p.b.s_v);
+    if (!lds) {
+        __syncthreads();
+        walk_list(p.b, h ? tot[1].cnt : 0, pb, xb);
+    }
+    if (threadIdx.x < 64) pot_walk(tot[1].cnt, pot_mass(P, v), pb, xb, p.b.s_v);
 }
 };
 
@@ -1003,7 +1019,7 @@ struct pot_rebuild_b_kernel {
     const int64_t n = p.s->n_max;
     const int64_t tile = kg_.bid, base = tile * CTILE;
     const int t = threadIdx.x;
-    if (base >= n || p.flag[0] || p.flag[1]) return;
+    if (base >= n || p.flag[0]) return;
     EsaArgs b = p.b;
     b.extra = n;
     const int64_t lb = p.lb(n);
@@ -1018,7 +1034,7 @@ struct pot_rebuild_b_kernel {
     TileItems it;
     double nv[CI], before;
     const int64_t bad = rebuild_tile(b, v, tile, lb, p.scal[2], p.scal[1], b.s_v, *b.s_n, sh, it, nv, &before);
-    if (bad < lb) p.flag[2] = 1;
+    if (bad < lb) p.flag[1] = 1;
     // 1/r_k - 1/r_{k+1} of the tile through LDS
     __syncthreads();                                  // tbuf free
 #pragma unroll
@@ -1042,7 +1058,7 @@ struct pot_classify_c_kernel {
 {
     __shared__ ChainLds sh;
     const int64_t n = p.s->n_max, tile = kg_.bid;
-    if (tile * CTILE >= n || p.flagged(3)) return;
+    if (tile * CTILE >= n || p.flagged(2)) return;
     double v[CI], pre_t, pre_t1;
     fetch_tile(ArraySrc{p.xc}, tile * CTILE, n, v);
     get_prefixes(p.c, tile, self_prefix, sh.d, &pre_t, &pre_t1);
@@ -1055,15 +1071,13 @@ struct pot_walk_c_kernel {
     static __device__ __forceinline__ void run(KGrid kg_, PotArgs p)
 {
     __shared__ WalkLds sh;
-    if (p.flagged(3)) return;
+    if (p.flagged(2)) return;
     Seg tot;
     tot = walk_scan(p.c, (p.s->n_max + CTILE - 1) / CTILE, sh.s);
-    if (tot.cnt > RAW_CAP) {
-        if (threadIdx.x == 0) p.flag[3] = 1;
-        return;
-    }
-    walk_list(p.c, tot.cnt, sh);
-    if (threadIdx.x < 64) pot_walk(tot.cnt, 0.0, sh.pre, sh.sx, p.c.s_v);
+    const bool lds = tot.cnt <= RAW_CAP;
+    double *pre = lds ? sh.pre : p.c.s_pre, *sx = lds ? sh.sx : p.c.s_v;
+    walk_list(p.c, tot.cnt, pre, sx);
+    if (threadIdx.x < 64) pot_walk(tot.cnt, 0.0, pre, sx, p.c.s_v);
 }
 };
 
@@ -1093,7 +1107,7 @@ struct pot_rebuild_c_kernel {
     const int64_t n = p.s->n_max;
     const int64_t tile = kg_.bid, base = tile * CTILE;
     const int t = threadIdx.x;
-    if (p.flagged(4)) return;
+    if (p.flagged(2)) return;
     if (n == 0 && kg_.bid == 0 && t == 0) put_ends(p, P, n, 0.0);
     if (base >= n) return;
     TileItems it;
@@ -1105,7 +1119,7 @@ struct pot_rebuild_c_kernel {
         rk[u] = j < n ? p.r[n - j] : 1.0;
     }
     const int64_t bad = rebuild_tile(p.c, v, tile, n, 0.0, 0.0, p.c.s_v, *p.c.s_n, sh, it, nv, &before);
-    if (bad < n) p.flag[4] = 1;
+    if (bad < n) p.flag[2] = 1;
     __syncthreads();                                  // tbuf free
 #pragma unroll
     for (int u = 0; u < CI; u++) sh.tbuf[tile_slot(t * CI + u)] = nv[u];
@@ -1124,8 +1138,8 @@ struct pot_rebuild_c_kernel {
 }
 };
 
-// The repair (a mass below zero, infinite or NaN, a list beyond RAW_CAP, a violated
-// recurrence: never an ordinary cluster; the test hook forces it): the three recurrences
+// The repair (a mass below zero, infinite or NaN, a violated recurrence: never an ordinary
+// cluster; the test hook forces it): the three recurrences
 // themselves, one thread over chunks that the block stages through LDS.
 constexpr int FIX_CHUNK = 2 * WALK_T;
 struct pot_finish_kernel {
@@ -1134,7 +1148,7 @@ struct pot_finish_kernel {
 {
     __shared__ double x[FIX_CHUNK], y[FIX_CHUNK];
     __shared__ double va, vm;
-    if (!p.flagged(5)) return;
+    if (!p.flagged(3)) return;
     const int64_t n = p.s->n_max;
     const int t = threadIdx.x;
     if (t == 0) va = 0.0;
@@ -1289,11 +1303,13 @@ EsaArgs report_chain0(const Scratch &sc, int slack, void *work, int64_t xs)
     e.raw_part = (int64_t *)(w + RAW_CAP);
     e.raw_bp = (int32_t *)(e.raw_part + RAW_CAP);
     e.raw_sx = (double *)(e.raw_part + 2 * RAW_CAP);
+    e.raw_cap = RAW_CAP;
     return e;
 }
 
-// The chains' per-tile and list buffers in the context's scratch (tile_sums: six
-// 8-byte words per tile).
+// The chains' per-tile buffers in the context's scratch (tile_sums: six 8-byte words per tile),
+// their lists, of as many elements as there are stars, in the sort's records (free between
+// sorts: 11 of their 16 words a star).
 // set: 0 or 1, for two chains that are classified together
 EsaArgs esa_args(const Scratch &sc, int slack, int set = 0)
 {
@@ -1307,16 +1323,19 @@ EsaArgs esa_args(const Scratch &sc, int slack, int set = 0)
     e.ttail = (int64_t *)(tb + 3 * T);
     e.toff = (int64_t *)(tb + 4 * T);
     e.tcarry = (int64_t *)(tb + 5 * T);
-    e.s_idx = sc.esa_idx;
-    e.s_pre = sc.esa_racc;
-    e.s_v = sc.esa_v;
     e.s_n = sc.esa_n;
-    e.smax = sc.esa_max;
     e.raw_n = sc.esa_n + 1 + set;
-    e.raw_idx = sc.esa_raw_idx + RAW_CAP * set;
-    e.raw_part = (int64_t *)sc.esa_raw_part + 3 * RAW_CAP * set;
-    e.raw_bp = (int32_t *)(e.raw_part + RAW_CAP);
-    e.raw_sx = (double *)(e.raw_part + 2 * RAW_CAP);
+    const int64_t cap = sc.sort_aos_cap;
+    double *w = (double *)sc.sort_aos;
+    e.smax = e.raw_cap = cap;
+    e.s_idx = (int64_t *)w;
+    e.s_pre = w + cap;
+    e.s_v = w + 2 * cap;
+    w += (3 + 4 * set) * cap;
+    e.raw_idx = (int64_t *)w;
+    e.raw_part = (int64_t *)(w + cap);
+    e.raw_bp = (int32_t *)(w + 2 * cap);
+    e.raw_sx = w + 3 * cap;
     return e;
 }
 } // namespace
@@ -1448,7 +1467,8 @@ hipError_t launch_potential(const DevFields &f, DevScalars *s, const KParams &P,
     p.b.sign = -1.0;
     p.c = p.a;                                       // A's tile sums and list are free when C needs its own
     p.c.raw_n = sc.esa_n + 3;
-    p.a.s_n = sc.esa_n + 4; p.a.s_idx = sc.esa_idx + RAW_CAP;   // walked at the same time as B's
+    p.a.s_n = sc.esa_n + 4;                          // walked at the same time as B's, for its last value alone
+    p.a.s_idx = nullptr;
     const dim3 gt((unsigned)ntiles), bt(CT);
     const int self_prefix = ntiles <= SELF_PREFIX_MAX;
     if (count) {

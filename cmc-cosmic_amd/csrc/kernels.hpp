@@ -84,14 +84,7 @@ struct Scratch {
     double *chain_x;
     double *chain_scal;         // 4 doubles
     int64_t *chain_fbad;        // 6
-    // potential chains: list of sensitive elements (index, int128 prefix, value)
-    int64_t *esa_idx;
-    double *esa_racc;           // regular sum before each listed element
-    double *esa_v;
     int64_t *esa_n;             // [0] sensitive count, [1]..[3] appended counts, [4] the total mass chain's [0]
-    int64_t *esa_raw_idx;       // appended sensitive elements (unordered), 2048 for each set
-    double *esa_raw_part;       // their in-tile regular sums (int64), binades (int32) and s x
-    int64_t esa_max;
     // deterministic block partials: 8 doubles per block
     double *partials;
     int64_t max_blocks;
