@@ -507,11 +507,12 @@ int cmcg_create(cmcg_ctx **out, int device, int64_t n_cap, const cmcg_params *pa
     const SortShape sort_max = sort_shape(n_cap);
     sc.sort_mat_cap = (size_t)sort_max.tiles * sort_max.buckets;
     sc.sort_aos_cap = n_cap + 4;
-    // about two radial-index buckets per star: 2^10 .. 2^23 buckets (at N = 4e6 one per
-    // star makes the orbit sampler 3% slower; four per star cost more to build than the
-    // sampler gains)
+    // about two radial-index buckets per star (at N = 4e6 one per star makes the orbit
+    // sampler 3% slower; four per star cost more to build than the sampler gains).  A limit of
+    // 2^23 buckets, about 4e6 stars' worth, left a crowded bucket's nodes to be bisected: the
+    // orbit phase 7.8 -> 4.7 ms at N = 1.8e7 without it, 22.0 -> 11.0 at 3.6e7.
     sc.ridx_bits = 10;
-    while (sc.ridx_bits < 23 && ((int64_t)1 << sc.ridx_bits) < 2 * (n_cap + 2)) sc.ridx_bits++;
+    while (sc.ridx_bits < 30 && ((int64_t)1 << sc.ridx_bits) < 2 * (n_cap + 2)) sc.ridx_bits++;
     if ((e = dalloc(c, &sc.ridx, (size_t)ridx_entries(sc.ridx_bits))) ||
         (e = dalloc(c, &sc.ridx_tb, (size_t)ridx_tiles(sc.ridx_bits) + 1))) { cmcg_destroy(c); return e; }
     if ((e = dalloc(c, &sc.tile_sums, (size_t)sc.max_tiles * 12)) || (e = dalloc(c, &sc.partials, (size_t)sc.max_blocks * 16)) ||
