@@ -251,11 +251,9 @@ struct SortSpec {
     uint64_t *dst[24];
     double **swap_a[24];
     double **swap_b[24];
-    int64_t **swap_ia = nullptr, **swap_ib = nullptr;
 };
 
-// fa, fb: the live/alternate pointer pair swapped after the sort (null for a scratch
-// array that the sort writes into a fixed destination)
+// fa, fb: the live/alternate pointer pair swapped after the sort
 void add_field(SortSpec &sp, double *src, double *dst, double **fa, double **fb)
 {
     sp.src[sp.nf] = (const uint64_t *)src;
@@ -298,21 +296,18 @@ static void swap_sorted(cmcg_ctx *c, const SortSpec &sp)
 {
     std::swap(c->f.r, c->alt.r);
     for (int i = 0; i < sp.nf - 1; i++)
-        if (sp.swap_a[i]) std::swap(*sp.swap_a[i], *sp.swap_b[i]);
+        std::swap(*sp.swap_a[i], *sp.swap_b[i]);
     std::swap(c->f.id, c->alt.id);
 }
 
-// Runs the sort and swaps every destination field into the live set.
-int run_sort(cmcg_ctx *c, bool fused)
+// Sorts by r and swaps every destination field into the live set.
+int run_sort(cmcg_ctx *c)
 {
     SortSpec sp;
-    sort_spec(c, fused, sp);
-    const double *key = fused ? c->f.rnew : c->f.r;
-    hipError_t e = launch_sort_fields(key, c->alt.r, sp.nf, sp.src, sp.dst, c->s, c->sc, c->n_ub,
-                                      fused ? (const int32_t *)c->f.knew : nullptr, c->stream);
+    sort_spec(c, false, sp);
+    hipError_t e = launch_sort_fields(c->f.r, c->alt.r, sp.nf, sp.src, sp.dst, c->s, c->sc, c->n_ub, nullptr, c->stream);
     if (e != hipSuccess) { cmcg_report_hip(e, "launch_sort_fields", __FILE__, __LINE__); return CMCG_E_HIP; }
     swap_sorted(c, sp);
-    // the old vr/vt buffers are now stale copies; vrnew/vtnew keep their values
     return CMCG_OK;
 }
 
@@ -794,7 +789,7 @@ int cmcg_sort_by_r(cmcg_ctx *c, int64_t *n_max)
     {
         PhaseTimer t(c, "sort");
         invalidate_graphs(c);
-        if (int e = run_sort(c, false)) return e;
+        if (int e = run_sort(c)) return e;
     }
     DevScalars h;
     if (int e = read_scalars(c, h)) return e;

@@ -693,13 +693,6 @@ __device__ __forceinline__ double potential_at_coarse_n(const N &nd, int64_t n_m
     }
     return potential_at_n(nd, n_max, x, lo, hi, bad, k_out);
 }
-__device__ __forceinline__ double potential_at_coarse(const double *__restrict__ r, const double *__restrict__ phi,
-                                                      int64_t n_max, double x, int64_t lo, int64_t hi,
-                                                      const Coarse &c, bool *bad)
-{
-    return potential_at_coarse_n(SplitNodes{r, phi}, n_max, x, lo, hi, c, bad);
-}
-
 // potential(x) through the radial index: the node below x's bucket and the two after it
 // (one index word, then three node loads that do not wait for each other) hold the
 // interval unless the bucket holds more nodes, which a bisection up to the next bucket's

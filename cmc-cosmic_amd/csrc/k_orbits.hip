@@ -389,7 +389,6 @@ struct orbits_kernel {
                                                              int64_t *__restrict__ defer_list,
                                                              int64_t *__restrict__ defer_kfirst,
                                                              const float2 *__restrict__ pred, float margin,
-                                                             const double2 *__restrict__ mid,
                                                              const double2 *__restrict__ nodes,
                                                              const double2 *__restrict__ coarse,
                                                              const uint32_t *__restrict__ ridx, int ridx_bits)
@@ -408,7 +407,6 @@ struct orbits_kernel {
     C.stride = coarse_stride(n, COARSE);
     C.inv_stride = 0xffffffffu / (uint32_t)C.stride;
     C.hint = false; C.lrp = C.lra = 0.f; C.margin = margin;
-    C.mid = mid;
     C.ri.t = nullptr;
     if (n >= 1) C.ri = ridx_of(ridx, nodes, n, ridx_bits);
     constexpr int NC = COARSE / THREADS;
@@ -811,8 +809,8 @@ struct ridx_clear_kernel {
 }
 };
 
-// The packed (r, phi) node table with its every MID_STEP-th entry (nodes 0..n+1), and
-// the radial index's marks (nodes 0..n), in one pass over r and phi: node k (node 0
+// The packed (r, phi) node table (nodes 0..n+1) and the radial index's marks
+// (nodes 0..n), in one pass over r and phi: node k (node 0
 // stands for "below every bucket") writes its index at its bucket when it is the
 // bucket's last node, and k at every multiple of RIDX_TILE in (bucket(r_k),
 // bucket(r_{k+1})] of the tile table.  The index array and *bad must be cleared before; *bad is
@@ -820,16 +818,14 @@ struct ridx_clear_kernel {
 struct node_index_kernel {
     static constexpr int LB = 1024, MB = 0;
     static __device__ __forceinline__ void run(KGrid kg_, const double *__restrict__ r, const double *__restrict__ phi, DevScalars *s,
-                                  double2 *__restrict__ nodes, double2 *__restrict__ mid, uint32_t *__restrict__ t,
+                                  double2 *__restrict__ nodes, uint32_t *__restrict__ t,
                                   uint32_t *__restrict__ tb, int bits, int32_t *bad)
 {
     const int64_t n = s->n_max;
     const int64_t k = (int64_t)kg_.bid * blockDim.x + threadIdx.x;
     if (k > n + 1) return;
     const double rk = r[k];
-    const double2 v = make_double2(rk, phi[k]);
-    nodes[k] = v;
-    if (k % MID_STEP == 0) mid[k / MID_STEP] = v;
+    nodes[k] = make_double2(rk, phi[k]);
     if (k > n) return;
     const int64_t nb = (int64_t)1 << bits;
     int64_t bk = -1, bn = nb + 1;
@@ -936,15 +932,15 @@ struct ridx_scan_kernel {
 // in a round (64: all idle lanes; fewer: less speculative work).  Every variant gives
 // the same stars; only the block order of the escape sums differs.
 using OrbFn = void (*)(dim3, dim3, hipStream_t, DevFields, DevScalars *, KParams, const JumpTables *,
-                       const Rng *, double *, int64_t *, int64_t *, const float2 *, float, const double2 *, const double2 *, const double2 *,
+                       const Rng *, double *, int64_t *, int64_t *, const float2 *, float, const double2 *, const double2 *,
                        const uint32_t *, int);
 template <int THREADS, int COARSE, int CAP, int MINB>
 void orbits_launch(dim3 g, dim3 b, hipStream_t st, DevFields f, DevScalars *s, KParams P, const JumpTables *jump,
                    const Rng *base, double *partials, int64_t *defer, int64_t *kfirst, const float2 *pred, float margin,
-                   const double2 *mid, const double2 *nodes, const double2 *coarse,
+                   const double2 *nodes, const double2 *coarse,
                    const uint32_t *ridx, int ridx_bits)
 {
-    kl<orbits_kernel<THREADS, COARSE, CAP, MINB>>(g, b, 0, st, f, s, P, jump, base, partials, defer, kfirst, pred, margin, mid, nodes,
+    kl<orbits_kernel<THREADS, COARSE, CAP, MINB>>(g, b, 0, st, f, s, P, jump, base, partials, defer, kfirst, pred, margin, nodes,
                                                   coarse, ridx, ridx_bits);
 }
 struct OrbVariant { OrbFn fn; int threads, coarse, cap, minb; };
@@ -989,9 +985,8 @@ hipError_t launch_orbits(const DevFields &f, DevScalars *s, const KParams &P, co
     }
     if (ev_a) hipEventRecord(ev_a, st);
     V.fn(dim3((unsigned)nblocks), dim3(V.threads), st, f, s, P, sc.jump, (const Rng *)sc.rng_base,
-                       sc.partials, sc.defer_list, sc.defer_kfirst, pred, margin, (const double2 *)sc.mid,
-                       (const double2 *)sc.nodes, (const double2 *)sc.coarse,
-                       (const uint32_t *)sc.ridx, sc.ridx_bits);
+                       sc.partials, sc.defer_list, sc.defer_kfirst, pred, margin,
+                       (const double2 *)sc.nodes, (const double2 *)sc.coarse, (const uint32_t *)sc.ridx, sc.ridx_bits);
     if (ev_b) hipEventRecord(ev_b, st);
     const int buckets = sort_shape(n_ub).buckets;
     kl<after_orbits_kernel>(dim3(RED2_BLOCKS + 1 + DEFER_BLOCKS + 1), dim3(DEFER_T), 0, st, f, s, P, (const double *)sc.partials,
@@ -1019,7 +1014,7 @@ hipError_t launch_node_index(const DevFields &f, DevScalars *s, const Scratch &s
     const int64_t entries = ridx_entries(sc.ridx_bits);
     if (!clear) kl<ridx_clear_kernel>(dim3(512), dim3(256), 0, st, sc.ridx, entries, sc.sort_uneven);
     kl<node_index_kernel>(dim3((unsigned)((n_ub + 2 + 255) / 256)), dim3(256), 0, st, f.r, f.phi, s,
-                       (double2 *)sc.nodes, (double2 *)sc.mid, sc.ridx, sc.ridx_tb, sc.ridx_bits, sc.sort_uneven);
+                       (double2 *)sc.nodes, sc.ridx, sc.ridx_tb, sc.ridx_bits, sc.sort_uneven);
     kl<ridx_scan_kernel>(dim3((unsigned)(ridx_tiles(sc.ridx_bits) + (coarse + 256) / 256)), dim3(256), 0, st, sc.ridx,
                        (const uint32_t *)sc.ridx_tb, sc.ridx_bits, (const double2 *)sc.nodes, s, coarse, sc.coarse);
     return hipGetLastError();

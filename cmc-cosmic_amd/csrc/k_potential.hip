@@ -823,7 +823,7 @@ struct PotArgs {
     // nonzero: the chains go through the repair.  A kernel reads only the words that earlier
     // kernels set: [0] classification of A and B, [1] rebuild of B, [2] rebuild of C
     int64_t *flag;
-    double2 *nodes, *mid;       // packed (r, phi) of every node and of every MID_STEP-th
+    double2 *nodes;             // packed (r, phi) of every node
     int counted;                // N_MAX from the count of radii below SF_INFINITY (pot_count_kernel)
     EsaArgs a, b, c;
     __device__ __forceinline__ int64_t lb(int64_t n) const { return n > 1 ? n - 1 : 0; }
@@ -1085,9 +1085,7 @@ struct pot_walk_c_kernel {
 // the orbit phase read
 __device__ __forceinline__ void put_node(const PotArgs &p, int64_t k, double r, double phi)
 {
-    const double2 v = make_double2(r, phi);
-    p.nodes[k] = v;
-    if (k % MID_STEP == 0) p.mid[k / MID_STEP] = v;
+    p.nodes[k] = make_double2(r, phi);
 }
 // nodes 0 (cmc_utils.c:729; phi1 = phi[1], the sentinel's 0 when there are no stars) and n + 1
 __device__ __forceinline__ void put_ends(const PotArgs &p, const KParams &P, int64_t n, double phi1)
@@ -1459,7 +1457,7 @@ hipError_t launch_potential(const DevFields &f, DevScalars *s, const KParams &P,
     p.xc = sc.chain_x;
     p.scal = sc.chain_scal;
     p.flag = sc.chain_fbad;
-    p.nodes = sc.nodes; p.mid = sc.mid;
+    p.nodes = sc.nodes;
     p.counted = count;
     p.a = esa_args(sc, P.chain_k_drop, 0);
     p.b = esa_args(sc, P.chain_k_drop, 1);
