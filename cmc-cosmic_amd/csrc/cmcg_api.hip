@@ -385,61 +385,18 @@ void noalloc_setup(int device)
 }  // namespace
 
 // ---- the jump tables (JumpLevel) ----
-// Constants of the generator (2.9 MB): one allocation on each GPU, filled when the first
-// context is created there, read by every context's kernels and freed with the last one.
+// Constants of the generator (2.9 MB): one allocation on each GPU, formed there when the first
+// context is created, read by every context's kernels and freed with the last one.
 
 namespace {
 JumpTables *g_jump_ptr[NOALLOC_MAX_DEVICES];
 int g_jump_users[NOALLOC_MAX_DEVICES];
 
-// t of one level: the unit's matrix `m` (columns), d = 0..63 of it by repeated products
-void fill_jump_level(const uint32_t m[4][32], JumpLevel *levels, int level)
-{
-    JumpLevel &L = levels[level];
-    const bool lanes = jump_over_lanes(level);
-    uint32_t col[4][32];
-    for (int c = 0; c < 4; c++)
-        for (int i = 0; i < 32; i++) col[c][i] = 1u << i;
-    for (int d = 0; d < 64; d++)
-        for (int c = 0; c < 4; c++) {
-            for (int q = 0; q < 8; q++)
-                for (int v = 0; v < 16; v++)
-                    L.t[jump_index(lanes, c, q, v, d)] = v ? L.t[jump_index(lanes, c, q, v & (v - 1), d)] ^
-                                                                 col[c][4 * q + __builtin_ctz(v)]
-                                                           : 0u;
-            for (int i = 0; i < 32; i++) col[c][i] = host_matvec(m[c], col[c][i]);
-        }
-}
-
-// The host's copy, made once (the generator's matrices are constants).
-const JumpTables *jump_host(const RngTable &T)
-{
-    auto *h = new JumpTables();
-    uint32_t m[4][32];
-    for (int k = 0; k < JL_PAIR_N; k++) {       // 3 64^k = 2^(6k) + 2^(6k + 1)
-        for (int c = 0; c < 4; c++)
-            for (int i = 0; i < 32; i++) m[c][i] = host_matvec(T.col[6 * k][c], T.col[6 * k + 1][c][i]);
-        fill_jump_level(m, h->level, JL_PAIR + k);
-    }
-    for (int k = 0; k < JL_SLOT_N; k++) fill_jump_level(T.col[20 + 6 * k], h->level, JL_SLOT + k);
-    fill_jump_level(T.col[66], h->level, JL_PHASE);
-    for (int k = 0; k < JL_STEP_N; k++)
-        if (72 + 6 * k < 128) fill_jump_level(T.col[72 + 6 * k], h->level, JL_STEP + k);
-    for (int d = 0; d < 8; d++)                 // d slots and 8 d slots, from the level's own table
-        for (int c = 0; c < 4; c++)
-            for (int q = 0; q < 8; q++)
-                for (int v = 0; v < 16; v++) {
-                    h->orbit.lo.t[c][q][v][d] = h->level[JL_SLOT].t[jump_index(false, c, q, v, d)];
-                    h->orbit.hi.t[c][q][v][d] = h->level[JL_SLOT].t[jump_index(false, c, q, v, 8 * d)];
-                }
-    return h;
-}
-
-// With `device` current: its jump tables, copied for the first user (null: failed).
-const JumpTables *jump_acquire(int device, const RngTable &T)
+// With `device` current: its jump tables, formed for the first user from the generator's
+// matrices T on the device (null: failed).
+const JumpTables *jump_acquire(int device, const RngTable *T, hipStream_t st)
 {
     if (device < 0 || device >= NOALLOC_MAX_DEVICES) return nullptr;
-    static const JumpTables *host = jump_host(T);
     std::lock_guard<std::mutex> lk(g_scratch_mu);
     if (g_jump_ptr[device]) {
         g_jump_users[device]++;
@@ -447,7 +404,7 @@ const JumpTables *jump_acquire(int device, const RngTable &T)
     }
     void *ptr = nullptr;
     if (hipMalloc(&ptr, sizeof(JumpTables)) != hipSuccess) return nullptr;
-    if (hipMemcpy(ptr, host, sizeof(JumpTables), hipMemcpyHostToDevice) != hipSuccess) {
+    if (launch_jump_build(T, (JumpTables *)ptr, st) != hipSuccess || hipStreamSynchronize(st) != hipSuccess) {
         hipFree(ptr);
         return nullptr;
     }
@@ -536,7 +493,7 @@ int cmcg_create(cmcg_ctx **out, int device, int64_t n_cap, const cmcg_params *pa
     c->seeded = host_seed(params->seed);
     bool ok = hipMemcpy(c->T, ht, sizeof(RngTable), hipMemcpyHostToDevice) == hipSuccess &&
               hipMemcpy(sc.rng_seeded, &c->seeded, sizeof(Rng), hipMemcpyHostToDevice) == hipSuccess;
-    if (ok) sc.jump = jump_acquire(device, *ht);
+    if (ok) sc.jump = jump_acquire(device, c->T, c->stream);
     ok = ok && sc.jump;
     delete ht;
     if (!ok) { cmcg_destroy(c); return CMCG_E_HIP; }
@@ -820,10 +777,10 @@ int cmcg_potential(cmcg_ctx *c, int64_t *n_max, double *mtotal, double *rtidal)
 constexpr int64_t QUERY_PACKED = 32768;
 
 // A batch of queries: the context's buffer, held by one thread at a time, of `arrays` 8-byte
-// arrays of `count`.  Up to QUERY_KEEP doubles stay with the context for the next batch; a
-// larger buffer goes back when the batch ends (64 MB take 5 ms to copy each way, and the
-// allocation and the free about 0.2).
-constexpr int64_t QUERY_KEEP = (int64_t)1 << 23;
+// arrays of `count`.  Up to QUERY_KEEP doubles (256 MB) stay with the context for the next
+// batch; a larger buffer goes back when the batch ends (an allocation and a free take 0.6 ms,
+// the copies of 256 MB 20).
+constexpr int64_t QUERY_KEEP = (int64_t)1 << 25;
 struct QueryBuffer {
     cmcg_ctx *c;
     std::lock_guard<std::mutex> lk;

@@ -156,6 +156,7 @@ constexpr int RELAX_NSHAPES = 4;
 hipError_t launch_relax(const DevFields &f, DevScalars *s, const KParams &P, const Scratch &sc,
                         int64_t n_ub, hipStream_t st,
                         bool with_ec1 = false, int threads = 256);
+hipError_t launch_jump_build(const RngTable *T, JumpTables *J, hipStream_t st);
 hipError_t launch_rng_bases(DevScalars *s, const Scratch &sc, hipStream_t st);
 hipError_t launch_rng_bases_step(DevScalars *s, const Scratch &sc, int64_t step, hipStream_t st);
 // the packed node table and the radial index in one pass over r and phi
