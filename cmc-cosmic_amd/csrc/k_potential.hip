@@ -23,11 +23,13 @@
 //   in between), then every element is rebuilt in parallel from the last sensitive
 //   value before it.  Four passes: tile sums (fused into the kernel that produces
 //   the increments), classification, walk, rebuild.
-// * Every element is verified against fl(v_{j-1} + s x_j), so the estimate's bound
-//   decides only the speed, never the result.  A violation (only when the bound or
-//   the sensitive-list capacity is exceeded) is repaired by running the recurrence
-//   itself from the first violating element.  The result equals the sequential
-//   chain exactly.
+// * Every element of chains B and C, and of the reports' chains, is rebuilt and verified
+//   against fl(v_{j-1} + s x_j), so there the estimate's bound decides only the speed, never
+//   the result.  A violation (only when the bound or a list's capacity is exceeded) is repaired
+//   by running the recurrence itself.
+// * Chain A needs only its last value and is not rebuilt: its exactness rests on the bound
+//   (err_bound), which is rigorous for masses that are not negative and finite (any other mass
+//   sends all three chains to the repair).
 #include "kernels.hpp"
 
 namespace {
@@ -159,8 +161,9 @@ __device__ __forceinline__ int interval_binade(double v, double e)
 // Bound on |v - P| for the estimate P of the chain value v after j elements: the
 // chain's own j roundings (at most 2^-53 |v| each, |v| <= vmax for a monotone chain)
 // and the roundings of the estimate's sums in any order (at most (j + 2) 2^-53
-// (|v0| + sum |s x|) <= (j + 2) 2^-52 vmax), with a factor 2 to spare.  A chain for
-// which it fails only takes the repair path: every element is verified.
+// (|v0| + sum |s x|) <= (j + 2) 2^-52 vmax), with a factor 2 to spare.  A chain that is verified
+// element by element would only take the repair if it failed; the total mass (the potential's
+// chain A) is not, and relies on it.
 __device__ __forceinline__ double err_bound(int64_t j, double vmax, int slack)
 {
     return ldexp(((double)j + 2.0) * vmax, slack - 50) * 1.001;
