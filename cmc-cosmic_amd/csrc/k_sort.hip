@@ -879,7 +879,7 @@ hipError_t sort_launch(const double *key_src, double *r_dst, const uint64_t *id_
     kl<sb_sort_kernel<W, CAP>>(dim3((unsigned)sh.buckets), dim3(BS_T), 0, st, s, (const uint32_t *)sc.sort_first,
                                (const uint64_t *)sc.sort_aos, sc.sort_order, sc.sort_aos_cap, r_dst, id_dst, sc.vals_a, g,
                                key_src, id_src, moved);
-    if (g.nf > W - 3)
+    if (g.nf > W - 3 && n_ub > 0)
         kl<sb_rest_kernel>(dim3((unsigned)((n_ub + 255) / 256)), dim3(256), 0, st, (const DevScalars *)s,
                            (const uint32_t *)sc.vals_a, W - 3, g);
     return hipGetLastError();
