@@ -1905,10 +1905,11 @@ int cmcg_central_calculate(cmcg_ctx *c, cmcg_central *out)
             c->cen_buf = nullptr;
             return CMCG_E_NOMEM;
         }
+        if (hipMemsetAsync(c->cen_buf, 0, central_out_bytes(), c->stream) != hipSuccess) return CMCG_E_HIP;
     }
     if (int e = report_reserve(c)) return e;
     LAUNCH(launch_central(c->f, c->s, c->kp, c->n_ub, c->sc, c->cen_buf, c->rep_buf, c->stream));
-    // layout: int64 nave, int32 error, int32 pad, then 13 doubles in cmcg_central's order
+    // layout: int64 nave, two int32 (the first the error), then 13 doubles in cmcg_central's order
     std::vector<char> host(central_out_bytes());
     if (hipMemcpyAsync(host.data(), c->cen_buf, host.size(), hipMemcpyDeviceToHost, c->stream) != hipSuccess ||
         sync(c) != hipSuccess)

@@ -1352,6 +1352,7 @@ struct MassPcOut {
     double v[8][MPC_MAX];        // mass_r, ave_mass_r, densities_r, ke_rad, ke_tan, v2_rad, v2_tan, (unused)
     int64_t k[MPC_MAX];          // no_star_r (the index k)
     int64_t reached;             // fractions assigned
+    int64_t negative;            // a mass is below zero (or NaN): the enclosed mass is not monotone
 };
 
 // Chain 0: star_m[k] / clus.N_STAR; 1 to 4: 0.5 m madhoc vr vr, 0.5 m madhoc vt vt, vr vr,
@@ -1359,7 +1360,7 @@ struct MassPcOut {
 struct mpc_prep_kernel {
     static constexpr int LB = 1024, MB = 0;
     static __device__ __forceinline__ void run(KGrid kg_, const DevFields f, const DevScalars *s, double nstar, double madhoc,
-                                  double mprev0, EsaArgs e, int64_t words, int64_t xs)
+                                  double mprev0, EsaArgs e, int64_t words, int64_t xs, MassPcOut *o)
 {
     const int64_t j = (int64_t)kg_.bid * blockDim.x + threadIdx.x, k = j + 1;
     const int64_t n = s->n_max, nn = s->n_max_new;
@@ -1368,7 +1369,11 @@ struct mpc_prep_kernel {
         const_cast<int64_t *>(e.Lp)[j * words] = j == 0 ? n : nn;
         const_cast<double *>(e.v0p)[j * words] = j == 0 ? mprev0 : 0.0;
     }
-    if (j < n) x[j] = f.m[k] / nstar;
+    if (j < n) {
+        const double m = f.m[k];
+        x[j] = m / nstar;
+        if (!(m >= 0.0)) o->negative = 1;
+    }
     if (j < nn) {
         const double m = f.m[k], vr = f.vr[k], vt = f.vt[k];
         x[xs + j] = 0.5 * m * madhoc * vr * vr;
@@ -1391,7 +1396,8 @@ __device__ __forceinline__ double cube_rn(double x)
 // The fractions' indices (one fraction per star at most, as the reference's loop) from the
 // enclosed-mass chain g[k-1] = mprev after star k, which does not decrease: a thread finds
 // each fraction's first k with g[k-1] > pc Mtotal, one thread then moves them past the
-// fraction before, and the threads take the values there.  (One thread searching for one
+// fraction before, and the threads take the values there.  With a negative mass it may decrease,
+// and the block looks at every star after the one before.  (One thread searching for one
 // fraction after another waited on 20 loads for each.)
 struct mpc_finish_kernel {
     static constexpr int LB = MPC_MAX, MB = 0;
@@ -1421,15 +1427,38 @@ struct mpc_finish_kernel {
         if (bh_include)
             for (; mc < count && mprev0 / Mtotal > pc[mc]; mc++) ks[mc] = 0;
         int64_t kprev = 0;
-        for (; mc < count; mc++) {
+        for (; mc < count && !o->negative; mc++) {
             const int64_t k = ks[mc] > kprev ? ks[mc] : kprev + 1;
             if (k > n) break;
             ks[mc] = kprev = k;
         }
         reached = mc;
-        o->reached = mc;
     }
     __syncthreads();
+    if (o->negative) {
+        __shared__ int64_t found;
+        int64_t k = 0;
+        for (int mc = reached; mc < count; mc++) {
+            const double thr = pc[mc] * Mtotal;
+            if (i == 0) found = n + 1;
+            __syncthreads();
+            for (k++; k <= n; k += MPC_MAX) {
+                if (k + i <= n && g[k + i - 1] > thr) atomicMin((unsigned long long *)&found, (unsigned long long)(k + i));
+                __syncthreads();
+                const bool hit = found <= n;
+                __syncthreads();                           // before the next round's stores
+                if (hit) break;
+            }
+            if (found > n) break;
+            k = found;
+            if (i == 0) {
+                ks[mc] = k;
+                reached = mc + 1;
+            }
+            __syncthreads();
+        }
+    }
+    if (i == 0) o->reached = reached;
     if (i >= reached) return;
     const int64_t k = ks[i];
     o->k[i] = k;
@@ -1517,7 +1546,7 @@ hipError_t launch_mass_percent(const DevFields &f, DevScalars *s, const KParams 
     const EsaArgs e = report_chain0(sc, P.chain_k_drop, work, xs);
     const double mprev0 = bh_include ? P.cenma_m * P.madhoc : 0.0;   // cmc_utils.c:878
     kl<mpc_prep_kernel>(dim3((unsigned)((n_ub + 256) / 256)), dim3(256), 0, st, f, (const DevScalars *)s, (double)P.n_star,
-                       P.madhoc, mprev0, e, words, xs);
+                       P.madhoc, mprev0, e, words, xs, (MassPcOut *)out);
     if (hipError_t err = run_chains(e, words, xs, 5, n_ub, st)) return err;
     kl<mpc_finish_kernel>(dim3(1), dim3(MPC_MAX), 0, st, (const double *)f.r, (const DevScalars *)s, (const double *)e.g, xs,
                        pc, count, bh_include, mprev0, itm, minimum_r, (MassPcOut *)out);
@@ -1539,7 +1568,7 @@ enum { CEN_OK = 0, CEN_E_STATE = 1, CEN_E_RANGE = 2 };
 
 struct CentralOut {
     int64_t nave;
-    int32_t error, pad;
+    int32_t error, negative;     // negative: a mass is below zero (or NaN); 0 between calls
     double rh, rhojsum, rhoj2sum, rho, v_rms, rc, rc_nb, m_ave, n, rc_spitzer, N_core, N_core_nb, Trc;
     double S[CEN_TERMS];
     unsigned long long mx[CEN_TERMS];     // bit patterns of the terms' maxima (non-negative doubles)
@@ -1592,7 +1621,11 @@ struct cen_begin_kernel {
         o->scale[j] = o->unscale[j] = 1.0;
         const_cast<double *>(e.v0p)[j * words] = 0.0;
     }
-    if (j < n) const_cast<double *>(e.x)[j] = m[j + 1] / nstar;
+    if (j < n) {
+        const double mj = m[j + 1];
+        const_cast<double *>(e.x)[j] = mj / nstar;
+        if (!(mj >= 0.0)) o->negative = 1;
+    }
 }
 };
 
@@ -1624,8 +1657,20 @@ struct cen_max_kernel {
     const int64_t n = s->n_max;
     const double thr = 0.5 * s->Mtotal;
     if (threadIdx.x < 64) {
-        // smallest k with !(g[k-1] < thr); g does not decrease
-        const int64_t k = wave_first_false(1, n + 1, [&](int64_t q) { return g[q - 1] < thr; });
+        // smallest k with !(g[k-1] < thr); g does not decrease, unless a mass is negative
+        int64_t k = 1;
+        if (!o->negative) {
+            k = wave_first_false(1, n + 1, [&](int64_t q) { return g[q - 1] < thr; });
+        } else {
+            for (; k <= n; k += 64) {
+                const uint64_t past = __ballot(k + threadIdx.x <= n && !(g[k + threadIdx.x - 1] < thr));
+                if (past) {
+                    k += __ffsll((unsigned long long)past) - 1;
+                    break;
+                }
+            }
+            if (k > n) k = n + 1;
+        }
         if (threadIdx.x == 0) found = k;
     }
     __syncthreads();
@@ -1723,6 +1768,7 @@ struct cen_final_kernel {
     static constexpr int LB = 64, MB = 0;
     static __device__ __forceinline__ void run(KGrid kg_, const double *__restrict__ g, int64_t xs, CentralOut *o)
 {
+    if (threadIdx.x == 0) o->negative = 0;
     if (o->error) return;
     if (threadIdx.x < CEN_TERMS) o->S[threadIdx.x] = g[threadIdx.x * xs + o->nave - 1] * o->unscale[threadIdx.x];
     __syncthreads();
