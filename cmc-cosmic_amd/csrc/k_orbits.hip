@@ -599,27 +599,30 @@ __device__ void orbits_part(const double *__restrict__ partials, int64_t nblocks
 }
 
 // Whether the new radii's indices cut the stars into even buckets for the step's sort: up to
-// SMP_MAX of them counted (one block).  A bucket is too long at twice its share and 40 more:
-// what a sample can miss, 40 of 8192, costs its block less than 0.4 ms at N = 4e6.  (The
+// BAL_MAX of them counted (one block).  A bucket is too long at twice its share and 10 more:
+// what a sample can miss, 10 of 2048, costs its block less than 0.4 ms at N = 4e6.  (The
 // deferred stars have the indices of their last orbits; counts decide only the speed.)
+// Bound by one CU's misses, a line a sample: the kernel that holds this block takes 12.0 us at
+// N = 4e6, as it does without the block; with 8192 samples and 40 more, 19.7.
+constexpr int BAL_MAX = 2048;
 __device__ void sort_balance(const int32_t *__restrict__ knew, int64_t n, int B, int32_t *uneven)
 {
     __shared__ uint32_t hist[SB_MAX_BUCKETS];
-    const int t = threadIdx.x, S = n < SMP_MAX ? (int)n : SMP_MAX;
+    const int t = threadIdx.x, S = n < BAL_MAX ? (int)n : BAL_MAX;
     for (int b = t; b < B; b += DEFER_T) hist[b] = 0;
     const StepBucket bucket(n, B);
     const double stride = (double)n / (double)S;           // at least 1
-    uint32_t k[SMP_MAX / DEFER_T];
+    uint32_t k[BAL_MAX / DEFER_T];
 #pragma unroll
-    for (int u = 0; u < SMP_MAX / DEFER_T; u++) {
+    for (int u = 0; u < BAL_MAX / DEFER_T; u++) {
         const int q = u * DEFER_T + t;
         k[u] = q < S ? bucket(knew[1 + (int64_t)(q * stride)]) : (uint32_t)SB_TAIL;
     }
     __syncthreads();
-    const uint32_t limit = 2 * (uint32_t)S / (uint32_t)B + 40;
+    const uint32_t limit = 2 * (uint32_t)S / (uint32_t)B + 10;
     bool over = false;
 #pragma unroll
-    for (int u = 0; u < SMP_MAX / DEFER_T; u++)
+    for (int u = 0; u < BAL_MAX / DEFER_T; u++)
         if (k[u] != SB_TAIL) over |= atomicAdd(&hist[k[u]], 1u) >= limit;
     if (over) *uneven = 2;
 }
@@ -946,10 +949,11 @@ void orbits_launch(dim3 g, dim3 b, hipStream_t st, DevFields f, DevScalars *s, K
 struct OrbVariant { OrbFn fn; int threads, coarse, cap, minb; };
 #define ORB_V(T, C, K, M) {orbits_launch<T, C, K, M>, T, C, K, M}
 const OrbVariant kOrbVariants[] = {
-    // the first is the default: five waves per SIMD hide the gathers best and at most four
-    // lanes per star waste few tries.  Sampler time, default / with 64 lanes / 128 threads (whose
-    // LDS allows fewer waves): N = 4e6 787 / 861 / 1006 us, 1e6 192 / 211 / 257, 3e5 60 / 71 / 87,
-    // 1e4 33 / 40 / 39.
+    // the first is the default: at most four lanes per star waste few tries.  Its bound of five
+    // waves per SIMD costs nothing and gains nothing: the allocation without it takes 91 registers
+    // for 89, five waves too (N = 4e6 795 us both, 1e6 185 and 180); the tuner tries both.
+    // Sampler time, default / with 64 lanes / 128 threads (whose LDS allows fewer waves): N = 4e6
+    // 795 / 868 / 972 us, 1e6 192 / 211 / 257, 3e5 60 / 71 / 87, 1e4 33 / 40 / 39.
     ORB_V(256, 1024, 4, 5),  ORB_V(256, 512, 64, 1), ORB_V(256, 2048, 64, 1), ORB_V(128, 1024, 64, 1),
     ORB_V(512, 1024, 64, 1), ORB_V(128, 512, 64, 1), ORB_V(256, 1024, 2, 1),  ORB_V(256, 1024, 4, 1),
     ORB_V(256, 1024, 8, 1),  ORB_V(256, 512, 4, 1),  ORB_V(256, 1024, 64, 1), ORB_V(256, 512, 4, 5),
