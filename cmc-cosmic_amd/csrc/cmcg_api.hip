@@ -1849,7 +1849,7 @@ int cmcg_autotune(cmcg_ctx *c, int reps, int32_t *variant, int32_t *threads, int
     return CMCG_OK;
 }
 
-// the reports' chain lists (9.5 MB and 0.2 words per star), allocated by the first of them
+// the reports' chain lists (9.5 MB and 0.14 bytes per star), allocated by the first of them
 static int report_reserve(cmcg_ctx *c)
 {
     if (c->rep_buf) return CMCG_OK;

@@ -18,15 +18,15 @@
 // * Segment and walk: a regular increment is an integer R in units of its binade's
 //   ulp, and a run of them between two sensitive elements stays in one binade, so
 //   an int64 scan that restarts at every sensitive element gives each run's exact
-//   sum.  One thread walks the sensitive elements in order, each getting
+//   sum.  One thread or wave walks the sensitive elements in order, each getting
 //   fl(v_prev + s x) from the exact value before it (the previous one plus the run
 //   in between), then every element is rebuilt in parallel from the last sensitive
 //   value before it.  Four passes: tile sums (fused into the kernel that produces
 //   the increments), classification, walk, rebuild.
 // * Every element of chains B and C, and of the reports' chains, is rebuilt and verified
 //   against fl(v_{j-1} + s x_j), so there the estimate's bound decides only the speed, never
-//   the result.  A violation (only when the bound or a list's capacity is exceeded) is repaired
-//   by running the recurrence itself.
+//   the result.  A violation (only when the bound is exceeded, or a report's list; the
+//   potential's hold every star) is repaired by running the recurrence itself.
 // * Chain A needs only its last value and is not rebuilt: its exactness rests on the bound
 //   (err_bound), which is rigorous for masses that are not negative and finite (any other mass
 //   sends all three chains to the repair).
@@ -36,7 +36,7 @@ namespace {
 constexpr int CT = 256;             // threads per tile
 constexpr int CI = 8;               // items per thread
 constexpr int CTILE = CT * CI;
-constexpr int RAW_CAP = 2048;         // sensitive elements sorted in LDS by the walk
+constexpr int RAW_CAP = 2048;         // sensitive elements that the walk puts in order in LDS (more: in memory)
 constexpr int WALK_T = 1024;          // threads of the one-block kernels
 constexpr int WALK_CHUNK = 256;       // sensitive elements staged per round of the walk
 constexpr int WALK_REG = 16;          // tiles per walk thread held in registers (N <= 8.4e6 at CT*CI = 2048)

@@ -24,11 +24,14 @@
 // split further by its block, in time proportional to its stars.
 //
 // Bound: HBM.  The payload (64 B a star) is read and written twice, 256 B a star, plus 4 B
-// of node indices.  It replaced an LSD radix sort of (key, slot) words, which packed the
-// records, moved the words through four histogram-scan-scatter passes and gathered the
-// records at the end (16 launches, now 3 or 4).  The step's sort, before -> now: N = 1e4
-// 0.099 -> 0.028 ms, 1e5 0.106 -> 0.034, 1e6 0.164 -> 0.092, 4e6 0.399 -> 0.277 (the
-// bucket pass 129 us for 528 MB, 4.1 TB/s; the scatter 112 us for 500 MB).
+// of node indices; the bucket pass reads the records a second time, in output order, mostly
+// from the caches below the L2.  It replaced an LSD radix sort of (key, slot) words, which
+// packed the records, moved the words through four histogram-scan-scatter passes and gathered
+// the records at the end (16 launches, now 3 or 4).  The step's sort, before -> now: N = 1e4
+// 0.099 -> 0.028 ms, 1e5 0.106 -> 0.034, 1e6 0.164 -> 0.092, 4e6 0.399 -> 0.282, 1.8e7
+// 1.82 -> 1.28.  At 4e6 the scatter takes 112 us for 532 MB measured at the L2 (4.7 TB/s, the
+// rate of a copy), the bucket pass 142 us for 889 MB (643 read, 245 written: 6.3 TB/s with
+// what the caches serve, 3.6 of the 512 MB it cannot do without).
 #include "kernels.hpp"
 
 namespace {
@@ -337,9 +340,10 @@ struct sb_scan_kernel {
 // Records of W words: r, id, slot, then the first W - 3 payload fields.  A wave packs 64
 // stars at a time through its own LDS patch (odd stride: no bank conflicts), so whole
 // records leave in each store instruction; the next 64 stars' loads are in flight
-// meanwhile.  knew: the step's form (bkt is read only where the indices would be uneven).  scanned: mat holds the tiles'
-// offsets and totals the bucket totals (sb_scan_kernel); otherwise both are formed here
-// from the raw histogram rows.  Bound by HBM: 500 MB in 112 us at N = 4e6.
+// meanwhile.  knew: the step's form (bkt is read only where the indices would be uneven).
+// scanned: mat holds the tiles' offsets and totals the bucket totals (sb_scan_kernel);
+// otherwise both are formed here
+// from the raw histogram rows.  Bound by HBM: 532 MB in 112 us at N = 4e6.
 constexpr int SC_T = 512, SC_W = SC_T / 64;
 template <int W, int BM>
 struct sb_scatter_kernel {
@@ -763,8 +767,9 @@ __device__ __forceinline__ void order_bucket(const uint64_t *__restrict__ rec, u
 // Block b orders bucket b and writes its stars' fields: the sorted records are read back in
 // output order, W/2 lanes per record, and leave through LDS with one coalesced store per
 // field.  (The general entry point's stars are often in order already; then the blocks only
-// copy them: 0.65 -> 0.45 ms at N = 4e6, 0.22 -> 0.16 at 1e6.)  Bound by HBM (N = 4e6, 8 words: 129 us); holding the records in registers
-// between the two reads, or 256 threads a block, changed nothing.
+// copy them: 0.65 -> 0.45 ms at N = 4e6, 0.22 -> 0.16 at 1e6.)  Bound by HBM (N = 4e6, 8 words:
+// 142 us); holding the records in registers between the two reads, or 256 threads a block,
+// changed nothing.
 template <int W, int CAP>
 struct sb_sort_kernel {
     static constexpr int LB = BS_T, MB = CAP <= 2048 ? 8 : 4;

@@ -77,15 +77,14 @@ __host__ __device__ constexpr int64_t ridx_entries(int bits) { return ((int64_t)
 __host__ __device__ constexpr int64_t ridx_tiles(int bits) { return (ridx_entries(bits) + RIDX_TILE - 1) / RIDX_TILE; }
 
 struct Scratch {
-    // potential chains: per-tile int128 sums and prefixes plus a boundary value
-    // (48 B per tile), chain increments / iterates / enclosed masses per star
-    double *tile_sums;         // two sets of 6 words per tile (potential chains)
+    // potential chains
+    double *tile_sums;          // two sets of 6 words per tile: estimates, counts, open runs and their prefixes
     int64_t max_tiles;
-    double *chain_x;
+    double *chain_x;            // chain C's increments
     double *chain_scal;         // 4 doubles
-    int64_t *chain_fbad;        // 6
+    int64_t *chain_fbad;        // [0]..[2]: a violation in the classification, in the rebuild of B, of C
     int64_t *esa_n;             // [0] sensitive count, [1]..[3] appended counts, [4] the total mass chain's [0]
-    // deterministic block partials: 8 doubles per block
+    // deterministic block partials: 8 doubles per block of the glue, 16 of the orbit sampler
     double *partials;
     int64_t max_blocks;
     // sort
@@ -114,7 +113,7 @@ struct Scratch {
     double *red2;               // second level of the block-partial reductions (RED2_BLOCKS x 16)
     int64_t sort_aos_cap;
     // set_velocities3 excess chain: per-star excess, ordered event list, per-event
-    // walk ends and merge flags, per-block counts, fallback flag
+    // walk ends and merge flags, per-block offsets, first failed check
     double *excess_c;
     int64_t *excess_list;
     int64_t *sv3_wend;
@@ -123,8 +122,8 @@ struct Scratch {
     int64_t *sv3_fallback;      // first presumed head that failed the check
     // tidal stripping loop flag
     int32_t *strip_done;
-    // orbit stars deferred to the linear-scan path (65536 slots)
-    int64_t *defer_list, *defer_kfirst, *defer_order;   // KParams::defer_cap entries
+    // orbit stars deferred to the linear-scan path: KParams::defer_cap entries
+    int64_t *defer_list, *defer_kfirst, *defer_order;
     // RNG bases of the current step: [0] relaxation, [1] orbits, [2] orbit slot 1; seeded state
     Rng *rng_base;
     Rng *rng_seeded;
