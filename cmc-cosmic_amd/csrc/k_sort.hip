@@ -342,8 +342,8 @@ struct sb_scan_kernel {
 // records leave in each store instruction; the next 64 stars' loads are in flight
 // meanwhile.  knew: the step's form (bkt is read only where the indices would be uneven).
 // scanned: mat holds the tiles' offsets and totals the bucket totals (sb_scan_kernel);
-// otherwise both are formed here
-// from the raw histogram rows.  Bound by HBM: 532 MB in 112 us at N = 4e6.
+// otherwise both are formed here from the raw histogram rows.  Bound by HBM: 532 MB in
+// 112 us at N = 4e6.
 constexpr int SC_T = 512, SC_W = SC_T / 64;
 template <int W, int BM>
 struct sb_scatter_kernel {
@@ -872,7 +872,7 @@ hipError_t sort_launch(const double *key_src, double *r_dst, const uint64_t *id_
         kl<sb_count_kernel<BM>>(dim3((unsigned)sh.tiles), dim3(1024), 0, st, key_src, s, (const uint64_t *)sc.sort_split,
                                 sh.buckets, sc.sort_bkt, sc.sort_mat, (const int64_t *)id_src, sc.sort_moved);
     }
-    const int32_t *moved = knew ? nullptr : sc.sort_moved;
+    const int32_t *moved = knew || W < 16 ? nullptr : sc.sort_moved;      // wide payloads alone are copied
     const int scanned = !sh.small;
     if (scanned)
         kl<sb_scan_kernel>(dim3((unsigned)((sh.buckets + 63) / 64)), dim3(1024), 0, st, sc.sort_mat, sc.sort_tot,
